@@ -8,9 +8,9 @@
 // (attention_paged.cu:58-59, 176); here the context is split into 1024-position pieces with an
 // online softmax each, merged by a second kernel: up to 1,048,576 positions per sequence.
 //
-// Work split: one wave per (query, kv head, block of up to 8 of its q heads, split). Each K
+// Work split: one workgroup per (query, kv head, block of up to 8 of its q heads, split). Each K
 // row crosses HBM once per (query, kv head) for up to 8 q heads. In causal prefill with fewer
-// than 8 q heads per kv head, a wave takes 8 / G consecutive queries instead, its columns
+// than 8 q heads per kv head, it takes 8 / G consecutive queries instead, its columns
 // being (query, head) pairs each masked to its own causal length, so that a K or V row is
 // read once for all of them. Per 32-position chunk (16 when head_dim is 256):
 //   QK on v_mfma_f32_16x16x32_f16: A = K rows (row = position, 8 consecutive dims per lane,
@@ -32,7 +32,6 @@ using namespace fhip;
 namespace {
 
 constexpr int kPSplit = 1024;  // positions per split: 64 pages, one per lane of the page cache
-constexpr int kPWaves = 2;     // waves per workgroup (independent work items)
 constexpr int kHeadsMax = 8;   // q heads per wave
 // Longest context a block table may describe (the combine kernel keeps one weight per
 // split in LDS: 4 KiB at this bound).
@@ -109,8 +108,14 @@ struct PQueries {
 // Split partials: per (query, q head, split) the running max m (natural log units), the sum
 // l and the unnormalised accumulator acc[hd]. Splits at or past the causal length are not
 // written; the combine kernel reads only the splits below it.
-template <int HD, int NH, class Pages>
-__global__ __launch_bounds__(64 * kPWaves) __attribute__((amdgpu_waves_per_eu(2))) void
+//
+// A workgroup of W waves takes one (query, kv head, head block, split); wave w scores the
+// split's positions [w, w + 1) * kPSplit / W and the waves' states are merged in LDS, so the
+// partials stay one per split whatever W is (kSplits8 / kSplits4 choose it). With a wave per split
+// the chunk's loads had nothing beside them to hide behind: 16 sequences of 500 .. 8192
+// positions (32 / 8 heads of 128, 285 MB) went from 136 to 72 us.
+template <int HD, int NH, int W, class Pages>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void
 paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, int qh, int kvh,
                         int nhb, float scale_log2, float* __restrict__ part_ml,
                         float* __restrict__ part_acc, int nsplit, int tok) {
@@ -120,31 +125,36 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
     constexpr int kDg = HD / 8;                  // lanes per V row, 8 dims each
     constexpr int kPpl = 64 / kDg;               // positions per V load
     constexpr int kVLoads = kChunk / kPpl;
+    constexpr int kPiece = kPSplit / W;  // positions per wave
     static_assert(kPpl <= 16 && 16 % kPpl == 0, "a V load stays inside one page");
+    static_assert(kPiece % kChunk == 0, "a wave's positions are whole chunks");
     // Every lane writes its own slot of these buffers (columns / entries past the wave's
     // heads are written and never read): a store guarded by the lane index followed by reads
     // of every lane lets the compiler sink the reads into the guarded block, where they run
     // with the other lanes switched off (seen in a variant of this loop at head_dim 32).
-    __shared__ __attribute__((aligned(16))) float pbuf[kPWaves][kChunk][16];
-    __shared__ __attribute__((aligned(16))) float abuf[kPWaves][64];
+    __shared__ __attribute__((aligned(16))) float pbuf[W][kChunk][16];
+    __shared__ __attribute__((aligned(16))) float abuf[W][64];
+    // the waves' states for the merge: (m, l) per column, and the accumulators
+    __shared__ float mlbuf[W][2][16];
+    __shared__ __attribute__((aligned(16))) float sbuf[W][NH][HD];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t item = (int64_t)blockIdx.x * kPWaves + wave;
+    const int64_t item = blockIdx.x;  // every exit before the merge is uniform over the workgroup
     const int64_t per_q = (int64_t)kvh * nhb * nsplit;
     // queries tq0 .. tq0 + ntok - 1 (tok > 1 only in causal prefill over one shared table
     // with nhb == 1, where causal lengths grow with the query index)
     const int tq0 = (int)(item / per_q) * tok;
     if (tq0 >= qs.count) return;
     const int ntok = min(tok, qs.count - tq0);
-    // kv head fastest: waves of one workgroup read neighbouring rows of the same pages
+    // kv head fastest: neighbouring workgroups read neighbouring rows of the same pages
     const int g = (int)(item % kvh);
     const int hb = (int)((item / kvh) % nhb);
     const int split = (int)((item / ((int64_t)kvh * nhb)) % nsplit);
     const int clen = qs.causal_len(tq0 + ntok - 1);
-    const int t_begin = split * kPSplit;
-    if (t_begin >= clen) return;
-    const int t_end = min(clen, t_begin + kPSplit);
+    if (split * kPSplit >= clen) return;
+    const int t_begin = split * kPSplit + wave * kPiece;  // may lie past t_end: an empty piece
+    const int t_end = min(clen, t_begin + kPiece);
     const int G = qh / kvh;
     const int h0 = g * G + hb * kHeadsMax;
     // MFMA columns (<= NH): with tok == 1 heads h0 .. h0 + ncols - 1 of query tq0, else
@@ -305,34 +315,52 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
         }
     }
 
-    // ---- partials: sum the position subsets (lanes with the same dim group), then lanes of
-    // subset 0 write dims 8 dg .. 8 dg + 7 of each head
+    // ---- the wave's state: sum the position subsets (lanes with the same dim group), then
+    // lanes of subset 0 leave dims 8 dg .. 8 dg + 7 of each column
 #pragma unroll
     for (int o = kDg; o < 64; o <<= 1)
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[h][i] += __shfl_xor(acc[h][i], o);
-    // column c's vector: (query tq0 + c / G, head h0 + c % G)
-    if (lane < ncols) {  // lane == n here
-        const int64_t v = (int64_t)(tq0 + ct) * qh + h0 + hn;
-        part_ml[(v * nsplit + split) * 2 + 0] = m_run * 0.6931471805599453f;
-        part_ml[(v * nsplit + split) * 2 + 1] = l_run;
+    if (lane < 16) {  // lane == n here
+        mlbuf[wave][0][lane] = m_run;
+        mlbuf[wave][1][lane] = l_run;
     }
     if (ps == 0) {
-        int hc = 0, hh = 0;  // column h is head h0 + hh of query tq0 + hc
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
-            if (h < ncols) {
-                const int64_t v = (int64_t)(tq0 + hc) * qh + h0 + hh;
-                float* dst = part_acc + (v * nsplit + split) * HD + 8 * dg;
-                *(f4_t*)dst = f4_t{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
-                *(f4_t*)(dst + 4) = f4_t{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
-            }
-            if (++hh == G) {
-                hh = 0;
-                ++hc;
-            }
+            float* dst = &sbuf[wave][h][8 * dg];
+            *(f4_t*)dst = f4_t{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+            *(f4_t*)(dst + 4) = f4_t{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
+        }
+    }
+    __syncthreads();
+    // ---- merge in wave order: column c's vector is (query tq0 + c / G, head h0 + c % G); a
+    // wave with m = -inf (an empty or fully masked piece) adds nothing
+    for (int i = threadIdx.x; i < ncols * (HD / 4); i += 64 * W) {
+        const int c = i / (HD / 4), d = 4 * (i - c * (HD / 4));
+        const int cq = tok > 1 ? c / G : 0;
+        float M = -__builtin_inff();
+#pragma unroll
+        for (int w = 0; w < W; ++w) M = fmaxf(M, mlbuf[w][0][c]);
+        float L = 0.0f;
+        f4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float mw = mlbuf[w][0][c];
+            if (mw == -__builtin_inff()) continue;
+            const float wt = __builtin_amdgcn_exp2f(mw - M);
+            L = fmaf(wt, mlbuf[w][1][c], L);
+            const f4_t a = *(const f4_t*)&sbuf[w][c][d];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[k] = fmaf(wt, a[k], o[k]);
+        }
+        const int64_t v = (int64_t)(tq0 + cq) * qh + h0 + (c - cq * G);
+        *(f4_t*)(part_acc + (v * nsplit + split) * HD + d) = o;
+        if (d == 0) {
+            part_ml[(v * nsplit + split) * 2 + 0] = M * 0.6931471805599453f;
+            part_ml[(v * nsplit + split) * 2 + 1] = L;
         }
     }
 }
@@ -759,19 +787,37 @@ bool paged_shape_ok(int qh, int kvh, int hd) {
     return kvh > 0 && qh > 0 && qh % kvh == 0 && hd >= 1 && hd <= 256;
 }
 
-template <int HD, int NH, class Pages>
-void launch_split_t(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
-                    int nhb, float* ml, float* acc, int nsplit, int tok, int64_t groups,
+// Waves per split by the launch's size (splits x kv heads x head blocks x query groups). Few
+// workgroups: eight waves each hide one another's memory latency (one sequence of 4000 positions,
+// 32 / 8 heads of 128: 94 us with a wave per split, 36 / 25 / 20 us with 2 / 4 / 8). Many: the
+// chip is full with two, and more only add merge work and empty pieces at the ragged ends (64
+// sequences of 500 .. 2000, 1024 workgroups: 77 / 93 / 85 us). In between, at 512 workgroups
+// (32 / 4 heads): 68 / 49 / 56 us.
+constexpr int64_t kSplits8 = 256, kSplits4 = 512;
+template <int HD, int NH, int W, class Pages>
+void launch_split_w(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
+                    int nhb, float* ml, float* acc, int nsplit, int tok, int64_t items,
                     hipStream_t s) {
     const float scale_log2 = 1.4426950408889634f / sqrtf((float)HD);
-    hipLaunchKernelGGL((paged_attn_split_kernel<HD, NH, Pages>), dim3((unsigned)groups),
-                       dim3(64 * kPWaves), 0, s, q, qs, pg, qh, kvh, nhb, scale_log2, ml, acc,
-                       nsplit, tok);
+    hipLaunchKernelGGL((paged_attn_split_kernel<HD, NH, W, Pages>), dim3((unsigned)items),
+                       dim3(64 * W), 0, s, q, qs, pg, qh, kvh, nhb, scale_log2, ml, acc, nsplit,
+                       tok);
+}
+template <int HD, int NH, class Pages>
+void launch_split_t(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
+                    int nhb, float* ml, float* acc, int nsplit, int tok, int64_t items,
+                    hipStream_t s) {
+    if (items <= kSplits8)
+        launch_split_w<HD, NH, 8>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+    else if (items <= kSplits4)
+        launch_split_w<HD, NH, 4>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+    else
+        launch_split_w<HD, NH, 2>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
 }
 
 template <int HD, class Pages>
 void launch_split_hd(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
-                     int nhb, float* ml, float* acc, int nsplit, int tok, int64_t groups,
+                     int nhb, float* ml, float* acc, int nsplit, int tok, int64_t items,
                      hipStream_t s) {
     if constexpr (HD <= 128) {
         if (tok > 1) {
@@ -786,9 +832,9 @@ void launch_split_hd(const uint16_t* q, const PQueries& qs, const Pages& pg, int
         }
     }
     if (qh / kvh * tok <= 4)
-        launch_split_t<HD, 4>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, groups, s);
+        launch_split_t<HD, 4>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
     else
-        launch_split_t<HD, 8>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, groups, s);
+        launch_split_t<HD, 8>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
 }
 
 template <class Pages>
@@ -810,8 +856,7 @@ int launch_paged(void* out, const void* q, const PQueries& qs, int nq, const Pag
                     : G < kHeadsMax                   ? kHeadsMax / G
                                                       : 1;
     const int64_t items = ceil_div((int64_t)nq, tok) * kvh * nhb * nsplit;
-    const int64_t groups = ceil_div(items, kPWaves);
-    if (groups > 0x7fffffff || (int64_t)nq * qh > 0x7fffffff) return hipErrorInvalidValue;
+    if (items > 0x7fffffff || (int64_t)nq * qh > 0x7fffffff) return hipErrorInvalidValue;
     PQueries q2 = qs;
     q2.count = nq;
     const uint16_t* qp = (const uint16_t*)q;
@@ -825,16 +870,16 @@ int launch_paged(void* out, const void* q, const PQueries& qs, int nq, const Pag
     } else {
     switch (hd) {
         case 32:
-            launch_split_hd<32>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, groups, s);
+            launch_split_hd<32>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
             break;
         case 64:
-            launch_split_hd<64>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, groups, s);
+            launch_split_hd<64>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
             break;
         case 128:
-            launch_split_hd<128>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, groups, s);
+            launch_split_hd<128>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
             break;
         default:
-            launch_split_hd<256>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, groups, s);
+            launch_split_hd<256>(qp, q2, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
             break;
     }
     }

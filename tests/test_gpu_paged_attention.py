@@ -66,6 +66,32 @@ def test_decode_small_contexts(dev, hd, qh, kvh):
                      f"seq {b} len {n}")
 
 
+@pytest.mark.parametrize("nseq,qh,kvh,hd", [
+    (32, 8, 8, 64), (33, 8, 8, 64), (33, 32, 8, 128), (64, 16, 8, 32), (65, 16, 8, 128), (65, 16, 8, 256)])
+def test_decode_waves_per_split(dev, nseq, qh, kvh, hd):
+    """8, 4 and 2 waves per split (up to 256, up to 512 and more workgroups): lengths that leave
+    waves empty, end inside each wave's piece and on its edges, and a masked page that is a
+    wave's whole piece of one chunk."""
+    rng = np.random.default_rng(nseq + hd)
+    edges = [0, 1, 127, 128, 129, 255, 257, 511, 512, 513, 640, 897, 1000, 1023, 1024]
+    lens = (edges * 5)[:nseq]
+    kp, vp, table = build_pool(rng, lens, kvh, hd)
+    for b, n in enumerate(lens):
+        if n == 640:
+            table[b, 32:40] = -1  # positions 512..639
+    q = (rng.standard_normal((len(lens), qh, hd)) * 2).astype(np.float16)
+    got = run_decode(dev, q, table, lens, kp, vp, kvh)
+    for b, n in enumerate(lens):
+        if b >= 20 and b < nseq - 5:
+            continue  # repeats of the same lengths
+        rows = table[b]
+        if n == 640:
+            rows, n = rows[:32], 512
+        want = oracle.paged_attention(q[b], rows, n, kp, vp, kvh) if n else np.zeros_like(q[b])
+        assert_close(got[b].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3,
+                     f"seq {b} len {n}")
+
+
 @pytest.mark.parametrize("hd", [128, 64, 80])
 def test_decode_split_edges(dev, hd):
     """Lengths around the 1024-position splits: the combine merges 1 to 3 splits."""
