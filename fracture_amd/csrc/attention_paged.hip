@@ -24,6 +24,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "fhip_common.h"
 #include "fracture_hip.h"
 
@@ -80,6 +82,11 @@ struct F16PoolPages {
     __device__ const uint8_t* k_page(int p) const { return k + p * sk; }
     __device__ const uint8_t* v_page(int p) const { return v + p * sv; }
 };
+
+// 16 bytes through a global pointer: page pointers read from memory are generic ones to the compiler,
+// and flat loads would also be waited for with every LDS read.
+typedef __attribute__((address_space(1))) const u32x4 g_u32x4;
+__device__ __forceinline__ u32x4 gld16(const uint8_t* p) { return *(g_u32x4*)p; }
 
 // Query i reads block-table row i (stride 0: one shared table) and attends to seq_lens[i]
 // positions, or min(start_pos + i + 1, kv_len) when seq_lens is null; never more than the
@@ -365,281 +372,24 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
     }
 }
 
-// Causal prefill groups with PV on the MFMA as well (head_dim 32 / 64 / 128, G <= 8 q heads per
-// kv head): a wave takes 16 / G consecutive queries, MFMA column c being head c % G of query
-// c / G. Per 32-position chunk:
-//   QK as in paged_attn_split_kernel, over 16 columns;
-//   PV on v_mfma_f32_16x16x32_f16, two products per 16-dim block: out[col][d] +=
-//     P[col][slot] V[slot][d] for columns 0..7, then 8..15. Slot 8q + i of lane group q is
-//     position 4q + i (i < 4) or 16 + 4q + i - 4: exactly the positions whose probabilities
-//     that lane group holds after QK. In the product for columns 8h .. 8h + 7, A row m < 8 is
-//     fp16(p) of column 8h + m and row 8 + m is fp16((p - fp16(p)) 2^12) of the same column
-//     (one DPP row rotation by 8 brings each lane its partner column's p), and the output
-//     is D[m] + 2^-12 D[8 + m]: fp32 weights to ~2^-22, V exact.
-//   The kPfWaves waves of a workgroup take consecutive query groups over the same kv head and
-//     split and share each chunk: the workgroup loads its K and V rows into LDS once and every
-//     wave reads all of them (the chunk's K and V cross L2 once per kPfWaves x 16 / G queries);
-//   B = V transposed: the chunk's V rows are staged in LDS row-major (rows padded so that the
-//     four rows one transposed read gathers sit on different banks), and
-//     ds_read_b64_tr_b16 gives lane (d, q) dim d of the 4 positions addressed by source
-//     lanes a + 4k of its 16-lane group (destination lane 4a + b takes element b of each).
-constexpr int kPfWaves = 4;  // prefill: waves (query groups) per workgroup sharing each chunk
-template <int HD, class Pages>
-__global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2))) void
-paged_attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, int qh,
-                               int kvh, float scale_log2, float* __restrict__ part_ml,
-                               float* __restrict__ part_acc, int nsplit, int tok) {
-    constexpr int kChunk = 32;
-    constexpr int kTiles = 2;
-    constexpr int kSteps = HD / 32;
-    constexpr int kBlk = HD / 16;  // PV output dim blocks
-    constexpr int kRow = HD * 2 + 32;   // bytes per staged V row
-    constexpr int kRowK = HD * 2 + 16;  // per staged K row: 16 rows' reads of one segment
-                                        // cover all banks
-    static_assert(HD >= 32 && HD <= 128, "head_dim 32, 64 or 128");
-    constexpr int kPieces = kChunk * HD / 8;  // 16-byte pieces of a chunk's K (and of its V)
-    constexpr int kPer = (kPieces + 64 * kPfWaves - 1) / (64 * kPfWaves);
-    __shared__ __attribute__((aligned(16))) uint8_t kbuf[kChunk * kRowK];
-    __shared__ __attribute__((aligned(16))) uint8_t vbuf[kChunk * kRow];
-    __shared__ __attribute__((aligned(16))) float abuf[kPfWaves][64];
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // workgroup (kPfWaves query groups, kv head, split); wave w takes the set's group w. Every
-    // exit before the chunk loop is uniform over the workgroup (the loop has barriers).
-    const int64_t wg = blockIdx.x;
-    const int64_t per_p = (int64_t)kvh * nsplit;
-    const int tp0 = (int)(wg / per_p) * kPfWaves * tok;  // the set's first query
-    if (tp0 >= qs.count) return;
-    const int tq0 = tp0 + wave * tok;
-    const int ntok = max(0, min(tok, qs.count - tq0));  // 0: a wave past the last query
-    const int g = (int)(wg % kvh);
-    const int split = (int)((wg / kvh) % nsplit);
-    // the set's longest causal length
-    const int clen = qs.causal_len(min(tp0 + kPfWaves * tok, qs.count) - 1);
-    const int t_begin = split * kPSplit;
-    if (t_begin >= clen) return;
-    const int t_end = min(clen, t_begin + kPSplit);
-    const int G = qh / kvh;
-    const int h0 = g * G;
-    const int ncols = ntok * G;  // <= 16
-    const int32_t* table = qs.table + (int64_t)tp0 * qs.table_stride;
-
-    static_assert(kPSplit == 64 * FHIP_PAGE_TOKENS, "one cached page per lane");
-    const int split_page =
-        t_begin + FHIP_PAGE_TOKENS * lane < t_end ? table[t_begin / FHIP_PAGE_TOKENS + lane] : -1;
-    const typename Pages::Lane pl = pg.lane_load(split_page);
-
-    // column n is head h0 + n % G of query tq0 + n / G
-    const int n = lane & 15, kg = lane >> 4;
-    const bool col_ok = n < ncols;
-    const int ct = col_ok ? n / G : 0;
-    const int hn = col_ok ? n - ct * G : 0;
-    const int lim = col_ok ? min(t_end, qs.causal_len(tq0 + ct)) : 0;
-    u32x4 bq[kSteps];
-    {
-        const uint16_t* qrow = q + ((int64_t)(col_ok ? tq0 + ct : tp0) * qh + h0 + hn) * HD + 8 * kg;
-#pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            const u32x4 v = ld16(qrow + 32 * s);
-            bq[s] = col_ok ? v : u32x4{0u, 0u, 0u, 0u};
-        }
-    }
-    const uint8_t* dummy = (const uint8_t*)q;
-    uint8_t* vb = vbuf;
-    // transposed-read source of this lane: row 4q + k (+16 for slots 4..7), dims 4a .. 4a + 3
-    // of each 16-dim block (q = lane / 16, k = (lane / 4) % 4, a = lane % 4)
-    const uint32_t tr_off =
-        (uint32_t)((4 * (lane >> 4) + ((lane >> 2) & 3)) * kRow + 8 * (lane & 3));
-
-    float m_run = -__builtin_inff(), l_run = 0.0f;
-    f4_t acc[2][kBlk];  // columns 0..7, 8..15
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int b = 0; b < kBlk; ++b) acc[h][b] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-
-    for (int t0 = t_begin; t0 < t_end; t0 += kChunk) {
-        const int j0 = (t0 - t_begin) / FHIP_PAGE_TOKENS;
-        bool pok[kTiles];
-#pragma unroll
-        for (int tt = 0; tt < kTiles; ++tt)
-            pok[tt] = pg.valid(__builtin_amdgcn_readlane(split_page, j0 + tt));
-        // ---- the chunk's K and V rows, 16-byte pieces spread over the workgroup: piece i is
-        // row i / (HD / 8), segment i % (HD / 8). Rows past the end or in invalid pages read
-        // `dummy` (finite); their V is staged as zeros (0 * NaN would poison PV).
-        const uint8_t* kpg[kTiles];
-        const uint8_t* vpg[kTiles];
-#pragma unroll
-        for (int tt = 0; tt < kTiles; ++tt) {
-            const int id = __builtin_amdgcn_readlane(split_page, j0 + tt);
-            kpg[tt] = pok[tt] ? pg.k_at(pl, j0 + tt, id) : dummy;
-            vpg[tt] = pok[tt] ? pg.v_at(pl, j0 + tt, id) : dummy;
-        }
-        u32x4 kr[kPer], vr[kPer];
-        bool rok[kPer];
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int i = min((int)threadIdx.x + 64 * kPfWaves * u, kPieces - 1);
-            const int r = i / (HD / 8), sg = i % (HD / 8);
-            rok[u] = pok[r / 16] && t0 + r < t_end;
-            const int64_t off = ((int64_t)(r % 16) * kvh + g) * (HD * 2) + 16 * sg;
-            kr[u] = ld16(rok[u] ? kpg[r / 16] + off : dummy);
-            vr[u] = ld16(rok[u] ? vpg[r / 16] + off : dummy);
-        }
-        // ---- stage: every wave has finished reading the previous chunk
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < kPer; ++u) {
-            const int i = (int)threadIdx.x + 64 * kPfWaves * u;
-            if (i < kPieces) {
-                const int r = i / (HD / 8), sg = i % (HD / 8);
-                *(u32x4*)(kbuf + r * kRowK + 16 * sg) = kr[u];
-                *(u32x4*)(vb + r * kRow + 16 * sg) = rok[u] ? vr[u] : u32x4{0u, 0u, 0u, 0u};
-            }
-        }
-        __syncthreads();
-
-        // ---- QK: lane (n, kg) gets positions 16 tt + 4 kg + e of column n
-        float sc[kTiles][4];
-#pragma unroll
-        for (int tt = 0; tt < kTiles; ++tt) {
-            f4_t d = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int st = 0; st < kSteps; ++st) {
-                const u32x4 kv =
-                    *(const u32x4*)(kbuf + (16 * tt + (lane & 15)) * kRowK + 64 * st + 16 * kg);
-                d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, kv),
-                                                           __builtin_bit_cast(h8_t, bq[st]), d,
-                                                           0, 0, 0);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int pos = t0 + 16 * tt + 4 * kg + e;
-                sc[tt][e] = pok[tt] && pos < lim ? d[e] * scale_log2 : -__builtin_inff();
-            }
-        }
-        // ---- online softmax per column (lanes n, n + 16, n + 32, n + 48)
-        float cmax = -__builtin_inff();
-#pragma unroll
-        for (int tt = 0; tt < kTiles; ++tt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) cmax = fmaxf(cmax, sc[tt][e]);
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 16));
-        cmax = fmaxf(cmax, __shfl_xor(cmax, 32));
-        const float m_new = fmaxf(m_run, cmax);
-        const float mref = m_new == -__builtin_inff() ? 0.0f : m_new;
-        const float alpha = __builtin_amdgcn_exp2f(m_run - mref);
-        float psum = 0.0f;
-        _Float16 a[2][8];  // A of the products for columns 0..7 and 8..15
-#pragma unroll
-        for (int tt = 0; tt < kTiles; ++tt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float p = __builtin_amdgcn_exp2f(sc[tt][e] - mref);
-                psum += p;
-                // p of column n ^ 8 (lane n of each 16-lane row takes lane n ^ 8)
-                const float po = __int_as_float(
-                    __builtin_amdgcn_mov_dpp(__float_as_int(p), 0x128, 0xF, 0xF, true));
-                const _Float16 ph = (_Float16)p, oh = (_Float16)po;
-                const _Float16 pl_ = (_Float16)((p - (float)ph) * 4096.0f);
-                const _Float16 ol = (_Float16)((po - (float)oh) * 4096.0f);
-                a[0][4 * tt + e] = n < 8 ? ph : ol;  // rows: hi of column n / lo of column n - 8
-                a[1][4 * tt + e] = n < 8 ? oh : pl_;  // hi of column n + 8 / lo of column n
-            }
-        psum += __shfl_xor(psum, 16);
-        psum += __shfl_xor(psum, 32);
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-        abuf[wave][lane] = alpha;
-        wave_lds_sync();
-        // ---- PV: rescale rows 4 kg + e (columns 8h + 4 (kg % 2) + e), then accumulate
-        const f4_t al0 = *(const f4_t*)&abuf[wave][4 * (kg & 1)];
-        const f4_t al1 = *(const f4_t*)&abuf[wave][8 + 4 * (kg & 1)];
-        const h8_t av0 = {a[0][0], a[0][1], a[0][2], a[0][3], a[0][4], a[0][5], a[0][6], a[0][7]};
-        const h8_t av1 = {a[1][0], a[1][1], a[1][2], a[1][3], a[1][4], a[1][5], a[1][6], a[1][7]};
-#pragma unroll
-        for (int b = 0; b < kBlk; ++b) {
-            typedef short v4s_t __attribute__((ext_vector_type(4)));
-            typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
-            const uint8_t* base = vb + tr_off + 32 * b;
-            const v4s_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (lds_v4s_t*)(__attribute__((address_space(3))) uint8_t*)base);
-            const v4s_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (lds_v4s_t*)(__attribute__((address_space(3))) uint8_t*)(base + 16 * kRow));
-            const h8_t bv = __builtin_bit_cast(
-                h8_t, (short __attribute__((ext_vector_type(8)))){lo4[0], lo4[1], lo4[2], lo4[3],
-                                                                  hi4[0], hi4[1], hi4[2], hi4[3]});
-            acc[0][b] *= al0;
-            acc[0][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av0, bv, acc[0][b], 0, 0, 0);
-            acc[1][b] *= al1;
-            acc[1][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av1, bv, acc[1][b], 0, 0, 0);
-        }
-    }
-
-    // ---- partials: in product h, lanes kg < 2 hold rows 4 kg + e (column 8h + 4 kg + e,
-    // fp16(p) part), lanes kg + 2 the matching 2^12 (p - fp16(p)) rows
-    if (lane < ncols) {  // lane == n here
-        const int64_t v = (int64_t)(tq0 + ct) * qh + h0 + hn;
-        part_ml[(v * nsplit + split) * 2 + 0] = m_run * 0.6931471805599453f;
-        part_ml[(v * nsplit + split) * 2 + 1] = l_run;
-    }
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-        float o[kBlk][4];
-#pragma unroll
-        for (int b = 0; b < kBlk; ++b)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                o[b][e] = acc[h][b][e] + __shfl_xor(acc[h][b][e], 32) * (1.0f / 4096.0f);
-        if (kg < 2) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int col = 8 * h + 4 * kg + e;
-                if (col < ncols) {
-                    const int cq = col / G;
-                    const int64_t v = (int64_t)(tq0 + cq) * qh + h0 + (col - cq * G);
-                    float* dst = part_acc + (v * nsplit + split) * HD + n;
-#pragma unroll
-                    for (int b = 0; b < kBlk; ++b) dst[16 * b] = o[b][e];
-                }
-            }
-        }
-    }
-}
-
-// Any other head_dim (1 .. 256; the reference kernel takes any width): one wave per (query,
-// q head, 1024-position split), same partials as paged_attn_split_kernel. Per 64-position
-// chunk, lane l scores position t0 + l against the query (fp32 dot over the dims in order,
-// the query staged in LDS), the wave updates the online softmax (natural-log units), and each
-// lane accumulates its dims l, l + 64, .. over the chunk's positions, their weights and row
-// addresses broadcast from the lanes that scored them. A fallback for widths no model on this
-// path uses at scale (the tiny test models' 16, odd widths): no MFMA, no vector loads.
-constexpr int kGenWaves = 4;
+// One wave's attention of one query row over positions [t_begin, t_end) of a kv head, any
+// head_dim up to 256. Per 64-position chunk, lane l scores position t0 + l against the query (fp32
+// dot over the dims in order, the query staged in `qv`, hd floats of LDS), the wave updates the
+// online softmax (natural-log units), and each lane accumulates its dims l, l + 64, .. over the
+// chunk's positions, their weights and row addresses broadcast from the lanes that scored them.
+// A position outside [t_begin, t_end) or in a page outside the pool is never read.
 template <class Pages>
-__global__ __launch_bounds__(64 * kGenWaves) void paged_attn_generic_kernel(
-    const uint16_t* __restrict__ q, PQueries qs, Pages pg, int qh, int kvh, int hd,
-    float scale, float* __restrict__ part_ml, float* __restrict__ part_acc, int nsplit,
-    int64_t items) {
-    __shared__ float qbuf[kGenWaves][256];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t item = (int64_t)blockIdx.x * kGenWaves + wave;
-    if (item >= items) return;
-    const int split = (int)(item % nsplit);
-    const int64_t vec = item / nsplit;  // query qi, q head h
-    const int qi = (int)(vec / qh), h = (int)(vec % qh);
-    const int clen = qs.causal_len(qi);
-    const int t_begin = split * kPSplit;
-    if (t_begin >= clen) return;  // not read by the combine (splits below the length only)
-    const int t_end = min(clen, t_begin + kPSplit);
-    const int g = h / (qh / kvh);
-    const int32_t* table = qs.table + (int64_t)qi * qs.table_stride;
-    float* qv = qbuf[wave];
-    for (int d = lane; d < hd; d += 64) qv[d] = h2f(q[vec * hd + d]);
+__device__ __forceinline__ void wave_attend(const uint16_t* qrow, const int32_t* table, const Pages& pg,
+                                            int t_begin, int t_end, int kvh, int g, int hd, float scale,
+                                            int lane, float* qv, float& m_run, float& l_run,
+                                            float (&acc)[4]) {
+    wave_lds_sync();  // an earlier call's reads of qv stay above these writes
+    for (int d = lane; d < hd; d += 64) qv[d] = h2f(qrow[d]);
     wave_lds_sync();  // every lane reads every dim below
-    float m_run = -__builtin_inff(), l_run = 0.0f;
-    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // dims lane + 64 i
+    m_run = -__builtin_inff();
+    l_run = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i] = 0.0f;  // dims lane + 64 i
     const int64_t row_bytes = (int64_t)hd * 2;
     for (int t0 = t_begin; t0 < t_end; t0 += 64) {
         const int pos = t0 + lane;
@@ -675,6 +425,365 @@ __global__ __launch_bounds__(64 * kGenWaves) void paged_attn_generic_kernel(
             }
         }
     }
+}
+
+// Causal prefill (head_dim 32 / 64 / 128, G <= 8 q heads per kv head): a workgroup of 4 waves takes
+// kPfCols columns of one kv head, column c being head c % G of query q0 + c / G, each wave 32 of
+// them, and walks a split of the positions in tiles of 64 that all its waves share.
+//   S^T = K Q^T on v_mfma_f32_32x32x16_f16: row = position, column = (query, head); lane
+//     (n, half) then holds 16 positions of column n per 32-position block, so the softmax of a
+//     column needs one exchange between the two halves (the maximum) per tile.
+//   out^T = V^T P^T on the same MFMA: slot j of lane half `half` in a 16-position step is
+//     position 4 half + j (j < 4) or 8 + 4 half + j - 4, exactly what the lane holds after S^T,
+//     so P goes into the B operand without moving between lanes. P = hi + lo in fp16, two
+//     products into one accumulator: the exponent is biased by kPfBias, so that lo is a normal
+//     fp16 number for every p above 2^-10 (p to ~2^-23; an absolute 2^-32 below that), and the
+//     bias cancels in out = acc / l. V is exact. A = V^T comes from the row-major tile by
+//     ds_read_b64_tr_b16.
+//   The next tile's rows are loaded into registers before the tile's products and stored to the
+//     other LDS buffer after them: one barrier per tile. Rows are padded so that the 16-byte
+//     reads of 16 K rows, and the transposed reads of 4 V rows x 32 dims, cover all banks.
+// Bound by the MFMA (48 products of 32 clocks per wave and tile at head_dim 128, a third of them
+// the lo parts) and by the VALU work of the softmax (~1360 clocks), which two waves per SIMD
+// overlap in part. 1000 queries at 3001 .. 4000, 32 / 8 heads of 128: 107 us (536 TFLOP/s of
+// attention); waves of 16 columns over chunks of 32 positions with two barriers each took 214.
+constexpr int kPfWaves = 4;                // waves per workgroup
+constexpr int kPfCols = 32 * kPfWaves;     // (query, head) columns per workgroup
+constexpr int kPfTile = 64;                // positions per tile
+constexpr float kPfBias = 7.0f;            // log2 of the scale that P carries
+constexpr float kPfScale = 128.0f;         // 2^kPfBias
+constexpr float kPfSlack = 8.0f;           // log2 that p may exceed it by (2^15 < fp16's largest)
+constexpr int64_t kPfGroups = 512;         // workgroups wanted: the two per CU that fit at once
+typedef float f16x_t __attribute__((ext_vector_type(16)));
+
+// (a, b) as fp16 pairs hi + lo, hi rounded to nearest, lo the fp16 of what it leaves.
+typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
+typedef float f2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t{a, b}), h2_t));
+    float la, lb;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(la) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(lb) : "v"(hi), "v"(b));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t{la, lb}), h2_t));
+}
+
+template <int HD, class Pages>
+__global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2))) void
+paged_attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, int qh,
+                               int kvh, float scale_log2, float* __restrict__ part_ml,
+                               float* __restrict__ part_acc, uint16_t* __restrict__ out,
+                               int nsplit, int split_pos, int nqb, int nblk) {
+    constexpr int kSteps = HD / 16;     // S^T steps per 32-position block
+    constexpr int kDt = HD / 32;        // 32-dim blocks of out^T
+    constexpr int kRowK = HD * 2 + 16;  // bytes per staged K row
+    constexpr int kRowV = HD * 2 + 64;  // bytes per staged V row
+    constexpr int kPer = kPfTile * HD / 8 / (64 * kPfWaves);  // 16-byte pieces of K (of V) per thread
+    constexpr int kSegs = HD / 8;                             // pieces per row
+    static_assert(HD == 32 || HD == 64 || HD == 128, "a wave's pieces lie in one page");
+    __shared__ __attribute__((aligned(16))) uint8_t kbuf[2][kPfTile * kRowK];
+    __shared__ __attribute__((aligned(16))) uint8_t vbuf[2][kPfTile * kRowV];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // kv head fastest (one head's rows stay in one XCD's L2 at 8 kv heads), then the split, then
+    // the query block from the last one down: the longest contexts start first
+    const int g = (int)(blockIdx.x % kvh);
+    const int rest = (int)(blockIdx.x / kvh);
+    const int split = rest % nsplit;
+    const int q0 = (nblk - 1 - rest / nsplit) * nqb;  // the block's first query
+    const int nq = min(nqb, qs.count - q0);
+    const int G = qh / kvh;
+    const int clen = qs.causal_len(q0 + nq - 1);  // the block's longest causal length
+    const int clen0 = qs.causal_len(q0);          // and its shortest
+    const int t_begin = split * split_pos;
+    // uniform: with several splits, a split past the block's length writes nothing
+    if (nsplit > 1 && t_begin >= clen) return;
+    const int t_end = min(clen, t_begin + split_pos);
+    const int32_t* table = qs.table + (int64_t)q0 * qs.table_stride;
+
+    // column n of the wave: head ch of query q0 + cq
+    const int n = lane & 31, half = lane >> 5;
+    const int ncols = nq * G;
+    const int col = 32 * wave + n;
+    const bool col_ok = col < ncols;
+    const bool wave_live = 32 * wave < ncols;
+    const int cq = col_ok ? col / G : 0;
+    const int64_t vec = (int64_t)(q0 + cq) * qh + g * G + (col_ok ? col - cq * G : 0);
+    const int lim = col_ok ? min(t_end, qs.causal_len(q0 + cq)) : 0;
+    u32x4 bq[kSteps];  // dims 16 s + 8 half + 0..7 of the column's query row
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) bq[s] = ld16(q + vec * HD + 16 * s + 8 * half);
+    // waited for here: left to the loop, the wait would also be for each next tile's loads
+#pragma unroll
+    for (int s = 0; s < kSteps; ++s) asm volatile("" : "+v"(bq[s]));
+
+    // The pages of 1024 positions from `win`, one per lane, refreshed when a tile leaves them.
+    const uint8_t* dummy = (const uint8_t*)q;  // >= 2 HD readable bytes
+    int win = t_begin, win_page;
+    typename Pages::Lane pl;
+    auto load_window = [&](int t0) {
+        win = t0;
+        win_page = t0 + FHIP_PAGE_TOKENS * lane < t_end ? table[t0 / FHIP_PAGE_TOKENS + lane] : -1;
+        pl = pg.lane_load(win_page);
+    };
+    // Piece u of a thread: row (threadIdx.x + 256 u) / kSegs of the tile, 16 bytes of it; the wave's
+    // rows of one u lie in one page (4, 8 or 16 rows a wave), whose row and offset do not depend
+    // on u. Pages outside the pool read `dummy`; their scores are masked. V rows past the end or
+    // in such pages are staged as zeros.
+    u32x4 kr[kPer], vr[kPer];
+    const uint32_t row_off = (uint32_t)(((int)threadIdx.x / kSegs % FHIP_PAGE_TOKENS * kvh + g) * (HD * 2) +
+                                        16 * ((int)threadIdx.x % kSegs));
+    uint32_t pok = 0;  // bit j: page j of the tile in the registers is in the pool
+    auto page_of = [&](int u) { return (64 * wave + 64 * kPfWaves * u) / kSegs / FHIP_PAGE_TOKENS; };
+    auto load_tile = [&](int t0) {
+        if (t0 >= win + 64 * FHIP_PAGE_TOKENS) load_window(t0);
+        const int j0 = (t0 - win) / FHIP_PAGE_TOKENS;
+        pok = (uint32_t)(__ballot(pg.valid(win_page)) >> j0) & 0xfu;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            const int j = page_of(u);
+            const int id = __builtin_amdgcn_readlane(win_page, j0 + j);
+            const bool ok = (pok >> j) & 1u;
+            const uint8_t* kp = ok ? pg.k_at(pl, j0 + j, id) : dummy;
+            const uint8_t* vp = ok ? pg.v_at(pl, j0 + j, id) : dummy;
+            const uint32_t off = ok ? row_off : 0u;
+            kr[u] = gld16(kp + off);
+            vr[u] = gld16(vp + off);
+        }
+    };
+    // Stores the tile of the registers. Where some column masks a position of the tile, also notes
+    // a V value that is infinite or NaN: 0 x inf would carry it to that column.
+    bool bad = false;
+    auto store_tile = [&](int t0, int b) {
+        const uint32_t off = ((uint32_t)threadIdx.x / kSegs) * kRowK + 16 * (threadIdx.x % kSegs);
+        const uint32_t offv = ((uint32_t)threadIdx.x / kSegs) * kRowV + 16 * (threadIdx.x % kSegs);
+        if (pok != 0xfu || t0 + kPfTile > t_end) {
+#pragma unroll
+            for (int u = 0; u < kPer; ++u) {
+                const int r = ((int)threadIdx.x + 64 * kPfWaves * u) / kSegs;
+                const bool rok = ((pok >> page_of(u)) & 1u) && t0 + r < t_end;
+                if (!rok) vr[u] = u32x4{0u, 0u, 0u, 0u};
+            }
+        }
+        if (t0 + kPfTile > clen0) {
+#pragma unroll
+            for (int u = 0; u < kPer; ++u)
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    bad |= (vr[u][k] & 0x7c00u) == 0x7c00u || (vr[u][k] & 0x7c000000u) == 0x7c000000u;
+        }
+#pragma unroll
+        for (int u = 0; u < kPer; ++u) {
+            *(u32x4*)(kbuf[b] + off + u * (64 * kPfWaves / kSegs) * kRowK) = kr[u];
+            *(u32x4*)(vbuf[b] + offv + u * (64 * kPfWaves / kSegs) * kRowV) = vr[u];
+        }
+    };
+
+    float m_run = -__builtin_inff(), l_run = 0.0f;  // l: the lane half's own positions
+    f16x_t acc[kDt];
+#pragma unroll
+    for (int d = 0; d < kDt; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] = 0.0f;
+
+    uint32_t tile_pok = 0;
+    if (t_begin < t_end) {
+        load_window(t_begin);
+        load_tile(t_begin);
+        tile_pok = pok;
+        store_tile(t_begin, 0);
+        lds_barrier();
+    }
+    int b = 0;
+    for (int t0 = t_begin; t0 < t_end; t0 += kPfTile, b ^= 1) {
+        const bool more = t0 + kPfTile < t_end;
+        if (more) load_tile(t0 + kPfTile);
+        if (wave_live) {
+            // ---- S^T: element i of block pt is position 32 pt + 8 (i / 4) + 4 half + i % 4
+            // K reads run kSteps products ahead of their use, across the two blocks
+            // (the priority lets this wave's products go first while the other wave of its SIMD is
+            // in its softmax: 114 -> 107 us)
+            __builtin_amdgcn_s_setprio(1);
+            f16x_t sc[2];
+            const uint8_t* ksrc = kbuf[b] + n * kRowK + 16 * half;
+            u32x4 ka[kSteps];
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s) ka[s] = *(const u32x4*)(ksrc + 32 * s);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sc[pt][i] = 0.0f;
+#pragma unroll
+                for (int s = 0; s < kSteps; ++s) {
+                    sc[pt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                        __builtin_bit_cast(h8_t, ka[s]), __builtin_bit_cast(h8_t, bq[s]), sc[pt], 0, 0, 0);
+                    if (pt == 0) {
+                        ka[s] = *(const u32x4*)(ksrc + 32 * kRowK + 32 * s);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+            // a tile with every page in the pool and inside every column's length needs no mask
+            if (!(tile_pok == 0xfu && t0 + kPfTile <= min(t_end, clen0))) {
+#pragma unroll
+                for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int pos = t0 + 32 * pt + 8 * (i / 4) + 4 * half + i % 4;
+                        const bool ok = ((tile_pok >> (2 * pt + i / 8)) & 1u) && pos < lim;
+                        sc[pt][i] = ok ? sc[pt][i] : -__builtin_inff();
+                    }
+            }
+            // ---- online softmax in log2 units, one column per lane pair (n, n + 32)
+            float cmax = sc[0][0];
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, sc[pt][i]);
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 32)) * scale_log2;
+            const float m_new = fmaxf(m_run, cmax);
+            // p may grow to 2^kPfSlack before the accumulators are rescaled: almost no tile after
+            // the first rescales, where following the maximum would on most (32 columns a wave)
+            if (__ballot(m_new > m_run + kPfSlack)) {
+                const float mref = m_new == -__builtin_inff() ? 0.0f : m_new;
+                const float alpha = __builtin_amdgcn_exp2f(m_run - mref);  // 0 while m_run is -inf
+                l_run *= alpha;
+#pragma unroll
+                for (int d = 0; d < kDt; ++d)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[d][i] *= alpha;
+                m_run = m_new;
+            }
+            const float ebias = kPfBias - (m_run == -__builtin_inff() ? 0.0f : m_run);
+            float psum = 0.0f;
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    sc[pt][i] = __builtin_amdgcn_exp2f(fmaf(sc[pt][i], scale_log2, ebias));
+                    psum += sc[pt][i];
+                }
+            l_run += psum;
+            __builtin_amdgcn_s_setprio(1);
+            // ---- out^T: 4 steps of 16 positions
+            const uint8_t* vsrc = vbuf[b] + (4 * half + ((lane & 15) >> 2)) * kRowV +
+                                  2 * (16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                uint32_t ph[4], pl_[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    split_pair(sc[ks >> 1][8 * (ks & 1) + 2 * j], sc[ks >> 1][8 * (ks & 1) + 2 * j + 1],
+                               ph[j], pl_[j]);
+                const h8_t bh = __builtin_bit_cast(h8_t, u32x4{ph[0], ph[1], ph[2], ph[3]});
+                const h8_t bl = __builtin_bit_cast(h8_t, u32x4{pl_[0], pl_[1], pl_[2], pl_[3]});
+#pragma unroll
+                for (int d = 0; d < kDt; ++d) {
+                    typedef short v4s_t __attribute__((ext_vector_type(4)));
+                    typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
+                    const uint8_t* src = vsrc + 16 * ks * kRowV + 64 * d;
+                    const v4s_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (lds_v4s_t*)(__attribute__((address_space(3))) uint8_t*)src);
+                    const v4s_t hi4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (lds_v4s_t*)(__attribute__((address_space(3))) uint8_t*)(src + 8 * kRowV));
+                    const h8_t av = __builtin_bit_cast(
+                        h8_t, (short __attribute__((ext_vector_type(8)))){
+                                  lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]});
+                    acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bh, acc[d], 0, 0, 0);
+                    acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bl, acc[d], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+        tile_pok = pok;
+        if (more) store_tile(t0 + kPfTile, b ^ 1);
+        lds_barrier();  // every wave is done with this tile's buffer, and the next one's is written
+    }
+
+    if (__syncthreads_or(bad)) {
+        // Rare: a V value past some column's causal length is not finite. Every column again, one
+        // at a time, its masked positions left out.
+        float* qv = (float*)(kbuf[0]) + wave * HD;
+        for (int c = 0; c < 32 && 32 * wave + c < ncols; ++c) {
+            const int c2 = 32 * wave + c, cq2 = c2 / G;
+            const int64_t v2 = (int64_t)(q0 + cq2) * qh + g * G + (c2 - cq2 * G);
+            float m, l, a[4];
+            wave_attend(q + v2 * HD, table, pg, t_begin, min(t_end, qs.causal_len(q0 + cq2)), kvh, g,
+                        HD, scale_log2 * 0.6931471805599453f, lane, qv, m, l, a);
+            if (lane == 0 && nsplit > 1) {  // in the units of the other splits' partials
+                part_ml[(v2 * nsplit + split) * 2 + 0] = m;
+                part_ml[(v2 * nsplit + split) * 2 + 1] = l * kPfScale;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int d = lane + 64 * i;
+                if (d >= HD) continue;
+                if (nsplit > 1)
+                    part_acc[(v2 * nsplit + split) * HD + d] = a[i] * kPfScale;
+                else
+                    out[v2 * HD + d] = (uint16_t)f2h(l > 0.0f ? a[i] / l : 0.0f);
+            }
+        }
+        return;
+    }
+
+    l_run += __shfl_xor(l_run, 32);
+    if (!col_ok) return;
+    if (nsplit == 1) {
+#pragma unroll
+        for (int d = 0; d < kDt; ++d)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                u32x2 w;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) {
+                    const float a0 = acc[d][4 * j + 2 * k], a1 = acc[d][4 * j + 2 * k + 1];
+                    w[k] = l_run > 0.0f ? f2h(a0 / l_run) | (f2h(a1 / l_run) << 16) : 0u;
+                }
+                *(u32x2*)(out + vec * HD + 32 * d + 8 * j + 4 * half) = w;
+            }
+        return;
+    }
+    if (half == 0) {
+        part_ml[(vec * nsplit + split) * 2 + 0] = m_run * 0.6931471805599453f;
+        part_ml[(vec * nsplit + split) * 2 + 1] = l_run;
+    }
+    float* dst = part_acc + (vec * nsplit + split) * HD + 4 * half;
+#pragma unroll
+    for (int d = 0; d < kDt; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            *(f4_t*)(dst + 32 * d + 8 * j) =
+                f4_t{acc[d][4 * j], acc[d][4 * j + 1], acc[d][4 * j + 2], acc[d][4 * j + 3]};
+}
+
+// Any other head_dim (1 .. 256; the reference kernel takes any width): one wave per (query,
+// q head, 1024-position split), same partials as paged_attn_split_kernel. A fallback for widths no
+// model on this path uses at scale (the tiny test models' 16, odd widths): no MFMA, no vector
+// loads.
+constexpr int kGenWaves = 4;
+template <class Pages>
+__global__ __launch_bounds__(64 * kGenWaves) void paged_attn_generic_kernel(
+    const uint16_t* __restrict__ q, PQueries qs, Pages pg, int qh, int kvh, int hd,
+    float scale, float* __restrict__ part_ml, float* __restrict__ part_acc, int nsplit,
+    int64_t items) {
+    __shared__ float qbuf[kGenWaves][256];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t item = (int64_t)blockIdx.x * kGenWaves + wave;
+    if (item >= items) return;
+    const int split = (int)(item % nsplit);
+    const int64_t vec = item / nsplit;  // query qi, q head h
+    const int qi = (int)(vec / qh), h = (int)(vec % qh);
+    const int clen = qs.causal_len(qi);
+    const int t_begin = split * kPSplit;
+    if (t_begin >= clen) return;  // not read by the combine (splits below the length only)
+    float m_run, l_run, acc[4];
+    wave_attend(q + vec * hd, qs.table + (int64_t)qi * qs.table_stride, pg, t_begin,
+                min(clen, t_begin + kPSplit), kvh, h / (qh / kvh), hd, scale, lane, qbuf[wave], m_run,
+                l_run, acc);
     if (lane == 0) {
         part_ml[(vec * nsplit + split) * 2 + 0] = m_run;
         part_ml[(vec * nsplit + split) * 2 + 1] = l_run;
@@ -692,13 +801,13 @@ __global__ __launch_bounds__(64 * kGenWaves) void paged_attn_generic_kernel(
 constexpr int kCombThreads = 128;
 __global__ __launch_bounds__(kCombThreads) void paged_attn_combine_kernel(
     PQueries qs, const float* __restrict__ ml, const float* __restrict__ acc,
-    uint16_t* __restrict__ out, int qh, int hd, int nsplit) {
+    uint16_t* __restrict__ out, int qh, int hd, int nsplit, int split_pos) {
     extern __shared__ float wts[];  // nsplit weights
     __shared__ float red[2][kCombThreads / kWave];
     const int64_t vec = blockIdx.x;
     const int qi = (int)(vec / qh);
     const int clen = qs.causal_len(qi);
-    const int ns = (clen + kPSplit - 1) / kPSplit;
+    const int ns = (clen + split_pos - 1) / split_pos;
     const float* m = ml + vec * nsplit * 2;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
     constexpr int kW = kCombThreads / kWave;
@@ -745,12 +854,12 @@ __global__ __launch_bounds__(kCombThreads) void paged_attn_combine_kernel(
 constexpr int kCombWaveMaxSplits = 8;
 __global__ __launch_bounds__(256) void paged_attn_combine_wave_kernel(
     PQueries qs, const float* __restrict__ ml, const float* __restrict__ acc,
-    uint16_t* __restrict__ out, int qh, int hd, int nsplit, int64_t nvec) {
+    uint16_t* __restrict__ out, int qh, int hd, int nsplit, int64_t nvec, int split_pos) {
     const int lane = threadIdx.x & 63;
     const int64_t vec = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (vec >= nvec) return;
     const int clen = qs.causal_len((int)(vec / qh));
-    const int ns = (clen + kPSplit - 1) / kPSplit;  // <= nsplit <= kCombWaveMaxSplits
+    const int ns = (clen + split_pos - 1) / split_pos;  // <= nsplit <= kCombWaveMaxSplits
     const float* m = ml + vec * nsplit * 2;
     const float ms = lane < ns ? m[2 * lane] : -__builtin_inff();
     const float ls = lane < ns ? m[2 * lane + 1] : 0.0f;
@@ -819,22 +928,33 @@ template <int HD, class Pages>
 void launch_split_hd(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
                      int nhb, float* ml, float* acc, int nsplit, int tok, int64_t items,
                      hipStream_t s) {
-    if constexpr (HD <= 128) {
-        if (tok > 1) {
-            // one workgroup per (kPfWaves query groups, kv head, split)
-            const int64_t sets = ceil_div(ceil_div((int64_t)qs.count, tok), kPfWaves);
-            const int64_t wgs = sets * kvh * nsplit;
-            const float scale_log2 = 1.4426950408889634f / sqrtf((float)HD);
-            hipLaunchKernelGGL((paged_attn_prefill_mfma_kernel<HD, Pages>), dim3((unsigned)wgs),
-                               dim3(64 * kPfWaves), 0, s, q, qs, pg, qh, kvh, scale_log2, ml, acc,
-                               nsplit, tok);
-            return;
-        }
-    }
     if (qh / kvh * tok <= 4)
         launch_split_t<HD, 4>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
     else
         launch_split_t<HD, 8>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+}
+
+template <int HD, class Pages>
+void launch_prefill_t(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
+                      float* ml, float* acc, uint16_t* out, int nsplit, int split_pos, int nqb,
+                      int nblk, hipStream_t s) {
+    const float scale_log2 = 1.4426950408889634f / sqrtf((float)HD);
+    hipLaunchKernelGGL((paged_attn_prefill_mfma_kernel<HD, Pages>),
+                       dim3((unsigned)((int64_t)nblk * nsplit * kvh)), dim3(64 * kPfWaves), 0, s, q,
+                       qs, pg, qh, kvh, scale_log2, ml, acc, out, nsplit, split_pos, nqb, nblk);
+}
+
+// The merge of nsplit splits of split_pos positions per vector.
+void launch_combine(const PQueries& qs, const float* ml, const float* acc, void* out, int64_t nvec,
+                    int qh, int hd, int nsplit, int split_pos, hipStream_t s) {
+    if (nsplit <= kCombWaveMaxSplits)
+        hipLaunchKernelGGL(paged_attn_combine_wave_kernel, dim3((unsigned)ceil_div(nvec, 4)),
+                           dim3(256), 0, s, qs, ml, acc, (uint16_t*)out, qh, hd, nsplit, nvec,
+                           split_pos);
+    else
+        hipLaunchKernelGGL(paged_attn_combine_kernel, dim3((unsigned)nvec), dim3(kCombThreads),
+                           (size_t)nsplit * sizeof(float), s, qs, ml, acc, (uint16_t*)out, qh, hd,
+                           nsplit, split_pos);
 }
 
 template <class Pages>
@@ -848,18 +968,44 @@ int launch_paged(void* out, const void* q, const PQueries& qs, int nq, const Pag
     float* acc = (float*)((char*)ws + off_acc);
     const int G = qh / kvh;
     const int nhb = (G + kHeadsMax - 1) / kHeadsMax;
-    // causal prefill over one shared table: 16 / G consecutive queries per wave on the MFMA
-    // prefill kernel (head_dim <= 128, G <= 8), else 8 / G (G < 8)
-    const bool prefill = !qs.seq_lens && qs.table_stride == 0 && nq > 1;
-    const int tok = !prefill                          ? 1
-                    : (hd <= 128 && G <= kHeadsMax)   ? 2 * kHeadsMax / G
-                    : G < kHeadsMax                   ? kHeadsMax / G
-                                                      : 1;
-    const int64_t items = ceil_div((int64_t)nq, tok) * kvh * nhb * nsplit;
-    if (items > 0x7fffffff || (int64_t)nq * qh > 0x7fffffff) return hipErrorInvalidValue;
+    const int64_t nvec = (int64_t)nq * qh;
     PQueries q2 = qs;
     q2.count = nq;
     const uint16_t* qp = (const uint16_t*)q;
+    // causal prefill over one shared table: kPfCols / G consecutive queries per workgroup on the
+    // MFMA prefill kernel (head_dim <= 128, G <= 8), else 8 / G per wave (G < 8)
+    const bool prefill = !qs.seq_lens && qs.table_stride == 0 && nq > 1;
+    if (prefill && (hd == 32 || hd == 64 || hd == 128) && G <= kHeadsMax) {
+        const int nqb = kPfCols / G;
+        const int nblk = (int)ceil_div((int64_t)nq, nqb);
+        const int64_t base = (int64_t)nblk * kvh;
+        // Splits only as far as the workgroups need to fill the chip (kPfGroups: 768 or 1024
+        // measured 129 and 120 us where 512 took 114), at most the
+        // workspace's one per kPSplit positions: every split adds partials to write and merge.
+        const int64_t extent =
+            std::max<int64_t>(std::min<int64_t>(qs.kv_len, (int64_t)qs.max_blocks * FHIP_PAGE_TOKENS), 1);
+        const int64_t want =
+            std::min<int64_t>(std::max<int64_t>(ceil_div(kPfGroups, base), 1), nsplit);
+        const int split_pos = (int)(ceil_div(ceil_div(extent, want), kPfTile) * kPfTile);
+        const int ns = (int)ceil_div(extent, split_pos);
+        if (base * ns > 0x7fffffff || nvec > 0x7fffffff) return hipErrorInvalidValue;
+        switch (hd) {
+            case 32:
+                launch_prefill_t<32>(qp, q2, pg, qh, kvh, ml, acc, (uint16_t*)out, ns, split_pos, nqb, nblk, s);
+                break;
+            case 64:
+                launch_prefill_t<64>(qp, q2, pg, qh, kvh, ml, acc, (uint16_t*)out, ns, split_pos, nqb, nblk, s);
+                break;
+            default:
+                launch_prefill_t<128>(qp, q2, pg, qh, kvh, ml, acc, (uint16_t*)out, ns, split_pos, nqb, nblk, s);
+                break;
+        }
+        if (ns > 1) launch_combine(q2, ml, acc, out, nvec, qh, hd, ns, split_pos, s);
+        return hipGetLastError();
+    }
+    const int tok = prefill && G < kHeadsMax ? kHeadsMax / G : 1;
+    const int64_t items = ceil_div((int64_t)nq, tok) * kvh * nhb * nsplit;
+    if (items > 0x7fffffff || nvec > 0x7fffffff) return hipErrorInvalidValue;
     if (hd != 32 && hd != 64 && hd != 128 && hd != 256) {
         const int64_t gitems = (int64_t)nq * qh * nsplit;
         const int64_t gwgs = ceil_div(gitems, kGenWaves);
@@ -883,14 +1029,7 @@ int launch_paged(void* out, const void* q, const PQueries& qs, int nq, const Pag
             break;
     }
     }
-    const int64_t nvec = (int64_t)nq * qh;
-    if (nsplit <= kCombWaveMaxSplits)
-        hipLaunchKernelGGL(paged_attn_combine_wave_kernel, dim3((unsigned)ceil_div(nvec, 4)),
-                           dim3(256), 0, s, q2, ml, acc, (uint16_t*)out, qh, hd, nsplit, nvec);
-    else
-        hipLaunchKernelGGL(paged_attn_combine_kernel, dim3((unsigned)nvec), dim3(kCombThreads),
-                           (size_t)nsplit * sizeof(float), s, q2, ml, acc, (uint16_t*)out, qh,
-                           hd, nsplit);
+    launch_combine(q2, ml, acc, out, nvec, qh, hd, nsplit, kPSplit, s);
     return hipGetLastError();
 }
 

@@ -222,3 +222,64 @@ def test_reference_interface_prefill_masked_page_and_no_blocks(dev, qh, kvh, hd)
     K.paged_attention(empty, tq_, dev_t(tab[:0], dev), kptr, vptr, kvh, 0, 0)
     torch.cuda.synchronize()
     assert not empty.cpu().numpy().any()
+
+
+@pytest.mark.parametrize("kv_len,T,start_pos,qh,kvh,hd", [
+    # two splits of 1056 positions: a split outlives the 64 pages a wave keeps at hand
+    (2100, 129, 1971, 128, 128, 32),
+    # full, partial and empty waves of columns; lengths on both sides of a 64-position tile
+    (64, 32, 32, 4, 1, 64), (129, 34, 95, 8, 2, 128), (65, 3, 62, 3, 1, 128), (193, 65, 128, 5, 1, 32)])
+def test_prefill_tiles(dev, kv_len, T, start_pos, qh, kvh, hd):
+    rng = np.random.default_rng(kv_len + qh)
+    kp, vp, table = build_pool(rng, [kv_len], kvh, hd, extra_pages=1)
+    q = (rng.standard_normal((T, qh, hd)) * 2).astype(np.float16)
+    got = prefill(dev, q, kp, vp, table[0], kvh, kv_len, start_pos)
+    for t in range(T):
+        want = oracle.paged_attention(q[t], table[0], start_pos + t + 1, kp, vp, kvh)
+        assert_close(got[t].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3, f"token {t}")
+
+
+def prefill(dev, q, kp, vp, table, kvh, kv_len, start_pos):
+    tk, tv = dev_t(kp, dev), dev_t(vp, dev)
+    kptr = torch.tensor([x.data_ptr() for x in tk], dtype=torch.int64, device=dev)
+    vptr = torch.tensor([x.data_ptr() for x in tv], dtype=torch.int64, device=dev)
+    tq_ = dev_t(q, dev)
+    out = torch.empty_like(tq_)
+    K.paged_attention(out, tq_, dev_t(table, dev), kptr, vptr, kvh, kv_len, start_pos)
+    torch.cuda.synchronize()
+    return out.cpu().numpy()
+
+
+@pytest.mark.parametrize("T,start_pos,hd", [(40, 30, 128), (20, 1100, 64)])
+def test_prefill_non_finite_values_stay_with_their_queries(dev, T, start_pos, hd):
+    """An infinity and a NaN among the V rows of the queries' own positions reach the queries that
+    attend to them and none before, and a K row of NaN likewise (its score makes the sum NaN,
+    which the merge writes as 0)."""
+    rng = np.random.default_rng(T)
+    qh, kvh = 8, 2
+    kv_len = start_pos + T
+    kp, vp, table = build_pool(rng, [kv_len], kvh, hd, extra_pages=1)
+    q = (rng.standard_normal((T, qh, hd)) * 2).astype(np.float16)
+    clean = [oracle.paged_attention(q[t], table[0], start_pos + t + 1, kp, vp, kvh) for t in range(T)]
+
+    def at(pages, pos):
+        return pages[table[0][pos // 16], pos % 16]
+
+    inf_t, nan_t, k_t = T // 3, T // 2, T - 5
+    at(vp, start_pos + inf_t)[1, 3] = np.inf
+    at(vp, start_pos + nan_t)[0, 5] = np.nan
+    at(kp, start_pos + k_t)[1, :] = np.nan
+    got = prefill(dev, q, kp, vp, table[0], kvh, kv_len, start_pos).astype(np.float32)
+    for t in range(T):
+        want = clean[t].astype(np.float32)
+        keep = np.ones((qh, hd), bool)
+        if t >= inf_t:
+            keep[4:, 3] = False
+            assert np.all(np.isposinf(got[t][4:, 3])) or t >= k_t
+        if t >= nan_t:
+            keep[:4, 5] = False
+            assert np.all(np.isnan(got[t][:4, 5]))
+        if t >= k_t:
+            keep[4:] = False
+            assert not got[t][4:].any()
+        assert_close(got[t][keep], want[keep], 1e-3, 1e-3, f"token {t}")
