@@ -533,11 +533,13 @@ __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// 2'. MFMA split kernel: head_dim 128, 4-bit K codes and 4- or 2-bit V codes (kV2: widened to
-//     4 bits on their way into LDS), G <= 8 query heads per kv head.
+// 2'. MFMA split kernel: head_dim 128, K and V codes of 2, 3, 4 or 8 bits (the pairs that
+//     launch_mfma_split lists), G <= 8 query heads per kv head. Codes of 2 and 3 bits are widened to
+//     4 on their way into registers (K) or LDS (V); 8-bit codes have one table entry each.
 //
-// A workgroup owns one (query, kv head, 1024-position block); each of its two waves walks
-// one 512-position split of it in 64-position chunks:
+// A workgroup owns one (query, kv head, 1024-position block); each of its W waves walks an
+// equal split of it in 64-position chunks (two waves of 512 positions, or eight of 128 where a
+// launch has few workgroups):
 //   QK  D[pos][col] = sum_k A[pos][k] B[k][col] on v_mfma_f32_16x16x32_f16. The K slots come
 //       in (hi, lo') pairs per coordinate: A = (c_hi, c_lo*2^12) of the position's centroid,
 //       B = (q_hi, 0) in column h and (q_lo*2^12, q_hi) in column 8+h, so one MFMA gives
@@ -556,10 +558,10 @@ __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
 // Online softmax per head (lanes n = h), lazily rescaling the accumulators.
 // ---------------------------------------------------------------------------------------
 constexpr int kChunkM = 64;     // positions per chunk
-constexpr int kSplitMfma = 512;  // positions per wave item (split)
+constexpr int kSplitMfma = 512;  // positions per wave (split) at two waves per workgroup
 constexpr int kXcds = 8;         // MI355X: accelerator complex dies, each with its own L2
-constexpr int kSplitPages = kSplitMfma / FHIP_PAGE_TOKENS;
-constexpr int kWavesM = 2;      // waves per workgroup (independent work items)
+constexpr int kWavesM = 2;      // waves per workgroup, large launches
+constexpr int kWavesWide = 8;   // and small ones
 static_assert(kChunkM == fhip_idx::kChunk && kSplitMfma == fhip_idx::kSplitPositions &&
                   kWavesM == fhip_idx::kBlockWaves && kXcds == fhip_idx::kXcdCount &&
                   FHIP_PAGE_TOKENS == fhip_idx::kPageTokens,
@@ -660,6 +662,11 @@ __device__ __forceinline__ u32x4 pair2(const u32x2* tab, uint32_t w) {
     return u32x4{e0[0], e0[1], e1[0], e1[1]};
 }
 
+// 8-bit codes: the words of the four codes of w (one table entry per code).
+__device__ __forceinline__ u32x4 quad8(const uint32_t* tab, uint32_t w) {
+    return u32x4{tab[w & 0xffu], tab[(w >> 8) & 0xffu], tab[(w >> 16) & 0xffu], tab[w >> 24]};
+}
+
 // The split's pages, read once per split into a per-wave LDS table: entry j holds the four
 // part addresses (K codes, V codes, K norms, V norms) of the split's page j. Where page j holds
 // no position of the split, or its table entry is outside the pool, the entry holds the split's
@@ -669,7 +676,7 @@ __device__ __forceinline__ u32x4 pair2(const u32x2* tab, uint32_t w) {
 struct PageAddrs {
     const uint8_t *k, *v, *kn, *vn;
 };
-template <class Pages>
+template <int kPages, class Pages>
 __device__ __forceinline__ uint64_t split_pages(const Pages& pg, const int32_t* table, int t_begin,
                                                 int t_end, int lane, PageAddrs* pages) {
     int column;
@@ -681,7 +688,7 @@ __device__ __forceinline__ uint64_t split_pages(const Pages& pg, const int32_t* 
     const int first = __builtin_amdgcn_readlane(id, (int)__builtin_ctzll(vmask));
     PageAddrs a;
     pg.addrs(ok ? id : first, a.k, a.kn, a.v, a.vn);
-    if (lane < kSplitPages) pages[lane] = a;
+    if (lane < kPages) pages[lane] = a;
     wave_lds_sync();  // the wave reads other lanes' entries next
     return vmask;
 }
@@ -725,13 +732,36 @@ __device__ __forceinline__ void dma16(const uint8_t* sbase, uint32_t voff, uint8
 // every address comes from the split's page lanes, so no load needs a per-position check.
 //
 // K codes, straight into the registers QK uses (LDS DMA streams markedly slower than vector
-// loads, and K needs no LDS stage): tile pt is position 4n + pt, bytes [16rg, 16rg + 16) for
-// lane (n, rg); the lane's page is j0 + n / 4 and the four tiles are 4 rows apart.
+// loads, and K needs no LDS stage): tile pt is position 4n + pt, the 4 KB bytes of coordinates
+// [32rg, 32rg + 32) for lane (n, rg); the lane's page is j0 + n / 4 and the four tiles are 4 rows
+// apart. Pages of other widths than 4 may lie at any address: their loads assume no alignment.
+typedef u32x4 u32x4_any __attribute__((aligned(1)));
+typedef u32x2 u32x2_any __attribute__((aligned(1)));
+typedef uint32_t u32_any __attribute__((aligned(1)));
+typedef __attribute__((address_space(1))) const u32x4_any g_u32x4_any;
+typedef __attribute__((address_space(1))) const u32x2_any g_u32x2_any;
+typedef __attribute__((address_space(1))) const u32_any g_u32_any;
+template <int KB>
+struct KCodes {
+    u32x4 w[4][KB == 8 ? 2 : 1];  // [pt]: KB words
+};
+template <int KB>
 __device__ __forceinline__ void load_k(const PageAddrs* pages, int j0, int kvh, int g, int lane,
-                                       u32x4 (&kc)[4]) {
-    const uint8_t* src = pages[j0 + fhip_idx::k_page(lane)].k + fhip_idx::k_offset(lane, kvh, g);
+                                       KCodes<KB>& kc) {
+    const uint8_t* src = pages[j0 + fhip_idx::k_page(lane)].k + fhip_idx::k_offset(lane, kvh, g, KB);
 #pragma unroll
-    for (int pt = 0; pt < 4; ++pt) kc[pt] = gld16(src + pt * fhip_idx::k_tile_stride(kvh));
+    for (int pt = 0; pt < 4; ++pt) {
+        const uint8_t* p = src + pt * fhip_idx::k_tile_stride(kvh, KB);
+        if constexpr (KB == 4) {
+            kc.w[pt][0] = gld16(p);
+        } else if constexpr (KB == 8) {
+            kc.w[pt][0] = *(g_u32x4_any*)p;
+            kc.w[pt][1] = *(g_u32x4_any*)(p + 16);
+        } else {
+            const u32x2 v = *(g_u32x2_any*)p;
+            kc.w[pt][0] = u32x4{v[0], v[1], KB == 3 ? *(g_u32_any*)(p + 8) : 0u, 0u};
+        }
+    }
 }
 // V codes by LDS DMA: copy i moves page j0 + i (positions 16i .. 16i + 15); lane L takes
 // position p = 16i + L / 4 and stores 16 bytes at 64p + 16(L % 4). The 16-byte segment it
@@ -760,12 +790,61 @@ __device__ __forceinline__ uint32_t widen2(uint32_t w, uint32_t sel) {
     return ((x & 0x00C000C0u) >> 2) | ((x & 0x00300030u) >> 4) | ((x & 0x0C000C00u) << 2) |
            (x & 0x03000300u);
 }
+// Eight 3-bit codes of the three bytes sel picks from (hi, lo), the first in the top bits of the
+// first byte, as four bytes of 4-bit codes, the first in the high nibble.
+__device__ __forceinline__ uint32_t widen3(uint32_t hi, uint32_t lo, uint32_t sel) {
+    uint32_t x = __builtin_amdgcn_perm(hi, lo, sel);          // 24 bits, the first code on top
+    x = ((x & 0x00FFF000u) << 4) | (x & 0x00000FFFu);         // 4 codes a half
+    x = ((x & 0x0FC00FC0u) << 2) | (x & 0x003F003Fu);         // 2 codes a byte
+    x = ((x & 0x38383838u) << 1) | (x & 0x07070707u);
+    return __builtin_amdgcn_perm(x, x, 0x00010203u);          // first byte lowest
+}
+// 32 codes of 2 or 3 bits (B words) as 4 words of 4-bit codes.
+template <int B, class Words>
+__device__ __forceinline__ u32x4 widen32(const Words& w) {
+    if constexpr (B == 2)
+        return u32x4{widen2(w[0], 0x01010000u), widen2(w[0], 0x03030202u), widen2(w[1], 0x01010000u),
+                     widen2(w[1], 0x03030202u)};
+    else  // bytes 3j .. 3j + 2 of the twelve, byte 3j on top
+        return u32x4{widen3(w[0], w[0], 0x0C000102u), widen3(w[1], w[0], 0x0C030405u),
+                     widen3(w[2], w[1], 0x0C020304u), widen3(w[2], w[2], 0x0C010203u)};
+}
 __device__ __forceinline__ void store_v2(const u32x2 (&r)[4], uint8_t* vb, int lane) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
         *(u32x4*)(vb + 1024 * i + 16 * lane) =
             u32x4{widen2(r[i][0], 0x01010000u), widen2(r[i][0], 0x03030202u),
                   widen2(r[i][1], 0x01010000u), widen2(r[i][1], 0x03030202u)};
+}
+
+// 3-bit V codes: the same with 12 bytes of rows of 48.
+struct V3Codes {
+    uint32_t w[4][3];
+};
+__device__ __forceinline__ void load_v3(const PageAddrs* pages, int j0, uint32_t voff, V3Codes& r) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint8_t* p = pages[j0 + i].v + voff;
+        const u32x2 v = *(g_u32x2_any*)p;
+        r.w[i][0] = v[0];
+        r.w[i][1] = v[1];
+        r.w[i][2] = *(g_u32_any*)(p + 8);
+    }
+}
+__device__ __forceinline__ void store_v3(const V3Codes& r, uint8_t* vb, int lane) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *(u32x4*)(vb + 1024 * i + 16 * lane) = widen32<3>(r.w[i]);
+}
+// 8-bit V codes: eight 16-byte loads of rows of 128 bytes, swizzled as v8_offset says.
+__device__ __forceinline__ void load_v8(const PageAddrs* pages, int j0, int kvh, int g, int lane,
+                                        u32x4 (&r)[8]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        r[i] = *(g_u32x4_any*)(pages[j0 + fhip_idx::v8_page(i)].v + fhip_idx::v8_offset(lane, i, kvh, g));
+}
+__device__ __forceinline__ void store_v8(const u32x4 (&r)[8], uint8_t* vb, int lane) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *(u32x4*)(vb + 1024 * i + 16 * lane) = r[i];
 }
 
 // Norms of position t0 + lane, loaded raw (fp16 bits): pack() gives (knorm, vnorm) in fp32
@@ -816,6 +895,34 @@ __device__ __forceinline__ void read_v_codes(const uint32_t (&seg)[4], v2i_t (&t
         : "memory");
 }
 
+// The same for 8-bit codes: dim tile c of position tiles 2 half, 2 half + 1; addr[c] is the lane's
+// address of segment c ^ swizzle of its row. ds_read_b64_tr_b8 gives lane n of each 16-lane group
+// byte n % 8 of source lanes 2 k + n / 8 (k = 0..7): word pt % 2 holds the four positions of tile pt.
+template <int kHalf>
+__device__ __forceinline__ void read_v_codes8(const uint32_t (&addr)[8], v2i_t (&tv)[8]) {
+#define FHIP_TR8(OFF)                                                                              \
+    asm volatile(                                                                                  \
+        "ds_read_b64_tr_b8 %0, %8" OFF "\n"                                                        \
+        "ds_read_b64_tr_b8 %1, %9" OFF "\n"                                                        \
+        "ds_read_b64_tr_b8 %2, %10" OFF "\n"                                                       \
+        "ds_read_b64_tr_b8 %3, %11" OFF "\n"                                                       \
+        "ds_read_b64_tr_b8 %4, %12" OFF "\n"                                                       \
+        "ds_read_b64_tr_b8 %5, %13" OFF "\n"                                                       \
+        "ds_read_b64_tr_b8 %6, %14" OFF "\n"                                                       \
+        "ds_read_b64_tr_b8 %7, %15" OFF "\n"                                                       \
+        "s_waitcnt lgkmcnt(0)"                                                                     \
+        : "=&v"(tv[0]), "=&v"(tv[1]), "=&v"(tv[2]), "=&v"(tv[3]), "=&v"(tv[4]), "=&v"(tv[5]),      \
+          "=&v"(tv[6]), "=&v"(tv[7])                                                               \
+        : "v"(addr[0]), "v"(addr[1]), "v"(addr[2]), "v"(addr[3]), "v"(addr[4]), "v"(addr[5]),      \
+          "v"(addr[6]), "v"(addr[7])                                                               \
+        : "memory")
+    if constexpr (kHalf == 0)
+        FHIP_TR8("");
+    else
+        FHIP_TR8(" offset:256");
+#undef FHIP_TR8
+}
+
 // kG4 score compaction: tile kPt's head-h score D[h] + 2^-12 D[8 + h] (MFMA columns h and 8 + h
 // of the lane's row) into lane 4 kPt + h, elements e = 0..3; the other banks keep theirs.
 template <int kPt>
@@ -839,31 +946,35 @@ __device__ __forceinline__ void expand_weights(uint32_t (&b)[4], const uint32_t 
     }
 }
 
-template <class Pages, bool kG4, bool kV2>
-__global__ __launch_bounds__(64 * kWavesM) __attribute__((amdgpu_waves_per_eu(3))) void
+// 8-bit codes hold twice the registers in flight, so two waves per SIMD instead of three.
+template <class Pages, bool kG4, int KB, int VB, int W>
+__global__ __launch_bounds__(64 * W)
+__attribute__((amdgpu_waves_per_eu(KB == 8 || VB == 8 ? 2 : 3))) void
 tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
                     const float* __restrict__ kcent, const float* __restrict__ vcent, int qh,
                     int kvh, float scale, float* __restrict__ part_ml,
                     float* __restrict__ part_acc, int nsplit, int nblk, int tok) {
     constexpr int hd = 128;
+    constexpr int kSwap = VB == 8 ? 0 : 1;  // element e of a dim tile holds dim e ^ kSwap
     // Code-byte tables: byte b -> the (c_hi | c_lo' << 16) words of its two codes, K as
     // {high nibble, low nibble} (the QK A operand's order), V as {low, high} (the PV B
     // operand's). One ds_read_b64 serves two codes: lookups at random entries of 2 KB tables
     // cost some bank conflicts, but half the LDS instructions and under half the address
     // arithmetic of per-code lookups in a 16-word table. The DMA
     // targets are separate objects: table reads never wait for DMA traffic.
-    __shared__ u32x2 pk[256], pv[256];
-    __shared__ __attribute__((aligned(16))) uint8_t vbuf[kWavesM][2][kChunkM * 64];  // by chunk parity
-    __shared__ __attribute__((aligned(16))) float2 nbuf[kWavesM][kChunkM];  // (knorm, vnorm)
-    __shared__ PageAddrs pagebuf[kWavesM][kSplitPages];  // the wave's split pages
+    __shared__ u32x2 pk[256], pv[256];  // 8-bit codes: 256 words, one per code
+    // two chunks of 4-bit V codes, by chunk parity, or one of 8-bit codes
+    __shared__ __attribute__((aligned(16))) uint8_t vbuf[W][2][kChunkM * 64];
+    __shared__ __attribute__((aligned(16))) float2 nbuf[W][kChunkM];  // (knorm, vnorm)
+    __shared__ PageAddrs pagebuf[W][kSplit / W / FHIP_PAGE_TOKENS];  // the wave's split pages
     __shared__ int waves_done;  // waves that have left their state for the merge
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, rg = lane >> 4;  // MFMA column / row group
     static_assert(kWavesM * kSplitMfma == kSplit, "a workgroup's splits make one partial's block");
 
-    // Workgroup (query, kv head, block of kWavesM consecutive splits); wave w takes split
-    // kWavesM * blk + w. Workgroups go to the 8 XCDs round-robin (workgroup b on XCD b % 8),
+    // Workgroup (query, kv head, block of W consecutive splits); wave w takes split
+    // W * blk + w. Workgroups go to the 8 XCDs round-robin (workgroup b on XCD b % 8),
     // and the kv heads of one token row share 128-byte lines, so the index puts every kv head
     // of one (query, block) item on the same XCD: item i = (query, block) and kv head g run
     // as workgroup (i / 8) (8 kvh) + 8 g + i % 8, and each line is filled into one L2 only.
@@ -881,19 +992,23 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     const int blk = (int)(item % nblk);
     const int clen = qs.causal_len(tq_last);  // the group's longest causal length
     if (blk * kSplit >= clen) return;
-    for (int b = threadIdx.x; b < 256; b += 64 * kWavesM) {
+    for (int b = threadIdx.x; b < 256; b += 64 * W) {
         float hf;
-        const uint32_t kh = hi_lo_pair(kcent[b >> 4], hf), kl = hi_lo_pair(kcent[b & 15], hf);
-        const int v0 = kV2 ? min(b >> 4, 3) : b >> 4, v1 = kV2 ? min(b & 15, 3) : b & 15;
-        const uint32_t vh = hi_lo_pair(vcent[v0], hf), vl = hi_lo_pair(vcent[v1], hf);
-        pk[b] = u32x2{kh, kl};
-        pv[b] = u32x2{vl, vh};
+        auto code = [](const float* cent, int c, int bits) { return cent[min(c, (1 << bits) - 1)]; };
+        if constexpr (KB == 8)
+            ((uint32_t*)pk)[b] = hi_lo_pair(kcent[b], hf);
+        else
+            pk[b] = u32x2{hi_lo_pair(code(kcent, b >> 4, KB), hf), hi_lo_pair(code(kcent, b & 15, KB), hf)};
+        if constexpr (VB == 8)
+            ((uint32_t*)pv)[b] = hi_lo_pair(vcent[b], hf);
+        else
+            pv[b] = u32x2{hi_lo_pair(code(vcent, b & 15, VB), hf), hi_lo_pair(code(vcent, b >> 4, VB), hf)};
         if (b == 0) waves_done = 0;
     }
     __syncthreads();
 
-    const int t_begin = fhip_idx::split_begin(blk, wave);
-    const int t_end = min(clen, t_begin + kSplitMfma);
+    const int t_begin = fhip_idx::split_begin(blk, wave, W);
+    const int t_end = min(clen, t_begin + kSplit / W);
     const int G = qh / kvh;
     const int32_t* table = qs.table + (int64_t)tq0 * qs.table_stride;
     uint8_t* vb = vbuf[wave][0];
@@ -915,23 +1030,36 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
 #pragma unroll
     for (int c = 0; c < 8; ++c) acc[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // The split's pages (at most kSplitPages), read once: the chunk loop then issues no memory
+    // The split's pages , read once: the chunk loop then issues no memory
     // instruction besides its loads and copies. A wave with no position to read (its split
     // starts past the end, or no page is in the pool) keeps the empty state.
     PageAddrs* pages = pagebuf[wave];
-    const uint64_t vmask = t_begin < clen ? split_pages(pg, table, t_begin, t_end, lane, pages) : 0;
+    const uint64_t vmask = t_begin < clen ? split_pages<kSplit / W / FHIP_PAGE_TOKENS>(pg, table, t_begin, t_end, lane, pages) : 0;
     if (vmask != 0) {
     // first chunk's copies go out before the Q set-up
-    const uint32_t v_lane_off = kV2 ? fhip_idx::v2_offset(lane, kvh, g) : fhip_idx::v_offset(lane, kvh, g);
+    const uint32_t v_lane_off = VB == 2   ? fhip_idx::v2_offset(lane, kvh, g)
+                                : VB == 3 ? fhip_idx::v3_offset(lane, kvh, g)
+                                          : fhip_idx::v_offset(lane, kvh, g);
     uint32_t pmask = (uint32_t)vmask & 0xfu;  // pages of the current chunk to read
-    u32x2 v2reg[kV2 ? 4 : 1];  // kV2: the next chunk's V codes, widened into LDS when it starts
-    if constexpr (kV2)
-        load_v2(pages, 0, v_lane_off, v2reg);
-    else
-        dma_v(pages, 0, v_lane_off, vb, lane);  // chunk 0: buffer 0
+    // the next chunk's V codes where they go through registers into LDS when it starts (all
+    // widths but 4)
+    u32x2 v2reg[VB == 2 ? 4 : 1];
+    V3Codes v3reg;
+    u32x4 v8reg[VB == 8 ? 8 : 1];
+    auto load_v = [&](int j0, uint8_t* dst) {
+        if constexpr (VB == 2)
+            load_v2(pages, j0, v_lane_off, v2reg);
+        else if constexpr (VB == 3)
+            load_v3(pages, j0, v_lane_off, v3reg);
+        else if constexpr (VB == 8)
+            load_v8(pages, j0, kvh, g, lane, v8reg);
+        else
+            dma_v(pages, j0, v_lane_off, dst, lane);
+    };
+    load_v(0, vb);  // chunk 0: buffer 0
     NormRegs nreg = load_norms(pages, 0, pmask, t_begin, t_end, kvh, g, lane);
-    u32x4 kreg[4];
-    load_k(pages, 0, kvh, g, lane, kreg);
+    KCodes<KB> kreg;
+    load_k<KB>(pages, 0, kvh, g, lane, kreg);
 
     // Q as the QK B operand, pre-scaled by scale * log2(e) so scores come out in log2 units:
     // step s, lane (n, rg) holds coordinates 32rg + 4s + c4.
@@ -970,14 +1098,21 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
         return __int_as_float(__builtin_amdgcn_ds_bpermute(bp, __float_as_int(v)));
     };
     // transposed V reads: source lane m of group rg reads position 16rg + 4(m % 4) + m / 4;
-    // segment s of that row sits at vrow[s ^ sw]
-    const int srow = 16 * rg + 4 * (n & 3) + (n >> 2);
-    const int sw = (srow >> 1) & 3;
-    uint32_t vseg[4];
+    // segment s of that row sits at vrow[s ^ sw]. 8-bit codes: lane m reads half m % 2 of the
+    // 16 dims of a tile at position 16rg + 4(k % 4) + k / 4 (+ 2 for tiles 2, 3), k = m / 2.
+    uint32_t vseg[VB == 8 ? 8 : 4];
+    const uint32_t vb32 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)vb;
+    if constexpr (VB == 8) {
+        const int k = n >> 1, srow = 16 * rg + 4 * (k & 3) + (k >> 2);
 #pragma unroll
-    for (int sg = 0; sg < 4; ++sg)
-        vseg[sg] = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)(
-            vb + 64 * srow + 16 * (sg ^ sw));
+        for (int c = 0; c < 8; ++c)
+            vseg[c] = vb32 + 128 * srow + 16 * (c ^ fhip_idx::v8_swizzle(srow)) + 8 * (n & 1);
+    } else {
+        const int srow = 16 * rg + 4 * (n & 3) + (n >> 2);
+        const int sw = (srow >> 1) & 3;
+#pragma unroll
+        for (int sg = 0; sg < 4; ++sg) vseg[sg] = vb32 + 64 * srow + 16 * (sg ^ sw);
+    }
 
     // kG4 (at most 4 query heads per kv head): scores, probabilities and weights are held
     // compactly, lane (n, rg) with n = 4 pt + h holding head h's 4 positions 16rg + 4e + pt of
@@ -1003,16 +1138,32 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         // the V buffer PV reads below (the sync after the norm records orders these writes
         // before the transposed reads)
-        if constexpr (kV2) store_v2(v2reg, vb + par * (kChunkM * 64), lane);
-        const u32x4 kcs[4] = {kreg[0], kreg[1], kreg[2], kreg[3]};
+        if constexpr (VB == 2) store_v2(v2reg, vb + par * (kChunkM * 64), lane);
+        if constexpr (VB == 3) store_v3(v3reg, vb + par * (kChunkM * 64), lane);
+        if constexpr (VB == 8) store_v8(v8reg, vb, lane);
+        u32x4 kcs[4][KB == 8 ? 2 : 1];
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt) {
+            if constexpr (KB == 2 || KB == 3) {
+                kcs[pt][0] = widen32<KB>(kreg.w[pt][0]);
+            } else {
+#pragma unroll
+                for (int k = 0; k < KB / 4; ++k) kcs[pt][k] = kreg.w[pt][k];
+            }
+        }
         // 32 MFMA steps t = (tile pt, word s2, half): the A operand of step t holds the table
-        // entries of bytes 2 half, 2 half + 1 of word s2 (coordinates 8 s2 + 4 half + 0..3).
+        // entries of bytes 2 half, 2 half + 1 of word s2 (coordinates 8 s2 + 4 half + 0..3; 8-bit
+        // codes: of word t % 8).
         // Table reads run kLookAhead steps ahead of their MFMA, so their LDS latency is
         // covered by the MFMAs in between.
         constexpr int kLookAhead = 2;
         auto qk_a = [&](int t) -> u32x4 {
-            const uint32_t w = kcs[t >> 3][(t >> 1) & 3];
-            return (t & 1) ? pair2<2>(pk, w) : pair2<0>(pk, w);
+            if constexpr (KB == 8) {
+                return quad8((const uint32_t*)pk, kcs[t >> 3][(t & 7) >> 2][t & 3]);
+            } else {
+                const uint32_t w = kcs[t >> 3][0][(t >> 1) & 3];
+                return (t & 1) ? pair2<2>(pk, w) : pair2<0>(pk, w);
+            }
         };
         {
             u32x4 ahead[kLookAhead + 1];
@@ -1062,12 +1213,9 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
         wave_lds_sync();
         uint8_t* vnext = vb + (par ^ 1) * (kChunkM * 64);
         if (tn < t_end) {
-            if constexpr (kV2)
-                load_v2(pages, jn, v_lane_off, v2reg);
-            else
-                dma_v(pages, jn, v_lane_off, vnext, lane);
+            load_v(jn, vnext);
             nreg = load_norms(pages, jn, pmask_n, tn, t_end, kvh, g, lane);
-            load_k(pages, jn, kvh, g, lane, kreg);
+            load_k<KB>(pages, jn, kvh, g, lane, kreg);
         }
         float m_new, alpha;
         uint32_t aw[4][4];  // !kG4 [pt][e]
@@ -1178,7 +1326,9 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
 
         // ---- PV: 8 dim tiles x 4 position tiles
         v2i_t tvs[8];
-        {
+        if constexpr (VB == 8) {
+            read_v_codes8<0>(vseg, tvs);
+        } else {
             const uint32_t vo = (uint32_t)par * (kChunkM * 64);
             const uint32_t seg[4] = {vseg[0] + vo, vseg[1] + vo, vseg[2] + vo, vseg[3] + vo};
             read_v_codes(seg, tvs);
@@ -1186,12 +1336,18 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
         // out^T = V^T W^T: the V entries are the A operand (row m: dim 16c + (m ^ 1)), the
         // weights the B operand (column n: head slot n). 32 MFMA steps t = (position tile pt,
         // dim tile c): nibble 4pt + c4 of dim tile c's transposed read is the code of position
-        // (pt, c4) at dim 16c + (n ^ 1); tile pt sits in word pt / 2, bytes 2 (pt % 2),
+        // (pt, c4) at dim 16c + (n ^ 1) (8-bit codes: a byte, at dim 16c + n); tile pt sits in word pt / 2, bytes 2 (pt % 2),
         // 2 (pt % 2) + 1. Table reads run kLookAhead steps ahead as in QK.
         auto pv_b = [&](int t) -> u32x4 {
             const int pt = t >> 3, c = t & 7;
-            const uint32_t w = (uint32_t)tvs[c][pt >> 1];
-            return (pt & 1) ? pair2<2>(pv, w) : pair2<0>(pv, w);
+            if constexpr (VB == 8) {
+                // the codes of tiles 2, 3 are read once tiles 0, 1 have used theirs
+                if (t == 16) read_v_codes8<1>(vseg, tvs);
+                return quad8((const uint32_t*)pv, (uint32_t)tvs[c][pt & 1]);
+            } else {
+                const uint32_t w = (uint32_t)tvs[c][pt >> 1];
+                return (pt & 1) ? pair2<2>(pv, w) : pair2<0>(pv, w);
+            }
         };
         {
             constexpr int kAheadPv = kLookAhead;
@@ -1239,13 +1395,13 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     // 16c + 4rg + 0..3 (element e holds dim e ^ 1), one 16-byte store.
     constexpr int kStRow = hd + 16;
     constexpr int kStM = kMaxG * kStRow, kStL = kStM + kMaxG;
-    float* st = (float*)vbuf[wave][0];
+    float* st = (float*)vb;
     static_assert(sizeof(vbuf[0]) >= (kStL + kMaxG) * sizeof(float), "merge state");
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         f32x4_t v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e ^ 1] = fmaf(ror8(acc[c][e]), 1.0f / 4096.0f, acc[c][e]);
+        for (int e = 0; e < 4; ++e) v[e ^ kSwap] = fmaf(ror8(acc[c][e]), 1.0f / 4096.0f, acc[c][e]);
         if (n < ncols) *(f32x4_t*)&st[n * kStRow + 16 * c + 4 * rg] = v;
     }
     if (n < ncols && rg == 0) {
@@ -1258,7 +1414,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     int arrived = 0;
     if (lane == 0) arrived = atomicAdd(&waves_done, 1);
     arrived = __builtin_amdgcn_readfirstlane(arrived);
-    if (arrived != kWavesM - 1) return;
+    if (arrived != W - 1) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     // one (head, 8-coordinate group) per lane and step: the head's wave weights once, then two
     // 16-byte reads per wave state and two 16-byte stores
@@ -1267,16 +1423,16 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
         if (tq0 + h / G >= qs.seq_lens_count) continue;  // a column past the queries
         const int64_t vec = fhip_idx::partial_vector(h, tq0, G, qh, g);
         const int64_t prow = fhip_idx::partial_row(vec, nsplit, blk);
-        float mw[kWavesM], M = -__builtin_inff();
+        float mw[W], M = -__builtin_inff();
 #pragma unroll
-        for (int w = 0; w < kWavesM; ++w) {
+        for (int w = 0; w < W; ++w) {
             mw[w] = ((const float*)vbuf[w][0])[kStM + h];
             M = fmaxf(M, mw[w]);
         }
         float L = 0.0f;
         f32x4_t A0 = {0.0f, 0.0f, 0.0f, 0.0f}, A1 = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int w = 0; w < kWavesM; ++w) {
+        for (int w = 0; w < W; ++w) {
             const float* sw = (const float*)vbuf[w][0];
             if (mw[w] != -__builtin_inff()) {
                 const float wt = __builtin_amdgcn_exp2f(mw[w] - M);
@@ -1300,10 +1456,39 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     }
 }
 
+// Eight waves per block up to this many workgroups, two beyond (32 / 8 heads, K4/V2: one sequence
+// of 4000, 32 workgroups: 38 -> 29 us; 16 sequences of 2000 .. 8000 at 8 heads a group, 512
+// workgroups: 53 -> 46; 64 of 500 .. 2000, 1024 workgroups: 53 with two, 58 with eight). 8-bit codes
+// keep twice the registers and buffers a wave: at 512 workgroups 50 us with two, 52 with eight.
+constexpr int64_t kWideGroups = 512, kWideGroups8 = 256;
+
+// The (K, V) code widths that the MFMA kernel is built for: the default cache, equal widths, and the
+// protected layers' 8 bits. On the VALU split kernel, which takes any other pair, 8 sequences of 1000
+// .. 8000 measured 438 us at 8 bits, 200 at 3 and 191 at 2, against 50, 43 and 44 here.
+bool mfma_widths(int kbits, int vbits) {
+    return (kbits == 4 && (vbits == 4 || vbits == 2)) ||
+           (kbits == vbits && (kbits == 2 || kbits == 3 || kbits == 8));
+}
+
+template <class Pages, int KB, int VB>
+void launch_mfma_t(const float* qrot, const Queries& q2, const Pages& pg, const float* kcent,
+                   const float* vcent, int qh, int kvh, int nsplit, int tok, int64_t wgs, float* ml,
+                   float* acc, hipStream_t s) {
+    const bool g4 = qh / kvh <= 4 && tok == 1;
+    const bool wide = wgs <= (KB == 8 ? kWideGroups8 : kWideGroups);
+    auto kern = g4 ? (wide ? tq_attn_mfma_kernel<Pages, true, KB, VB, kWavesWide>
+                           : tq_attn_mfma_kernel<Pages, true, KB, VB, kWavesM>)
+                   : (wide ? tq_attn_mfma_kernel<Pages, false, KB, VB, kWavesWide>
+                           : tq_attn_mfma_kernel<Pages, false, KB, VB, kWavesM>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * (wide ? kWavesWide : kWavesM)), 0, s, qrot,
+                       q2, pg, kcent, vcent, qh, kvh, 1.0f / sqrtf(128.0f), ml, acc, nsplit, nsplit,
+                       tok);
+}
+
 template <class Pages>
 void launch_mfma_split(const float* qrot, const Queries& qsv, const Pages& pg,
                        const float* kcent, const float* vcent, int nq, int qh, int kvh,
-                       int nsplit, bool v2, float* ml, float* acc, hipStream_t s) {
+                       int nsplit, int kbits, int vbits, float* ml, float* acc, hipStream_t s) {
     // Causal prefill (queries at consecutive positions of one sequence: one shared block table,
     // lengths from start_pos) groups 8 / G consecutive queries per item so that they share the
     // MFMA columns and every code lookup; decode keeps one query per item.
@@ -1316,11 +1501,16 @@ void launch_mfma_split(const float* qrot, const Queries& qsv, const Pages& pg,
     const int64_t wgs = ceil_div(items * nsplit, kXcds) * kXcds * kvh;
     Queries q2 = qsv;
     q2.seq_lens_count = nq;
-    const bool g4 = G <= 4 && tok == 1;
-    auto kern = v2 ? (g4 ? tq_attn_mfma_kernel<Pages, true, true> : tq_attn_mfma_kernel<Pages, false, true>)
-                   : (g4 ? tq_attn_mfma_kernel<Pages, true, false> : tq_attn_mfma_kernel<Pages, false, false>);
-    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * kWavesM), 0, s, qrot, q2, pg, kcent,
-                       vcent, qh, kvh, 1.0f / sqrtf(128.0f), ml, acc, nsplit, nsplit, tok);
+    if (kbits == 8)
+        launch_mfma_t<Pages, 8, 8>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+    else if (kbits == 3)
+        launch_mfma_t<Pages, 3, 3>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+    else if (kbits == 2)
+        launch_mfma_t<Pages, 2, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+    else if (vbits == 2)
+        launch_mfma_t<Pages, 4, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+    else
+        launch_mfma_t<Pages, 4, 4>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
 }
 
 struct AttnArgs {
@@ -1380,9 +1570,9 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
         hipLaunchKernelGGL(tq_attn_prerotate_kernel, dim3(rot_groups), dim3(256), 0, s,
                            (const uint16_t*)a.q, a.krot, qrot, a.hd, nvec);
     }
-    if (a.kbits == 4 && (a.vbits == 4 || a.vbits == 2) && a.hd == 128 && a.qh / a.kvh <= 8)
-        launch_mfma_split(qrot, a.qs, pg, a.kcent, a.vcent, a.nq, a.qh, a.kvh, nsplit,
-                          a.vbits == 2, ml, acc, s);
+    if (mfma_widths(a.kbits, a.vbits) && a.hd == 128 && a.qh / a.kvh <= 8)
+        launch_mfma_split(qrot, a.qs, pg, a.kcent, a.vcent, a.nq, a.qh, a.kvh, nsplit, a.kbits,
+                          a.vbits, ml, acc, s);
     else if (a.kbits == 4 && a.vbits == 4)
         launch_split<4, 4>(a, pg, nsplit, ml, acc, s);
     else if (a.kbits == 4 && a.vbits == 2)

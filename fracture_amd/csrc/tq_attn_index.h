@@ -1,9 +1,9 @@
-// Index arithmetic of the MFMA decode-attention kernel (tq_attn_mfma_kernel, head_dim 128,
-// 4-bit K codes, 4- or 2-bit V codes), shared by the kernel and by a host build of the functions
+// Index arithmetic of the MFMA decode-attention kernel (tq_attn_mfma_kernel, head_dim 128, K and V
+// codes of 2, 3, 4 or 8 bits), shared by the kernel and by a host build of the functions
 // (tq_attn_index_host.cpp). The CPU bounds check of every global access the kernel makes
 // calls the host build, so it covers the arithmetic the kernel runs rather than a restatement
 // of it. Page layout (quantized_paged_kv_cache.rs:86-128): a page holds 16 positions; its K
-// codes are [16][kvh][64] bytes, its K norms [16][kvh] fp16, and the same for V.
+// codes are [16][kvh][16 bits] bytes (64 at 4 bits), its K norms [16][kvh] fp16, and the same for V.
 #pragma once
 #include <stdint.h>
 
@@ -57,6 +57,11 @@ FHIP_IDX void split_grid_item(int64_t lin, int64_t total, int nsplit, int kvh, i
 // First position of wave `wave`'s split in block blk.
 FHIP_IDX int split_begin(int blk, int wave) { return (kBlockWaves * blk + wave) * kSplitPositions; }
 
+// The same with `waves` waves per workgroup (2, 4 or 8) sharing the block.
+FHIP_IDX int split_begin(int blk, int wave, int waves) {
+    return (blk * waves + wave) * (kBlockWaves * kSplitPositions / waves);
+}
+
 // Lane j of a wave reads the block-table column of its split's page j, if that page holds
 // positions of the split [t_begin, t_end).
 FHIP_IDX bool split_page_column(int t_begin, int t_end, int lane, int& column) {
@@ -75,6 +80,11 @@ FHIP_IDX uint32_t k_offset(int lane, int kvh, int g) {
     return (uint32_t)((4 * ((lane & 15) & 3) * kvh + g) * kCodeRow + 16 * (lane >> 4));
 }
 FHIP_IDX uint32_t k_tile_stride(int kvh) { return (uint32_t)(kvh * kCodeRow); }
+// The same for rows of `bits`-bit codes: 4 bits bytes (32 codes) at 4 bits rg of the row.
+FHIP_IDX uint32_t k_offset(int lane, int kvh, int g, int bits) {
+    return (uint32_t)((4 * ((lane & 15) & 3) * kvh + g) * 16 * bits + 4 * bits * (lane >> 4));
+}
+FHIP_IDX uint32_t k_tile_stride(int kvh, int bits) { return (uint32_t)(kvh * 16 * bits); }
 
 // V codes of a chunk by LDS DMA: copy i (0..3) moves split page chunk_first_page + i; lane L
 // copies position L / 4 of that page, 16-byte segment (L % 4) ^ ((L / 8) % 4) of kv head g's
@@ -86,6 +96,21 @@ FHIP_IDX uint32_t v_offset(int lane, int kvh, int g) {
 // the codes of the 16-byte segment v_offset names, and widens them to it.
 FHIP_IDX uint32_t v2_offset(int lane, int kvh, int g) {
     return (uint32_t)(((lane >> 2) * kvh + g) * (kCodeRow / 2) + 8 * ((lane & 3) ^ ((lane >> 3) & 3)));
+}
+
+// The same with 3-bit codes: 12 bytes of a 48-byte row.
+FHIP_IDX uint32_t v3_offset(int lane, int kvh, int g) {
+    return (uint32_t)(((lane >> 2) * kvh + g) * 48 + 12 * ((lane & 3) ^ ((lane >> 3) & 3)));
+}
+// 8-bit V codes: load i (0..7) reads split page chunk_first_page + i / 2; lane L takes chunk
+// position 8 i + L / 8, 16-byte segment (L % 8) ^ v8_swizzle(position) of its 128-byte row, and
+// stores it at 16 (64 i + L) of the wave's LDS buffer. The swizzle gives the 32 rows that one
+// transposed read touches all eight segments.
+FHIP_IDX int v8_swizzle(int pos) { return ((pos >> 2) & 3) | (((pos >> 4) & 1) << 2); }
+FHIP_IDX int v8_page(int i) { return i >> 1; }
+FHIP_IDX uint32_t v8_offset(int lane, int i, int kvh, int g) {
+    const int pos = 8 * i + (lane >> 3);
+    return (uint32_t)(((pos & 15) * kvh + g) * 128 + 16 * ((lane & 7) ^ v8_swizzle(pos)));
 }
 
 // Norms of a chunk: lane L reads split page chunk_first_page + norm_page(L), the fp16 norm of

@@ -33,6 +33,36 @@ int fhip_idx_v2_offsets(int kvh, int g, uint32_t* v2_off) {
     return 0;
 }
 
+// Codes of 2, 3, 4 or 8 bits: K offsets k_off[pt][lane] (pt = 0..3) and V load offsets
+// v_off[i][lane] with their split page slots v_page[i] (i < 4, or i < 8 at 8 bits); kw and vw are
+// the bytes of one K and one V load.
+int fhip_idx_code_tables(int kvh, int g, int kbits, int vbits, uint32_t* k_off, uint32_t* v_off,
+                         int32_t* v_page, int32_t* kw, int32_t* vw) {
+    if (kvh < 1 || g < 0 || g >= kvh || !k_off || !v_off || !v_page || !kw || !vw) return -1;
+    if ((kbits != 2 && kbits != 3 && kbits != 4 && kbits != 8) ||
+        (vbits != 2 && vbits != 3 && vbits != 4 && vbits != 8))
+        return -1;
+    *kw = 4 * kbits;
+    *vw = vbits == 8 ? 16 : 4 * vbits;
+    for (int lane = 0; lane < 64; ++lane) {
+        for (int pt = 0; pt < 4; ++pt)
+            k_off[pt * 64 + lane] =
+                fhip_idx::k_offset(lane, kvh, g, kbits) + pt * fhip_idx::k_tile_stride(kvh, kbits);
+        for (int i = 0; i < (vbits == 8 ? 8 : 4); ++i)
+            v_off[i * 64 + lane] = vbits == 8   ? fhip_idx::v8_offset(lane, i, kvh, g)
+                                   : vbits == 4 ? fhip_idx::v_offset(lane, kvh, g)
+                                   : vbits == 3 ? fhip_idx::v3_offset(lane, kvh, g)
+                                                : fhip_idx::v2_offset(lane, kvh, g);
+    }
+    for (int i = 0; i < 8; ++i) v_page[i] = vbits == 8 ? fhip_idx::v8_page(i) : i;
+    return 0;
+}
+
+// First position of wave `wave` of `waves` in block blk.
+int32_t fhip_idx_split_begin(int blk, int wave, int waves) {
+    return fhip_idx::split_begin(blk, wave, waves);
+}
+
 // Workgroup wg of a launch with kvh kv heads -> its item and kv head.
 int fhip_idx_wg_item(int64_t wg, int kvh, int64_t* item, int32_t* g) {
     if (kvh < 1 || wg < 0 || !item || !g) return -1;

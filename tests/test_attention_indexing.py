@@ -388,3 +388,75 @@ def test_split_grid_item_covers_grid_and_balances_xcds():
     assert load.sum() == naive.sum()
     assert load.max() / load.mean() < 1.05, load / load.mean()
     assert naive.max() / naive.mean() > 1.20, naive / naive.mean()
+
+
+WIDTHS = [(4, 4), (4, 2), (8, 8), (3, 3), (2, 2)]
+
+
+@pytest.mark.parametrize("kbits,vbits", WIDTHS)
+@pytest.mark.parametrize("kvh", [1, 3, 8])
+def test_code_loads_cover_each_page_once(kbits, vbits, kvh):
+    """The K and V code loads of one chunk (4 pages) at each width the MFMA kernel takes: every byte
+    of every position's row of kv head g is read exactly once, and nothing else."""
+    import ctypes as C
+    L = index_lib().lib
+    for g in range(kvh):
+        k_off, v_off = np.zeros((4, 64), np.uint32), np.zeros((8, 64), np.uint32)
+        v_page, kw, vw = np.zeros(8, np.int32), C.c_int32(), C.c_int32()
+        assert L.fhip_idx_code_tables(kvh, g, kbits, vbits, k_off.ctypes.data_as(C.c_void_p),
+                                      v_off.ctypes.data_as(C.c_void_p), v_page.ctypes.data_as(C.c_void_p),
+                                      C.byref(kw), C.byref(vw)) == 0
+        for bits, width, loads in (
+                (kbits, kw.value, [(p, (np.arange(64) & 15) >> 2, k_off[p]) for p in range(4)]),
+                (vbits, vw.value, [(i, np.full(64, v_page[i]), v_off[i])
+                                   for i in range(8 if vbits == 8 else 4)])):
+            row = 16 * bits
+            seen = np.zeros((4, PAGE, kvh, row), np.int32)
+            flat = seen.reshape(4, -1)
+            for _, page, off in loads:
+                for lane in range(64):
+                    flat[page[lane], off[lane]:off[lane] + width] += 1
+            assert (seen[:, :, g] == 1).all()
+            assert seen.sum() == 4 * PAGE * row
+
+
+def test_transposed_reads_of_8_bit_codes():
+    """The LDS image of a chunk's 8-bit V codes (stored as v8_offset loads them) read back by the
+    transposed reads' addresses: tile c, half r, lane (n, rg) must get, in byte k, dim 16 c + n of
+    position 16 rg + 4 (k % 4) + 2 r + k / 4."""
+    import ctypes as C
+    L = index_lib().lib
+    k_off, v_off = np.zeros((4, 64), np.uint32), np.zeros((8, 64), np.uint32)
+    v_page, kw, vw = np.zeros(8, np.int32), C.c_int32(), C.c_int32()
+    assert L.fhip_idx_code_tables(1, 0, 8, 8, k_off.ctypes.data_as(C.c_void_p),
+                                  v_off.ctypes.data_as(C.c_void_p), v_page.ctypes.data_as(C.c_void_p),
+                                  C.byref(kw), C.byref(vw)) == 0
+    pages = np.arange(64 * 128).reshape(4, 16 * 128)  # value = position * 128 + dim
+    lds = np.full(64 * 128, -1)
+    for i in range(8):
+        for lane in range(64):
+            lds[1024 * i + 16 * lane:1024 * i + 16 * lane + 16] = \
+                pages[v_page[i], v_off[i, lane]:v_off[i, lane] + 16]
+    assert (np.sort(lds) == np.arange(64 * 128)).all()
+    for c in range(8):
+        for r in range(2):
+            for rg in range(4):
+                src = []
+                for m in range(16):  # source lane m reads 8 bytes
+                    k = m >> 1
+                    row = 16 * rg + 4 * (k & 3) + (k >> 2)
+                    sw = ((row >> 2) & 3) | (((row >> 4) & 1) << 2)
+                    a = 128 * row + 16 * (c ^ sw) + 8 * (m & 1) + 256 * r
+                    src.append(lds[a:a + 8])
+                for n in range(16):
+                    for k in range(8):  # the read's own exchange: byte n % 8 of lane 2 k + n / 8
+                        got = src[2 * k + n // 8][n % 8]
+                        pos = 16 * rg + 4 * (k % 4) + 2 * r + k // 4
+                        assert got == pos * 128 + 16 * c + n
+
+
+@pytest.mark.parametrize("waves", [2, 8])
+def test_split_begin_tiles_the_block(waves):
+    L = index_lib().lib
+    begins = [L.fhip_idx_split_begin(3, w, waves) for w in range(waves)]
+    assert begins == [3 * SPLIT + w * (SPLIT // waves) for w in range(waves)]

@@ -135,3 +135,69 @@ def test_reference_interface_prefill_causal(dev):
                                    pool["VP"], pool["VN"], pool["krot"], pool["vrot"],
                                    pool["kc"], pool["vc"], kbits, vbits, kvh)
         assert_close(got[t].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3, f"token {t}")
+
+
+@pytest.mark.parametrize("kbits,vbits", [(8, 8), (3, 3), (2, 2), (4, 2), (4, 4)])
+@pytest.mark.parametrize("qh,kvh,reps", [(8, 2, 1), (8, 1, 1), (16, 8, 13)])
+def test_decode_widths_and_waves(dev, kbits, vbits, qh, kvh, reps):
+    """Every width pair of the MFMA kernel, at up to 4 and up to 8 q heads per kv head, eight waves
+    per block (small launches) and two (13 x 5 sequences over 8 kv heads): lengths on the edges of
+    chunks, of the waves' splits and of pages, a masked page, an empty sequence."""
+    rng = np.random.default_rng(kbits * 10 + vbits + qh)
+    hd = 128
+    lens = ([1, 65, 128, 0, 300] if reps > 1 else [1, 63, 64, 65, 127, 129, 511, 513, 0, 1023, 1025])
+    pool = build_pool(rng, lens, kvh, hd, kbits, vbits)
+    pool["table"][2, 1] = -1  # the third sequence (of 128 or 64): positions 16..31 masked
+    table, lens = np.tile(pool["table"], (reps, 1)), lens * reps
+    q = rng.standard_normal((len(lens), qh, hd)).astype(np.float16)
+    out = torch.empty(q.shape, dtype=torch.float16, device=dev)
+    K.attention_tq_decode(out, dev_t(q, dev), dev_t(table, dev), dev_t(np.array(lens, np.int32), dev),
+                          *(dev_t(pool[n], dev) for n in ("KP", "KN", "VP", "VN", "krot", "vrot", "kc", "vc")),
+                          kbits, vbits, kvh)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    for b, n in enumerate(lens):
+        rows = table[b]
+        if n == 0:
+            assert not got[b].any()
+            continue
+        if rows[1] == -1 and n > 32:
+            rows, n = np.delete(rows, 1), n - 16
+        want = oracle.tq_attention(q[b], rows, n, pool["KP"], pool["KN"], pool["VP"], pool["VN"],
+                                   pool["krot"], pool["vrot"], pool["kc"], pool["vc"], kbits, vbits, kvh)
+        assert_close(got[b].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3, f"seq {b} len {n}")
+
+
+@pytest.mark.parametrize("bits", [8, 3, 2])
+def test_code_pages_at_odd_addresses(dev, bits):
+    """Code pages that start at any byte (the widths other than 4 assume no alignment), through the
+    per-block pointer arrays."""
+    rng = np.random.default_rng(bits)
+    qh, kvh, hd, n = 4, 2, 128, 100
+    pool = build_pool(rng, [n], kvh, hd, bits, bits)
+    P = pool["KP"].shape[0]
+    held, ptrs = [], []
+    for name in ("KP", "KN", "VP", "VN"):
+        t = []
+        for i in range(P):
+            raw = np.ascontiguousarray(pool[name][i]).view(np.uint8).ravel()
+            buf = torch.zeros(raw.size + 16, dtype=torch.uint8, device=dev)
+            off = (2 * i + 1) % 16 if name in ("KP", "VP") else 0
+            buf[off:off + raw.size] = torch.from_numpy(raw.copy()).to(dev)
+            held.append(buf)
+            t.append(buf.data_ptr() + off)
+        ptrs.append(torch.tensor(t, dtype=torch.int64, device=dev))
+    q = rng.standard_normal((1, qh, hd)).astype(np.float16)
+    tq_, table = dev_t(q, dev), dev_t(pool["table"][0], dev)
+    tabs = [dev_t(pool[x], dev) for x in ("krot", "vrot", "kc", "vc")]
+    out = torch.empty_like(tq_)
+    pd = oracle.packed_dim(hd, bits)
+    code = K._L().fhip_launch_attention_paged_tq(
+        out.data_ptr(), tq_.data_ptr(), table.data_ptr(), *(p.data_ptr() for p in ptrs),
+        *(t.data_ptr() for t in tabs), 1, qh, kvh, hd, n, n - 1, bits, bits, pd, pd,
+        torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    torch.cuda.synchronize()
+    want = oracle.tq_attention(q[0], pool["table"][0], n, pool["KP"], pool["KN"], pool["VP"], pool["VN"],
+                               pool["krot"], pool["vrot"], pool["kc"], pool["vc"], bits, bits, kvh)
+    assert_close(out.cpu().numpy()[0].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3)
