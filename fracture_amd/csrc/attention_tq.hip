@@ -14,6 +14,9 @@
 //   1. q_rot = Pi_k q                  (per query head)
 //   2. split partials                  (the HBM stream over the pages)
 //   3. merge + unrotate -> fp16 output
+#include <algorithm>
+#include <type_traits>
+
 #include "fhip_internal.h"
 #include "tq_attn_index.h"
 #include "tq_quant.h"
@@ -23,6 +26,8 @@ using namespace fhip;
 namespace {
 
 constexpr int kSplit = 1024;   // positions per split workgroup
+constexpr int kFinePart = 256; // and in launches too small to fill the chip with those
+constexpr size_t kFineBytes = (size_t)24 << 20;  // the largest workspace that finer splits may ask for
 constexpr int kSub = 256;      // positions per pass (one per lane in the score phase)
 constexpr int kMaxG = 8;       // q heads per kv head
 constexpr int kMaxHd = 256;
@@ -390,12 +395,12 @@ size_t combine_lds_bytes(int hd, int nsplit, bool merge_only = false) {
 constexpr int kMergeWaveMaxSplits = 8;
 __global__ __launch_bounds__(256) void tq_attn_merge_wave_kernel(
     Queries qs, const float* __restrict__ part_ml, const float* __restrict__ part_acc, int qh,
-    int hd, int nsplit, int64_t nvec, float* __restrict__ merged) {
+    int hd, int nsplit, int64_t nvec, float* __restrict__ merged, int split_pos) {
     const int lane = threadIdx.x & 63;
     const int64_t vec = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (vec >= nvec) return;
     const int clen = qs.causal_len((int)(vec / qh));
-    const int ns = (clen + kSplit - 1) / kSplit;  // <= nsplit <= kMergeWaveMaxSplits
+    const int ns = (clen + split_pos - 1) / split_pos;  // <= nsplit <= kMergeWaveMaxSplits
     const float* ml = part_ml + vec * nsplit * 2;
     const float ms = lane < ns ? ml[2 * lane] : -__builtin_inff();
     const float ls = lane < ns ? ml[2 * lane + 1] : 0.0f;
@@ -424,7 +429,7 @@ template <bool kRotLds, bool kMergeOnly = false>
 __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
     Queries qs, const float* __restrict__ part_ml, const float* __restrict__ part_acc,
     const float* __restrict__ vrot, uint16_t* __restrict__ out, int qh, int hd, int nsplit,
-    int64_t nvec, float* __restrict__ merged = nullptr) {
+    int64_t nvec, float* __restrict__ merged, int split_pos) {
     __shared__ float o[kCombHeads][kMaxHd];
     __shared__ float linv[kCombHeads];
     __shared__ int nsv[kCombHeads];
@@ -452,7 +457,7 @@ __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
         int ns = 0;
         if (mine && head < nvec) {
             const int clen = qs.causal_len((int)(head / qh));
-            ns = (clen + kSplit - 1) / kSplit;
+            ns = (clen + split_pos - 1) / split_pos;
         }
         const float* ml = part_ml + head * nsplit * 2;
         float M = -__builtin_inff();
@@ -947,7 +952,7 @@ __device__ __forceinline__ void expand_weights(uint32_t (&b)[4], const uint32_t 
 }
 
 // 8-bit codes hold twice the registers in flight, so two waves per SIMD instead of three.
-template <class Pages, bool kG4, int KB, int VB, int W>
+template <class Pages, bool kG4, int KB, int VB, int W, int kPart>
 __global__ __launch_bounds__(64 * W)
 __attribute__((amdgpu_waves_per_eu(KB == 8 || VB == 8 ? 2 : 3))) void
 tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
@@ -966,12 +971,13 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     // two chunks of 4-bit V codes, by chunk parity, or one of 8-bit codes
     __shared__ __attribute__((aligned(16))) uint8_t vbuf[W][2][kChunkM * 64];
     __shared__ __attribute__((aligned(16))) float2 nbuf[W][kChunkM];  // (knorm, vnorm)
-    __shared__ PageAddrs pagebuf[W][kSplit / W / FHIP_PAGE_TOKENS];  // the wave's split pages
+    __shared__ PageAddrs pagebuf[W][kPart / W / FHIP_PAGE_TOKENS];  // the wave's split pages
     __shared__ int waves_done;  // waves that have left their state for the merge
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, rg = lane >> 4;  // MFMA column / row group
-    static_assert(kWavesM * kSplitMfma == kSplit, "a workgroup's splits make one partial's block");
+    static_assert(kPart / W % kChunkM == 0 && kPart / W <= 64 * FHIP_PAGE_TOKENS,
+                  "a wave's split is whole chunks, its pages one per lane");
 
     // Workgroup (query, kv head, block of W consecutive splits); wave w takes split
     // W * blk + w. Workgroups go to the 8 XCDs round-robin (workgroup b on XCD b % 8),
@@ -991,7 +997,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     const int tq_last = min(tq0 + tok, qs.seq_lens_count) - 1;
     const int blk = (int)(item % nblk);
     const int clen = qs.causal_len(tq_last);  // the group's longest causal length
-    if (blk * kSplit >= clen) return;
+    if (blk * kPart >= clen) return;
     for (int b = threadIdx.x; b < 256; b += 64 * W) {
         float hf;
         auto code = [](const float* cent, int c, int bits) { return cent[min(c, (1 << bits) - 1)]; };
@@ -1007,8 +1013,8 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     }
     __syncthreads();
 
-    const int t_begin = fhip_idx::split_begin(blk, wave, W);
-    const int t_end = min(clen, t_begin + kSplit / W);
+    const int t_begin = blk * kPart + wave * (kPart / W);
+    const int t_end = min(clen, t_begin + kPart / W);
     const int G = qh / kvh;
     const int32_t* table = qs.table + (int64_t)tq0 * qs.table_stride;
     uint8_t* vb = vbuf[wave][0];
@@ -1034,7 +1040,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     // instruction besides its loads and copies. A wave with no position to read (its split
     // starts past the end, or no page is in the pool) keeps the empty state.
     PageAddrs* pages = pagebuf[wave];
-    const uint64_t vmask = t_begin < clen ? split_pages<kSplit / W / FHIP_PAGE_TOKENS>(pg, table, t_begin, t_end, lane, pages) : 0;
+    const uint64_t vmask = t_begin < clen ? split_pages<kPart / W / FHIP_PAGE_TOKENS>(pg, table, t_begin, t_end, lane, pages) : 0;
     if (vmask != 0) {
     // first chunk's copies go out before the Q set-up
     const uint32_t v_lane_off = VB == 2   ? fhip_idx::v2_offset(lane, kvh, g)
@@ -1456,8 +1462,423 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     }
 }
 
-// Eight waves per block up to this many workgroups, two beyond (32 / 8 heads, K4/V2: one sequence
-// of 4000, 32 workgroups: 38 -> 29 us; 16 sequences of 2000 .. 8000 at 8 heads a group, 512
+// ---------------------------------------------------------------------------------------
+// 2''. Causal prefill (many queries of one sequence over one block table; head_dim 128, the MFMA
+//      kernel's width pairs, G <= 8). The decode kernel would look every code up again for each 8
+//      columns; here a workgroup of 4 waves takes kPqCols (query, head) columns of one kv head,
+//      32 per wave, and expands each tile of 64 positions once, into fp16 hi and lo rows of K and
+//      V centroids in LDS, which all its waves read:
+//   S^T = K Q^T and out^T = V^T W^T on v_mfma_f32_32x32x16_f16, each product as hi hi + hi lo +
+//   lo hi into one accumulator (what is left out is 2^-22 of the product). lo = x - hi stays a
+//   normal fp16 number because every factor is scaled by a power of two first: the centroids by
+//   their table's largest magnitude, a query by its own, the weights w = p norm_v by the largest
+//   value norm so far (e_run, for which the accumulators are rescaled like for the running
+//   maximum) and by 2^kPqBias. The scales are exact and leave with the score or the output.
+//   Lane layouts are those of the FP16 prefill kernel: lane (n, half) holds 16 positions of column n
+//   per 32-position block, which are its own slots of W^T.
+// Bound by the MFMA (96 products of 32 clocks per wave and tile) with the lookups (16 8-byte LDS
+// reads a thread and tile at 4 bits) and the softmax beside it. 2048 queries from
+// position 0, 32 / 8 heads, K4/V2: 177 us in all (194 TFLOP/s of attention, three products each),
+// 324 with the decode kernel; 1500 at 1000: 246 and 389 us.
+// ---------------------------------------------------------------------------------------
+constexpr int kPqWaves = 4;
+constexpr int kPqCols = 32 * kPqWaves;  // columns per workgroup
+constexpr int kPqTile = 64;             // positions per tile
+constexpr int kPqRowK = 256 + 16;       // bytes per K row in LDS: 16 rows' 16-byte reads on all banks
+constexpr int kPqRowV = 256 + 64;       // per V row: the transposed reads of 4 rows x 32 dims
+constexpr float kPqBias = 7.0f;         // log2 of the scale that p carries
+constexpr float kPqSlack = 8.0f;        // log2 that p may exceed it by before a rescale
+constexpr int kPqScaleExp = 8;          // centroids and queries are scaled below 2^8
+constexpr int64_t kPqGroups = 512;      // workgroups wanted: the two per CU that fit at once
+typedef float f32x16_t __attribute__((ext_vector_type(16)));
+typedef _Float16 f16x2c_t __attribute__((ext_vector_type(2)));
+typedef float f32x2c_t __attribute__((ext_vector_type(2)));
+
+// x = hi + lo as fp16 pairs, hi rounded to nearest, lo the fp16 of what it leaves.
+__device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2c_t{a, b}), f16x2c_t));
+    float la, lb;
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(la) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(lb) : "v"(hi), "v"(b));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2c_t{la, lb}), f16x2c_t));
+}
+// e with |x| < 2^e (and >= 2^(e-1)) for normal x; infinities and NaN give 129, 0 gives -126.
+__device__ __forceinline__ int exponent_above(float x) {
+    return (int)((__float_as_uint(x) >> 23) & 0xffu) - 126;
+}
+__device__ __forceinline__ float exp2i(int e) { return ldexpf(1.0f, e); }
+
+// Codes of one thread's quarter row (32 codes) of a tile: 4 B bytes.
+template <int B>
+struct Codes32 {
+    u32x4 w[B == 8 ? 2 : 1];
+};
+template <int B>
+__device__ __forceinline__ void load_codes32(const uint8_t* p, Codes32<B>& c) {
+    if constexpr (B == 8) {
+        c.w[0] = *(g_u32x4_any*)p;
+        c.w[1] = *(g_u32x4_any*)(p + 16);
+    } else if constexpr (B == 4) {
+        c.w[0] = *(g_u32x4_any*)p;
+    } else {
+        const u32x2 v = *(g_u32x2_any*)p;
+        c.w[0] = u32x4{v[0], v[1], B == 3 ? *(g_u32_any*)(p + 8) : 0u, 0u};
+    }
+}
+// Expands them: 32 fp16 hi parts at `hi`, lo parts at `lo` (64 bytes each). Tables: B == 8, one
+// (hi | lo << 16) word per code; else per byte of two 4-bit codes the words (hi, hi) and (lo, lo).
+template <int B>
+__device__ __forceinline__ void expand_codes32(const Codes32<B>& c, const u32x2* tab, uint8_t* hi,
+                                               uint8_t* lo) {
+    u32x4 w = c.w[0];
+    if constexpr (B == 2 || B == 3) w = widen32<B>(c.w[0]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // 8 codes
+        u32x4 h, l;
+        if constexpr (B == 8) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const u32x4 v = quad8((const uint32_t*)tab, c.w[j >> 1][2 * (j & 1) + k]);
+                h[2 * k] = __builtin_amdgcn_perm(v[1], v[0], 0x05040100u);
+                h[2 * k + 1] = __builtin_amdgcn_perm(v[3], v[2], 0x05040100u);
+                l[2 * k] = __builtin_amdgcn_perm(v[1], v[0], 0x07060302u);
+                l[2 * k + 1] = __builtin_amdgcn_perm(v[3], v[2], 0x07060302u);
+            }
+        } else {
+            const u32x4 a = pair2<0>(tab, w[j]), b = pair2<2>(tab, w[j]);
+            h = u32x4{a[0], a[2], b[0], b[2]};
+            l = u32x4{a[1], a[3], b[1], b[3]};
+        }
+        *(u32x4*)(hi + 16 * j) = h;
+        *(u32x4*)(lo + 16 * j) = l;
+    }
+}
+
+template <int KB, int VB>
+__global__ __launch_bounds__(64 * kPqWaves) __attribute__((amdgpu_waves_per_eu(2))) void
+tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
+                       const float* __restrict__ kcent, const float* __restrict__ vcent, int qh,
+                       int kvh, float scale_log2, float* __restrict__ part_ml,
+                       float* __restrict__ part_acc, int nsplit, int split_pos, int nqb, int nblk,
+                       int fold, bool merged) {
+    constexpr int hd = 128;
+    __shared__ u32x2 tabs[2][256];
+    __shared__ __attribute__((aligned(16))) uint8_t kbuf[2][kPqTile * kPqRowK];  // hi, lo
+    __shared__ __attribute__((aligned(16))) uint8_t vbuf[2][kPqTile * kPqRowV];
+    __shared__ __attribute__((aligned(16))) float nbuf[2][kPqTile];  // norm_k scale log2(e), norm_v
+    __shared__ float tmax[2];  // the largest centroid magnitudes, then [0] the tile's largest norm_v
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // kv head fastest, then the split, then the query block: see the launcher for its order
+    const int g = (int)(blockIdx.x % kvh);
+    const int rest = (int)(blockIdx.x / kvh);
+    const int split = rest % nsplit;
+    const int bi = rest / nsplit;
+    const int q0 = (fold > 0 && bi >= fold ? bi - fold : nblk - 1 - bi) * nqb;
+    const int nq = min(nqb, qs.seq_lens_count - q0);
+    const int G = qh / kvh;
+    const int clen = qs.causal_len(q0 + nq - 1), clen0 = qs.causal_len(q0);
+    const int t_begin = split * split_pos;
+    // uniform; merged (a single split): every column is written, also one that attends to nothing
+    if (!merged && t_begin >= clen) return;
+    const int t_end = min(clen, t_begin + split_pos);
+    const int32_t* table = qs.table + (int64_t)q0 * qs.table_stride;
+
+    // ---- centroid tables, scaled to below 2^kPqScaleExp
+    float cmaxk = 0.0f, cmaxv = 0.0f;
+    for (int i = lane; i < (1 << KB); i += 64) cmaxk = fmaxf(cmaxk, fabsf(kcent[i]));
+    for (int i = lane; i < (1 << VB); i += 64) cmaxv = fmaxf(cmaxv, fabsf(vcent[i]));
+    const int ek = kPqScaleExp - max(exponent_above(wave_max(cmaxk)), -100);
+    const int ev = kPqScaleExp - max(exponent_above(wave_max(cmaxv)), -100);
+    {
+        auto fill = [&](u32x2* tab, const float* cent, int bits, int e) {
+            for (int b = threadIdx.x; b < 256; b += 64 * kPqWaves) {
+                uint32_t h, l;
+                if (bits == 8) {
+                    split_pair(ldexpf(cent[b], e), 0.0f, h, l);
+                    ((uint32_t*)tab)[b] = (h & 0xffffu) | (l << 16);
+                } else {
+                    const int top = (1 << bits) - 1;
+                    split_pair(ldexpf(cent[min(b >> 4, top)], e), ldexpf(cent[min(b & 15, top)], e), h, l);
+                    tab[b] = u32x2{h, l};
+                }
+            }
+        };
+        fill(tabs[0], kcent, KB, ek);
+        fill(tabs[1], vcent, VB, ev);
+    }
+
+    // ---- column n of the wave: head col % G of query q0 + col / G
+    const int n = lane & 31, half = lane >> 5;
+    const int ncols = nq * G;
+    const int col = 32 * wave + n;
+    const bool col_ok = col < ncols;
+    const bool wave_live = 32 * wave < ncols;
+    const int cq = col_ok ? col / G : 0;
+    const int64_t vec = (int64_t)(q0 + cq) * qh + g * G + (col_ok ? col - cq * G : 0);
+    const int lim = col_ok ? min(t_end, qs.causal_len(q0 + cq)) : 0;
+    u32x4 bh[8], bl[8];  // the query's hi and lo, dims 16 s + 8 half + 0..7, scaled to below 2^8
+    float colscale;      // what a score is multiplied by, with norm_k's factor
+    {
+        f32x4_t v[8][2];
+        const float* src = qrot + vec * hd + 8 * half;
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+            v[s][0] = *(const f32x4_t*)(src + 16 * s);
+            v[s][1] = *(const f32x4_t*)(src + 16 * s + 4);
+        }
+        float m = 0.0f;
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) m = fmaxf(m, fabsf(v[s][k >> 2][k & 3]));
+        m = fmaxf(m, __shfl_xor(m, 32));
+        const int eq = kPqScaleExp - max(exponent_above(m), -100);
+#pragma unroll
+        for (int s = 0; s < 8; ++s)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                uint32_t h, l;
+                split_pair(ldexpf(v[s][k >> 1][2 * (k & 1)], eq), ldexpf(v[s][k >> 1][2 * (k & 1) + 1], eq), h, l);
+                bh[s][k] = h;
+                bl[s][k] = l;
+            }
+        colscale = exp2i(-eq - ek);
+    }
+
+    // ---- tile loads: thread -> row tid / 4, quarter tid % 4 (32 codes); threads of wave 0 the norms.
+    // The row's page is looked up per thread (a wave's 16 rows are one page).
+    const int row = threadIdx.x >> 2, quarter = threadIdx.x & 3;
+    const uint32_t koff = (uint32_t)((((row & 15) * kvh + g) * 16 + 4 * quarter) * KB);
+    const uint32_t voff = (uint32_t)((((row & 15) * kvh + g) * 16 + 4 * quarter) * VB);
+    const uint32_t noff = (uint32_t)(((lane & 15) * kvh + g) * 2);
+    Codes32<KB> kc;
+    Codes32<VB> vc;
+    uint32_t kn = 0, vn = 0;
+    bool nok = false;
+    // pages of the next tile (lane j < 4: page j), read one tile ahead of their rows
+    int page_next = -1;
+    auto load_pages = [&](int t0) {
+        page_next = lane < 4 && t0 + FHIP_PAGE_TOKENS * lane < t_end ? table[t0 / FHIP_PAGE_TOKENS + lane] : -1;
+    };
+    uint32_t pok = 0, pages_ok = 0;
+    const uint8_t *pk_ = nullptr, *pkn = nullptr, *pv_ = nullptr, *pvn = nullptr;  // lane j < 4: page j
+    auto load_addrs = [&]() {
+        const bool ok = lane < 4 && pg.valid(page_next);
+        pages_ok = (uint32_t)__ballot(ok) & 0xfu;
+        if (ok) pg.addrs(page_next, pk_, pkn, pv_, pvn);
+    };
+    auto load_tile = [&](int t0) {
+        pok = pages_ok;
+        if ((pok >> wave) & 1u) {  // the wave's rows: page `wave` of the tile
+            load_codes32<KB>(addr_of_lane(pk_, wave) + koff, kc);
+            load_codes32<VB>(addr_of_lane(pv_, wave) + voff, vc);
+        } else {  // any codes: the scores are masked
+#pragma unroll
+            for (int k = 0; k < (KB == 8 ? 2 : 1); ++k) kc.w[k] = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int k = 0; k < (VB == 8 ? 2 : 1); ++k) vc.w[k] = u32x4{0u, 0u, 0u, 0u};
+        }
+        if (wave == 0) {
+            const int j = lane >> 4;
+            const uint8_t* a = (const uint8_t*)__shfl((long long)(uintptr_t)pkn, j);
+            const uint8_t* b = (const uint8_t*)__shfl((long long)(uintptr_t)pvn, j);
+            nok = ((pok >> j) & 1u) && t0 + lane < t_end;
+            if (nok) {
+                kn = gld2(a + noff);
+                vn = gld2(b + noff);
+            }
+        }
+    };
+    auto store_tile = [&]() {
+        expand_codes32<KB>(kc, tabs[0], kbuf[0] + row * kPqRowK + 64 * quarter, kbuf[1] + row * kPqRowK + 64 * quarter);
+        expand_codes32<VB>(vc, tabs[1], vbuf[0] + row * kPqRowV + 64 * quarter, vbuf[1] + row * kPqRowV + 64 * quarter);
+        if (wave == 0) {
+            const float a = nok ? h2f(kn) * scale_log2 : 0.0f, b = nok ? h2f(vn) : 0.0f;
+            nbuf[0][lane] = a;
+            nbuf[1][lane] = b;
+            const float m = wave_max(fabsf(b));
+            if (lane == 0) tmax[0] = m;
+        }
+    };
+
+    float m_run = -__builtin_inff(), l_run = 0.0f;  // l: the lane half's own positions
+    int e_run = -100;  // the accumulators are in units of 2^e_run (norm_v below it)
+    f32x16_t acc[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[d][i] = 0.0f;
+
+    if (t_begin < t_end) {
+        load_pages(t_begin);
+        load_addrs();
+        load_tile(t_begin);
+        if (t_begin + kPqTile < t_end) {
+            load_pages(t_begin + kPqTile);
+            load_addrs();
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < 8; ++s) asm volatile("" : "+v"(bh[s]), "+v"(bl[s]));
+    for (int t0 = t_begin; t0 < t_end; t0 += kPqTile) {
+        __syncthreads();  // the tables are written; every wave is done with the previous tile
+        store_tile();
+        const uint32_t tile_pok = pok;
+        lds_barrier();
+        if (t0 + kPqTile < t_end) {
+            load_tile(t0 + kPqTile);
+            if (t0 + 2 * kPqTile < t_end) load_pages(t0 + 2 * kPqTile);
+        }
+        if (wave_live) {
+            __builtin_amdgcn_s_setprio(1);
+            // ---- S^T: element i of block pt is position 32 pt + 8 (i / 4) + 4 half + i % 4
+            f32x16_t sc[2];
+            const uint8_t* ksrc = kbuf[0] + n * kPqRowK + 16 * half;
+            constexpr int kLoPart = kPqTile * kPqRowK;
+            constexpr int kAhead = 3;
+            auto k_hi = [&](int t) { return *(const u32x4*)(ksrc + (t >> 3) * 32 * kPqRowK + 32 * (t & 7)); };
+            auto k_lo = [&](int t) { return *(const u32x4*)(ksrc + kLoPart + (t >> 3) * 32 * kPqRowK + 32 * (t & 7)); };
+            u32x4 kh[kAhead + 1], kl[kAhead + 1];
+#pragma unroll
+            for (int t = 0; t < kAhead; ++t) {
+                kh[t] = k_hi(t);
+                kl[t] = k_lo(t);
+            }
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) sc[pt][i] = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                if (t + kAhead < 16) {
+                    kh[(t + kAhead) % (kAhead + 1)] = k_hi(t + kAhead);
+                    kl[(t + kAhead) % (kAhead + 1)] = k_lo(t + kAhead);
+                }
+                const f16x8_t h = __builtin_bit_cast(f16x8_t, kh[t % (kAhead + 1)]);
+                const f16x8_t l = __builtin_bit_cast(f16x8_t, kl[t % (kAhead + 1)]);
+                const f16x8_t qhi = __builtin_bit_cast(f16x8_t, bh[t & 7]), qlo = __builtin_bit_cast(f16x8_t, bl[t & 7]);
+                sc[t >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(l, qhi, sc[t >> 3], 0, 0, 0);
+                sc[t >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h, qlo, sc[t >> 3], 0, 0, 0);
+                sc[t >> 3] = __builtin_amdgcn_mfma_f32_32x32x16_f16(h, qhi, sc[t >> 3], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_s_setprio(0);
+            const bool masked = !(tile_pok == 0xfu && t0 + kPqTile <= min(t_end, clen0));
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const f32x4_t nk = *(const f32x4_t*)&nbuf[0][32 * pt + 8 * j + 4 * half];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) sc[pt][4 * j + k] *= nk[k];
+                }
+            if (masked) {
+#pragma unroll
+                for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int pos = t0 + 32 * pt + 8 * (i / 4) + 4 * half + i % 4;
+                        const bool ok = ((tile_pok >> (2 * pt + i / 8)) & 1u) && pos < lim;
+                        sc[pt][i] = ok ? sc[pt][i] : -__builtin_inff();
+                    }
+            }
+            // ---- online softmax in log2 units
+            float cmax = sc[0][0];
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, sc[pt][i]);
+            cmax = fmaxf(cmax, __shfl_xor(cmax, 32)) * colscale;
+            const float m_new = fmaxf(m_run, cmax);
+            const int e_new = max(e_run, min(exponent_above(tmax[0]), 17));
+            if (__ballot(m_new > m_run + kPqSlack) != 0 || e_new > e_run) {
+                const float mref = m_new == -__builtin_inff() ? 0.0f : m_new;
+                const float alpha = __builtin_amdgcn_exp2f(m_run - mref);  // 0 while m_run is -inf
+                l_run *= alpha;
+                const float beta = alpha * exp2i(e_run - e_new);
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[d][i] *= beta;
+                m_run = m_new;
+                e_run = e_new;
+            }
+            const float ebias = kPqBias - (m_run == -__builtin_inff() ? 0.0f : m_run);
+            const float nscale = exp2i(-e_run);
+            float psum = 0.0f;
+#pragma unroll
+            for (int pt = 0; pt < 2; ++pt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    f32x4_t nv = *(const f32x4_t*)&nbuf[1][32 * pt + 8 * j + 4 * half];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const float p = __builtin_amdgcn_exp2f(fmaf(sc[pt][4 * j + k], colscale, ebias));
+                        psum += p;
+                        const float w = p * (nv[k] * nscale);
+                        // a masked position's norm may be infinite or NaN
+                        sc[pt][4 * j + k] = masked && p == 0.0f ? 0.0f : w;
+                    }
+                }
+            l_run += psum;
+            __builtin_amdgcn_s_setprio(1);
+            // ---- out^T: 4 steps of 16 positions
+            const uint8_t* vsrc = vbuf[0] + (4 * half + ((lane & 15) >> 2)) * kPqRowV +
+                                  2 * (16 * ((lane >> 4) & 1) + 4 * (lane & 3));
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                uint32_t ph[4], pl[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    split_pair(sc[ks >> 1][8 * (ks & 1) + 2 * j], sc[ks >> 1][8 * (ks & 1) + 2 * j + 1], ph[j], pl[j]);
+                const f16x8_t wh = __builtin_bit_cast(f16x8_t, u32x4{ph[0], ph[1], ph[2], ph[3]});
+                const f16x8_t wl = __builtin_bit_cast(f16x8_t, u32x4{pl[0], pl[1], pl[2], pl[3]});
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    auto tr = [&](const uint8_t* src) -> f16x8_t {
+                        typedef short v4s_t __attribute__((ext_vector_type(4)));
+                        typedef __attribute__((address_space(3))) v4s_t lds_v4s_t;
+                        const v4s_t a = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (lds_v4s_t*)(__attribute__((address_space(3))) uint8_t*)src);
+                        const v4s_t b = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                            (lds_v4s_t*)(__attribute__((address_space(3))) uint8_t*)(src + 8 * kPqRowV));
+                        return __builtin_bit_cast(f16x8_t, (short __attribute__((ext_vector_type(8)))){
+                                                               a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]});
+                    };
+                    const uint8_t* src = vsrc + 16 * ks * kPqRowV + 64 * d;
+                    const f16x8_t vh = tr(src), vl = tr(src + kPqTile * kPqRowV);
+                    acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vl, wh, acc[d], 0, 0, 0);
+                    acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, wl, acc[d], 0, 0, 0);
+                    acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vh, wh, acc[d], 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        if (t0 + 2 * kPqTile < t_end) load_addrs();
+    }
+
+    l_run += __shfl_xor(l_run, 32);
+    if (!col_ok) return;
+    // merged: acc / l replaces the query in q_rot, which only this column's lanes have read
+    const float unit = exp2i(e_run - ev) * (merged ? (l_run > 0.0f ? 1.0f / l_run : 0.0f) : 1.0f);
+    float* dst = merged ? qrot + vec * hd : part_acc + (vec * nsplit + split) * hd;
+    if (!merged && half == 0) {
+        part_ml[(vec * nsplit + split) * 2 + 0] = m_run * 0.6931471805599453f;
+        part_ml[(vec * nsplit + split) * 2 + 1] = l_run;
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            *(f32x4_t*)(dst + 32 * d + 8 * j + 4 * half) =
+                f32x4_t{acc[d][4 * j] * unit, acc[d][4 * j + 1] * unit, acc[d][4 * j + 2] * unit,
+                        acc[d][4 * j + 3] * unit};
+}
+
+// Eight waves per block up to this many workgroups, two beyond (32 / 8 heads, K4/V2: 16 sequences of
+// 500 .. 2000, 256 workgroups: 39 -> 30 us; 16 sequences of 2000 .. 8000 at 8 heads a group, 512
 // workgroups: 53 -> 46; 64 of 500 .. 2000, 1024 workgroups: 53 with two, 58 with eight). 8-bit codes
 // keep twice the registers and buffers a wave: at 512 workgroups 50 us with two, 52 with eight.
 constexpr int64_t kWideGroups = 512, kWideGroups8 = 256;
@@ -1470,47 +1891,58 @@ bool mfma_widths(int kbits, int vbits) {
            (kbits == vbits && (kbits == 2 || kbits == 3 || kbits == 8));
 }
 
+int decode_group(const Queries& qs, int nq, int G) {
+    return (!qs.seq_lens && qs.table_stride == 0 && nq > 1 && G < 8) ? 8 / G : 1;
+}
+int64_t decode_groups(int nq, int tok, int kvh, int nsplit) {
+    return ceil_div(ceil_div((int64_t)nq, tok) * nsplit, kXcds) * kXcds * kvh;
+}
+
 template <class Pages, int KB, int VB>
 void launch_mfma_t(const float* qrot, const Queries& q2, const Pages& pg, const float* kcent,
-                   const float* vcent, int qh, int kvh, int nsplit, int tok, int64_t wgs, float* ml,
-                   float* acc, hipStream_t s) {
+                   const float* vcent, int qh, int kvh, int nsplit, int part, int tok, int64_t wgs,
+                   float* ml, float* acc, hipStream_t s) {
     const bool g4 = qh / kvh <= 4 && tok == 1;
-    const bool wide = wgs <= (KB == 8 ? kWideGroups8 : kWideGroups);
-    auto kern = g4 ? (wide ? tq_attn_mfma_kernel<Pages, true, KB, VB, kWavesWide>
-                           : tq_attn_mfma_kernel<Pages, true, KB, VB, kWavesM>)
-                   : (wide ? tq_attn_mfma_kernel<Pages, false, KB, VB, kWavesWide>
-                           : tq_attn_mfma_kernel<Pages, false, KB, VB, kWavesM>);
-    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * (wide ? kWavesWide : kWavesM)), 0, s, qrot,
-                       q2, pg, kcent, vcent, qh, kvh, 1.0f / sqrtf(128.0f), ml, acc, nsplit, nsplit,
-                       tok);
+    auto go = [&](auto kern, int waves) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * waves), 0, s, qrot, q2, pg, kcent, vcent,
+                           qh, kvh, 1.0f / sqrtf(128.0f), ml, acc, nsplit, nsplit, tok);
+    };
+    if (part == kFinePart)
+        go(g4 ? tq_attn_mfma_kernel<Pages, true, KB, VB, 4, kFinePart>
+              : tq_attn_mfma_kernel<Pages, false, KB, VB, 4, kFinePart>, 4);
+    else if (wgs <= (KB == 8 ? kWideGroups8 : kWideGroups))
+        go(g4 ? tq_attn_mfma_kernel<Pages, true, KB, VB, kWavesWide, kSplit>
+              : tq_attn_mfma_kernel<Pages, false, KB, VB, kWavesWide, kSplit>, kWavesWide);
+    else
+        go(g4 ? tq_attn_mfma_kernel<Pages, true, KB, VB, kWavesM, kSplit>
+              : tq_attn_mfma_kernel<Pages, false, KB, VB, kWavesM, kSplit>, kWavesM);
 }
 
 template <class Pages>
 void launch_mfma_split(const float* qrot, const Queries& qsv, const Pages& pg,
                        const float* kcent, const float* vcent, int nq, int qh, int kvh,
-                       int nsplit, int kbits, int vbits, float* ml, float* acc, hipStream_t s) {
+                       int nsplit, int part, int kbits, int vbits, float* ml, float* acc,
+                       hipStream_t s) {
     // Causal prefill (queries at consecutive positions of one sequence: one shared block table,
     // lengths from start_pos) groups 8 / G consecutive queries per item so that they share the
     // MFMA columns and every code lookup; decode keeps one query per item.
-    const int G = qh / kvh;
-    const int tok = (!qsv.seq_lens && qsv.table_stride == 0 && nq > 1 && G < 8) ? 8 / G : 1;
-    const int64_t items = ceil_div((int64_t)nq, tok);
-    // one workgroup per (item, kv head, kSplit-position block): the block count is the
+    const int tok = decode_group(qsv, nq, qh / kvh);
+    // one workgroup per (item, kv head, part-position block): the block count is the
     // partial layout's split count; the (item, block) pairs are padded to a multiple of the
     // XCD count (the kernel's index spreads them, not heads, over the XCDs)
-    const int64_t wgs = ceil_div(items * nsplit, kXcds) * kXcds * kvh;
+    const int64_t wgs = decode_groups(nq, tok, kvh, nsplit);
     Queries q2 = qsv;
     q2.seq_lens_count = nq;
     if (kbits == 8)
-        launch_mfma_t<Pages, 8, 8>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 8, 8>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
     else if (kbits == 3)
-        launch_mfma_t<Pages, 3, 3>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 3, 3>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
     else if (kbits == 2)
-        launch_mfma_t<Pages, 2, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 2, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
     else if (vbits == 2)
-        launch_mfma_t<Pages, 4, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 4, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
     else
-        launch_mfma_t<Pages, 4, 4>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 4, 4>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
 }
 
 struct AttnArgs {
@@ -1521,11 +1953,14 @@ struct AttnArgs {
     const float *krot, *vrot, *kcent, *vcent;
     int qh, kvh, hd, kbits, vbits;
     void* ws;
+    size_t ws_bytes = kFineBytes;  // what `ws` holds, at least ws_layout's at kSplit positions
 };
 
-size_t ws_layout(int nq, int qh, int hd, int max_tokens, size_t* off_ml, size_t* off_acc,
+// The workspace: q_rot, then (m, l) and the accumulators of the split partials, one split per `part`
+// positions.
+size_t ws_layout(int nq, int qh, int hd, int max_tokens, int part, size_t* off_ml, size_t* off_acc,
                  int* nsplit) {
-    const int ns = max_tokens > 0 ? (max_tokens + kSplit - 1) / kSplit : 1;
+    const int ns = max_tokens > 0 ? (max_tokens + part - 1) / part : 1;
     const size_t qrot = (size_t)nq * qh * hd * sizeof(float);
     const size_t ml = (size_t)nq * qh * ns * 2 * sizeof(float);
     const size_t acc = (size_t)nq * qh * ns * hd * sizeof(float);
@@ -1534,6 +1969,14 @@ size_t ws_layout(int nq, int qh, int hd, int max_tokens, size_t* off_ml, size_t*
     if (off_acc) *off_acc = al(qrot) + al(ml);
     if (nsplit) *nsplit = ns;
     return al(qrot) + al(ml) + al(acc);
+}
+// Small launches may split finer, where the layout of kFinePart positions stays within kFineBytes. The
+// size a caller is asked for covers that layout at every smaller size too (it never falls as an
+// argument grows), so a workspace warmed up at the largest call serves the smaller ones.
+size_t ws_bytes_for(int nq, int qh, int hd, int max_tokens) {
+    return std::max(ws_layout(nq, qh, hd, max_tokens, kSplit, nullptr, nullptr, nullptr),
+                    std::min(ws_layout(nq, qh, hd, max_tokens, kFinePart, nullptr, nullptr, nullptr),
+                             kFineBytes));
 }
 
 template <int KB, int VB, class Pages>
@@ -1547,12 +1990,68 @@ void launch_split(const AttnArgs& a, const Pages& pg, int nsplit, float* ml, flo
                        a.kvh, a.hd, 1.0f / sqrtf((float)a.hd), ml, acc, nsplit);
 }
 
+// Workgroups of the prefill kernel with up to nsplit splits. Below kPqMinGroups the decode kernel,
+// whose waves share a split, is the faster one (16 queries at 100, 16 workgroups: 26 against 32 us);
+// above it this one is (64 at 2000, 144: 48 against 55; 200 at 1000, K8/V8, 280: 62 against 88).
+constexpr int64_t kPqMinGroups = 96;
+int64_t prefill_groups(const AttnArgs& a, int nsplit) {
+    const int64_t base = ceil_div((int64_t)a.nq, kPqCols / (a.qh / a.kvh)) * a.kvh;
+    return a.nq > 1 ? base * std::min<int64_t>(std::max<int64_t>(ceil_div(kPqGroups, base), 1), nsplit) : 0;
+}
+// Decode launches of up to this many 1024-position workgroups split at kFinePart positions, four waves
+// of one chunk each: four times the workgroups (one sequence of 4000, 32 of them: 29 -> 23 us; at
+// 256, 16 sequences of 500 .. 2000: 30 us either way).
+constexpr int64_t kFineGroups = 256;
+
+// Launches the prefill kernel; *nsplit (in: what the workspace holds) and *split_pos become its own,
+// *merged tells whether it left merged vectors in qrot.
+void launch_prefill(float* qrot, const AttnArgs& a, const PtrPages& pg, bool batched_rot, int* nsplit,
+                    int* split_pos, bool* merged, float* ml, float* acc, hipStream_t s) {
+    const int G = a.qh / a.kvh;
+    const int nqb = kPqCols / G;
+    const int nblk = (int)ceil_div((int64_t)a.nq, nqb);
+    const int64_t base = (int64_t)nblk * a.kvh;
+    const int extent = std::max(std::min(a.qs.kv_len, a.qs.max_blocks * FHIP_PAGE_TOKENS), 1);
+    const int64_t want = std::min<int64_t>(std::max<int64_t>(ceil_div(kPqGroups, base), 1), *nsplit);
+    *split_pos = (int)(ceil_div(ceil_div(extent, want), kPqTile) * kPqTile);
+    *nsplit = (int)ceil_div(extent, *split_pos);
+    *merged = *nsplit == 1 && batched_rot;
+    // Blocks start from the last (the longest contexts) down. Where all fit at once, two to a CU, the
+    // second half goes up from the first instead, so that a long block shares its CU with a short one.
+    const int64_t wgs = base * *nsplit;
+    const int cus = fhip_host::cu_count();
+    const int fold = *nsplit == 1 && wgs > cus && wgs <= 2 * cus ? (int)(cus / a.kvh) : 0;
+    Queries q2 = a.qs;
+    q2.seq_lens_count = a.nq;
+    auto kern = a.kbits == 8   ? tq_attn_prefill_kernel<8, 8>
+                : a.kbits == 3 ? tq_attn_prefill_kernel<3, 3>
+                : a.kbits == 2 ? tq_attn_prefill_kernel<2, 2>
+                : a.vbits == 2 ? tq_attn_prefill_kernel<4, 2>
+                               : tq_attn_prefill_kernel<4, 4>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * kPqWaves), 0, s, qrot, q2, pg, a.kcent,
+                       a.vcent, a.qh, a.kvh, 1.4426950408889634f / sqrtf(128.0f), ml, acc, *nsplit,
+                       *split_pos, nqb, nblk, fold, *merged);
+}
+
 template <class Pages>
 int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
     if (a.nq == 0) return hipSuccess;
+    const int G = a.qh / a.kvh, max_tokens = a.qs.max_blocks * FHIP_PAGE_TOKENS;
+    const bool mfma = mfma_widths(a.kbits, a.vbits) && a.hd == 128 && G <= 8;
+    int split_pos = kSplit, nsplit;
+    bool prefill = false;
+    if (mfma) {
+        const bool fine = ws_layout(a.nq, a.qh, a.hd, max_tokens, kFinePart, nullptr, nullptr, &nsplit) <=
+                          std::min(a.ws_bytes, kFineBytes);
+        if constexpr (std::is_same_v<Pages, PtrPages>)
+            prefill = !a.qs.seq_lens && a.qs.table_stride == 0 &&
+                      prefill_groups(a, fine ? nsplit : (int)ceil_div(max_tokens, kSplit)) >= kPqMinGroups;
+        if (fine && (prefill || decode_groups(a.nq, decode_group(a.qs, a.nq, G), a.kvh,
+                                              (int)ceil_div(max_tokens, kSplit)) <= kFineGroups))
+            split_pos = kFinePart;
+    }
     size_t off_ml, off_acc;
-    int nsplit;
-    ws_layout(a.nq, a.qh, a.hd, a.qs.max_blocks * FHIP_PAGE_TOKENS, &off_ml, &off_acc, &nsplit);
+    ws_layout(a.nq, a.qh, a.hd, max_tokens, split_pos, &off_ml, &off_acc, &nsplit);
     float* qrot = (float*)a.ws;
     float* ml = (float*)((char*)a.ws + off_ml);
     float* acc = (float*)((char*)a.ws + off_acc);
@@ -1570,9 +2069,13 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
         hipLaunchKernelGGL(tq_attn_prerotate_kernel, dim3(rot_groups), dim3(256), 0, s,
                            (const uint16_t*)a.q, a.krot, qrot, a.hd, nvec);
     }
-    if (mfma_widths(a.kbits, a.vbits) && a.hd == 128 && a.qh / a.kvh <= 8)
-        launch_mfma_split(qrot, a.qs, pg, a.kcent, a.vcent, a.nq, a.qh, a.kvh, nsplit, a.kbits,
-                          a.vbits, ml, acc, s);
+    bool merged = false;  // the split kernel has left the merged vectors in q_rot
+    if (prefill) {
+        if constexpr (std::is_same_v<Pages, PtrPages>)
+            launch_prefill(qrot, a, pg, batched_rot, &nsplit, &split_pos, &merged, ml, acc, s);
+    } else if (mfma)
+        launch_mfma_split(qrot, a.qs, pg, a.kcent, a.vcent, a.nq, a.qh, a.kvh, nsplit, split_pos,
+                          a.kbits, a.vbits, ml, acc, s);
     else if (a.kbits == 4 && a.vbits == 4)
         launch_split<4, 4>(a, pg, nsplit, ml, acc, s);
     else if (a.kbits == 4 && a.vbits == 2)
@@ -1580,15 +2083,17 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
     else
         launch_split<0, 0>(a, pg, nsplit, ml, acc, s);
     if (batched_rot) {
-        if (nsplit <= kMergeWaveMaxSplits)
+        if (merged)
+            ;
+        else if (nsplit <= kMergeWaveMaxSplits)
             hipLaunchKernelGGL(tq_attn_merge_wave_kernel, dim3((unsigned)ceil_div(nvec, 4)),
                                dim3(256), 0, s, a.qs, ml, acc, a.qh, a.hd, nsplit, (int64_t)nvec,
-                               qrot);
+                               qrot, split_pos);
         else
             hipLaunchKernelGGL((tq_attn_combine_kernel<true, true>),
                                dim3((unsigned)ceil_div(nvec, kCombHeads)), dim3(256),
                                combine_lds_bytes(a.hd, nsplit, true), s, a.qs, ml, acc, a.vrot,
-                               (uint16_t*)a.out, a.qh, a.hd, nsplit, (int64_t)nvec, qrot);
+                               (uint16_t*)a.out, a.qh, a.hd, nsplit, (int64_t)nvec, qrot, split_pos);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         return fhip_internal::tq_rotate_back_rows(qrot, a.vrot, a.out, nvec, s);
@@ -1596,7 +2101,7 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
     auto comb = a.hd <= kRotLdsMaxHd ? tq_attn_combine_kernel<true> : tq_attn_combine_kernel<false>;
     hipLaunchKernelGGL(comb, dim3((unsigned)ceil_div(nvec, kCombHeads)), dim3(256),
                        combine_lds_bytes(a.hd, nsplit), s, a.qs, ml, acc, a.vrot,
-                       (uint16_t*)a.out, a.qh, a.hd, nsplit, (int64_t)nvec, nullptr);
+                       (uint16_t*)a.out, a.qh, a.hd, nsplit, (int64_t)nvec, nullptr, split_pos);
     return hipGetLastError();
 }
 
@@ -1648,8 +2153,7 @@ extern "C" {
 size_t fhip_attention_tq_workspace_bytes(int batch, int num_q_heads, int head_dim,
                                          int max_blocks) {
     if (batch <= 0 || num_q_heads <= 0 || head_dim <= 0 || max_blocks <= 0) return 0;
-    return ws_layout(batch, num_q_heads, head_dim, max_blocks * FHIP_PAGE_TOKENS, nullptr, nullptr,
-                     nullptr);
+    return ws_bytes_for(batch, num_q_heads, head_dim, max_blocks * FHIP_PAGE_TOKENS);
 }
 
 int fhip_launch_attention_tq_decode(void* output, const void* q, const int32_t* block_table,
@@ -1820,12 +2324,12 @@ static int attention_paged_tq_ref(void* output, const void* q, const int* block_
                         !v_norms_ptrs))
         return hipErrorInvalidValue;
     const int mb = nblocks > 0 ? nblocks : 1;
-    const size_t bytes = ws_layout(num_tokens, num_q_heads, head_dim, mb * FHIP_PAGE_TOKENS,
-                                   nullptr, nullptr, nullptr);
+    const size_t need = ws_bytes_for(num_tokens, num_q_heads, head_dim, mb * FHIP_PAGE_TOKENS);
     const bool own = ws == nullptr;
-    if (!own && ws_bytes < bytes) return hipErrorInvalidValue;
+    if (!own && ws_bytes < need) return hipErrorInvalidValue;
     if (own) {
-        hipError_t e = hipMallocAsync(&ws, bytes, s);
+        ws_bytes = need;
+        hipError_t e = hipMallocAsync(&ws, ws_bytes, s);
         if (e != hipSuccess) return e;
     }
     AttnArgs a;
@@ -1843,6 +2347,7 @@ static int attention_paged_tq_ref(void* output, const void* q, const int* block_
     a.kbits = key_bits;
     a.vbits = value_bits;
     a.ws = ws;
+    a.ws_bytes = ws_bytes;
     PtrPages pg{(const uint8_t* const*)k_packed_ptrs, (const uint8_t* const*)k_norms_ptrs,
                 (const uint8_t* const*)v_packed_ptrs, (const uint8_t* const*)v_norms_ptrs,
                 0x7fffffff};
@@ -1884,9 +2389,9 @@ int fhip_launch_attention_paged_tq_noalloc(void* output, const void* q, const in
         return hipErrorInvalidValue;
     if (num_tokens == 0) return hipSuccess;
     const int nblocks = (kv_len + FHIP_PAGE_TOKENS - 1) / FHIP_PAGE_TOKENS;
-    const size_t need = ws_layout(num_tokens, num_q_heads, head_dim,
-                                  (nblocks > 0 ? nblocks : 1) * FHIP_PAGE_TOKENS, nullptr,
-                                  nullptr, nullptr);
+    const size_t need = ws_bytes_for(num_tokens, num_q_heads, head_dim,
+                                     (nblocks > 0 ? nblocks : 1) * FHIP_PAGE_TOKENS);
+    static_assert(kFineBytes <= kNoAllocScratchBytes, "finer splits never make a call too large");
     if (need > kNoAllocScratchBytes) return hipErrorOutOfMemory;
     hipStream_t s = fhip_host::as_stream(stream);
     int dev = -1;

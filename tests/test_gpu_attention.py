@@ -201,3 +201,52 @@ def test_code_pages_at_odd_addresses(dev, bits):
     want = oracle.tq_attention(q[0], pool["table"][0], n, pool["KP"], pool["KN"], pool["VP"], pool["VN"],
                                pool["krot"], pool["vrot"], pool["kc"], pool["vc"], bits, bits, kvh)
     assert_close(out.cpu().numpy()[0].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3)
+
+
+def run_prefill(dev, pool, q, kvh, kv_len, start_pos, kbits, vbits):
+    P, T, qh, hd = pool["KP"].shape[0], *q.shape
+    parts = [dev_t(pool[n], dev) for n in ("KP", "KN", "VP", "VN")]
+    ptrs = [torch.tensor([x.data_ptr() for x in t], dtype=torch.int64, device=dev) for t in parts]
+    tq_, table = dev_t(q, dev), dev_t(pool["table"][0], dev)
+    tabs = [dev_t(pool[x], dev) for x in ("krot", "vrot", "kc", "vc")]
+    out = torch.empty_like(tq_)
+    code = K._L().fhip_launch_attention_paged_tq(
+        out.data_ptr(), tq_.data_ptr(), table.data_ptr(), *(p.data_ptr() for p in ptrs),
+        *(t.data_ptr() for t in tabs), T, qh, kvh, hd, kv_len, start_pos, kbits, vbits,
+        oracle.packed_dim(hd, kbits), oracle.packed_dim(hd, vbits), torch.cuda.current_stream().cuda_stream)
+    assert code == 0
+    torch.cuda.synchronize()
+    return out.cpu().numpy().astype(np.float32)
+
+
+@pytest.mark.parametrize("kbits,vbits,qh,kvh,T,kv_len", [
+    # several splits, ragged columns: G = 2, 4, 8, 3, 1 (5 splits of the positions or more)
+    (4, 2, 16, 8, 130, 1100), (4, 4, 16, 4, 65, 1800), (8, 8, 16, 2, 60, 3000), (3, 3, 24, 8, 45, 1301),
+    (2, 2, 8, 8, 130, 1537),
+    # one split and a batch of vectors that skips the merge, blocks going up after those going down
+    (4, 2, 32, 8, 2048, 2048)])
+def test_prefill_tiles(dev, kbits, vbits, qh, kvh, T, kv_len):
+    """The causal prefill kernel against the oracle, with a masked page and with a value norm of
+    infinity and a key norm of NaN at late positions, which no earlier query may see; the value norms
+    span 2^-10 .. 2^10."""
+    rng = np.random.default_rng(kbits * 100 + T)
+    hd, start = 128, kv_len - T
+    pool = build_pool(rng, [kv_len], kvh, hd, kbits, vbits)
+    table = pool["table"][0]
+    pool["VN"] *= np.exp2(rng.uniform(-10, 10, pool["VN"].shape[:2]))[..., None].astype(np.float16)
+    table[2] = -5  # positions 32..47 masked
+    pool["VN"][table[(kv_len - 3) // 16], (kv_len - 3) % 16] = np.inf
+    pool["KN"][table[(kv_len - 2) // 16], (kv_len - 2) % 16] = np.nan
+    q = rng.standard_normal((T, qh, hd)).astype(np.float16)
+    got = run_prefill(dev, pool, q, kvh, kv_len, start, kbits, vbits)
+    for t in sorted({0, 1, T // 3, T // 2, T - 5, T - 4} | set(range(0, T - 4, max(1, T // 12)))):
+        n = start + t + 1
+        if n <= 48:
+            n = min(n, 32)
+            rows = table
+        else:
+            rows, n = np.delete(table, 2), n - 16
+        want = oracle.tq_attention(q[t], rows, n, pool["KP"], pool["KN"], pool["VP"], pool["VN"],
+                                   pool["krot"], pool["vrot"], pool["kc"], pool["vc"], kbits, vbits, kvh)
+        scale = max(1.0, float(np.abs(want.astype(np.float32)).max()))  # norms up to 2^10
+        assert_close(got[t] / scale, want.astype(np.float32) / scale, 1e-3, 1e-3, f"token {t}")
