@@ -165,6 +165,42 @@ __global__ __launch_bounds__(256) void tq_attn_prerotate_kernel(const uint16_t* 
     }
 }
 
+// The same at head_dim 128: 4 vectors per workgroup of 512 lanes, lane (row i, quarter jq) holding 32
+// coordinates of Pi_k's row i, read as eight 16-byte loads that are all in flight with the vectors'
+// own; the quarters are summed by DPP. The general kernel walks a row of 128 loads a lane, one
+// latency after another, over half the workgroups: 6.4 us for 32 vectors and 9.9 for 2048 against
+// 4.5 and 8.4 here (kernel trace; a kernel that does nothing takes 2).
+constexpr int kRot128Vecs = 4;
+__global__ __launch_bounds__(512) void tq_attn_prerotate128_kernel(const uint16_t* __restrict__ q,
+                                                                   const float* __restrict__ rot,
+                                                                   float* __restrict__ qrot, int nvec) {
+    __shared__ __attribute__((aligned(16))) float qs[kRot128Vecs][4][36];  // quarters on distinct banks
+    const int v0 = blockIdx.x * kRot128Vecs;
+    const int tid = threadIdx.x, i = tid >> 2, jq = tid & 3;
+    f32x4 r[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) r[k] = *(const f32x4*)(rot + 128 * i + 32 * jq + 4 * k);
+    const int lv = tid >> 7, lj = tid & 127;
+    const uint16_t raw = v0 + lv < nvec ? q[(int64_t)(v0 + lv) * 128 + lj] : 0;
+    qs[lv][lj >> 5][lj & 31] = h2f(raw);
+    __syncthreads();
+    float mine = 0.0f;
+#pragma unroll
+    for (int v = 0; v < kRot128Vecs; ++v) {
+        float dot = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const f32x4 x = *(const f32x4*)&qs[v][jq][4 * k];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dot = fmaf(r[k][e], x[e], dot);
+        }
+        dot += __builtin_amdgcn_update_dpp(0.0f, dot, 0xB1, 0xF, 0xF, true);  // lane ^ 1
+        dot += __builtin_amdgcn_update_dpp(0.0f, dot, 0x4E, 0xF, 0xF, true);  // lane ^ 2
+        mine = v == jq ? dot : mine;
+    }
+    if (v0 + jq < nvec) qrot[(int64_t)(v0 + jq) * 128 + i] = mine;
+}
+
 // 2. One (split, kv head, query) per workgroup of 256 lanes. Each pass of 256 positions
 // stages the positions' packed K and V rows in LDS (row stride padded to an odd number of
 // words, so lanes reading different rows hit different banks), scores them one position per
@@ -535,6 +571,82 @@ __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
             if (head < nvec) out[head * hd + i] = (uint16_t)f2h(dot[k]);
         }
     }
+}
+
+// Merge and unrotation at head_dim 128: 4 vectors per workgroup of 512 lanes. Everything that does not
+// depend on the rest is loaded at once: lane (i, quarter jq) its 32 entries of Pi_v's column i, lane
+// (vector, d) up to 16 splits' (m, l) and accumulator d, folded as an online softmax over chunks of
+// 16 splits. The merged vectors cross LDS once, then each lane sums its 32 products for the 4
+// vectors and the quarters meet in LDS. The general kernel above stages Pi_v in LDS, then waits for
+// (m, l), for the accumulators and for 128 LDS reads in turn: 8.3 us for 32 vectors of 4 splits
+// against 5.3 here (2048 vectors of up to 32 splits are bound by their 34 MB either way: 20 us).
+constexpr int kComb128Vecs = 4;
+__global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
+    Queries qs, const float* __restrict__ part_ml, const float* __restrict__ part_acc,
+    const float* __restrict__ vrot, uint16_t* __restrict__ out, int qh, int nsplit, int64_t nvec,
+    int split_pos) {
+    constexpr int kChunk = 16;
+    __shared__ __attribute__((aligned(16))) float o[kComb128Vecs][128];
+    __shared__ float red[4][kComb128Vecs][128];
+    const int tid = threadIdx.x, i = tid & 127;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 7);  // the lane's vector, then its quarter
+    float r[32];
+#pragma unroll
+    for (int k = 0; k < 32; ++k) r[k] = vrot[(32 * w + k) * 128 + i];
+    const int64_t vec = (int64_t)blockIdx.x * kComb128Vecs + w;
+    float M = -__builtin_inff(), L = 0.0f, sum = 0.0f;
+    if (vec < nvec) {
+        const float* ml = part_ml + vec * nsplit * 2;
+        const float* a = part_acc + vec * nsplit * 128 + i;
+        const int ns = (qs.causal_len((int)(vec / qh)) + split_pos - 1) / split_pos;
+        for (int s0 = 0; s0 < (s0 == 0 ? nsplit : ns); s0 += kChunk) {
+            // the first chunk goes by the layout, so that its loads need not wait for the length;
+            // what lies past the length is not used
+            const int top = s0 == 0 ? nsplit : ns;
+            float m[kChunk], l[kChunk], av[kChunk];
+#pragma unroll
+            for (int u = 0; u < kChunk; ++u) {
+                const int sp = min(s0 + u, top - 1);
+                m[u] = ml[2 * sp];
+                l[u] = ml[2 * sp + 1];
+                av[u] = a[(int64_t)sp * 128];
+            }
+            float mx = M;
+#pragma unroll
+            for (int u = 0; u < kChunk; ++u) {
+                m[u] = s0 + u < ns ? m[u] : -__builtin_inff();
+                mx = fmaxf(mx, m[u]);
+            }
+            const float old = M == -__builtin_inff() ? 0.0f : expf(M - mx);
+            L *= old;
+            sum *= old;
+#pragma unroll
+            for (int u = 0; u < kChunk; ++u) {
+                if (m[u] == -__builtin_inff()) continue;  // uniform over the wave
+                const float wt = expf(m[u] - mx);
+                L = fmaf(wt, l[u], L);
+                sum = fmaf(wt, av[u], sum);
+            }
+            M = mx;
+        }
+    }
+    o[w][i] = L > 0.0f ? sum / L : 0.0f;
+    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < kComb128Vecs; ++v) {
+        float dot = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const f32x4 x = *(const f32x4*)&o[v][32 * w + 4 * k];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dot = fmaf(r[4 * k + e], x[e], dot);
+        }
+        red[w][v][i] = dot;
+    }
+    __syncthreads();
+    if (vec < nvec)
+        out[vec * 128 + i] =
+            (uint16_t)f2h((red[0][w][i] + red[1][w][i]) + (red[2][w][i] + red[3][w][i]));
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2064,6 +2176,9 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
     if (batched_rot) {
         const int e = fhip_internal::tq_rotate_rows(a.q, a.krot, qrot, nvec, s);
         if (e != hipSuccess) return e;
+    } else if (a.hd == 128 && fhip_host::aligned16(a.krot)) {
+        hipLaunchKernelGGL(tq_attn_prerotate128_kernel, dim3((unsigned)ceil_div(nvec, kRot128Vecs)),
+                           dim3(512), 0, s, (const uint16_t*)a.q, a.krot, qrot, nvec);
     } else {
         const unsigned rot_groups = (unsigned)ceil_div(nvec, kRotVecs);
         hipLaunchKernelGGL(tq_attn_prerotate_kernel, dim3(rot_groups), dim3(256), 0, s,
@@ -2097,6 +2212,12 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         return fhip_internal::tq_rotate_back_rows(qrot, a.vrot, a.out, nvec, s);
+    }
+    if (a.hd == 128) {
+        hipLaunchKernelGGL(tq_attn_combine128_kernel, dim3((unsigned)ceil_div(nvec, kComb128Vecs)),
+                           dim3(512), 0, s, a.qs, ml, acc, a.vrot, (uint16_t*)a.out, a.qh, nsplit,
+                           (int64_t)nvec, split_pos);
+        return hipGetLastError();
     }
     auto comb = a.hd <= kRotLdsMaxHd ? tq_attn_combine_kernel<true> : tq_attn_combine_kernel<false>;
     hipLaunchKernelGGL(comb, dim3((unsigned)ceil_div(nvec, kCombHeads)), dim3(256),
