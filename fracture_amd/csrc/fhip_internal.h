@@ -30,4 +30,8 @@ int tq_rotate_rows(const void* input, const float* rotation, float* out, int64_t
 int tq_rotate_back_rows(const float* input, const float* rotation, void* out, int64_t rows,
                         hipStream_t stream);
 
+// C[m, n] = A[m, k] B[n, k]^T for few rows of A (matmul_skinny.hip), where matmul_skinny_takes.
+bool matmul_skinny_takes(const void* c, const void* a, const void* b, int m, int n, int k);
+int matmul_skinny(void* c, const void* a, const void* b, int m, int n, int k, hipStream_t stream);
+
 }  // namespace fhip_internal

@@ -1,8 +1,9 @@
 // Dense fp16 GEMM for the Backend::matmul surface: C[M, N] = A[M, K] · B[N, K]ᵀ, row-major,
 // fp16 in and out with fp32 accumulation — the contract of CudaBackend::matmul
 // (cuda/src/backend.rs:75-128: weights stored [out_features, in_features], y = x Wᵀ,
-// cublasGemmEx with CUBLAS_COMPUTE_32F). A plain library GEMM: rocBLAS gemm_ex on the
-// caller's stream, which dispatches to the library's tuned gfx950 MFMA kernels.
+// cublasGemmEx with CUBLAS_COMPUTE_32F). A few rows of A on a B of moderate size go to
+// matmul_skinny.hip; any other product is a plain library GEMM: rocBLAS gemm_ex on the caller's
+// stream, which dispatches to the library's tuned gfx950 MFMA kernels.
 //
 // Row-major operands are column-major transposes, so the call computes Cᵀ (N × M,
 // column-major, ld N) = op(B) · Aᵀ with B read transposed (ld K) and A as is (ld K).
@@ -12,6 +13,7 @@
 #include <mutex>
 #include <vector>
 
+#include "fhip_internal.h"
 #include "fracture_hip.h"
 
 namespace {
@@ -51,6 +53,8 @@ int fhip_launch_matmul(void* c, const void* a, const void* b, int m, int n, int 
     if (m < 0 || n < 0 || k < 0) return hipErrorInvalidValue;
     if (m == 0 || n == 0) return hipSuccess;
     if (!c || (k > 0 && (!a || !b))) return hipErrorInvalidValue;
+    if (fhip_internal::matmul_skinny_takes(c, a, b, m, n, k))
+        return fhip_internal::matmul_skinny(c, a, b, m, n, k, (hipStream_t)stream);
     std::lock_guard<std::mutex> g(handles().mu);
     rocblas_handle h;
     int e = device_handle(&h);

@@ -54,6 +54,25 @@ def test_matmul_vs_float64(dev, m, n, k):
                  f"matmul {m}x{n}x{k}")
 
 
+@pytest.mark.parametrize("m,n,k", [
+    # few rows: rows of B past the last full 16, K of one lane's 8, short of a 32-wide step, of the
+    # waves' shares and of their unrolled loads; the last m and sizes each kernel takes
+    (1, 1, 8), (1, 17, 24), (2, 1000, 4088), (3, 33, 1000), (8, 1024, 4096), (16, 100, 264), (17, 100, 264),
+    (5, 64, 36), (2, 16384, 2056), (3, 16384, 2056), (1, 40, 20000)])
+def test_matmul_few_rows(dev, m, n, k):
+    rng = np.random.default_rng(m * n + k)
+    a = rng.standard_normal((m, k)).astype(np.float16)
+    b = (rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float16)
+    ta, tb = torch.from_numpy(a).to(dev), torch.from_numpy(b).to(dev)
+    c = torch.full((m + 1, n), 7.0, dtype=torch.float16, device=dev)
+    K.matmul(c[:m], ta, tb)
+    torch.cuda.synchronize()
+    want = a.astype(np.float64) @ b.astype(np.float64).T
+    assert_close(c[:m].cpu().numpy().astype(np.float32), want.astype(np.float32), 1e-3, 1e-3,
+                 f"matmul {m}x{n}x{k}")
+    assert bool((c[m] == 7.0).all())
+
+
 def test_matmul_through_trait_checks_shapes(backend):
     a = backend.alloc([4, 8], DType.FP16)
     b = backend.alloc([3, 9], DType.FP16)
