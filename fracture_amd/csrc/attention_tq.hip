@@ -1125,7 +1125,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     }
     __syncthreads();
 
-    const int t_begin = blk * kPart + wave * (kPart / W);
+    const int t_begin = fhip_idx::split_begin(blk, wave, W, kPart);
     const int t_end = min(clen, t_begin + kPart / W);
     const int G = qh / kvh;
     const int32_t* table = qs.table + (int64_t)tq0 * qs.table_stride;

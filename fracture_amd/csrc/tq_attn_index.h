@@ -57,9 +57,9 @@ FHIP_IDX void split_grid_item(int64_t lin, int64_t total, int nsplit, int kvh, i
 // First position of wave `wave`'s split in block blk.
 FHIP_IDX int split_begin(int blk, int wave) { return (kBlockWaves * blk + wave) * kSplitPositions; }
 
-// The same with `waves` waves per workgroup (2, 4 or 8) sharing the block.
-FHIP_IDX int split_begin(int blk, int wave, int waves) {
-    return (blk * waves + wave) * (kBlockWaves * kSplitPositions / waves);
+// The same with `waves` waves per workgroup sharing a block of `part` positions.
+FHIP_IDX int split_begin(int blk, int wave, int waves, int part) {
+    return blk * part + wave * (part / waves);
 }
 
 // Lane j of a wave reads the block-table column of its split's page j, if that page holds

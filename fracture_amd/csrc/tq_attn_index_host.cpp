@@ -58,9 +58,9 @@ int fhip_idx_code_tables(int kvh, int g, int kbits, int vbits, uint32_t* k_off, 
     return 0;
 }
 
-// First position of wave `wave` of `waves` in block blk.
-int32_t fhip_idx_split_begin(int blk, int wave, int waves) {
-    return fhip_idx::split_begin(blk, wave, waves);
+// First position of wave `wave` of `waves` in block blk of `part` positions.
+int32_t fhip_idx_split_begin(int blk, int wave, int waves, int part) {
+    return fhip_idx::split_begin(blk, wave, waves, part);
 }
 
 // Workgroup wg of a launch with kvh kv heads -> its item and kv head.

@@ -455,8 +455,10 @@ def test_transposed_reads_of_8_bit_codes():
                         assert got == pos * 128 + 16 * c + n
 
 
-@pytest.mark.parametrize("waves", [2, 8])
-def test_split_begin_tiles_the_block(waves):
+@pytest.mark.parametrize("waves,part", [(2, SPLIT), (8, SPLIT), (4, 256)])
+def test_split_begin_tiles_the_block(waves, part):
     L = index_lib().lib
-    begins = [L.fhip_idx_split_begin(3, w, waves) for w in range(waves)]
-    assert begins == [3 * SPLIT + w * (SPLIT // waves) for w in range(waves)]
+    begins = [L.fhip_idx_split_begin(3, w, waves, part) for w in range(waves)]
+    assert begins == [3 * part + w * (part // waves) for w in range(waves)]
+    if (waves, part) == (2, SPLIT):  # the split that the model above walks
+        assert begins[1] == index_lib().split(3, 1, 1 << 20)[0]

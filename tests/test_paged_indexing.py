@@ -144,3 +144,55 @@ def test_column_mapping_error_is_caught():
     """The model fails when the acc loop's column counter wraps at the wrong head count."""
     with pytest.raises(AssertionError):
         model_split_kernel(13, 8, 4, 300, 0, wrap=3, hd=256)
+
+
+def prefill_split(nq, qh, kvh, extent, nsplit_ws, cols=128, tile=64, groups=512):
+    """The launchers' choice for the tiled prefill kernels: queries per block, blocks, splits."""
+    nqb = cols // (qh // kvh)
+    nblk = -(-nq // nqb)
+    base = nblk * kvh
+    want = min(max(-(-groups // base), 1), nsplit_ws)
+    pos = -(-(-(-extent // want)) // tile) * tile
+    return nqb, nblk, -(-extent // pos), pos
+
+
+@pytest.mark.parametrize("nq,qh,kvh,kv_len,start_pos", [
+    (2, 8, 8, 40, 38), (130, 32, 8, 1130, 1000), (129, 128, 128, 2100, 1971), (37, 24, 3, 1200, 1163),
+    (1000, 32, 8, 4001, 3001), (70, 7, 1, 70, 0), (65, 16, 2, 5000, 4000)])
+@pytest.mark.parametrize("fold", [False, True])
+def test_tiled_prefill_covers_every_partial(nq, qh, kvh, kv_len, start_pos, fold):
+    """Workgroups of the tiled prefill kernels (128 columns of one kv head, one split): each
+    (vector, split) below the vector's causal length is written once, no split count exceeds the
+    workspace's, tiles start inside a 64-page window with their four pages, and the order of blocks
+    (from the last down, or folded) is a permutation."""
+    G = qh // kvh
+    ws = max(1, -(-(-(-kv_len // PAGE) * PAGE) // SPLIT))
+    nqb, nblk, nsplit, pos = prefill_split(nq, qh, kvh, kv_len, ws)
+    assert nsplit <= ws and pos % 64 == 0
+    half = max(1, nblk // 2) if fold else 0
+    order = [bi - half if fold and bi >= half else nblk - 1 - bi for bi in range(nblk)]
+    assert sorted(order) == list(range(nblk))
+    written = {}
+    for blk in order:
+        q0 = blk * nqb
+        n = min(nqb, nq - q0)
+        clen = min(start_pos + q0 + n, kv_len)
+        for split in range(nsplit):
+            t_begin = split * pos
+            if nsplit > 1 and t_begin >= clen:
+                continue
+            win = t_begin
+            for t0 in range(t_begin, min(clen, t_begin + pos), 64):
+                if t0 >= win + 64 * PAGE:
+                    win = t0
+                assert 0 <= (t0 - win) // PAGE <= 60 and (t0 - win) % PAGE == 0
+            for col in range(n * G):
+                for g in range(kvh):
+                    key = ((q0 + col // G) * qh + g * G + col % G, split)
+                    assert key not in written
+                    written[key] = min(clen, t_begin + pos)
+    for qi in range(nq):
+        c = min(start_pos + qi + 1, kv_len)
+        for s in range(-(-c // pos)):
+            for h in range(qh):
+                assert written[(qi * qh + h, s)] >= min(c, (s + 1) * pos)
