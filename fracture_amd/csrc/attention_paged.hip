@@ -121,8 +121,9 @@ struct PQueries {
 // partials stay one per split whatever W is (kSplits8 / kSplits4 choose it). With a wave per split
 // the chunk's loads had nothing beside them to hide behind: 16 sequences of 500 .. 8192
 // positions (32 / 8 heads of 128, 285 MB) went from 136 to 72 us.
+// W = 1 puts two splits of neighbouring kv heads, each a wave's own, in a workgroup instead.
 template <int HD, int NH, int W, class Pages>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void
+__global__ __launch_bounds__(64 * (W == 1 ? 2 : W)) __attribute__((amdgpu_waves_per_eu(2))) void
 paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, int qh, int kvh,
                         int nhb, float scale_log2, float* __restrict__ part_ml,
                         float* __restrict__ part_acc, int nsplit, int tok) {
@@ -139,15 +140,18 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
     // heads are written and never read): a store guarded by the lane index followed by reads
     // of every lane lets the compiler sink the reads into the guarded block, where they run
     // with the other lanes switched off (seen in a variant of this loop at head_dim 32).
-    __shared__ __attribute__((aligned(16))) float pbuf[W][kChunk][16];
-    __shared__ __attribute__((aligned(16))) float abuf[W][64];
+    constexpr int kWaves = W == 1 ? 2 : W;  // of the workgroup
+    __shared__ __attribute__((aligned(16))) float pbuf[kWaves][kChunk][16];
+    __shared__ __attribute__((aligned(16))) float abuf[kWaves][64];
     // the waves' states for the merge: (m, l) per column, and the accumulators
-    __shared__ float mlbuf[W][2][16];
-    __shared__ __attribute__((aligned(16))) float sbuf[W][NH][HD];
+    __shared__ float mlbuf[kWaves][2][16];
+    __shared__ __attribute__((aligned(16))) float sbuf[kWaves][NH][HD];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t item = blockIdx.x;  // every exit before the merge is uniform over the workgroup
+    // W > 1: every exit before the merge's barrier is uniform over the workgroup
+    const int64_t item = W == 1 ? (int64_t)blockIdx.x * 2 + wave : blockIdx.x;
+    const int piece = W == 1 ? 0 : wave;  // of the split
     const int64_t per_q = (int64_t)kvh * nhb * nsplit;
     // queries tq0 .. tq0 + ntok - 1 (tok > 1 only in causal prefill over one shared table
     // with nhb == 1, where causal lengths grow with the query index)
@@ -160,7 +164,7 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
     const int split = (int)((item / ((int64_t)kvh * nhb)) % nsplit);
     const int clen = qs.causal_len(tq0 + ntok - 1);
     if (split * kPSplit >= clen) return;
-    const int t_begin = split * kPSplit + wave * kPiece;  // may lie past t_end: an empty piece
+    const int t_begin = split * kPSplit + piece * kPiece;  // may lie past t_end: an empty piece
     const int t_end = min(clen, t_begin + kPiece);
     const int G = qh / kvh;
     const int h0 = g * G + hb * kHeadsMax;
@@ -342,24 +346,28 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
             *(f4_t*)(dst + 4) = f4_t{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
         }
     }
-    __syncthreads();
+    if constexpr (W == 1)
+        wave_lds_sync();
+    else
+        __syncthreads();
     // ---- merge in wave order: column c's vector is (query tq0 + c / G, head h0 + c % G); a
     // wave with m = -inf (an empty or fully masked piece) adds nothing
-    for (int i = threadIdx.x; i < ncols * (HD / 4); i += 64 * W) {
+    const int own = W == 1 ? wave : 0;  // the split's first wave
+    for (int i = W == 1 ? lane : (int)threadIdx.x; i < ncols * (HD / 4); i += 64 * W) {
         const int c = i / (HD / 4), d = 4 * (i - c * (HD / 4));
         const int cq = tok > 1 ? c / G : 0;
         float M = -__builtin_inff();
 #pragma unroll
-        for (int w = 0; w < W; ++w) M = fmaxf(M, mlbuf[w][0][c]);
+        for (int w = 0; w < W; ++w) M = fmaxf(M, mlbuf[own + w][0][c]);
         float L = 0.0f;
         f4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int w = 0; w < W; ++w) {
-            const float mw = mlbuf[w][0][c];
+            const float mw = mlbuf[own + w][0][c];
             if (mw == -__builtin_inff()) continue;
             const float wt = __builtin_amdgcn_exp2f(mw - M);
-            L = fmaf(wt, mlbuf[w][1][c], L);
-            const f4_t a = *(const f4_t*)&sbuf[w][c][d];
+            L = fmaf(wt, mlbuf[own + w][1][c], L);
+            const f4_t a = *(const f4_t*)&sbuf[own + w][c][d];
 #pragma unroll
             for (int k = 0; k < 4; ++k) o[k] = fmaf(wt, a[k], o[k]);
         }
@@ -847,37 +855,53 @@ __global__ __launch_bounds__(kCombThreads) void paged_attn_combine_kernel(
     }
 }
 
-// The same merge with one wave per vector, four vectors per workgroup, for launches with at
-// most 8 splits per vector (contexts up to 8192 positions; causal prefill): lane s holds split
-// s's (m, l) and the weights reach the dim loop by lane broadcasts, so no LDS and no barrier.
-// A workgroup per vector spent most of its time being scheduled at prefill sizes.
+// The same merge for launches with at most 8 splits per vector (contexts up to 8192 positions; causal
+// prefill) and head_dim a multiple of 4: half a wave per vector, eight vectors per workgroup. Lane s
+// of the half holds split s's (m, l), the weights reach the dim loop by lane broadcasts, and every lane
+// loads 16 bytes of each split: no LDS, no barrier. A workgroup per vector spent most of its time
+// being scheduled at prefill sizes. The call of 32000 vectors of 2 splits (1000 queries at 3001):
+// 108.9 us with a wave per vector and 4-byte loads, 103.8 with this.
 constexpr int kCombWaveMaxSplits = 8;
-__global__ __launch_bounds__(256) void paged_attn_combine_wave_kernel(
+__global__ __launch_bounds__(256) void paged_attn_combine_half_kernel(
     PQueries qs, const float* __restrict__ ml, const float* __restrict__ acc,
     uint16_t* __restrict__ out, int qh, int hd, int nsplit, int64_t nvec, int split_pos) {
-    const int lane = threadIdx.x & 63;
-    const int64_t vec = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (vec >= nvec) return;
-    const int clen = qs.causal_len((int)(vec / qh));
+    const int l32 = threadIdx.x & 31;
+    const int64_t vec = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
+    const bool live = vec < nvec;  // dead halves join the shuffles on vector 0's numbers
+    const int64_t v = live ? vec : 0;
+    const int clen = qs.causal_len((int)(v / qh));
     const int ns = (clen + split_pos - 1) / split_pos;  // <= nsplit <= kCombWaveMaxSplits
-    const float* m = ml + vec * nsplit * 2;
-    const float ms = lane < ns ? m[2 * lane] : -__builtin_inff();
-    const float ls = lane < ns ? m[2 * lane + 1] : 0.0f;
-    const float M = wave_max(ms);
-    const float w = lane < ns && M != -__builtin_inff() ? expf(ms - M) : 0.0f;
-    const float L = wave_sum(w * ls);
-    float ws[kCombWaveMaxSplits];
+    const float* m = ml + v * nsplit * 2;
+    const float ms = l32 < ns ? m[2 * l32] : -__builtin_inff();
+    const float ls = l32 < ns ? m[2 * l32 + 1] : 0.0f;
+    float M = ms;
 #pragma unroll
-    for (int j = 0; j < kCombWaveMaxSplits; ++j) ws[j] = __shfl(w, j);
-    const float* a = acc + vec * nsplit * hd;
-    for (int d = lane; d < hd; d += 64) {
-        float av[kCombWaveMaxSplits];
+    for (int o = 4; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));  // lanes 0..7 of the half
+    M = __shfl(M, threadIdx.x & 32);
+    const float w = l32 < ns && M != -__builtin_inff() ? expf(ms - M) : 0.0f;
+    float ws[kCombWaveMaxSplits], L = 0.0f;
 #pragma unroll
-        for (int j = 0; j < kCombWaveMaxSplits; ++j) av[j] = j < ns ? a[(int64_t)j * hd + d] : 0.0f;
-        float o = 0.0f;
+    for (int j = 0; j < kCombWaveMaxSplits; ++j) {
+        ws[j] = __shfl(w, (threadIdx.x & 32) + j);
+        L += ws[j] * __shfl(ls, (threadIdx.x & 32) + j);
+    }
+    if (!live) return;
+    const float* a = acc + v * nsplit * hd;
+    for (int d = 4 * l32; d < hd; d += 128) {
+        f4_t av[kCombWaveMaxSplits];
 #pragma unroll
-        for (int j = 0; j < kCombWaveMaxSplits; ++j) o = fmaf(ws[j], av[j], o);
-        out[vec * hd + d] = (uint16_t)f2h(L > 0.0f ? o / L : 0.0f);
+        for (int j = 0; j < kCombWaveMaxSplits; ++j)
+            av[j] = j < ns ? *(const f4_t*)(a + (int64_t)j * hd + d) : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        f4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int j = 0; j < kCombWaveMaxSplits; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[k] = fmaf(ws[j], av[j][k], o[k]);
+        u32x2 r;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            r[k] = f2h(L > 0.0f ? o[2 * k] / L : 0.0f) | (f2h(L > 0.0f ? o[2 * k + 1] / L : 0.0f) << 16);
+        *(u32x2*)(out + v * hd + d) = r;
     }
 }
 
@@ -901,15 +925,18 @@ bool paged_shape_ok(int qh, int kvh, int hd) {
 // 32 / 8 heads of 128: 94 us with a wave per split, 36 / 25 / 20 us with 2 / 4 / 8). Many: the
 // chip is full with two, and more only add merge work and empty pieces at the ragged ends (64
 // sequences of 500 .. 2000, 1024 workgroups: 77 / 93 / 85 us). In between, at 512 workgroups
-// (32 / 4 heads): 68 / 49 / 56 us.
-constexpr int64_t kSplits8 = 256, kSplits4 = 512;
+// (32 / 4 heads): 68 / 49 / 56 us. One wave per split where even that fills every CU several times
+// over, two splits to a workgroup (64 sequences up to 32768, 16384 splits: 810 us, 820 with two waves
+// per split, 848 with one-wave workgroups).
+constexpr int64_t kSplits8 = 256, kSplits4 = 512, kSplits2 = 4096;
 template <int HD, int NH, int W, class Pages>
 void launch_split_w(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
                     int nhb, float* ml, float* acc, int nsplit, int tok, int64_t items,
                     hipStream_t s) {
     const float scale_log2 = 1.4426950408889634f / sqrtf((float)HD);
-    hipLaunchKernelGGL((paged_attn_split_kernel<HD, NH, W, Pages>), dim3((unsigned)items),
-                       dim3(64 * W), 0, s, q, qs, pg, qh, kvh, nhb, scale_log2, ml, acc, nsplit,
+    const int64_t wgs = W == 1 ? ceil_div(items, 2) : items;
+    hipLaunchKernelGGL((paged_attn_split_kernel<HD, NH, W, Pages>), dim3((unsigned)wgs),
+                       dim3(64 * (W == 1 ? 2 : W)), 0, s, q, qs, pg, qh, kvh, nhb, scale_log2, ml, acc, nsplit,
                        tok);
 }
 template <int HD, int NH, class Pages>
@@ -920,8 +947,10 @@ void launch_split_t(const uint16_t* q, const PQueries& qs, const Pages& pg, int 
         launch_split_w<HD, NH, 8>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
     else if (items <= kSplits4)
         launch_split_w<HD, NH, 4>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
-    else
+    else if (items <= kSplits2)
         launch_split_w<HD, NH, 2>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+    else
+        launch_split_w<HD, NH, 1>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
 }
 
 template <int HD, class Pages>
@@ -947,8 +976,9 @@ void launch_prefill_t(const uint16_t* q, const PQueries& qs, const Pages& pg, in
 // The merge of nsplit splits of split_pos positions per vector.
 void launch_combine(const PQueries& qs, const float* ml, const float* acc, void* out, int64_t nvec,
                     int qh, int hd, int nsplit, int split_pos, hipStream_t s) {
-    if (nsplit <= kCombWaveMaxSplits)
-        hipLaunchKernelGGL(paged_attn_combine_wave_kernel, dim3((unsigned)ceil_div(nvec, 4)),
+    if (nsplit <= kCombWaveMaxSplits && hd % 4 == 0 && fhip_host::aligned16(acc) &&
+        ((uintptr_t)out & 7) == 0)
+        hipLaunchKernelGGL(paged_attn_combine_half_kernel, dim3((unsigned)ceil_div(nvec, 8)),
                            dim3(256), 0, s, qs, ml, acc, (uint16_t*)out, qh, hd, nsplit, nvec,
                            split_pos);
     else

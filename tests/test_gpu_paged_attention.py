@@ -67,9 +67,10 @@ def test_decode_small_contexts(dev, hd, qh, kvh):
 
 
 @pytest.mark.parametrize("nseq,qh,kvh,hd", [
-    (32, 8, 8, 64), (33, 8, 8, 64), (33, 32, 8, 128), (64, 16, 8, 32), (65, 16, 8, 128), (65, 16, 8, 256)])
+    (32, 8, 8, 64), (33, 8, 8, 64), (33, 32, 8, 128), (64, 16, 8, 32), (65, 16, 8, 128), (65, 16, 8, 256),
+    (65, 64, 64, 32)])
 def test_decode_waves_per_split(dev, nseq, qh, kvh, hd):
-    """8, 4 and 2 waves per split (up to 256, up to 512 and more workgroups): lengths that leave
+    """8, 4, 2 and 1 waves per split (up to 256, 512, 4096 and more workgroups): lengths that leave
     waves empty, end inside each wave's piece and on its edges, and a masked page that is a
     wave's whole piece of one chunk."""
     rng = np.random.default_rng(nseq + hd)
