@@ -1397,7 +1397,10 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
                 for (int pt = 0; pt < 4; ++pt)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (!(row_ok && t0 + 16 * rg + 4 * e + pt < lim)) sc[pt][e] = -__builtin_inff();
+                        if (!(row_ok && t0 + 16 * rg + 4 * e + pt < lim)) {
+                            sc[pt][e] = -__builtin_inff();
+                            vn[4 * e + pt] = 0.0f;  // an infinite or NaN norm past the column's length
+                        }
             }
             float cmax = -__builtin_inff();
 #pragma unroll

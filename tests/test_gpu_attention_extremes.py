@@ -1,0 +1,53 @@
+"""Attention where its inputs leave the ordinary range: norms that are not finite past a query's
+length, centroid tables far from 1, weights far below the largest, NaN scores."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from fracture_amd import kernels as K
+from test_gpu_attention import build_pool, dev_t, run_prefill
+from test_gpu_paged_attention import run_decode
+
+pytestmark = pytest.mark.gpu
+
+WIDTHS = [(8, 8), (4, 2), (4, 4), (3, 3), (2, 2)]
+
+
+def tq_want(pool, q, n, kbits, vbits, kvh, rows=None):
+    rows = pool["table"][0] if rows is None else rows
+    return oracle.tq_attention(q, rows, n, pool["KP"], pool["KN"], pool["VP"], pool["VN"], pool["krot"],
+                               pool["vrot"], pool["kc"], pool["vc"], kbits, vbits, kvh).astype(np.float32)
+
+
+def assert_rel(got, want, rel, what=""):
+    """|got - want| <= rel * the row's largest magnitude."""
+    err = np.abs(got - want).max(-1) / np.abs(want).max(-1)
+    assert np.isfinite(got).all() and err.max() <= rel, f"{what}: {err.max()}"
+
+
+def run_tq_decode(dev, pool, q, lens, kbits, vbits, kvh):
+    out = torch.empty(q.shape, dtype=torch.float16, device=dev)
+    K.attention_tq_decode(out, dev_t(q, dev), dev_t(pool["table"], dev), dev_t(np.array(lens, np.int32), dev),
+                          *(dev_t(pool[n], dev) for n in ("KP", "KN", "VP", "VN", "krot", "vrot", "kc", "vc")),
+                          kbits, vbits, kvh)
+    torch.cuda.synchronize()
+    return out.cpu().numpy().astype(np.float32)
+
+
+@pytest.mark.parametrize("kbits,vbits", WIDTHS)
+@pytest.mark.parametrize("qh,kvh,T,kv_len", [(8, 2, 6, 90), (8, 4, 8, 131), (8, 8, 9, 300)])
+def test_short_prefill_hides_later_norms(dev, kbits, vbits, qh, kvh, T, kv_len):
+    """Queries that share MFMA columns (8 / G of them): a value norm of infinity and a key norm of NaN at
+    the last two positions reach the queries that see them and no earlier one."""
+    rng = np.random.default_rng(kbits * 10 + T)
+    pool = build_pool(rng, [kv_len], kvh, 128, kbits, vbits)
+    table = pool["table"][0]
+    pool["VN"][table[(kv_len - 2) // 16], (kv_len - 2) % 16] = np.inf
+    pool["KN"][table[(kv_len - 1) // 16], (kv_len - 1) % 16] = np.nan
+    q = rng.standard_normal((T, qh, 128)).astype(np.float16)
+    got = run_prefill(dev, pool, q, kvh, kv_len, kv_len - T, kbits, vbits)
+    for t in range(T - 2):
+        # fp16 rounding of the output (2^-11) and of the oracle's, plus fp32 sums
+        assert_rel(got[t], tq_want(pool, q[t], kv_len - T + t + 1, kbits, vbits, kvh), 2e-3, f"token {t}")
+    assert not np.isfinite(got[T - 2]).any()
