@@ -698,6 +698,31 @@ __device__ __forceinline__ uint32_t hi_lo_pair(float v, float& hi_f) {
     return (uint32_t)__builtin_bit_cast(uint16_t, hi) |
            ((uint32_t)__builtin_bit_cast(uint16_t, lo) << 16);
 }
+// e with |x| < 2^e (and >= 2^(e-1)) for normal x; infinities and NaN give 129, 0 gives -126.
+__device__ __forceinline__ int exponent_above(float x) {
+    return (int)((__float_as_uint(x) >> 23) & 0xffu) - 126;
+}
+__device__ __forceinline__ float exp2i(int e) { return ldexpf(1.0f, e); }
+// The power of two that brings magnitudes up to x below 2^kScaleExp, so that an fp16 hi + lo pair of a
+// scaled value holds 22 bits whatever range the fp32 values come in.
+constexpr int kScaleExp = 8;
+__device__ __forceinline__ int scale_exponent(float x) { return kScaleExp - max(exponent_above(x), -100); }
+// A table of 2^B centroids in a wave's registers (centroid 64 k + lane, the last one repeated), and the
+// exponent that scales it.
+template <int B>
+struct Centroids {
+    float v[B == 8 ? 4 : 1];
+    int e;
+    __device__ void load(const float* cent) {
+        const int lane = threadIdx.x & 63;
+        for (int k = 0; k < (B == 8 ? 4 : 1); ++k) v[k] = cent[min(64 * k + lane, (1 << B) - 1)];
+    }
+    __device__ void find_exponent() {
+        float m = 0.0f;
+        for (int k = 0; k < (B == 8 ? 4 : 1); ++k) m = fmaxf(m, fabsf(v[k]));
+        e = __builtin_amdgcn_readfirstlane(scale_exponent(wave_max(m)));
+    }
+};
 __device__ __forceinline__ float ror8(float v) {  // lane n of each 16-lane row gets lane n^8
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xF, 0xF, true));
 }
@@ -964,7 +989,11 @@ __device__ __forceinline__ void store_v8(const u32x4 (&r)[8], uint8_t* vb, int l
     for (int i = 0; i < 8; ++i) *(u32x4*)(vb + 1024 * i + 16 * lane) = r[i];
 }
 
-// Norms of position t0 + lane, loaded raw (fp16 bits): pack() gives (knorm, vnorm) in fp32
+// Value norms enter the weights as quarters: a weight's w_hi, rounded toward zero, then leaves less than
+// 8, and lo' = 2^12 of that stays in fp16's range up to the largest norm.
+constexpr float kNormVUnit = 0.25f;
+constexpr int kNormVExp = 2;  // 1 / kNormVUnit = 2^kNormVExp
+// Norms of position t0 + lane, loaded raw (fp16 bits): pack() gives (knorm, vnorm kNormVUnit) in fp32
 // once they are needed (0 where there is none), so each norm is converted once, by the lane
 // that loaded it. Packing later keeps the wait for them away from the copies issued after them.
 struct NormRegs {
@@ -975,7 +1004,7 @@ struct NormRegs {
         // pins the pack here: the compiler would otherwise pack right after the loads
         asm volatile("" : "+v"(a), "+v"(b));
         const float fk = (float)__builtin_bit_cast(_Float16, (uint16_t)a);
-        const float fv = (float)__builtin_bit_cast(_Float16, (uint16_t)b);
+        const float fv = (float)__builtin_bit_cast(_Float16, (uint16_t)b) * kNormVUnit;
         return ok ? float2{fk, fv} : float2{0.0f, 0.0f};
     }
 };
@@ -1110,18 +1139,38 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     const int blk = (int)(item % nblk);
     const int clen = qs.causal_len(tq_last);  // the group's longest causal length
     if (blk * kPart >= clen) return;
-    for (int b = threadIdx.x; b < 256; b += 64 * W) {
-        float hf;
-        auto code = [](const float* cent, int c, int bits) { return cent[min(c, (1 << bits) - 1)]; };
-        if constexpr (KB == 8)
-            ((uint32_t*)pk)[b] = hi_lo_pair(kcent[b], hf);
-        else
-            pk[b] = u32x2{hi_lo_pair(code(kcent, b >> 4, KB), hf), hi_lo_pair(code(kcent, b & 15, KB), hf)};
-        if constexpr (VB == 8)
-            ((uint32_t*)pv)[b] = hi_lo_pair(vcent[b], hf);
-        else
-            pv[b] = u32x2{hi_lo_pair(code(vcent, b & 15, VB), hf), hi_lo_pair(code(vcent, b >> 4, VB), hf)};
-        if (b == 0) waves_done = 0;
+    int ek, ev;
+    {
+        Centroids<KB> ck;
+        Centroids<VB> cv;
+        ck.load(kcent);
+        cv.load(vcent);
+        ck.find_exponent();
+        cv.find_exponent();
+        ek = ck.e;
+        ev = cv.e;
+        // each wave fills its share of the entries 64 k + lane
+        auto fill = [&](auto& c, u32x2* tab, int bits, bool high_first) {
+            float hf;
+            if (bits == 8) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (k % W == wave) ((uint32_t*)tab)[64 * k + lane] = hi_lo_pair(ldexpf(c.v[k % (sizeof(c.v) / 4)], c.e), hf);
+            } else {
+                const int word = (int)hi_lo_pair(ldexpf(c.v[0], c.e), hf);  // lane: its code's
+                const int low = __shfl(word, lane & 15);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const int high = __shfl(word, 4 * k + (lane >> 4));
+                    if (k % W == wave)
+                        tab[64 * k + lane] = high_first ? u32x2{(uint32_t)high, (uint32_t)low}
+                                                        : u32x2{(uint32_t)low, (uint32_t)high};
+                }
+            }
+        };
+        fill(ck, pk, KB, true);
+        fill(cv, pv, VB, false);
+        if (threadIdx.x == 0) waves_done = 0;
     }
     __syncthreads();
 
@@ -1179,17 +1228,30 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     KCodes<KB> kreg;
     load_k<KB>(pages, 0, kvh, g, lane, kreg);
 
-    // Q as the QK B operand, pre-scaled by scale * log2(e) so scores come out in log2 units:
-    // step s, lane (n, rg) holds coordinates 32rg + 4s + c4.
+    // Q as the QK B operand, scaled like the tables: step s, lane (n, rg) holds coordinates
+    // 32rg + 4s + c4. What a score is then multiplied by, with the key's norm, to be in log2 units
+    // (never 0: a masked score stays -inf):
+    float colscale;
     uint32_t bq[8][4];
     {
         // heads past G read head 0 and are zeroed by the multiplier
         // columns past the group's heads read the group's first vector and are zeroed
         const float* qsrc = qrot + qvec * hd;
-        const float qmul = col_ok ? scale * 1.4426950408889634f : 0.0f;
         f32x4_t qv[8];
 #pragma unroll
         for (int s8 = 0; s8 < 8; ++s8) qv[s8] = *(const f32x4_t*)(qsrc + fhip_idx::q_lane_offset(lane, s8));
+        float qmax = 0.0f;
+#pragma unroll
+        for (int s8 = 0; s8 < 8; ++s8)
+#pragma unroll
+            for (int c4 = 0; c4 < 4; ++c4) qmax = fmaxf(qmax, fabsf(qv[s8][c4]));
+        qmax = fmaxf(qmax, __shfl_xor(qmax, 16));
+        qmax = fmaxf(qmax, __shfl_xor(qmax, 32));
+        const int eq = scale_exponent(qmax);
+        const float qmul = col_ok ? exp2i(eq) : 0.0f;
+        colscale = fmaxf(ldexpf(scale * 1.4426950408889634f, -eq - ek), 0x1p-126f);
+        // kG4: lane 4 pt + h holds head h's scores
+        if constexpr (kG4) colscale = __shfl(colscale, (lane & 48) | (lane & 3));
 #pragma unroll
         for (int s8 = 0; s8 < 8; ++s8) {
 #pragma unroll
@@ -1355,13 +1417,13 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
             cmax = bank_max(cmax);
             cmax = fmaxf(cmax, xrow(bp16, cmax));
             cmax = fmaxf(cmax, xrow(bp32, cmax));
-            m_new = fmaxf(m_run, cmax);
+            m_new = fmaxf(m_run, cmax * colscale);
             alpha = m_run == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
             float psum = 0.0f;
             const float mref = m_new == -__builtin_inff() ? 0.0f : m_new;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float pr = __builtin_amdgcn_exp2f(scc[e] - mref);
+                const float pr = __builtin_amdgcn_exp2f(fmaf(scc[e], colscale, -mref));
                 psum += pr;
                 const float w = pr * vn[e];
                 // w_hi = w rounded toward zero; lo' = f16(2^12 (w - w_hi)) in place of r.lo
@@ -1409,7 +1471,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
                 for (int e = 0; e < 4; ++e) cmax = fmaxf(cmax, sc[pt][e]);
             cmax = fmaxf(cmax, xrow(bp16, cmax));
             cmax = fmaxf(cmax, xrow(bp32, cmax));
-            m_new = fmaxf(m_run, cmax);
+            m_new = fmaxf(m_run, cmax * colscale);
             alpha = m_run == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
             // ---- probabilities, weights, B operands of PV
             float psum = 0.0f;
@@ -1418,7 +1480,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
             for (int pt = 0; pt < 4; ++pt) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float pr = __builtin_amdgcn_exp2f(sc[pt][e] - mref);
+                    const float pr = __builtin_amdgcn_exp2f(fmaf(sc[pt][e], colscale, -mref));
                     psum += pr;
                     const float w = pr * vn[4 * e + pt];
                     uint32_t r = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(w, w));
@@ -1518,11 +1580,12 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     constexpr int kStM = kMaxG * kStRow, kStL = kStM + kMaxG;
     float* st = (float*)vb;
     static_assert(sizeof(vbuf[0]) >= (kStL + kMaxG) * sizeof(float), "merge state");
+    const float vunit = exp2i(kNormVExp - ev), vunit_lo = vunit * (1.0f / 4096.0f);
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
         f32x4_t v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e ^ kSwap] = fmaf(ror8(acc[c][e]), 1.0f / 4096.0f, acc[c][e]);
+        for (int e = 0; e < 4; ++e) v[e ^ kSwap] = fmaf(ror8(acc[c][e]), vunit_lo, acc[c][e] * vunit);
         if (n < ncols) *(f32x4_t*)&st[n * kStRow + 16 * c + 4 * rg] = v;
     }
     if (n < ncols && rg == 0) {
@@ -1603,7 +1666,6 @@ constexpr int kPqRowK = 256 + 16;       // bytes per K row in LDS: 16 rows' 16-b
 constexpr int kPqRowV = 256 + 64;       // per V row: the transposed reads of 4 rows x 32 dims
 constexpr float kPqBias = 7.0f;         // log2 of the scale that p carries
 constexpr float kPqSlack = 8.0f;        // log2 that p may exceed it by before a rescale
-constexpr int kPqScaleExp = 8;          // centroids and queries are scaled below 2^8
 constexpr int64_t kPqGroups = 512;      // workgroups wanted: the two per CU that fit at once
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x2c_t __attribute__((ext_vector_type(2)));
@@ -1617,12 +1679,6 @@ __device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint3
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(lb) : "v"(hi), "v"(b));
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2c_t{la, lb}), f16x2c_t));
 }
-// e with |x| < 2^e (and >= 2^(e-1)) for normal x; infinities and NaN give 129, 0 gives -126.
-__device__ __forceinline__ int exponent_above(float x) {
-    return (int)((__float_as_uint(x) >> 23) & 0xffu) - 126;
-}
-__device__ __forceinline__ float exp2i(int e) { return ldexpf(1.0f, e); }
-
 // Codes of one thread's quarter row (32 codes) of a tile: 4 B bytes.
 template <int B>
 struct Codes32 {
@@ -1700,12 +1756,14 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
     const int t_end = min(clen, t_begin + split_pos);
     const int32_t* table = qs.table + (int64_t)q0 * qs.table_stride;
 
-    // ---- centroid tables, scaled to below 2^kPqScaleExp
-    float cmaxk = 0.0f, cmaxv = 0.0f;
-    for (int i = lane; i < (1 << KB); i += 64) cmaxk = fmaxf(cmaxk, fabsf(kcent[i]));
-    for (int i = lane; i < (1 << VB); i += 64) cmaxv = fmaxf(cmaxv, fabsf(vcent[i]));
-    const int ek = kPqScaleExp - max(exponent_above(wave_max(cmaxk)), -100);
-    const int ev = kPqScaleExp - max(exponent_above(wave_max(cmaxv)), -100);
+    // ---- centroid tables, scaled
+    Centroids<KB> ck;
+    Centroids<VB> cv;
+    ck.load(kcent);
+    cv.load(vcent);
+    ck.find_exponent();
+    cv.find_exponent();
+    const int ek = ck.e, ev = cv.e;
     {
         auto fill = [&](u32x2* tab, const float* cent, int bits, int e) {
             for (int b = threadIdx.x; b < 256; b += 64 * kPqWaves) {
@@ -1749,7 +1807,7 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
 #pragma unroll
             for (int k = 0; k < 8; ++k) m = fmaxf(m, fabsf(v[s][k >> 2][k & 3]));
         m = fmaxf(m, __shfl_xor(m, 32));
-        const int eq = kPqScaleExp - max(exponent_above(m), -100);
+        const int eq = scale_exponent(m);
 #pragma unroll
         for (int s = 0; s < 8; ++s)
 #pragma unroll

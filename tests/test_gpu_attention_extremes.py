@@ -51,3 +51,41 @@ def test_short_prefill_hides_later_norms(dev, kbits, vbits, qh, kvh, T, kv_len):
         # fp16 rounding of the output (2^-11) and of the oracle's, plus fp32 sums
         assert_rel(got[t], tq_want(pool, q[t], kv_len - T + t + 1, kbits, vbits, kvh), 2e-3, f"token {t}")
     assert not np.isfinite(got[T - 2]).any()
+
+
+@pytest.mark.parametrize("kbits,vbits", WIDTHS)
+@pytest.mark.parametrize("exp", [18, -18])
+@pytest.mark.parametrize("G,T", [(4, 1), (8, 1), (2, 5), (4, 130)])
+def test_centroid_tables_of_any_scale(dev, kbits, vbits, exp, G, T):
+    """Centroids times 2^exp, with norms and queries that bring scores and outputs back: past fp16's
+    range on either side, inside fp32's. Decode and the two prefill kernels."""
+    rng = np.random.default_rng(kbits + G)
+    kvh, kv_len = (8, 700) if T > 100 else (2, 300)
+    pool = build_pool(rng, [kv_len], kvh, 128, kbits, vbits)
+    pool["kc"], pool["vc"] = (pool[n] * np.float32(2.0 ** exp) for n in ("kc", "vc"))
+    back = np.float16(2.0 ** (-exp // 2))
+    pool["KN"], pool["VN"] = pool["KN"] * back, pool["VN"] * back
+    q = (rng.standard_normal((T, kvh * G, 128)) * float(back)).astype(np.float16)
+    if T == 1:
+        got = run_tq_decode(dev, pool, q, [kv_len], kbits, vbits, kvh)
+    else:
+        got = run_prefill(dev, pool, q, kvh, kv_len, kv_len - T, kbits, vbits)
+    for t in range(0, T, max(1, T // 10)):
+        assert_rel(got[t], tq_want(pool, q[t], kv_len - T + t + 1, kbits, vbits, kvh), 2e-3, f"token {t}")
+
+
+@pytest.mark.parametrize("kbits,vbits", WIDTHS)
+@pytest.mark.parametrize("G,T", [(4, 1), (8, 1), (2, 5), (4, 130)])
+def test_value_norms_up_to_the_largest(dev, kbits, vbits, G, T):
+    """Value norms of 2^15 and more: the low parts of the weights stay finite."""
+    rng = np.random.default_rng(kbits + G)
+    kvh, kv_len = (8, 700) if T > 100 else (2, 300)
+    pool = build_pool(rng, [kv_len], kvh, 128, kbits, vbits)
+    pool["VN"] = rng.uniform(3e4, 65504, pool["VN"].shape).astype(np.float16)
+    q = rng.standard_normal((T, kvh * G, 128)).astype(np.float16)
+    if T == 1:
+        got = run_tq_decode(dev, pool, q, [kv_len], kbits, vbits, kvh)
+    else:
+        got = run_prefill(dev, pool, q, kvh, kv_len, kv_len - T, kbits, vbits)
+    for t in range(0, T, max(1, T // 10)):
+        assert_rel(got[t], tq_want(pool, q[t], kv_len - T + t + 1, kbits, vbits, kvh), 2e-3, f"token {t}")
