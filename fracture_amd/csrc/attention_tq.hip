@@ -1110,7 +1110,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     // targets are separate objects: table reads never wait for DMA traffic.
     __shared__ u32x2 pk[256], pv[256];  // 8-bit codes: 256 words, one per code
     // two chunks of 4-bit V codes, by chunk parity, or one of 8-bit codes
-    __shared__ __attribute__((aligned(16))) uint8_t vbuf[W][2][kChunkM * 64];
+    __shared__ __attribute__((aligned(64))) uint8_t vbuf[W][2][kChunkM * 64];
     __shared__ __attribute__((aligned(16))) float2 nbuf[W][kChunkM];  // (knorm, vnorm)
     __shared__ PageAddrs pagebuf[W][kPart / W / FHIP_PAGE_TOKENS];  // the wave's split pages
     __shared__ int waves_done;  // waves that have left their state for the merge
@@ -1280,7 +1280,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     // transposed V reads: source lane m of group rg reads position 16rg + 4(m % 4) + m / 4;
     // segment s of that row sits at vrow[s ^ sw]. 8-bit codes: lane m reads half m % 2 of the
     // 16 dims of a tile at position 16rg + 4(k % 4) + k / 4 (+ 2 for tiles 2, 3), k = m / 2.
-    uint32_t vseg[VB == 8 ? 8 : 4];
+    uint32_t vseg[VB == 8 ? 8 : 1];
     const uint32_t vb32 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)vb;
     if constexpr (VB == 8) {
         const int k = n >> 1, srow = 16 * rg + 4 * (k & 3) + (k >> 2);
@@ -1290,8 +1290,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     } else {
         const int srow = 16 * rg + 4 * (n & 3) + (n >> 2);
         const int sw = (srow >> 1) & 3;
-#pragma unroll
-        for (int sg = 0; sg < 4; ++sg) vseg[sg] = vb32 + 64 * srow + 16 * (sg ^ sw);
+        vseg[0] = vb32 + 64 * srow + 16 * sw;  // segment s: exclusive or with 16 s (rows are aligned)
     }
 
     // kG4 (at most 4 query heads per kv head): scores, probabilities and weights are held
@@ -1513,7 +1512,8 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
             read_v_codes8<0>(vseg, tvs);
         } else {
             const uint32_t vo = (uint32_t)par * (kChunkM * 64);
-            const uint32_t seg[4] = {vseg[0] + vo, vseg[1] + vo, vseg[2] + vo, vseg[3] + vo};
+            const uint32_t s0 = vseg[0] + vo;
+            const uint32_t seg[4] = {s0, s0 ^ 16, s0 ^ 32, s0 ^ 48};
             read_v_codes(seg, tvs);
         }
         // out^T = V^T W^T: the V entries are the A operand (row m: dim 16c + (m ^ 1)), the
