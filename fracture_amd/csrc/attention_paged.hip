@@ -445,7 +445,7 @@ __device__ __forceinline__ void wave_attend(const uint16_t* qrow, const int32_t*
 //     position 4 half + j (j < 4) or 8 + 4 half + j - 4, exactly what the lane holds after S^T,
 //     so P goes into the B operand without moving between lanes. P = hi + lo in fp16, two
 //     products into one accumulator: the exponent is biased by kPfBias, so that lo is a normal
-//     fp16 number for every p above 2^-10 (p to ~2^-23; an absolute 2^-32 below that), and the
+//     fp16 number for every p above 2^-14 (p to ~2^-23; an absolute 2^-37 below that), and the
 //     bias cancels in out = acc / l. V is exact. A = V^T comes from the row-major tile by
 //     ds_read_b64_tr_b16.
 //   The next tile's rows are loaded into registers before the tile's products and stored to the
@@ -458,9 +458,9 @@ __device__ __forceinline__ void wave_attend(const uint16_t* qrow, const int32_t*
 constexpr int kPfWaves = 4;                // waves per workgroup
 constexpr int kPfCols = 32 * kPfWaves;     // (query, head) columns per workgroup
 constexpr int kPfTile = 64;                // positions per tile
-constexpr float kPfBias = 7.0f;            // log2 of the scale that P carries
-constexpr float kPfScale = 128.0f;         // 2^kPfBias
-constexpr float kPfSlack = 8.0f;           // log2 that p may exceed it by (2^15 < fp16's largest)
+constexpr float kPfBias = 12.0f;           // log2 of the scale that P carries
+constexpr float kPfScale = 4096.0f;        // 2^kPfBias
+constexpr float kPfSlack = 3.75f;          // log2 that p may exceed it by (2^15.75 < fp16's largest)
 constexpr int64_t kPfGroups = 512;         // workgroups wanted: the two per CU that fit at once
 typedef float f16x_t __attribute__((ext_vector_type(16)));
 

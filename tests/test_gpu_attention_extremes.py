@@ -89,3 +89,33 @@ def test_value_norms_up_to_the_largest(dev, kbits, vbits, G, T):
         got = run_prefill(dev, pool, q, kvh, kv_len, kv_len - T, kbits, vbits)
     for t in range(0, T, max(1, T // 10)):
         assert_rel(got[t], tq_want(pool, q[t], kv_len - T + t + 1, kbits, vbits, kvh), 2e-3, f"token {t}")
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128])
+@pytest.mark.parametrize("kv_len", [200, 5000])
+def test_fp16_prefill_small_weights(dev, hd, kv_len):
+    """One position holds nearly all the weight and no value; the output is what the others, at about
+    2^-24 of it, add up to. 2^-11 is the rounding of the output; a weight is right to 2^-37 of the largest,
+    2^-13 of itself here."""
+    T, qh, kvh = 64, 8, 2
+    P = (kv_len + 15) // 16
+    kp = np.zeros((P, 16, kvh, hd), np.float16)
+    vp = np.zeros((P, 16, kvh, hd), np.float16)
+    rng = np.random.default_rng(hd)
+    vp[:] = rng.uniform(4e4, 6e4, (kvh, hd)).astype(np.float16)
+    vp[0, 0] = 0
+    top = 16.6  # nats: 2^-24 = exp(-16.6)
+    kp[0, 0] = np.float16(top / np.sqrt(hd))
+    q = (np.ones((T, qh, hd)) * rng.uniform(0.93, 1.0, (T, qh, 1))).astype(np.float16)
+    tk, tv = dev_t(kp, dev), dev_t(vp, dev)
+    ptr = [torch.tensor([x.data_ptr() for x in t], dtype=torch.int64, device=dev) for t in (tk, tv)]
+    out = torch.empty(q.shape, dtype=torch.float16, device=dev)
+    K.paged_attention(out, dev_t(q, dev), torch.arange(P, dtype=torch.int32, device=dev), *ptr, kvh, kv_len,
+                      kv_len - T)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy().astype(np.float64)
+    s = q.astype(np.float64)[:, :, 0] * float(kp[0, 0, 0, 0]) * hd / np.sqrt(hd)
+    n = kv_len - T + 1 + np.arange(T)
+    w = (n[:, None] - 1) * np.exp(-s) / (1 + (n[:, None] - 1) * np.exp(-s))
+    want = w[:, :, None] * np.repeat(vp[1, 1].astype(np.float64), qh // kvh, 0)
+    assert np.abs(got / want - 1).max() <= 2.0 ** -11 + 2.0 ** -12
