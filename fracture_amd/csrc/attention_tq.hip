@@ -1650,8 +1650,9 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
 //   lo hi into one accumulator (what is left out is 2^-22 of the product). lo = x - hi stays a
 //   normal fp16 number because every factor is scaled by a power of two first: the centroids by
 //   their table's largest magnitude, a query by its own, the weights w = p norm_v by the largest
-//   value norm so far (e_run, for which the accumulators are rescaled like for the running
-//   maximum) and by 2^kPqBias. The scales are exact and leave with the score or the output.
+//   value norm that the column has seen (e_run, for which the accumulators are rescaled like for
+//   the running maximum) and by 2^kPqBias: an absolute 2^-38 of the largest w, in fp16 pairs. The
+//   scales are exact and leave with the score or the output.
 //   Lane layouts are those of the FP16 prefill kernel: lane (n, half) holds 16 positions of column n
 //   per 32-position block, which are its own slots of W^T.
 // Bound by the MFMA (96 products of 32 clocks per wave and tile) with the lookups (16 8-byte LDS
@@ -1664,8 +1665,10 @@ constexpr int kPqCols = 32 * kPqWaves;  // columns per workgroup
 constexpr int kPqTile = 64;             // positions per tile
 constexpr int kPqRowK = 256 + 16;       // bytes per K row in LDS: 16 rows' 16-byte reads on all banks
 constexpr int kPqRowV = 256 + 64;       // per V row: the transposed reads of 4 rows x 32 dims
-constexpr float kPqBias = 7.0f;         // log2 of the scale that p carries
-constexpr float kPqSlack = 8.0f;        // log2 that p may exceed it by before a rescale
+constexpr float kPqBias = 13.0f;        // log2 of the scale that p carries
+// log2 that p may exceed it by before a rescale: w < 2^16 (1 - 2^-11) (an fp16 norm's largest share of
+// its power of two), which fp16 holds
+constexpr float kPqSlack = 3.0f;
 constexpr int64_t kPqGroups = 512;      // workgroups wanted: the two per CU that fit at once
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x2c_t __attribute__((ext_vector_type(2)));
@@ -1737,7 +1740,7 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
     __shared__ __attribute__((aligned(16))) uint8_t kbuf[2][kPqTile * kPqRowK];  // hi, lo
     __shared__ __attribute__((aligned(16))) uint8_t vbuf[2][kPqTile * kPqRowV];
     __shared__ __attribute__((aligned(16))) float nbuf[2][kPqTile];  // norm_k scale log2(e), norm_v
-    __shared__ float tmax[2];  // the largest centroid magnitudes, then [0] the tile's largest norm_v
+    __shared__ float tmax;  // the tile's largest norm_v
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1872,12 +1875,12 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
             nbuf[0][lane] = a;
             nbuf[1][lane] = b;
             const float m = wave_max(fabsf(b));
-            if (lane == 0) tmax[0] = m;
+            if (lane == 0) tmax = m;
         }
     };
 
     float m_run = -__builtin_inff(), l_run = 0.0f;  // l: the lane half's own positions
-    int e_run = -100;  // the accumulators are in units of 2^e_run (norm_v below it)
+    int e_run = -100;  // the column's accumulators are in units of 2^e_run (norm_v below it)
     f32x16_t acc[4];
 #pragma unroll
     for (int d = 0; d < 4; ++d)
@@ -1947,15 +1950,24 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
 #pragma unroll
                     for (int k = 0; k < 4; ++k) sc[pt][4 * j + k] *= nk[k];
                 }
+            float vmax = tmax;
             if (masked) {
+                vmax = 0.0f;  // of the positions that the column sees
 #pragma unroll
                 for (int pt = 0; pt < 2; ++pt)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) {
-                        const int pos = t0 + 32 * pt + 8 * (i / 4) + 4 * half + i % 4;
-                        const bool ok = ((tile_pok >> (2 * pt + i / 8)) & 1u) && pos < lim;
-                        sc[pt][i] = ok ? sc[pt][i] : -__builtin_inff();
+                    for (int j = 0; j < 4; ++j) {
+                        const int p = 32 * pt + 8 * j + 4 * half;
+                        const f32x4_t nv = *(const f32x4_t*)&nbuf[1][p];
+                        const int end = (tile_pok >> (2 * pt + j / 2)) & 1u ? lim - t0 - p : 0;
+#pragma unroll
+                        for (int k = 0; k < 4; ++k) {
+                            sc[pt][4 * j + k] = k < end ? sc[pt][4 * j + k] : -__builtin_inff();
+                            vmax = fmaxf(vmax, k < end ? fabsf(nv[k]) : 0.0f);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
+                vmax = fmaxf(vmax, __shfl_xor(vmax, 32));
             }
             // ---- online softmax in log2 units
             float cmax = sc[0][0];
@@ -1965,8 +1977,8 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
                 for (int i = 0; i < 16; ++i) cmax = fmaxf(cmax, sc[pt][i]);
             cmax = fmaxf(cmax, __shfl_xor(cmax, 32)) * colscale;
             const float m_new = fmaxf(m_run, cmax);
-            const int e_new = max(e_run, min(exponent_above(tmax[0]), 17));
-            if (__ballot(m_new > m_run + kPqSlack) != 0 || e_new > e_run) {
+            const int e_new = max(e_run, min(exponent_above(vmax), 17));
+            if (__ballot(m_new > m_run + kPqSlack || e_new > e_run) != 0) {
                 const float mref = m_new == -__builtin_inff() ? 0.0f : m_new;
                 const float alpha = __builtin_amdgcn_exp2f(m_run - mref);  // 0 while m_run is -inf
                 l_run *= alpha;

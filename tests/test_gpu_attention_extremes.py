@@ -119,3 +119,33 @@ def test_fp16_prefill_small_weights(dev, hd, kv_len):
     w = (n[:, None] - 1) * np.exp(-s) / (1 + (n[:, None] - 1) * np.exp(-s))
     want = w[:, :, None] * np.repeat(vp[1, 1].astype(np.float64), qh // kvh, 0)
     assert np.abs(got / want - 1).max() <= 2.0 ** -11 + 2.0 ** -12
+
+
+@pytest.mark.parametrize("kbits,vbits", WIDTHS)
+@pytest.mark.parametrize("late", [np.inf, 6e4])
+def test_tq_prefill_late_norm_costs_no_precision(dev, kbits, vbits, late):
+    """The first position holds nearly all the weight and a value norm of 0; what the others add, at
+    about 2^-18 of it, is the output. A large value norm at position 40, in the first tile of all the
+    first block's queries, changes none before it."""
+    rng = np.random.default_rng(kbits)
+    T, qh, kvh = 400, 32, 8
+    pool = build_pool(rng, [T], kvh, 128, kbits, vbits)
+    rows = pool["table"][0]
+    pos = lambda n, t: pool[n][rows[t // 16], t % 16]
+    for t in range(1, T):
+        pos("KP", t)[:] = pos("KP", 0)
+        pos("VP", t)[:] = pos("VP", 1)
+        pos("KN", t)[:] = np.float16(0.125)
+        pos("VN", t)[:] = np.float16(1024)
+    pos("KN", 0)[:] = np.float16(8)
+    pos("VN", 0)[:] = 0
+    pos("VN", 40)[:] = late
+    # q along the first key: a score of about 12.5 nats (2^-18) against a sixty-fourth of it
+    codes = oracle.tq_unpack_rows(pos("KP", 0).reshape(kvh, -1), 128, kbits)
+    k = pool["kc"][codes] @ pool["krot"]
+    a = 12.5 * np.sqrt(128) / 8 / (k * k).sum(-1, keepdims=True)
+    q = ((a * k)[None, :, None] * rng.uniform(0.97, 1.0, (T, kvh, qh // kvh, 1))).reshape(T, qh, 128).astype(np.float16)
+    got = run_prefill(dev, pool, q, kvh, T, 0, kbits, vbits)
+    for t in range(2, 40, 3):
+        # the rounding of the output and of the oracle's, 2^-11 each of the larger elements
+        assert_rel(got[t], tq_want(pool, q[t], t + 1, kbits, vbits, kvh), 1.2e-3, f"token {t}")
