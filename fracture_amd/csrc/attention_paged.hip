@@ -351,7 +351,8 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
     else
         __syncthreads();
     // ---- merge in wave order: column c's vector is (query tq0 + c / G, head h0 + c % G); a
-    // wave with m = -inf (an empty or fully masked piece) adds nothing
+    // wave with m = -inf adds nothing (an empty or fully masked piece), or the NaN that all its
+    // scores were
     const int own = W == 1 ? wave : 0;  // the split's first wave
     for (int i = W == 1 ? lane : (int)threadIdx.x; i < ncols * (HD / 4); i += 64 * W) {
         const int c = i / (HD / 4), d = 4 * (i - c * (HD / 4));
@@ -364,8 +365,7 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             const float mw = mlbuf[own + w][0][c];
-            if (mw == -__builtin_inff()) continue;
-            const float wt = __builtin_amdgcn_exp2f(mw - M);
+            const float wt = mw == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
             L = fmaf(wt, mlbuf[own + w][1][c], L);
             const f4_t a = *(const f4_t*)&sbuf[own + w][c][d];
 #pragma unroll

@@ -614,7 +614,10 @@ __global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
             float mx = M;
 #pragma unroll
             for (int u = 0; u < kChunk; ++u) {
-                m[u] = s0 + u < ns ? m[u] : -__builtin_inff();
+                const bool live = s0 + u < ns;
+                m[u] = live ? m[u] : -__builtin_inff();
+                l[u] = live ? l[u] : 0.0f;
+                av[u] = live ? av[u] : 0.0f;
                 mx = fmaxf(mx, m[u]);
             }
             const float old = M == -__builtin_inff() ? 0.0f : expf(M - mx);
@@ -622,15 +625,14 @@ __global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
             sum *= old;
 #pragma unroll
             for (int u = 0; u < kChunk; ++u) {
-                if (m[u] == -__builtin_inff()) continue;  // uniform over the wave
-                const float wt = expf(m[u] - mx);
+                const float wt = m[u] == -__builtin_inff() ? 0.0f : expf(m[u] - mx);  // NaN sums stay
                 L = fmaf(wt, l[u], L);
                 sum = fmaf(wt, av[u], sum);
             }
             M = mx;
         }
     }
-    o[w][i] = L > 0.0f ? sum / L : 0.0f;
+    o[w][i] = sum * (L > 0.0f ? 1.0f / L : 0.0f);
     __syncthreads();
 #pragma unroll
     for (int v = 0; v < kComb128Vecs; ++v) {
@@ -1572,7 +1574,8 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     // then m (log2 units) and l per head, and counts itself done; the last wave to finish
     // merges (no barrier: the others leave at once and free their slots). Each output (h, d)
     // sums the waves in wave order, weighted by exp2(m_w - max m) (0 for a wave with
-    // m = -inf), whichever wave merges.
+    // m = -inf: one with nothing to add, or with nothing but NaN scores, which stay NaN), whichever
+    // wave merges.
     // Head rows are kStRow floats apart (144: the 16 writing lanes of a 16-byte store, 4 heads
     // x 4 row groups, land in distinct banks); a lane's 4 values of dim tile c are dims
     // 16c + 4rg + 0..3 (element e holds dim e ^ 1), one 16-byte store.
@@ -1618,16 +1621,14 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             const float* sw = (const float*)vbuf[w][0];
-            if (mw[w] != -__builtin_inff()) {
-                const float wt = __builtin_amdgcn_exp2f(mw[w] - M);
-                L = fmaf(wt, sw[kStL + h], L);
-                const f32x4_t a0 = *(const f32x4_t*)&sw[h * kStRow + d0];
-                const f32x4_t a1 = *(const f32x4_t*)&sw[h * kStRow + d0 + 4];
+            const float wt = mw[w] == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(mw[w] - M);
+            L = fmaf(wt, sw[kStL + h], L);
+            const f32x4_t a0 = *(const f32x4_t*)&sw[h * kStRow + d0];
+            const f32x4_t a1 = *(const f32x4_t*)&sw[h * kStRow + d0 + 4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    A0[k] = fmaf(wt, a0[k], A0[k]);
-                    A1[k] = fmaf(wt, a1[k], A1[k]);
-                }
+            for (int k = 0; k < 4; ++k) {
+                A0[k] = fmaf(wt, a0[k], A0[k]);
+                A1[k] = fmaf(wt, a1[k], A1[k]);
             }
         }
         float* pa = part_acc + prow * hd + d0;

@@ -149,3 +149,41 @@ def test_tq_prefill_late_norm_costs_no_precision(dev, kbits, vbits, late):
     for t in range(2, 40, 3):
         # the rounding of the output and of the oracle's, 2^-11 each of the larger elements
         assert_rel(got[t], tq_want(pool, q[t], t + 1, kbits, vbits, kvh), 1.2e-3, f"token {t}")
+
+
+@pytest.mark.parametrize("n,bad", [(1000, (0, 64)), (1000, (128, 256)), (1000, (256, 512)), (3000, (1024, 2048)),
+                                   (40000, (2048, 2304))])
+def test_nan_scores_of_a_whole_piece(dev, n, bad):
+    """Key rows of NaN over positions that make up a whole wave's piece, a 256-position part or a split:
+    the result is what one such row gives anywhere: NaN over TurboQuant pages, zeros over FP16 pages."""
+    rng = np.random.default_rng(n)
+    qh, kvh = 8, 2
+    pool = build_pool(rng, [n], kvh, 128, 4, 4)
+    rows = pool["table"][0]
+    for t in range(*bad):
+        pool["KN"][rows[t // 16], t % 16] = np.nan
+    q = rng.standard_normal((1, qh, 128)).astype(np.float16)
+    assert np.isnan(run_tq_decode(dev, pool, q, [n], 4, 4, kvh)).all()
+    kp = rng.standard_normal((len(rows), 16, kvh, 128)).astype(np.float16)
+    vp = rng.standard_normal(kp.shape).astype(np.float16)
+    for t in range(*bad):
+        kp[t // 16, t % 16] = np.nan
+    table = np.arange(len(rows), dtype=np.int32)[None]
+    assert not run_decode(dev, q, table, [n], kp, vp, kvh).any()
+
+
+@pytest.mark.parametrize("kbits,vbits", [(4, 4), (8, 8), (8, 2)])
+@pytest.mark.parametrize("T", [1, 5, 130])
+def test_nan_query_gives_nan(dev, kbits, vbits, T):
+    """A query with NaN among its elements gives NaN, as the reference's sums do
+    (attention_paged_tq.cu:56-257), and disturbs no other one."""
+    rng = np.random.default_rng(T)
+    qh, kvh, n = 32, 8, 700
+    pool = build_pool(rng, [n], kvh, 128, kbits, vbits)
+    q = rng.standard_normal((T, qh, 128)).astype(np.float16)
+    clean = run_prefill(dev, pool, q, kvh, n, n - T, kbits, vbits)
+    q[T // 2, 3, 7] = np.nan
+    got = run_prefill(dev, pool, q, kvh, n, n - T, kbits, vbits)
+    assert np.isnan(got[T // 2, 3]).all()
+    got[T // 2, 3] = clean[T // 2, 3]
+    np.testing.assert_array_equal(got, clean)
