@@ -1003,20 +1003,11 @@ __device__ __forceinline__ void decode_group(const DequantLds& t, const CodeHalf
 // MFMA dequantize of one tile by one wave, head_dim 128 (turboquant_decompress.cu:21-94):
 //   unpack -> c[idx] -> x_hat = Pi^T y_hat -> fp16(x_hat * float(norm)).
 // Lane (r, h) ends block c holding coordinates 32c + 8g + 4h + e of row r; neighbouring
-// chunks are exchanged with the partner lane so every lane stores 16 contiguous bytes.
+// chunks are exchanged with the partner lane so every lane has 16 contiguous bytes.
 // ---------------------------------------------------------------------------------------
-// The dequantize's stores. A lane ends a block with pieces of one row, so storing them from there
-// touches 32 rows of 32 bytes an instruction, and an output line is completed by four of them, some
-// time apart. The wave gathers two blocks (128 bytes of each of its 32 rows) in its own 4 KB of LDS
-// instead and stores whole 128-byte lines, eight an instruction, past the L2 (the reader of so much
-// output does not find it there). Pieces are XOR-swizzled by their row. 32768 tokens of 8 heads, K4/V4,
-// 134 MB of output: 64.5 us with the lanes' own stores, 47.3 with lines, 43.8 past the L2 (3.9 TB/s).
-struct OutStage {
-    u32x4 piece[kTile * 8];  // [row][16-byte piece ^ row % 8]
-};
-// Block c of the lane's row (its 32 coordinates are pieces 4 (c % 2) .. + 3).
-__device__ __forceinline__ void stage_block(const f32x16& acc, float nrm, OutStage& st, int c) {
-    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+// Where the blocks of a tile go. fp16 of a block: pieces m = 0, 1 of the lane, 16 bytes each, at
+// coordinates 32c + 16m + 8h.
+__device__ __forceinline__ void block_pieces(const f32x16& acc, float nrm, u32x4 (&piece)[2]) {
     uint32_t ch[4][2];
 #pragma unroll
     for (int g = 0; g < 4; ++g)
@@ -1027,29 +1018,62 @@ __device__ __forceinline__ void stage_block(const f32x16& acc, float nrm, OutSta
     for (int m = 0; m < 2; ++m) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) swap_halves(ch[2 * m][e], ch[2 * m + 1][e]);
-        st.piece[8 * r + ((4 * (c & 1) + 2 * m + h) ^ (r & 7))] =
-            u32x4{ch[2 * m][0], ch[2 * m][1], ch[2 * m + 1][0], ch[2 * m + 1][1]};
+        piece[m] = u32x4{ch[2 * m][0], ch[2 * m][1], ch[2 * m + 1][0], ch[2 * m + 1][1]};
     }
 }
-// Blocks 2 pair, 2 pair + 1 of the tile's rows to out.
-__device__ __forceinline__ void flush_blocks(const OutStage& st, uint16_t* __restrict__ out, int64_t m0,
-                                             int nvalid, int pair) {
-    const int lane = threadIdx.x & 63, r8 = lane >> 3, p = lane & 7;
-    wave_lds_sync();  // the pieces come from other lanes
-    u32x4 v[4];
+// The lanes' own stores, into the L2: 32 rows of 32 bytes an instruction, an output line completed by
+// four of them, some time apart.
+struct LaneOut {
+    __device__ __forceinline__ void block(const f32x16& acc, float nrm, int c, uint16_t* __restrict__ out,
+                                          int64_t m0, int nvalid) {
+        const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+        u32x4 piece[2];
+        block_pieces(acc, nrm, piece);
+        uint16_t* orow = out + m0 * kHd + (r * kHd + 8 * h);
+        if (r < nvalid) {
+            *(u32x4*)&orow[32 * c] = piece[0];
+            *(u32x4*)&orow[32 * c + 16] = piece[1];
+        }
+    }
+};
+// Whole lines: the wave gathers two blocks (128 bytes of each of its 32 rows) in its own 4 KB of LDS and
+// stores 128-byte lines, eight an instruction, past the L2. Pieces are XOR-swizzled by their row.
+struct LineOut {
+    u32x4 piece[kTile * 8];  // [row][16-byte piece ^ row % 8]
+    __device__ __forceinline__ void block(const f32x16& acc, float nrm, int c, uint16_t* __restrict__ out,
+                                          int64_t m0, int nvalid) {
+        const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+        u32x4 mine[2];
+        block_pieces(acc, nrm, mine);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = st.piece[8 * (8 * j + r8) + (p ^ r8)];
-    wave_lds_sync();  // the next pair's pieces overwrite them
-    char* dst = (char*)(out + m0 * kHd) + r8 * (2 * kHd) + 128 * pair + 16 * p;
+        for (int m = 0; m < 2; ++m) piece[8 * r + ((4 * (c & 1) + 2 * m + h) ^ (r & 7))] = mine[m];
+        if ((c & 1) == 0) return;
+        const int r8 = lane >> 3, p = lane & 7;
+        wave_lds_sync();  // the pieces come from other lanes
+        u32x4 v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        if (8 * j + r8 < nvalid) st16_stream(dst + j * 8 * (2 * kHd), v[j]);
-}
+        for (int j = 0; j < 4; ++j) v[j] = piece[8 * (8 * j + r8) + (p ^ r8)];
+        wave_lds_sync();  // the next pair's pieces overwrite them
+        char* dst = (char*)(out + m0 * kHd) + r8 * (2 * kHd) + 128 * (c >> 1) + 16 * p;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (8 * j + r8 < nvalid) st16_stream(dst + j * 8 * (2 * kHd), v[j]);
+    }
+};
+// Lines from this many rows (8 MB of output a tensor), codes of up to 4 bits; the lanes' stores below,
+// where the LDS pass costs more than it saves and the next kernel finds the output in the L2, and at
+// 8 bits, where the pass spills registers. Keys and values of N tokens x 8 heads, K4/V4,
+// us with the lanes' stores and with lines (and with a reader of both behind them): N = 256 7.0 / 7.4
+// (9.1 / 9.8), 1024 7.5 / 7.8 (10.5 / 10.9), 3072 8.9 / 8.3 (13.6 / 13.9), 4096 9.5 / 8.6 (15.8 /
+// 15.5), 8192 16.5 / 14.4, 32768 44 / 43 repeated (100 / 74), and on new outputs 64.5 / 43.8. K8/V8: 1024
+// 8.7 / 11.0, 8192 19.2 / 19.6, 32768 46.8 / 50.9.
+constexpr int64_t kLineRows = 32768;
 
 // x = Pi^T y of the lane's row from the (hi, lo') fp16 B fragments of y (three fp16
 // products per step), stored as fp16(x * nrm).
+template <class Out>
 __device__ __forceinline__ void rotate_back_store(const RotLds& L, const f16x8 (&bh)[8],
-                                                  const f16x8 (&bl)[8], float nrm, OutStage& st,
+                                                  const f16x8 (&bl)[8], float nrm, Out& st,
                                                   uint16_t* __restrict__ out, int64_t m0,
                                                   int nvalid) {
     const int lane = threadIdx.x & 63;
@@ -1067,8 +1091,7 @@ __device__ __forceinline__ void rotate_back_store(const RotLds& L, const f16x8 (
         f32x16 x;
 #pragma unroll
         for (int v = 0; v < 16; ++v) x[v] = fmaf(acc2[v], kLoInv, acc1[v]);
-        stage_block(x, nrm, st, c);
-        if (c & 1) flush_blocks(st, out, m0, nvalid, c >> 1);
+        st.block(x, nrm, c, out, m0, nvalid);
     }
 }
 
@@ -1079,9 +1102,9 @@ __device__ __forceinline__ i32x8 deq_a8(const DeqLds& L, int c, int u, int t, in
                  (int)b[0], (int)b[1], (int)b[2], (int)b[3]};
 }
 
-template <int kBits>
+template <int kBits, class Out>
 __device__ __forceinline__ void dequant_tile(const DequantLds& t, const DeqLds& L,
-                                             const CodeHalf<kBits>& cw, OutStage& st,
+                                             const CodeHalf<kBits>& cw, Out& st,
                                              uint16_t* __restrict__ out, int64_t m0, int nvalid) {
     const int lane = threadIdx.x & 63;
     CodeOps ops;
@@ -1125,14 +1148,10 @@ __device__ __forceinline__ void dequant_tile(const DequantLds& t, const DeqLds& 
                     f8r[j & 1], ops.b8[u][1], acc[b], 0, 0, 0, sa_hi, 0, sb_lo);
         }
         // block c - 1's stores, two steps into block c (its last product has finished)
-        if (c > 0 && s == 2) {
-            stage_block(acc[b ^ 1], nrm, st, c - 1);
-            if (c == 2) flush_blocks(st, out, m0, nvalid, 0);
-        }
+        if (c > 0 && s == 2) st.block(acc[b ^ 1], nrm, c - 1, out, m0, nvalid);
     }
     __builtin_amdgcn_sched_barrier(0);
-    stage_block(acc[1], nrm, st, 3);
-    flush_blocks(st, out, m0, nvalid, 1);
+    st.block(acc[1], nrm, 3, out, m0, nvalid);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1154,7 +1173,8 @@ __device__ __forceinline__ void load_row_half(const float* __restrict__ y, int64
 #pragma unroll
     for (int i = 0; i < 16; ++i) rh.v[i] = *(const f32x4*)(src + 4 * i);
 }
-__device__ __forceinline__ void rotate_back_tile(const RotLds& L, const RowHalf& rh, OutStage& st,
+template <class Out>
+__device__ __forceinline__ void rotate_back_tile(const RotLds& L, const RowHalf& rh, Out& st,
                                                  uint16_t* __restrict__ out, int64_t m0,
                                                  int nvalid) {
     f16x8 bh[8], bl[8];
@@ -1180,11 +1200,12 @@ __device__ __forceinline__ void rotate_back_tile(const RotLds& L, const RowHalf&
     rotate_back_store(L, bh, bl, 1.0f, st, out, m0, nvalid);
 }
 constexpr int kWavesR = 4;  // waves per workgroup of the back-rotation (two workgroups per CU)
+template <class Out>
 __global__ __launch_bounds__(64 * kWavesR) __attribute__((amdgpu_waves_per_eu(2))) void
 tq_rotate_back_kernel(const float* __restrict__ y, const float* __restrict__ rot,
                       uint16_t* __restrict__ out, int64_t rows) {
     __shared__ RotLds rl;
-    __shared__ OutStage st[kWavesR];
+    __shared__ Out st[kWavesR];
     const int64_t ntiles = ceil_div(rows, kTile);
     const int64_t stride = (int64_t)gridDim.x * kWavesR;
     int64_t tile = (int64_t)blockIdx.x * kWavesR + wave_id();
@@ -1205,8 +1226,8 @@ tq_rotate_back_kernel(const float* __restrict__ y, const float* __restrict__ rot
 
 // The wave's tile loop: ca holds its first tile (loads issued); each tile's successor is in
 // flight while it computes.
-template <int kBits>
-__device__ __forceinline__ void dequant_waves(const DequantLds& t, const DeqLds& rl, OutStage& st,
+template <int kBits, class Out>
+__device__ __forceinline__ void dequant_waves(const DequantLds& t, const DeqLds& rl, Out& st,
                                               const uint8_t* __restrict__ packed,
                                               const uint16_t* __restrict__ norms,
                                               uint16_t* __restrict__ out, int64_t rows,
@@ -1245,8 +1266,8 @@ __device__ __forceinline__ const RotLds& plan_compress_frags(const TqPlanDev* p)
 
 // The planned dequantize of one tensor by workgroup blk of nblk: the tables and fragments are
 // copied from the plan into LDS while the first tile's loads are in flight.
-template <int kBits>
-__device__ __forceinline__ void dequant_planned(DequantLds& t, DeqLds& rl, OutStage* st,
+template <int kBits, class Out>
+__device__ __forceinline__ void dequant_planned(DequantLds& t, DeqLds& rl, Out* st,
                                                 const uint8_t* __restrict__ packed,
                                                 const uint16_t* __restrict__ norms,
                                                 const TqPlanDev* __restrict__ plan,
@@ -1269,7 +1290,7 @@ __device__ __forceinline__ void dequant_planned(DequantLds& t, DeqLds& rl, OutSt
     dequant_waves<kBits>(t, rl, st[wave_id()], packed, norms, out, rows, tile, stride, ntiles, ca, cb);
 }
 
-template <int kBits, bool kPlanned>
+template <int kBits, bool kPlanned, class Out>
 __global__ __launch_bounds__(64 * kWavesD) __attribute__((amdgpu_waves_per_eu(3))) void
 tq_dequant_mfma_kernel(const uint8_t* __restrict__ packed, const uint16_t* __restrict__ norms,
                        const float* __restrict__ rot, const float* __restrict__ cent, int L,
@@ -1277,7 +1298,7 @@ tq_dequant_mfma_kernel(const uint8_t* __restrict__ packed, const uint16_t* __res
                        int64_t rows) {
     __shared__ DequantLds t;
     __shared__ DeqLds rl;
-    __shared__ OutStage st[kWavesD];
+    __shared__ Out st[kWavesD];
     if constexpr (kPlanned) {
         dequant_planned<kBits>(t, rl, st, packed, norms, plan, out, rows, blockIdx.x, gridDim.x);
         return;
@@ -1310,7 +1331,7 @@ tq_dequant_mfma_kernel(const uint8_t* __restrict__ packed, const uint16_t* __res
 
 // Keys and values of one layer in one launch: even workgroups dequantize the keys, odd ones
 // the values (as the K+V compress kernel).
-template <int kKBits, int kVBits>
+template <int kKBits, int kVBits, class Out>
 __global__ __launch_bounds__(64 * kWavesD) __attribute__((amdgpu_waves_per_eu(3))) void
 tq_dequant_kv_mfma_kernel(const uint8_t* __restrict__ k_packed, const uint16_t* __restrict__ k_norms,
                           const uint8_t* __restrict__ v_packed, const uint16_t* __restrict__ v_norms,
@@ -1319,7 +1340,7 @@ tq_dequant_kv_mfma_kernel(const uint8_t* __restrict__ k_packed, const uint16_t* 
                           int64_t rows) {
     __shared__ DequantLds t;
     __shared__ DeqLds rl;
-    __shared__ OutStage st[kWavesD];
+    __shared__ Out st[kWavesD];
     const int64_t blk = blockIdx.x >> 1, nblk = gridDim.x >> 1;
     if (blockIdx.x & 1)
         dequant_planned<kVBits>(t, rl, st, v_packed, v_norms, vplan, v_out, rows, blk, nblk);
@@ -1458,16 +1479,15 @@ int launch_dequant(const void* packed_in, const void* norms_in, const float* rot
     if (head_dim == kHd && mfma_bits && packed_dim_per_head == 16 * bits &&
         fhip_host::aligned16(output) && fhip_host::aligned16(packed_in) &&
         (((uintptr_t)norms_in) & 1u) == 0) {
+        const bool lines = rows >= kLineRows;
         auto pick = [&](auto planned) {
             constexpr bool kP = decltype(planned)::value;
-            auto kern = tq_dequant_mfma_kernel<4, kP>;
             switch (bits) {
-                case 2: kern = tq_dequant_mfma_kernel<2, kP>; break;
-                case 3: kern = tq_dequant_mfma_kernel<3, kP>; break;
-                case 8: kern = tq_dequant_mfma_kernel<8, kP>; break;
-                default: break;
+                case 2: return lines ? tq_dequant_mfma_kernel<2, kP, LineOut> : tq_dequant_mfma_kernel<2, kP, LaneOut>;
+                case 3: return lines ? tq_dequant_mfma_kernel<3, kP, LineOut> : tq_dequant_mfma_kernel<3, kP, LaneOut>;
+                case 8: return tq_dequant_mfma_kernel<8, kP, LaneOut>;
+                default: return lines ? tq_dequant_mfma_kernel<4, kP, LineOut> : tq_dequant_mfma_kernel<4, kP, LaneOut>;
             }
-            return kern;
         };
         auto kern = plan ? pick(std::true_type{}) : pick(std::false_type{});
         hipLaunchKernelGGL(kern, dim3(mfma_grid(ceil_div(rows, kTile), kWavesD)),
@@ -1518,13 +1538,18 @@ bool launch_dequant_kv(const TqPlanDev* kp, const TqPlanDev* vp, int kbits, int 
     if (!fhip_host::aligned16(kpk) || !fhip_host::aligned16(vpk) || !fhip_host::aligned16(kout) ||
         !fhip_host::aligned16(vout) || (((uintptr_t)knm) & 1u) || (((uintptr_t)vnm) & 1u))
         return false;
-    auto kern = tq_dequant_kv_mfma_kernel<4, 4>;
-    if (kbits == 4 && vbits == 4) kern = tq_dequant_kv_mfma_kernel<4, 4>;
-    else if (kbits == 3 && vbits == 3) kern = tq_dequant_kv_mfma_kernel<3, 3>;
-    else if (kbits == 2 && vbits == 2) kern = tq_dequant_kv_mfma_kernel<2, 2>;
-    else if (kbits == 8 && vbits == 8) kern = tq_dequant_kv_mfma_kernel<8, 8>;
-    else if (kbits == 4 && vbits == 2) kern = tq_dequant_kv_mfma_kernel<4, 2>;
-    else return false;
+    const bool lines = rows >= kLineRows;
+    auto kern = tq_dequant_kv_mfma_kernel<8, 8, LaneOut>;
+    if (kbits == 4 && vbits == 4)
+        kern = lines ? tq_dequant_kv_mfma_kernel<4, 4, LineOut> : tq_dequant_kv_mfma_kernel<4, 4, LaneOut>;
+    else if (kbits == 3 && vbits == 3)
+        kern = lines ? tq_dequant_kv_mfma_kernel<3, 3, LineOut> : tq_dequant_kv_mfma_kernel<3, 3, LaneOut>;
+    else if (kbits == 2 && vbits == 2)
+        kern = lines ? tq_dequant_kv_mfma_kernel<2, 2, LineOut> : tq_dequant_kv_mfma_kernel<2, 2, LaneOut>;
+    else if (kbits == 4 && vbits == 2)
+        kern = lines ? tq_dequant_kv_mfma_kernel<4, 2, LineOut> : tq_dequant_kv_mfma_kernel<4, 2, LaneOut>;
+    else if (!(kbits == 8 && vbits == 8))
+        return false;
     hipLaunchKernelGGL(kern, dim3(mfma_grid_kv(ceil_div(rows, kTile), kWavesD)),
                        dim3(64 * kWavesD), 0, s, (const uint8_t*)kpk, (const uint16_t*)knm,
                        (const uint8_t*)vpk, (const uint16_t*)vnm, kp, vp, (uint16_t*)kout,
@@ -1573,7 +1598,8 @@ int tq_rotate_back_rows(const float* input, const float* rotation, void* out, in
     if (rows == 0) return hipSuccess;
     const int64_t need = ceil_div(ceil_div(rows, kTile), kWavesR);
     const int64_t cap = 2 * (int64_t)fhip_host::cu_count();
-    hipLaunchKernelGGL(tq_rotate_back_kernel, dim3((unsigned)(need < cap ? need : cap)),
+    auto kern = rows >= kLineRows ? tq_rotate_back_kernel<LineOut> : tq_rotate_back_kernel<LaneOut>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(need < cap ? need : cap)),
                        dim3(64 * kWavesR), 0, stream, input, rotation, (uint16_t*)out, rows);
     return hipGetLastError();
 }

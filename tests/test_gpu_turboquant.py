@@ -565,3 +565,32 @@ def test_kv_planned_layer_scale(dev):
         K.tq_dequant_planned(plans[i], *fused[i], want)
         torch.cuda.synchronize()
         assert torch.equal(want.view(torch.int16), outs[i].view(torch.int16))
+
+
+@pytest.mark.parametrize("kb,vb", [(4, 4), (4, 2), (3, 3), (2, 2), (8, 8)])
+@pytest.mark.parametrize("N", [4095, 4096, 4101])
+def test_dequant_stores_agree_across_sizes(dev, kb, vb, N):
+    """Calls of 32768 rows and more store whole lines, smaller ones each lane's pieces: the same bits, in
+    whole tensors and in single ones, and nothing past the last row."""
+    rng = np.random.default_rng(N + kb)
+    H, hd = 8, 128
+    plans, packs = [], []
+    for bits, seed in ((kb, 1), (vb, 2)):
+        plans.append(K.TqPlan(dev_t(tq.rotation_matrix(hd, seed), dev), dev_t(tq.codebook(hd, bits)[0], dev), bits))
+        packs.append((dev_t(rng.integers(0, 256, (N, H * 16 * bits)).astype(np.uint8), dev),
+                      dev_t(rng.uniform(1, 20, (N, H)).astype(np.float16), dev)))
+    def run(a, b):
+        outs = []
+        for _ in range(2):
+            o = torch.full((b - a + 1, H, hd), 7.0, dtype=torch.float16, device=dev)
+            outs.append(o)
+        K.tq_dequant_kv_planned(*plans, *(x[a:b].contiguous() for p in packs for x in p), *(o[:-1] for o in outs))
+        single = torch.full_like(outs[0], 7.0)
+        K.tq_dequant_planned(plans[0], packs[0][0][a:b].contiguous(), packs[0][1][a:b].contiguous(), single[:-1])
+        torch.cuda.synchronize()
+        for o in (*outs, single):
+            assert (o[-1] == 7.0).all()
+        return [o[:-1].cpu().numpy().view(np.uint16) for o in (*outs, single)]
+    whole = run(0, N)
+    for w, p, q in zip(whole, run(0, 2000), run(2000, N)):
+        np.testing.assert_array_equal(w, np.concatenate([p, q]))
