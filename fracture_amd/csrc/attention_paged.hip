@@ -26,6 +26,7 @@
 
 #include <algorithm>
 
+#include "attn_rules.h"
 #include "fhip_common.h"
 #include "fracture_hip.h"
 
@@ -118,7 +119,7 @@ struct PQueries {
 //
 // A workgroup of W waves takes one (query, kv head, head block, split); wave w scores the
 // split's positions [w, w + 1) * kPSplit / W and the waves' states are merged in LDS, so the
-// partials stay one per split whatever W is (kSplits8 / kSplits4 choose it). With a wave per split
+// partials stay one per split whatever W is (paged_waves in attn_rules.h). With a wave per split
 // the chunk's loads had nothing beside them to hide behind: 16 sequences of 500 .. 8192
 // positions (32 / 8 heads of 128, 285 MB) went from 136 to 72 us.
 // W = 1 puts two splits of neighbouring kv heads, each a wave's own, in a workgroup instead.
@@ -334,7 +335,27 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
         for (int h = 0; h < NH; ++h)
 #pragma unroll
             for (int i = 0; i < 8; ++i) acc[h][i] += __shfl_xor(acc[h][i], o);
-    if (lane < 16) {  // lane == n here
+    // column c's vector is (query tq0 + c / G, head h0 + c % G)
+    if constexpr (W == 1) {  // the split's state is the wave's
+        if (lane < ncols) {  // lane == n here
+            const int64_t v = (int64_t)(tq0 + ct) * qh + h0 + hn;
+            part_ml[(v * nsplit + split) * 2 + 0] = m_run * 0.6931471805599453f;
+            part_ml[(v * nsplit + split) * 2 + 1] = l_run;
+        }
+        if (ps == 0) {
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                if (h >= ncols) break;
+                const int cq = tok > 1 ? h / G : 0;
+                const int64_t v = (int64_t)(tq0 + cq) * qh + h0 + (h - cq * G);
+                float* dst = part_acc + (v * nsplit + split) * HD + 8 * dg;
+                *(f4_t*)dst = f4_t{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+                *(f4_t*)(dst + 4) = f4_t{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
+            }
+        }
+        return;
+    }
+    if (lane < 16) {
         mlbuf[wave][0][lane] = m_run;
         mlbuf[wave][1][lane] = l_run;
     }
@@ -346,28 +367,23 @@ paged_attn_split_kernel(const uint16_t* __restrict__ q, PQueries qs, Pages pg, i
             *(f4_t*)(dst + 4) = f4_t{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
         }
     }
-    if constexpr (W == 1)
-        wave_lds_sync();
-    else
-        __syncthreads();
-    // ---- merge in wave order: column c's vector is (query tq0 + c / G, head h0 + c % G); a
-    // wave with m = -inf adds nothing (an empty or fully masked piece), or the NaN that all its
-    // scores were
-    const int own = W == 1 ? wave : 0;  // the split's first wave
-    for (int i = W == 1 ? lane : (int)threadIdx.x; i < ncols * (HD / 4); i += 64 * W) {
+    __syncthreads();
+    // ---- merge in wave order; a wave with m = -inf adds nothing (an empty or fully masked piece), or
+    // the NaN that all its scores were
+    for (int i = threadIdx.x; i < ncols * (HD / 4); i += 64 * W) {
         const int c = i / (HD / 4), d = 4 * (i - c * (HD / 4));
         const int cq = tok > 1 ? c / G : 0;
         float M = -__builtin_inff();
 #pragma unroll
-        for (int w = 0; w < W; ++w) M = fmaxf(M, mlbuf[own + w][0][c]);
+        for (int w = 0; w < W; ++w) M = fmaxf(M, mlbuf[w][0][c]);
         float L = 0.0f;
         f4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int w = 0; w < W; ++w) {
-            const float mw = mlbuf[own + w][0][c];
+            const float mw = mlbuf[w][0][c];
             const float wt = mw == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
-            L = fmaf(wt, mlbuf[own + w][1][c], L);
-            const f4_t a = *(const f4_t*)&sbuf[own + w][c][d];
+            L = fmaf(wt, mlbuf[w][1][c], L);
+            const f4_t a = *(const f4_t*)&sbuf[w][c][d];
 #pragma unroll
             for (int k = 0; k < 4; ++k) o[k] = fmaf(wt, a[k], o[k]);
         }
@@ -856,52 +872,65 @@ __global__ __launch_bounds__(kCombThreads) void paged_attn_combine_kernel(
 }
 
 // The same merge for launches with at most 8 splits per vector (contexts up to 8192 positions; causal
-// prefill) and head_dim a multiple of 4: half a wave per vector, eight vectors per workgroup. Lane s
-// of the half holds split s's (m, l), the weights reach the dim loop by lane broadcasts, and every lane
-// loads 16 bytes of each split: no LDS, no barrier. A workgroup per vector spent most of its time
-// being scheduled at prefill sizes. The call of 32000 vectors of 2 splits (1000 queries at 3001):
-// 108.9 us with a wave per vector and 4-byte loads, 103.8 with this.
+// prefill): kLanes lanes per vector, 256 / kLanes vectors per workgroup. Lane s of the group holds split
+// s's (m, l), the weights reach the dim loop by lane broadcasts: no LDS, no barrier. A workgroup per vector
+// spent most of its time being scheduled at prefill sizes. Half a wave per vector, every lane loading
+// 16 bytes of each split, from head_dim 128 on (32000 vectors of 2 splits, 1000 queries at 3001: the call
+// 103.8 us, 108.9 with a wave per vector and 4-byte loads); below, half of those lanes would be idle, and
+// a whole wave is the faster one (64 sequences of 100, 16 / 8 heads of 64: 11.4 us and 11.0).
 constexpr int kCombWaveMaxSplits = 8;
-__global__ __launch_bounds__(256) void paged_attn_combine_half_kernel(
+template <int kLanes, int kVec>
+__global__ __launch_bounds__(256) void paged_attn_combine_wave_kernel(
     PQueries qs, const float* __restrict__ ml, const float* __restrict__ acc,
     uint16_t* __restrict__ out, int qh, int hd, int nsplit, int64_t nvec, int split_pos) {
-    const int l32 = threadIdx.x & 31;
-    const int64_t vec = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
-    const bool live = vec < nvec;  // dead halves join the shuffles on vector 0's numbers
+    typedef float vec_t __attribute__((ext_vector_type(kVec)));
+    const int gl = threadIdx.x & (kLanes - 1), g0 = threadIdx.x & 63 & ~(kLanes - 1);
+    const int64_t vec = (int64_t)blockIdx.x * (256 / kLanes) + threadIdx.x / kLanes;
+    const bool live = vec < nvec;  // dead groups join the shuffles on vector 0's numbers
     const int64_t v = live ? vec : 0;
     const int clen = qs.causal_len((int)(v / qh));
     const int ns = (clen + split_pos - 1) / split_pos;  // <= nsplit <= kCombWaveMaxSplits
     const float* m = ml + v * nsplit * 2;
-    const float ms = l32 < ns ? m[2 * l32] : -__builtin_inff();
-    const float ls = l32 < ns ? m[2 * l32 + 1] : 0.0f;
-    float M = ms;
+    const float ms = gl < ns ? m[2 * gl] : -__builtin_inff();
+    const float ls = gl < ns ? m[2 * gl + 1] : 0.0f;
+    float M = ms, L = 0.0f;
+    if constexpr (kLanes == 64) {
+        M = wave_max(ms);
+    } else {
 #pragma unroll
-    for (int o = 4; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));  // lanes 0..7 of the half
-    M = __shfl(M, threadIdx.x & 32);
-    const float w = l32 < ns && M != -__builtin_inff() ? expf(ms - M) : 0.0f;
-    float ws[kCombWaveMaxSplits], L = 0.0f;
+        for (int o = 4; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));  // lanes 0..7 of the group
+        M = __shfl(M, g0);
+    }
+    const float w = gl < ns && M != -__builtin_inff() ? expf(ms - M) : 0.0f;
+    float ws[kCombWaveMaxSplits];
 #pragma unroll
-    for (int j = 0; j < kCombWaveMaxSplits; ++j) {
-        ws[j] = __shfl(w, (threadIdx.x & 32) + j);
-        L += ws[j] * __shfl(ls, (threadIdx.x & 32) + j);
+    for (int j = 0; j < kCombWaveMaxSplits; ++j) ws[j] = __shfl(w, g0 + j);
+    if constexpr (kLanes == 64) {
+        L = wave_sum(w * ls);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kCombWaveMaxSplits; ++j) L += ws[j] * __shfl(ls, g0 + j);
     }
     if (!live) return;
     const float* a = acc + v * nsplit * hd;
-    for (int d = 4 * l32; d < hd; d += 128) {
-        f4_t av[kCombWaveMaxSplits];
+    for (int d = kVec * gl; d < hd; d += kVec * kLanes) {
+        vec_t av[kCombWaveMaxSplits];
 #pragma unroll
-        for (int j = 0; j < kCombWaveMaxSplits; ++j)
-            av[j] = j < ns ? *(const f4_t*)(a + (int64_t)j * hd + d) : f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        f4_t o = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int j = 0; j < kCombWaveMaxSplits; ++j) av[j] = j < ns ? *(const vec_t*)(a + (int64_t)j * hd + d) : (vec_t)0.0f;
+        float o[kVec];
 #pragma unroll
-        for (int j = 0; j < kCombWaveMaxSplits; ++j)
+        for (int k = 0; k < kVec; ++k) {
+            o[k] = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) o[k] = fmaf(ws[j], av[j][k], o[k]);
-        u32x2 r;
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-            r[k] = f2h(L > 0.0f ? o[2 * k] / L : 0.0f) | (f2h(L > 0.0f ? o[2 * k + 1] / L : 0.0f) << 16);
-        *(u32x2*)(out + v * hd + d) = r;
+            for (int j = 0; j < kCombWaveMaxSplits; ++j) o[k] = fmaf(ws[j], av[j][k], o[k]);
+            o[k] = L > 0.0f ? o[k] / L : 0.0f;
+        }
+        if constexpr (kVec == 1) {
+            out[v * hd + d] = (uint16_t)f2h(o[0]);
+        } else {
+            *(u32x2*)(out + v * hd + d) =
+                u32x2{f2h(o[0]) | (f2h(o[1]) << 16), f2h(o[2]) | (f2h(o[3]) << 16)};
+        }
     }
 }
 
@@ -920,15 +949,6 @@ bool paged_shape_ok(int qh, int kvh, int hd) {
     return kvh > 0 && qh > 0 && qh % kvh == 0 && hd >= 1 && hd <= 256;
 }
 
-// Waves per split by the launch's size (splits x kv heads x head blocks x query groups). Few
-// workgroups: eight waves each hide one another's memory latency (one sequence of 4000 positions,
-// 32 / 8 heads of 128: 94 us with a wave per split, 36 / 25 / 20 us with 2 / 4 / 8). Many: the
-// chip is full with two, and more only add merge work and empty pieces at the ragged ends (64
-// sequences of 500 .. 2000, 1024 workgroups: 77 / 93 / 85 us). In between, at 512 workgroups
-// (32 / 4 heads): 68 / 49 / 56 us. One wave per split where even that fills every CU several times
-// over, two splits to a workgroup (64 sequences up to 32768, 16384 splits: 810 us, 820 with two waves
-// per split, 848 with one-wave workgroups).
-constexpr int64_t kSplits8 = 256, kSplits4 = 512, kSplits2 = 4096;
 template <int HD, int NH, int W, class Pages>
 void launch_split_w(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
                     int nhb, float* ml, float* acc, int nsplit, int tok, int64_t items,
@@ -943,14 +963,12 @@ template <int HD, int NH, class Pages>
 void launch_split_t(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
                     int nhb, float* ml, float* acc, int nsplit, int tok, int64_t items,
                     hipStream_t s) {
-    if (items <= kSplits8)
-        launch_split_w<HD, NH, 8>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
-    else if (items <= kSplits4)
-        launch_split_w<HD, NH, 4>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
-    else if (items <= kSplits2)
-        launch_split_w<HD, NH, 2>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
-    else
-        launch_split_w<HD, NH, 1>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+    switch (fhip_rules::paged_waves(items, HD, qs.max_blocks * FHIP_PAGE_TOKENS)) {
+        case 8: return launch_split_w<HD, NH, 8>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+        case 4: return launch_split_w<HD, NH, 4>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+        case 2: return launch_split_w<HD, NH, 2>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+        default: return launch_split_w<HD, NH, 1>(q, qs, pg, qh, kvh, nhb, ml, acc, nsplit, tok, items, s);
+    }
 }
 
 template <int HD, class Pages>
@@ -976,9 +994,13 @@ void launch_prefill_t(const uint16_t* q, const PQueries& qs, const Pages& pg, in
 // The merge of nsplit splits of split_pos positions per vector.
 void launch_combine(const PQueries& qs, const float* ml, const float* acc, void* out, int64_t nvec,
                     int qh, int hd, int nsplit, int split_pos, hipStream_t s) {
-    if (nsplit <= kCombWaveMaxSplits && hd % 4 == 0 && fhip_host::aligned16(acc) &&
+    if (nsplit <= kCombWaveMaxSplits && hd % 128 == 0 && fhip_host::aligned16(acc) &&
         ((uintptr_t)out & 7) == 0)
-        hipLaunchKernelGGL(paged_attn_combine_half_kernel, dim3((unsigned)ceil_div(nvec, 8)),
+        hipLaunchKernelGGL((paged_attn_combine_wave_kernel<32, 4>), dim3((unsigned)ceil_div(nvec, 8)),
+                           dim3(256), 0, s, qs, ml, acc, (uint16_t*)out, qh, hd, nsplit, nvec,
+                           split_pos);
+    else if (nsplit <= kCombWaveMaxSplits)
+        hipLaunchKernelGGL((paged_attn_combine_wave_kernel<64, 1>), dim3((unsigned)ceil_div(nvec, 4)),
                            dim3(256), 0, s, qs, ml, acc, (uint16_t*)out, qh, hd, nsplit, nvec,
                            split_pos);
     else

@@ -1,8 +1,9 @@
 // Host build of the MFMA decode-attention kernel's index arithmetic (tq_attn_index.h), for the
-// CPU bounds check of the kernel's global accesses. Each entry evaluates the same inline
+// CPU bounds check of the kernel's global accesses, and of the launchers' rules (attn_rules.h). Each entry evaluates the same inline
 // functions the kernel calls, over all 64 lanes where an index depends on the lane.
 #include <stdint.h>
 
+#include "attn_rules.h"
 #include "tq_attn_index.h"
 
 extern "C" {
@@ -120,6 +121,11 @@ int fhip_idx_q_vectors(int tq0, int tok, int G, int nq, int qh, int g, int64_t* 
 // block blk).
 int64_t fhip_idx_partial_row(int h, int tq0, int G, int qh, int g, int nsplit, int blk) {
     return fhip_idx::partial_row(fhip_idx::partial_vector(h, tq0, G, qh, g), nsplit, blk);
+}
+
+// Waves per split of an FP16 decode launch (attn_rules.h).
+int fhip_rule_paged_waves(int64_t items, int hd, int max_tokens) {
+    return fhip_rules::paged_waves(items, hd, max_tokens);
 }
 
 }  // extern "C"

@@ -1,0 +1,18 @@
+"""Which kernel and split the attention launchers choose (fracture_amd/csrc/attn_rules.h), on the CPU."""
+import pytest
+
+import rules
+
+
+@pytest.mark.parametrize("queries,qh,kvh,hd,tokens,waves", [
+    # up to 256, 512, 1024 splits and more, tables of whole splits
+    (1, 32, 8, 128, 4000, 8), (32, 32, 8, 128, 1024, 8), (33, 32, 8, 128, 1024, 4), (64, 32, 8, 128, 1000, 4),
+    (65, 32, 8, 128, 1024, 2), (128, 32, 8, 128, 1024, 2), (129, 32, 8, 128, 1024, 1),
+    (64, 32, 8, 128, 4000, 1), (256, 32, 8, 128, 1100, 1), (64, 32, 32, 128, 1000, 1),
+    (16, 64, 8, 64, 8000, 2), (16, 8, 8, 32, 8000, 1), (256, 16, 4, 256, 1000, 1), (128, 16, 4, 256, 1000, 4),
+    # short tables: no waves past their end, at head_dim 128 not below two
+    (1, 32, 8, 128, 128, 2), (1, 32, 8, 128, 144, 8), (64, 32, 8, 128, 256, 2), (64, 32, 8, 128, 272, 4),
+    (128, 32, 8, 128, 100, 2), (256, 32, 8, 128, 16, 1), (8, 16, 8, 64, 64, 1), (8, 16, 8, 64, 208, 8),
+    (64, 16, 8, 64, 368, 1), (64, 16, 8, 64, 400, 4), (64, 8, 8, 32, 16, 1), (8, 16, 4, 256, 100, 1)])
+def test_waves_of_a_paged_decode(queries, qh, kvh, hd, tokens, waves):
+    assert rules.paged_waves(queries, qh, kvh, hd, tokens) == waves

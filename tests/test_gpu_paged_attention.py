@@ -12,6 +12,7 @@ import pytest
 import torch
 
 import oracle
+import rules
 from conftest import assert_close
 from fracture_amd import kernels as K
 
@@ -66,13 +67,13 @@ def test_decode_small_contexts(dev, hd, qh, kvh):
                      f"seq {b} len {n}")
 
 
-@pytest.mark.parametrize("nseq,qh,kvh,hd", [
-    (32, 8, 8, 64), (33, 8, 8, 64), (33, 32, 8, 128), (64, 16, 8, 32), (65, 16, 8, 128), (65, 16, 8, 256),
-    (65, 64, 64, 32)])
-def test_decode_waves_per_split(dev, nseq, qh, kvh, hd):
-    """8, 4, 2 and 1 waves per split (up to 256, 512, 4096 and more workgroups): lengths that leave
-    waves empty, end inside each wave's piece and on its edges, and a masked page that is a
-    wave's whole piece of one chunk."""
+@pytest.mark.parametrize("nseq,qh,kvh,hd,waves", [
+    (32, 8, 8, 64, 8), (33, 8, 8, 64, 4), (33, 32, 8, 128, 4), (64, 16, 8, 32, 4), (65, 16, 8, 128, 2),
+    (65, 16, 8, 64, 2), (65, 16, 8, 256, 1), (65, 64, 64, 32, 1)])
+def test_decode_waves_per_split(dev, nseq, qh, kvh, hd, waves):
+    """8, 4, 2 and 1 waves per split: lengths that leave waves empty, end inside each wave's piece and on
+    its edges, and a masked page that is a wave's whole piece of one chunk."""
+    assert rules.paged_waves(nseq, qh, kvh, hd, 1024) == waves
     rng = np.random.default_rng(nseq + hd)
     edges = [0, 1, 127, 128, 129, 255, 257, 511, 512, 513, 640, 897, 1000, 1023, 1024]
     lens = (edges * 5)[:nseq]
@@ -91,6 +92,33 @@ def test_decode_waves_per_split(dev, nseq, qh, kvh, hd):
         want = oracle.paged_attention(q[b], rows, n, kp, vp, kvh) if n else np.zeros_like(q[b])
         assert_close(got[b].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3,
                      f"seq {b} len {n}")
+
+
+@pytest.mark.parametrize("nseq,qh,kvh,hd,widest", [
+    (343, 4, 1, 128, 2100),   # 1029 splits: the last workgroup's second wave has none
+    (343, 8, 1, 128, 2100), (172, 16, 2, 128, 2100), (172, 8, 2, 64, 3000), (515, 4, 2, 256, 20),
+    (257, 8, 2, 256, 1100), (1025, 1, 1, 32, 100)])
+def test_decode_one_wave_per_split(dev, nseq, qh, kvh, hd, widest):
+    """Two splits of neighbouring kv heads to a workgroup, each a wave's own: odd counts of splits, pairs
+    across a split and a sequence, a wave whose split lies past its sequence beside one that goes on,
+    a masked page, empty sequences."""
+    assert rules.paged_waves(nseq, qh, kvh, hd, -(-widest // 16) * 16) == 1
+    rng = np.random.default_rng(nseq + hd)
+    some = [n for n in (0, 1, 15, 17, 33, 640, 1000, 1023, 1024, 1025, 2048, widest) if n <= widest]
+    lens = [some[b] if b < len(some) else (b * 7) % 40 for b in range(nseq)]
+    lens[-1] = widest
+    kp, vp, table = build_pool(rng, lens, kvh, hd)
+    masked = {}
+    for b in (5, nseq - 1):
+        if lens[b] >= 48:
+            table[b, 1] = -1  # positions 16..31
+            masked[b] = np.delete(table[b], 1)
+    q = (rng.standard_normal((nseq, qh, hd)) * 2).astype(np.float16)
+    got = run_decode(dev, q, table, lens, kp, vp, kvh)
+    for b in sorted(set(range(len(some) + 4)) | {nseq // 2, nseq - 2, nseq - 1}):
+        n = lens[b] - 16 if b in masked else lens[b]
+        want = oracle.paged_attention(q[b], masked.get(b, table[b]), n, kp, vp, kvh) if n else np.zeros_like(q[b])
+        assert_close(got[b].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3, f"seq {b} len {lens[b]}")
 
 
 @pytest.mark.parametrize("hd", [128, 64, 80])
