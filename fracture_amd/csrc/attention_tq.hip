@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "attn_rules.h"
 #include "fhip_internal.h"
 #include "tq_attn_index.h"
 #include "tq_quant.h"
@@ -25,9 +26,8 @@ using namespace fhip;
 
 namespace {
 
-constexpr int kSplit = 1024;   // positions per split workgroup
-constexpr int kFinePart = 256; // and in launches too small to fill the chip with those
-constexpr size_t kFineBytes = (size_t)24 << 20;  // the largest workspace that finer splits may ask for
+constexpr int kSplit = fhip_rules::kTqSplit;        // positions per split workgroup
+constexpr int kFinePart = fhip_rules::kTqFinePart;  // and in small launches
 constexpr int kSub = 256;      // positions per pass (one per lane in the score phase)
 constexpr int kMaxG = 8;       // q heads per kv head
 constexpr int kMaxHd = 256;
@@ -657,8 +657,9 @@ __global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
 //     4 on their way into registers (K) or LDS (V); 8-bit codes have one table entry each.
 //
 // A workgroup owns one (query, kv head, 1024-position block); each of its W waves walks an
-// equal split of it in 64-position chunks (two waves of 512 positions, or eight of 128 where a
-// launch has few workgroups):
+// equal split of it in 64-position chunks (two waves of 512 positions, four of 256 where a launch
+// has few workgroups, or four of 64 over a block of 256 positions where it has very few; tq_route
+// in attn_rules.h):
 //   QK  D[pos][col] = sum_k A[pos][k] B[k][col] on v_mfma_f32_16x16x32_f16. The K slots come
 //       in (hi, lo') pairs per coordinate: A = (c_hi, c_lo*2^12) of the position's centroid,
 //       B = (q_hi, 0) in column h and (q_lo*2^12, q_hi) in column 8+h, so one MFMA gives
@@ -680,7 +681,7 @@ constexpr int kChunkM = 64;     // positions per chunk
 constexpr int kSplitMfma = 512;  // positions per wave (split) at two waves per workgroup
 constexpr int kXcds = 8;         // MI355X: accelerator complex dies, each with its own L2
 constexpr int kWavesM = 2;      // waves per workgroup, large launches
-constexpr int kWavesWide = 8;   // and small ones
+constexpr int kWavesWide = 4;   // and small ones
 static_assert(kChunkM == fhip_idx::kChunk && kSplitMfma == fhip_idx::kSplitPositions &&
                   kWavesM == fhip_idx::kBlockWaves && kXcds == fhip_idx::kXcdCount &&
                   FHIP_PAGE_TOKENS == fhip_idx::kPageTokens,
@@ -1662,15 +1663,15 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
 // 324 with the decode kernel; 1500 at 1000: 246 and 389 us.
 // ---------------------------------------------------------------------------------------
 constexpr int kPqWaves = 4;
-constexpr int kPqCols = 32 * kPqWaves;  // columns per workgroup
-constexpr int kPqTile = 64;             // positions per tile
+constexpr int kPqCols = fhip_rules::kPqCols;
+constexpr int kPqTile = fhip_rules::kPqTile;
+static_assert(kPqCols == 32 * kPqWaves, "a wave has the 32 columns of its MFMA");
 constexpr int kPqRowK = 256 + 16;       // bytes per K row in LDS: 16 rows' 16-byte reads on all banks
 constexpr int kPqRowV = 256 + 64;       // per V row: the transposed reads of 4 rows x 32 dims
 constexpr float kPqBias = 13.0f;        // log2 of the scale that p carries
 // log2 that p may exceed it by before a rescale: w < 2^16 (1 - 2^-11) (an fp16 norm's largest share of
 // its power of two), which fp16 holds
 constexpr float kPqSlack = 3.0f;
-constexpr int64_t kPqGroups = 512;      // workgroups wanted: the two per CU that fit at once
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x2c_t __attribute__((ext_vector_type(2)));
 typedef float f32x2c_t __attribute__((ext_vector_type(2)));
@@ -2063,40 +2064,20 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
                         acc[d][4 * j + 3] * unit};
 }
 
-// Eight waves per block up to this many workgroups, two beyond (32 / 8 heads, K4/V2: 16 sequences of
-// 500 .. 2000, 256 workgroups: 39 -> 30 us; 16 sequences of 2000 .. 8000 at 8 heads a group, 512
-// workgroups: 53 -> 46; 64 of 500 .. 2000, 1024 workgroups: 53 with two, 58 with eight). 8-bit codes
-// keep twice the registers and buffers a wave: at 512 workgroups 50 us with two, 52 with eight.
-constexpr int64_t kWideGroups = 512, kWideGroups8 = 256;
-
-// The (K, V) code widths that the MFMA kernel is built for: the default cache, equal widths, and the
-// protected layers' 8 bits. On the VALU split kernel, which takes any other pair, 8 sequences of 1000
-// .. 8000 measured 438 us at 8 bits, 200 at 3 and 191 at 2, against 50, 43 and 44 here.
-bool mfma_widths(int kbits, int vbits) {
-    return (kbits == 4 && (vbits == 4 || vbits == 2)) ||
-           (kbits == vbits && (kbits == 2 || kbits == 3 || kbits == 8));
-}
-
-int decode_group(const Queries& qs, int nq, int G) {
-    return (!qs.seq_lens && qs.table_stride == 0 && nq > 1 && G < 8) ? 8 / G : 1;
-}
-int64_t decode_groups(int nq, int tok, int kvh, int nsplit) {
-    return ceil_div(ceil_div((int64_t)nq, tok) * nsplit, kXcds) * kXcds * kvh;
-}
-
 template <class Pages, int KB, int VB>
 void launch_mfma_t(const float* qrot, const Queries& q2, const Pages& pg, const float* kcent,
-                   const float* vcent, int qh, int kvh, int nsplit, int part, int tok, int64_t wgs,
-                   float* ml, float* acc, hipStream_t s) {
+                   const float* vcent, int qh, int kvh, int nsplit, const fhip_rules::TqRoute& route,
+                   int64_t wgs, float* ml, float* acc, hipStream_t s) {
+    const int tok = route.tok;
     const bool g4 = qh / kvh <= 4 && tok == 1;
     auto go = [&](auto kern, int waves) {
         hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * waves), 0, s, qrot, q2, pg, kcent, vcent,
                            qh, kvh, 1.0f / sqrtf(128.0f), ml, acc, nsplit, nsplit, tok);
     };
-    if (part == kFinePart)
+    if (route.part == kFinePart)
         go(g4 ? tq_attn_mfma_kernel<Pages, true, KB, VB, 4, kFinePart>
               : tq_attn_mfma_kernel<Pages, false, KB, VB, 4, kFinePart>, 4);
-    else if (wgs <= (KB == 8 ? kWideGroups8 : kWideGroups))
+    else if (route.waves == kWavesWide)
         go(g4 ? tq_attn_mfma_kernel<Pages, true, KB, VB, kWavesWide, kSplit>
               : tq_attn_mfma_kernel<Pages, false, KB, VB, kWavesWide, kSplit>, kWavesWide);
     else
@@ -2107,28 +2088,27 @@ void launch_mfma_t(const float* qrot, const Queries& q2, const Pages& pg, const 
 template <class Pages>
 void launch_mfma_split(const float* qrot, const Queries& qsv, const Pages& pg,
                        const float* kcent, const float* vcent, int nq, int qh, int kvh,
-                       int nsplit, int part, int kbits, int vbits, float* ml, float* acc,
-                       hipStream_t s) {
+                       int nsplit, const fhip_rules::TqRoute& route, int kbits, int vbits, float* ml,
+                       float* acc, hipStream_t s) {
     // Causal prefill (queries at consecutive positions of one sequence: one shared block table,
     // lengths from start_pos) groups 8 / G consecutive queries per item so that they share the
     // MFMA columns and every code lookup; decode keeps one query per item.
-    const int tok = decode_group(qsv, nq, qh / kvh);
     // one workgroup per (item, kv head, part-position block): the block count is the
     // partial layout's split count; the (item, block) pairs are padded to a multiple of the
     // XCD count (the kernel's index spreads them, not heads, over the XCDs)
-    const int64_t wgs = decode_groups(nq, tok, kvh, nsplit);
+    const int64_t wgs = fhip_rules::tq_decode_workgroups(nq, route.tok, kvh, nsplit);
     Queries q2 = qsv;
     q2.seq_lens_count = nq;
     if (kbits == 8)
-        launch_mfma_t<Pages, 8, 8>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 8, 8>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, route, wgs, ml, acc, s);
     else if (kbits == 3)
-        launch_mfma_t<Pages, 3, 3>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 3, 3>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, route, wgs, ml, acc, s);
     else if (kbits == 2)
-        launch_mfma_t<Pages, 2, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 2, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, route, wgs, ml, acc, s);
     else if (vbits == 2)
-        launch_mfma_t<Pages, 4, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 4, 2>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, route, wgs, ml, acc, s);
     else
-        launch_mfma_t<Pages, 4, 4>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, part, tok, wgs, ml, acc, s);
+        launch_mfma_t<Pages, 4, 4>(qrot, q2, pg, kcent, vcent, qh, kvh, nsplit, route, wgs, ml, acc, s);
 }
 
 struct AttnArgs {
@@ -2139,31 +2119,8 @@ struct AttnArgs {
     const float *krot, *vrot, *kcent, *vcent;
     int qh, kvh, hd, kbits, vbits;
     void* ws;
-    size_t ws_bytes = kFineBytes;  // what `ws` holds, at least ws_layout's at kSplit positions
+    size_t ws_bytes = fhip_rules::kTqFineBytes;  // what `ws` holds, at least tq_layout's at kSplit positions
 };
-
-// The workspace: q_rot, then (m, l) and the accumulators of the split partials, one split per `part`
-// positions.
-size_t ws_layout(int nq, int qh, int hd, int max_tokens, int part, size_t* off_ml, size_t* off_acc,
-                 int* nsplit) {
-    const int ns = max_tokens > 0 ? (max_tokens + part - 1) / part : 1;
-    const size_t qrot = (size_t)nq * qh * hd * sizeof(float);
-    const size_t ml = (size_t)nq * qh * ns * 2 * sizeof(float);
-    const size_t acc = (size_t)nq * qh * ns * hd * sizeof(float);
-    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    if (off_ml) *off_ml = al(qrot);
-    if (off_acc) *off_acc = al(qrot) + al(ml);
-    if (nsplit) *nsplit = ns;
-    return al(qrot) + al(ml) + al(acc);
-}
-// Small launches may split finer, where the layout of kFinePart positions stays within kFineBytes. The
-// size a caller is asked for covers that layout at every smaller size too (it never falls as an
-// argument grows), so a workspace warmed up at the largest call serves the smaller ones.
-size_t ws_bytes_for(int nq, int qh, int hd, int max_tokens) {
-    return std::max(ws_layout(nq, qh, hd, max_tokens, kSplit, nullptr, nullptr, nullptr),
-                    std::min(ws_layout(nq, qh, hd, max_tokens, kFinePart, nullptr, nullptr, nullptr),
-                             kFineBytes));
-}
 
 template <int KB, int VB, class Pages>
 void launch_split(const AttnArgs& a, const Pages& pg, int nsplit, float* ml, float* acc,
@@ -2176,37 +2133,13 @@ void launch_split(const AttnArgs& a, const Pages& pg, int nsplit, float* ml, flo
                        a.kvh, a.hd, 1.0f / sqrtf((float)a.hd), ml, acc, nsplit);
 }
 
-// Workgroups of the prefill kernel with up to nsplit splits. Below kPqMinGroups the decode kernel,
-// whose waves share a split, is the faster one (16 queries at 100, 16 workgroups: 26 against 32 us);
-// above it this one is (64 at 2000, 144: 48 against 55; 200 at 1000, K8/V8, 280: 62 against 88).
-constexpr int64_t kPqMinGroups = 96;
-int64_t prefill_groups(const AttnArgs& a, int nsplit) {
-    const int64_t base = ceil_div((int64_t)a.nq, kPqCols / (a.qh / a.kvh)) * a.kvh;
-    return a.nq > 1 ? base * std::min<int64_t>(std::max<int64_t>(ceil_div(kPqGroups, base), 1), nsplit) : 0;
-}
-// Decode launches of up to this many 1024-position workgroups split at kFinePart positions, four waves
-// of one chunk each: four times the workgroups (one sequence of 4000, 32 of them: 29 -> 23 us; at
-// 256, 16 sequences of 500 .. 2000: 30 us either way).
-constexpr int64_t kFineGroups = 256;
-
-// Launches the prefill kernel; *nsplit (in: what the workspace holds) and *split_pos become its own,
-// *merged tells whether it left merged vectors in qrot.
-void launch_prefill(float* qrot, const AttnArgs& a, const PtrPages& pg, bool batched_rot, int* nsplit,
-                    int* split_pos, bool* merged, float* ml, float* acc, hipStream_t s) {
-    const int G = a.qh / a.kvh;
-    const int nqb = kPqCols / G;
-    const int nblk = (int)ceil_div((int64_t)a.nq, nqb);
-    const int64_t base = (int64_t)nblk * a.kvh;
-    const int extent = std::max(std::min(a.qs.kv_len, a.qs.max_blocks * FHIP_PAGE_TOKENS), 1);
-    const int64_t want = std::min<int64_t>(std::max<int64_t>(ceil_div(kPqGroups, base), 1), *nsplit);
-    *split_pos = (int)(ceil_div(ceil_div(extent, want), kPqTile) * kPqTile);
-    *nsplit = (int)ceil_div(extent, *split_pos);
-    *merged = *nsplit == 1 && batched_rot;
+// Launches the prefill kernel; `merged`: it leaves merged vectors in qrot.
+void launch_prefill(float* qrot, const AttnArgs& a, const PtrPages& pg, const fhip_rules::PrefillSplit& ps,
+                    bool merged, float* ml, float* acc, hipStream_t s) {
     // Blocks start from the last (the longest contexts) down. Where all fit at once, two to a CU, the
     // second half goes up from the first instead, so that a long block shares its CU with a short one.
-    const int64_t wgs = base * *nsplit;
     const int cus = fhip_host::cu_count();
-    const int fold = *nsplit == 1 && wgs > cus && wgs <= 2 * cus ? (int)(cus / a.kvh) : 0;
+    const int fold = ps.nsplit == 1 && ps.workgroups > cus && ps.workgroups <= 2 * cus ? (int)(cus / a.kvh) : 0;
     Queries q2 = a.qs;
     q2.seq_lens_count = a.nq;
     auto kern = a.kbits == 8   ? tq_attn_prefill_kernel<8, 8>
@@ -2214,33 +2147,27 @@ void launch_prefill(float* qrot, const AttnArgs& a, const PtrPages& pg, bool bat
                 : a.kbits == 2 ? tq_attn_prefill_kernel<2, 2>
                 : a.vbits == 2 ? tq_attn_prefill_kernel<4, 2>
                                : tq_attn_prefill_kernel<4, 4>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)wgs), dim3(64 * kPqWaves), 0, s, qrot, q2, pg, a.kcent,
-                       a.vcent, a.qh, a.kvh, 1.4426950408889634f / sqrtf(128.0f), ml, acc, *nsplit,
-                       *split_pos, nqb, nblk, fold, *merged);
+    hipLaunchKernelGGL(kern, dim3((unsigned)ps.workgroups), dim3(64 * kPqWaves), 0, s, qrot, q2, pg, a.kcent,
+                       a.vcent, a.qh, a.kvh, 1.4426950408889634f / sqrtf(128.0f), ml, acc, ps.nsplit,
+                       ps.split_pos, ps.nqb, ps.nblk, fold, merged);
 }
 
 template <class Pages>
 int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
     if (a.nq == 0) return hipSuccess;
-    const int G = a.qh / a.kvh, max_tokens = a.qs.max_blocks * FHIP_PAGE_TOKENS;
-    const bool mfma = mfma_widths(a.kbits, a.vbits) && a.hd == 128 && G <= 8;
-    int split_pos = kSplit, nsplit;
-    bool prefill = false;
-    if (mfma) {
-        const bool fine = ws_layout(a.nq, a.qh, a.hd, max_tokens, kFinePart, nullptr, nullptr, &nsplit) <=
-                          std::min(a.ws_bytes, kFineBytes);
-        if constexpr (std::is_same_v<Pages, PtrPages>)
-            prefill = !a.qs.seq_lens && a.qs.table_stride == 0 &&
-                      prefill_groups(a, fine ? nsplit : (int)ceil_div(max_tokens, kSplit)) >= kPqMinGroups;
-        if (fine && (prefill || decode_groups(a.nq, decode_group(a.qs, a.nq, G), a.kvh,
-                                              (int)ceil_div(max_tokens, kSplit)) <= kFineGroups))
-            split_pos = kFinePart;
+    const int max_tokens = a.qs.max_blocks * FHIP_PAGE_TOKENS;
+    const bool causal = std::is_same_v<Pages, PtrPages> && !a.qs.seq_lens && a.qs.table_stride == 0;
+    const fhip_rules::TqRoute route = fhip_rules::tq_route({a.nq, a.qh, a.kvh, a.hd, a.kbits, a.vbits, max_tokens,
+                                                            a.qs.kv_len, causal, a.ws_bytes});
+    const fhip_rules::TqLayout layout = fhip_rules::tq_layout(a.nq, a.qh, a.hd, max_tokens, route.part);
+    int nsplit = layout.nsplit, split_pos = route.part;
+    if (route.kind == fhip_rules::TqRoute::kPrefill) {
+        nsplit = route.prefill.nsplit;
+        split_pos = route.prefill.split_pos;
     }
-    size_t off_ml, off_acc;
-    ws_layout(a.nq, a.qh, a.hd, max_tokens, split_pos, &off_ml, &off_acc, &nsplit);
     float* qrot = (float*)a.ws;
-    float* ml = (float*)((char*)a.ws + off_ml);
-    float* acc = (float*)((char*)a.ws + off_acc);
+    float* ml = (float*)((char*)a.ws + layout.off_ml);
+    float* acc = (float*)((char*)a.ws + layout.off_acc);
     const int nvec = a.nq * a.qh;
     // Many vectors (prefill): both rotations as batched MFMA products (the VALU kernels'
     // per-workgroup copies of Pi would cross L2 once per 8 vectors); the merged outputs reuse
@@ -2258,12 +2185,13 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
         hipLaunchKernelGGL(tq_attn_prerotate_kernel, dim3(rot_groups), dim3(256), 0, s,
                            (const uint16_t*)a.q, a.krot, qrot, a.hd, nvec);
     }
-    bool merged = false;  // the split kernel has left the merged vectors in q_rot
-    if (prefill) {
+    // one split: the prefill kernel leaves the merged vectors in q_rot
+    const bool merged = route.kind == fhip_rules::TqRoute::kPrefill && nsplit == 1 && batched_rot;
+    if (route.kind == fhip_rules::TqRoute::kPrefill) {
         if constexpr (std::is_same_v<Pages, PtrPages>)
-            launch_prefill(qrot, a, pg, batched_rot, &nsplit, &split_pos, &merged, ml, acc, s);
-    } else if (mfma)
-        launch_mfma_split(qrot, a.qs, pg, a.kcent, a.vcent, a.nq, a.qh, a.kvh, nsplit, split_pos,
+            launch_prefill(qrot, a, pg, route.prefill, merged, ml, acc, s);
+    } else if (route.kind == fhip_rules::TqRoute::kDecode)
+        launch_mfma_split(qrot, a.qs, pg, a.kcent, a.vcent, a.nq, a.qh, a.kvh, nsplit, route,
                           a.kbits, a.vbits, ml, acc, s);
     else if (a.kbits == 4 && a.vbits == 4)
         launch_split<4, 4>(a, pg, nsplit, ml, acc, s);
@@ -2348,7 +2276,7 @@ extern "C" {
 size_t fhip_attention_tq_workspace_bytes(int batch, int num_q_heads, int head_dim,
                                          int max_blocks) {
     if (batch <= 0 || num_q_heads <= 0 || head_dim <= 0 || max_blocks <= 0) return 0;
-    return ws_bytes_for(batch, num_q_heads, head_dim, max_blocks * FHIP_PAGE_TOKENS);
+    return fhip_rules::tq_workspace_bytes(batch, num_q_heads, head_dim, max_blocks * FHIP_PAGE_TOKENS);
 }
 
 int fhip_launch_attention_tq_decode(void* output, const void* q, const int32_t* block_table,
@@ -2519,7 +2447,7 @@ static int attention_paged_tq_ref(void* output, const void* q, const int* block_
                         !v_norms_ptrs))
         return hipErrorInvalidValue;
     const int mb = nblocks > 0 ? nblocks : 1;
-    const size_t need = ws_bytes_for(num_tokens, num_q_heads, head_dim, mb * FHIP_PAGE_TOKENS);
+    const size_t need = fhip_rules::tq_workspace_bytes(num_tokens, num_q_heads, head_dim, mb * FHIP_PAGE_TOKENS);
     const bool own = ws == nullptr;
     if (!own && ws_bytes < need) return hipErrorInvalidValue;
     if (own) {
@@ -2584,9 +2512,9 @@ int fhip_launch_attention_paged_tq_noalloc(void* output, const void* q, const in
         return hipErrorInvalidValue;
     if (num_tokens == 0) return hipSuccess;
     const int nblocks = (kv_len + FHIP_PAGE_TOKENS - 1) / FHIP_PAGE_TOKENS;
-    const size_t need = ws_bytes_for(num_tokens, num_q_heads, head_dim,
+    const size_t need = fhip_rules::tq_workspace_bytes(num_tokens, num_q_heads, head_dim,
                                      (nblocks > 0 ? nblocks : 1) * FHIP_PAGE_TOKENS);
-    static_assert(kFineBytes <= kNoAllocScratchBytes, "finer splits never make a call too large");
+    static_assert(fhip_rules::kTqFineBytes <= kNoAllocScratchBytes, "finer splits never make a call too large");
     if (need > kNoAllocScratchBytes) return hipErrorOutOfMemory;
     hipStream_t s = fhip_host::as_stream(stream);
     int dev = -1;

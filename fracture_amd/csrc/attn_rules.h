@@ -37,4 +37,134 @@ inline int paged_waves(int64_t items, int hd, int max_tokens) {
     return span * w >= 1536 ? w : 1;
 }
 
+// ---------------------------------------------------------------------------------------
+// Causal prefill on the tiled kernels: query blocks of `cols` (query, head) columns, and as many splits of
+// the positions as bring the launch to `groups` workgroups, of whole tiles each.
+// ---------------------------------------------------------------------------------------
+struct PrefillSplit {
+    int nqb, nblk;          // queries per block, blocks
+    int nsplit, split_pos;  // splits, positions of each
+    int64_t workgroups;
+};
+inline PrefillSplit prefill_split(int nq, int G, int kvh, int cols, int tile, int64_t groups, int extent,
+                                  int max_splits) {
+    PrefillSplit p;
+    p.nqb = cols / G;
+    p.nblk = (int)div_up(nq, p.nqb);
+    const int64_t base = (int64_t)p.nblk * kvh;
+    extent = std::max(extent, 1);
+    const int64_t want = std::min<int64_t>(std::max<int64_t>(div_up(groups, base), 1), max_splits);
+    p.split_pos = (int)(div_up(div_up(extent, want), tile) * tile);
+    p.nsplit = (int)div_up(extent, p.split_pos);
+    p.workgroups = base * p.nsplit;
+    return p;
+}
+
+// ---------------------------------------------------------------------------------------
+// TurboQuant attention
+// ---------------------------------------------------------------------------------------
+constexpr int kTqSplit = 1024;     // positions per split partial
+constexpr int kTqFinePart = 256;   // and in launches too small to fill the chip with those
+constexpr size_t kTqFineBytes = (size_t)24 << 20;  // the largest workspace that finer splits may ask for
+
+// The workspace: q_rot, then (m, l) and the accumulators of the split partials, one split per `part`
+// positions.
+struct TqLayout {
+    size_t off_ml, off_acc, bytes;
+    int nsplit;
+};
+inline TqLayout tq_layout(int nq, int qh, int hd, int max_tokens, int part) {
+    TqLayout l;
+    l.nsplit = max_tokens > 0 ? (max_tokens + part - 1) / part : 1;
+    auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
+    const size_t qrot = (size_t)nq * qh * hd * sizeof(float);
+    const size_t ml = (size_t)nq * qh * l.nsplit * 2 * sizeof(float);
+    const size_t acc = (size_t)nq * qh * l.nsplit * hd * sizeof(float);
+    l.off_ml = al(qrot);
+    l.off_acc = l.off_ml + al(ml);
+    l.bytes = l.off_acc + al(acc);
+    return l;
+}
+// Small launches may split finer, where the layout of kTqFinePart positions stays within kTqFineBytes. The
+// size a caller is asked for covers that layout at every smaller size too (it never falls as an
+// argument grows), so a workspace warmed up at the largest call serves the smaller ones.
+inline size_t tq_workspace_bytes(int nq, int qh, int hd, int max_tokens) {
+    return std::max(tq_layout(nq, qh, hd, max_tokens, kTqSplit).bytes,
+                    std::min(tq_layout(nq, qh, hd, max_tokens, kTqFinePart).bytes, kTqFineBytes));
+}
+
+// The (K, V) code widths that the MFMA kernels are built for: the default cache, equal widths, and the
+// protected layers' 8 bits. On the VALU split kernel, which takes any other pair, 8 sequences of 1000
+// .. 8000 measured 438 us at 8 bits, 200 at 3 and 191 at 2, against 50, 43 and 44 on the MFMA kernel.
+inline bool tq_mfma_widths(int kbits, int vbits) {
+    return (kbits == 4 && (vbits == 4 || vbits == 2)) ||
+           (kbits == vbits && (kbits == 2 || kbits == 3 || kbits == 8));
+}
+
+struct TqCall {
+    int nq, qh, kvh, hd, kbits, vbits;
+    int max_tokens;   // positions that the block table describes
+    int kv_len;       // causal: positions of the sequence
+    bool causal;      // consecutive queries of one sequence over one table
+    size_t ws_bytes;  // of the workspace, at least tq_layout's at kTqSplit
+};
+struct TqRoute {
+    enum Kind { kValu, kDecode, kPrefill } kind;
+    int part;   // positions per partial of the layout
+    int waves;  // kDecode: per workgroup
+    int tok;    // kDecode: queries per workgroup (its MFMA columns are tok x G)
+    PrefillSplit prefill;
+};
+constexpr int kXcds = 8;
+inline int64_t tq_decode_workgroups(int nq, int tok, int kvh, int nsplit) {
+    return div_up(div_up(nq, tok) * nsplit, kXcds) * kXcds * kvh;
+}
+constexpr int kPqCols = 128;        // prefill kernel: columns per workgroup
+constexpr int kPqTile = 64;         // positions per tile
+constexpr int64_t kPqGroups = 512;  // workgroups wanted: the two per CU that fit at once
+
+// The route of a call. Times in us at K4/V2 unless said otherwise.
+//   The decode kernel in 256-position parts, four waves of one chunk each, where that makes at most three
+//   workgroups per CU and 48 parts: four times the workgroups of 1024-position parts (one sequence of
+//   1000, 32 / 8 heads: 16.5 us; 23.3 in 1024-position blocks of four waves, 31.2 of two). More
+//   workgroups run in turns (512 queries' worth, 64 sequences of 1000: 39.9 and 35.5), and more parts
+//   make the merge the larger half (one sequence of 20000, 79 parts: 28.3 and 25.6; 32000: 37.3 and 26.8).
+//   Else 1024-position parts: four waves up to 512 workgroups (64 sequences of 1000: 35.5 us, with two
+//   42.8, with eight 39.6; of 16: 21.3, 21.5, 24.1), two beyond (64 of 3000, 1536 workgroups: 62.6 us,
+//   with four 64.8).
+//   The prefill kernel takes causal calls that give it 96 workgroups (64 queries at 2000, 144 workgroups:
+//   48, decoded 55; 16 at 100, 16 workgroups: 32 and 26).
+inline TqRoute tq_route(const TqCall& c) {
+    TqRoute r;
+    const int G = c.qh / c.kvh;
+    r.kind = TqRoute::kValu;
+    r.part = kTqSplit;
+    r.waves = 0;
+    r.tok = 1;
+    r.prefill = {};
+    if (!tq_mfma_widths(c.kbits, c.vbits) || c.hd != 128 || G > 8) return r;
+    r.kind = TqRoute::kDecode;
+    r.tok = c.causal && c.nq > 1 && G < 8 ? 8 / G : 1;
+    const TqLayout fine = tq_layout(c.nq, c.qh, c.hd, c.max_tokens, kTqFinePart);
+    const bool fits = fine.bytes <= std::min(c.ws_bytes, kTqFineBytes);
+    const int nsplit = tq_layout(c.nq, c.qh, c.hd, c.max_tokens, kTqSplit).nsplit;
+    const int64_t wgs = tq_decode_workgroups(c.nq, r.tok, c.kvh, nsplit);
+    if (c.causal && c.nq > 1) {
+        r.prefill = prefill_split(c.nq, G, c.kvh, kPqCols, kPqTile, kPqGroups,
+                                  std::min(c.kv_len, c.max_tokens), fits ? fine.nsplit : nsplit);
+        if (r.prefill.workgroups >= 96) {
+            r.kind = TqRoute::kPrefill;
+            r.part = fits ? kTqFinePart : kTqSplit;
+            return r;
+        }
+    }
+    if (fits && fine.nsplit <= 48 && tq_decode_workgroups(c.nq, r.tok, c.kvh, fine.nsplit) <= 768) {
+        r.part = kTqFinePart;
+        r.waves = 4;
+    } else {
+        r.waves = wgs <= 512 ? 4 : 2;
+    }
+    return r;
+}
+
 }  // namespace fhip_rules

@@ -123,6 +123,28 @@ int64_t fhip_idx_partial_row(int h, int tq0, int G, int qh, int g, int nsplit, i
     return fhip_idx::partial_row(fhip_idx::partial_vector(h, tq0, G, qh, g), nsplit, blk);
 }
 
+// Route of a TurboQuant attention call (attn_rules.h): out[0..5] = kind (0 VALU, 1 decode, 2 prefill), positions per
+// partial, waves, queries per workgroup, splits, positions per split; returns the workspace bytes of its
+// layout.
+int64_t fhip_rule_tq_route(int nq, int qh, int kvh, int hd, int kbits, int vbits, int max_tokens, int kv_len,
+                           int causal, int64_t ws_bytes, int32_t* out) {
+    const fhip_rules::TqRoute r = fhip_rules::tq_route(
+        {nq, qh, kvh, hd, kbits, vbits, max_tokens, kv_len, causal != 0, (size_t)ws_bytes});
+    const fhip_rules::TqLayout l = fhip_rules::tq_layout(nq, qh, hd, max_tokens, r.part);
+    const bool prefill = r.kind == fhip_rules::TqRoute::kPrefill;
+    out[0] = r.kind;
+    out[1] = r.part;
+    out[2] = r.waves;
+    out[3] = r.tok;
+    out[4] = prefill ? r.prefill.nsplit : l.nsplit;
+    out[5] = prefill ? r.prefill.split_pos : r.part;
+    return (int64_t)l.bytes;
+}
+// The workspace size a caller is asked for.
+int64_t fhip_rule_tq_workspace(int nq, int qh, int hd, int max_tokens) {
+    return (int64_t)fhip_rules::tq_workspace_bytes(nq, qh, hd, max_tokens);
+}
+
 // Waves per split of an FP16 decode launch (attn_rules.h).
 int fhip_rule_paged_waves(int64_t items, int hd, int max_tokens) {
     return fhip_rules::paged_waves(items, hd, max_tokens);

@@ -16,3 +16,24 @@ import rules
     (64, 16, 8, 64, 368, 1), (64, 16, 8, 64, 400, 4), (64, 8, 8, 32, 16, 1), (8, 16, 4, 256, 100, 1)])
 def test_waves_of_a_paged_decode(queries, qh, kvh, hd, tokens, waves):
     assert rules.paged_waves(queries, qh, kvh, hd, tokens) == waves
+
+
+@pytest.mark.parametrize("queries,qh,kvh,kbits,vbits,kv_len,part,waves", [
+    # 256-position parts: at most 768 of their workgroups and 48 parts
+    (1, 32, 8, 4, 2, 4001, 256, 4), (32, 32, 8, 4, 2, 700, 256, 4), (64, 32, 8, 4, 4, 16, 256, 4),
+    (1, 32, 8, 4, 2, 12288, 256, 4), (1, 32, 8, 4, 2, 12289, 1024, 4), (1, 32, 8, 8, 8, 32000, 1024, 4),
+    (40, 32, 8, 4, 2, 700, 1024, 4), (64, 32, 8, 3, 3, 1000, 1024, 4), (8, 32, 8, 8, 8, 8000, 1024, 4),
+    # above 512 workgroups two waves
+    (65, 32, 8, 4, 2, 1024, 1024, 2), (64, 32, 8, 4, 2, 32768, 1024, 2), (256, 32, 8, 2, 2, 16, 1024, 2)])
+def test_route_of_a_tq_decode(queries, qh, kvh, kbits, vbits, kv_len, part, waves):
+    r = rules.TqRoute(queries, qh, kvh, kbits, vbits, kv_len)
+    assert (r.kind, r.part, r.waves, r.tok) == (rules.DECODE, part, waves, 1)
+    assert r.nsplit == -(-(-(-kv_len // 16) * 16) // part)
+
+
+@pytest.mark.parametrize("qh,kvh,hd,kbits,vbits", [(8, 2, 64, 4, 4), (8, 2, 256, 4, 2), (8, 2, 128, 8, 2), (8, 2, 128, 3, 4),
+                                                  (8, 2, 128, 5, 5)])
+def test_other_widths_and_head_dims_stay_on_the_valu_kernel(qh, kvh, hd, kbits, vbits):
+    for causal in (False, True):
+        r = rules.TqRoute(300, qh, kvh, kbits, vbits, 3000, causal, hd=hd)
+        assert (r.kind, r.part, r.nsplit) == (rules.VALU, 1024, 3)

@@ -11,6 +11,7 @@ import pytest
 import torch
 
 import oracle
+import rules
 from conftest import assert_close
 from fracture_amd import kernels as K
 from fracture_amd import turboquant as tq
@@ -138,14 +139,18 @@ def test_reference_interface_prefill_causal(dev):
 
 
 @pytest.mark.parametrize("kbits,vbits", [(8, 8), (3, 3), (2, 2), (4, 2), (4, 4)])
-@pytest.mark.parametrize("qh,kvh,reps", [(8, 2, 1), (8, 1, 1), (16, 8, 13)])
-def test_decode_widths_and_waves(dev, kbits, vbits, qh, kvh, reps):
-    """Every width pair of the MFMA kernel, at up to 4 and up to 8 q heads per kv head, eight waves
-    per block (small launches) and two (13 x 5 sequences over 8 kv heads): lengths on the edges of
-    chunks, of the waves' splits and of pages, a masked page, an empty sequence."""
+@pytest.mark.parametrize("qh,kvh,reps,part,waves", [
+    (8, 2, 1, 256, 4), (8, 1, 1, 256, 4), (16, 8, 13, 1024, 2), (64, 8, 13, 1024, 2), (16, 4, 4, 1024, 4),
+    (32, 4, 4, 1024, 4)])
+def test_decode_widths_and_waves(dev, kbits, vbits, qh, kvh, reps, part, waves):
+    """Every width pair of the MFMA kernel, at up to 4 and up to 8 q heads per kv head, in 256-position
+    parts, in 1024-position blocks of four waves and of two: lengths on the edges of chunks, of the
+    waves' splits and of pages, a masked page, an empty sequence."""
     rng = np.random.default_rng(kbits * 10 + vbits + qh)
     hd = 128
-    lens = ([1, 65, 128, 0, 300] if reps > 1 else [1, 63, 64, 65, 127, 129, 511, 513, 0, 1023, 1025])
+    lens = ([1, 65, 128, 0, 300] if waves == 2 else [1, 63, 64, 65, 127, 129, 255, 257, 511, 513, 0, 1023, 1025])
+    route = rules.TqRoute(len(lens) * reps, qh, kvh, kbits, vbits, max(lens))
+    assert (route.kind, route.part, route.waves) == (rules.DECODE, part, waves)
     pool = build_pool(rng, lens, kvh, hd, kbits, vbits)
     pool["table"][2, 1] = -1  # the third sequence (of 128 or 64): positions 16..31 masked
     table, lens = np.tile(pool["table"], (reps, 1)), lens * reps
