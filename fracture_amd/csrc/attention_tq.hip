@@ -123,7 +123,7 @@ __device__ __forceinline__ void row_group(const uint32_t* w, int g, int bits_rt,
 // A workgroup rotates kRotVecs vectors so Pi_k is read once per workgroup: work unit
 // (row i, half) computes row i of vectors 4 half .. 4 half + 3.
 constexpr int kRotVecs = 8;
-constexpr int kMfmaRotVecs = 4096;  // from this many query vectors on, batched MFMA rotations
+constexpr int kMfmaRotVecs = fhip_rules::kRotBatch;  // from this many query vectors on, batched MFMA rotations
 __global__ __launch_bounds__(256) void tq_attn_prerotate_kernel(const uint16_t* __restrict__ q,
                                                                 const float* __restrict__ rot,
                                                                 float* __restrict__ qrot, int hd,
@@ -428,7 +428,7 @@ size_t combine_lds_bytes(int hd, int nsplit, bool merge_only = false) {
 // (m, l), the weights reach the dim loop by lane broadcasts, and each merged vector (fp32,
 // divided by its sum) goes to merged[vector]. The combine kernel's 16-split load batches
 // would be mostly clamped repeats at these sizes.
-constexpr int kMergeWaveMaxSplits = 8;
+constexpr int kMergeWaveMaxSplits = fhip_rules::kMergeSplits;
 __global__ __launch_bounds__(256) void tq_attn_merge_wave_kernel(
     Queries qs, const float* __restrict__ part_ml, const float* __restrict__ part_acc, int qh,
     int hd, int nsplit, int64_t nvec, float* __restrict__ merged, int split_pos) {

@@ -122,6 +122,8 @@ inline int64_t tq_decode_workgroups(int nq, int tok, int kvh, int nsplit) {
 constexpr int kPqCols = 128;        // prefill kernel: columns per workgroup
 constexpr int kPqTile = 64;         // positions per tile
 constexpr int64_t kPqGroups = 512;  // workgroups wanted: the two per CU that fit at once
+constexpr int kRotBatch = 4096;     // vectors from which both rotations are batched MFMA products ...
+constexpr int kMergeSplits = 8;     // ... and the splits that the merge before the second takes in one wave
 
 // The route of a call. Times in us at K4/V2 unless said otherwise.
 //   The decode kernel in 256-position parts, four waves of one chunk each, where that makes at most three
@@ -132,8 +134,12 @@ constexpr int64_t kPqGroups = 512;  // workgroups wanted: the two per CU that fi
 //   Else 1024-position parts: four waves up to 512 workgroups (64 sequences of 1000: 35.5 us, with two
 //   42.8, with eight 39.6; of 16: 21.3, 21.5, 24.1), two beyond (64 of 3000, 1536 workgroups: 62.6 us,
 //   with four 64.8).
-//   The prefill kernel takes causal calls that give it 96 workgroups (64 queries at 2000, 144 workgroups:
-//   48, decoded 55; 16 at 100, 16 workgroups: 32 and 26).
+//   Causal calls of more workgroups than that (than 256 where the codes' expansion is dearer, at 3 and 8
+//   bits) go to the prefill kernel where it is the shorter one: a tile takes a workgroup 4.3 us, with up to
+//   one workgroup per CU, and a decode workgroup of 1024 positions 0.042 us of the whole chip, twice that at
+//   3 and 8 bits. It also has to have 96 workgroups, 128 where its partials are merged by a kernel of their
+//   own. 32 / 8 heads, decoded and tiled: 8 queries at 8000 26.6 and 31.9, 32 at 3000 33.2 and 32.9, 32 at
+//   8000 52 and 40, 8 at 30000 51 and 59, 200 at 1000 of 64 / 8 heads (104 workgroups of 16 tiles) 90 and 92.
 inline TqRoute tq_route(const TqCall& c) {
     TqRoute r;
     const int G = c.qh / c.kvh;
@@ -149,20 +155,25 @@ inline TqRoute tq_route(const TqCall& c) {
     const bool fits = fine.bytes <= std::min(c.ws_bytes, kTqFineBytes);
     const int nsplit = tq_layout(c.nq, c.qh, c.hd, c.max_tokens, kTqSplit).nsplit;
     const int64_t wgs = tq_decode_workgroups(c.nq, r.tok, c.kvh, nsplit);
-    if (c.causal && c.nq > 1) {
-        r.prefill = prefill_split(c.nq, G, c.kvh, kPqCols, kPqTile, kPqGroups,
-                                  std::min(c.kv_len, c.max_tokens), fits ? fine.nsplit : nsplit);
-        if (r.prefill.workgroups >= 96) {
-            r.kind = TqRoute::kPrefill;
-            r.part = fits ? kTqFinePart : kTqSplit;
-            return r;
-        }
-    }
     if (fits && fine.nsplit <= 48 && tq_decode_workgroups(c.nq, r.tok, c.kvh, fine.nsplit) <= 768) {
         r.part = kTqFinePart;
         r.waves = 4;
-    } else {
-        r.waves = wgs <= 512 ? 4 : 2;
+        return r;
+    }
+    r.waves = wgs <= 512 ? 4 : 2;
+    const bool dear = c.kbits == 3 || c.kbits == 8;
+    if (c.causal && c.nq > 1 && wgs > (dear ? 256 : 512)) {
+        const bool batch = (int64_t)c.nq * c.qh >= kRotBatch;
+        // splits beyond what the wave merge takes would go to the merge in LDS, 25 us slower (64 queries at
+        // 3000, 64 / 8 heads: 96 us in 12 splits)
+        const int most = std::min(fits ? fine.nsplit : nsplit, batch ? kMergeSplits : 1 << 30);
+        r.prefill = prefill_split(c.nq, G, c.kvh, kPqCols, kPqTile, kPqGroups,
+                                  std::min(c.kv_len, c.max_tokens), most);
+        const int64_t tiles = r.prefill.split_pos / kPqTile * div_up(r.prefill.workgroups, 256);
+        if (r.prefill.workgroups >= (batch && r.prefill.nsplit > 1 ? 128 : 96) && tiles * (dear ? 50 : 105) < wgs) {
+            r.kind = TqRoute::kPrefill;
+            r.part = fits ? kTqFinePart : kTqSplit;
+        }
     }
     return r;
 }

@@ -37,3 +37,20 @@ def test_other_widths_and_head_dims_stay_on_the_valu_kernel(qh, kvh, hd, kbits, 
     for causal in (False, True):
         r = rules.TqRoute(300, qh, kvh, kbits, vbits, 3000, causal, hd=hd)
         assert (r.kind, r.part, r.nsplit) == (rules.VALU, 1024, 3)
+
+
+@pytest.mark.parametrize("queries,qh,kvh,kbits,vbits,kv_len,kind,part,nsplit,split_pos", [
+    # few columns or short: the decode kernel, in the parts a decode would take
+    (2, 32, 8, 4, 2, 8000, rules.DECODE, 256, 32, 256), (16, 32, 8, 4, 2, 100, rules.DECODE, 256, 1, 256),
+    (8, 32, 8, 4, 2, 8000, rules.DECODE, 1024, 8, 1024), (32, 32, 8, 4, 2, 3000, rules.DECODE, 1024, 3, 1024),
+    # many
+    (2048, 32, 8, 4, 2, 2048, rules.PREFILL, 1024, 1, 2048), (130, 32, 8, 4, 4, 1000, rules.PREFILL, 256, 4, 256),
+    # the codes' expansion is dearer at 8 and 3 bits
+    (32, 32, 8, 8, 8, 3000, rules.PREFILL, 256, 12, 256), (32, 32, 8, 3, 3, 3000, rules.PREFILL, 256, 12, 256),
+    # from 4096 vectors on at most the 8 splits that a wave merges, and 128 workgroups
+    (130, 32, 8, 4, 2, 2560, rules.PREFILL, 256, 8, 320), (600, 8, 8, 4, 4, 600, rules.DECODE, 1024, 1, 1024),
+    # long tiles on a part of the chip lose to the decode kernel
+    (200, 64, 8, 4, 2, 1000, rules.DECODE, 1024, 1, 1024), (8, 32, 8, 4, 2, 30000, rules.DECODE, 1024, 30, 1024)])
+def test_route_of_a_tq_prefill(queries, qh, kvh, kbits, vbits, kv_len, kind, part, nsplit, split_pos):
+    r = rules.TqRoute(queries, qh, kvh, kbits, vbits, kv_len, causal=True)
+    assert (r.kind, r.part, r.nsplit, r.split_pos) == (kind, part, nsplit, split_pos)

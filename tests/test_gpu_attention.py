@@ -224,16 +224,22 @@ def run_prefill(dev, pool, q, kvh, kv_len, start_pos, kbits, vbits):
     return out.cpu().numpy().astype(np.float32)
 
 
-@pytest.mark.parametrize("kbits,vbits,qh,kvh,T,kv_len", [
+@pytest.mark.parametrize("kbits,vbits,qh,kvh,T,kv_len,tiled", [
     # several splits, ragged columns: G = 2, 4, 8, 3, 1 (5 splits of the positions or more)
-    (4, 2, 16, 8, 130, 1100), (4, 4, 16, 4, 65, 1800), (8, 8, 16, 2, 60, 3000), (3, 3, 24, 8, 45, 1301),
-    (2, 2, 8, 8, 130, 1537),
+    (4, 2, 16, 8, 130, 1100, True), (4, 4, 16, 4, 300, 1800, True), (8, 8, 16, 2, 60, 3000, True),
+    (3, 3, 24, 8, 45, 1301, True), (2, 2, 8, 8, 260, 1537, True),
+    # the same with too few columns for it, on the decode kernel
+    (4, 4, 16, 4, 65, 1800, False), (2, 2, 8, 8, 130, 1537, False),
     # one split and a batch of vectors that skips the merge, blocks going up after those going down
-    (4, 2, 32, 8, 2048, 2048)])
-def test_prefill_tiles(dev, kbits, vbits, qh, kvh, T, kv_len):
+    (4, 2, 32, 8, 2048, 2048, True),
+    # a batch of vectors whose splits the wave merge takes
+    (4, 2, 32, 8, 130, 2560, True)])
+def test_prefill_tiles(dev, kbits, vbits, qh, kvh, T, kv_len, tiled):
     """The causal prefill kernel against the oracle, with a masked page and with a value norm of
     infinity and a key norm of NaN at late positions, which no earlier query may see; the value norms
     span 2^-10 .. 2^10."""
+    route = rules.TqRoute(T, qh, kvh, kbits, vbits, kv_len, causal=True)
+    assert (route.kind == rules.PREFILL) == tiled
     rng = np.random.default_rng(kbits * 100 + T)
     hd, start = 128, kv_len - T
     pool = build_pool(rng, [kv_len], kvh, hd, kbits, vbits)
