@@ -26,7 +26,7 @@
 
 #include <algorithm>
 
-#include "attn_rules.h"
+#include "launch_rules.h"
 #include "fhip_common.h"
 #include "fracture_hip.h"
 
@@ -119,7 +119,7 @@ struct PQueries {
 //
 // A workgroup of W waves takes one (query, kv head, head block, split); wave w scores the
 // split's positions [w, w + 1) * kPSplit / W and the waves' states are merged in LDS, so the
-// partials stay one per split whatever W is (paged_waves in attn_rules.h). With a wave per split
+// partials stay one per split whatever W is (paged_waves in launch_rules.h). With a wave per split
 // the chunk's loads had nothing beside them to hide behind: 16 sequences of 500 .. 8192
 // positions (32 / 8 heads of 128, 285 MB) went from 136 to 72 us.
 // W = 1 puts two splits of neighbouring kv heads, each a wave's own, in a workgroup instead.

@@ -17,7 +17,7 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "attn_rules.h"
+#include "launch_rules.h"
 #include "fhip_internal.h"
 #include "tq_attn_index.h"
 #include "tq_quant.h"
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
 // A workgroup owns one (query, kv head, 1024-position block); each of its W waves walks an
 // equal split of it in 64-position chunks (two waves of 512 positions, four of 256 where a launch
 // has few workgroups, or four of 64 over a block of 256 positions where it has very few; tq_route
-// in attn_rules.h):
+// in launch_rules.h):
 //   QK  D[pos][col] = sum_k A[pos][k] B[k][col] on v_mfma_f32_16x16x32_f16. The K slots come
 //       in (hi, lo') pairs per coordinate: A = (c_hi, c_lo*2^12) of the position's centroid,
 //       B = (q_hi, 0) in column h and (q_lo*2^12, q_hi) in column 8+h, so one MFMA gives

@@ -178,4 +178,25 @@ inline TqRoute tq_route(const TqCall& c) {
     return r;
 }
 
+// ---------------------------------------------------------------------------------------
+// Matmul: whether C[M, N] = A[M, K] B[N, K]^T takes the streaming kernel of matmul_skinny.hip instead of the
+// library. Two times count: the kernel's, and a call's among others, where the library's host path takes
+// 23 us and this one's 9. A decode step between graph launches is bound by the second: 2 layers and a head at
+// batch 16, 987 us with it for the 4096-wide projections and 1094 without, at batch 1, 358 with it for
+// all of them, 376 for up to 2^25 elements, 433 without.
+//   A workgroup's 8 waves share a row's K, so K bounds the kernel: N = 1024, M = 1 / 4 / 16, us of this one and
+//   of the library, K = 2048 5.1 / 5.5 / 6.6 and 10.6 / 8.0 / 7.9, 4096 8.3 / 8.5 / 10.4 and 11.0 / 8.3 /
+//   8.2, 8192 13.1 / 14.2 / 18.1 and 11.6 / 9.2 / 9.3, 2^18 on N = 16 315 / 351 / 475 and 94 / 80 / 80. It is
+//   taken while it stays below the library's call: to 8192 with up to 4 rows, to 4096 with up to 16.
+//   Up to 2^25 elements (M = 16, 8192 x 4096: 19.5, the library 15.9, its call 23), and 2^27 with one or two
+//   rows, whose product is bound by B's stream either way (14336 x 4096 25.4 and 24.8, 4096 x 14336 25.4 and
+//   24.1, 32000 x 4096 48.5 and 54.5; in the step 1.8 us a product faster for all three).
+//   Up to 65536 rows of B: beyond, its many short workgroups are the longer way (524288 x 64: 38 and 29).
+inline bool matmul_skinny(int m, int n, int k) {
+    const int64_t elems = (int64_t)n * k;
+    if (m < 1 || m > 16 || n > 65536 || k < 8 || k % 8 != 0) return false;
+    if (elems <= (int64_t)1 << 25 && k <= (m <= 4 ? 8192 : 4096)) return true;
+    return m <= 2 && elems <= (int64_t)1 << 27 && n >= 4096 && k <= 16384;
+}
+
 }  // namespace fhip_rules

@@ -8,6 +8,7 @@
 // sum crosses lanes. The waves meet in LDS, in wave order.
 #include <hip/hip_runtime.h>
 
+#include "launch_rules.h"
 #include "fhip_common.h"
 #include "fhip_internal.h"
 
@@ -75,16 +76,8 @@ __global__ __launch_bounds__(64 * W) void matmul_skinny_kernel(uint16_t* __restr
 
 namespace fhip_internal {
 
-// Up to 16 rows on up to 2^25 elements of B (64 MiB: the library's kernels are launched and drained too
-// slowly there: 8 rows on 1024 x 4096 and 4096 x 4096, call after call, 25 us each against 10 here,
-// their kernels alone 11.4 and 12.6 us), and one or two rows on up to 2^27 (1 row on 14336 x 4096: 26.9
-// against 25.6, on 32000 x 4096: 57 against 49). Beyond, the library's larger tiles are the better
-// ones: each of the 16-row workgroups here reads all of A again (8 rows on 14336 x 4096: 26.4 against
-// 29.6; 1 row on 128256 x 4096: 183 against 184).
 bool matmul_skinny_takes(const void* c, const void* a, const void* b, int m, int n, int k) {
-    const int64_t elems = (int64_t)n * k;
-    return m >= 1 && m <= 16 && k >= 8 && k % 8 == 0 && elems <= (m <= 2 ? (int64_t)1 << 27 : (int64_t)1 << 25) &&
-           fhip_host::aligned16(a) && fhip_host::aligned16(b);
+    return fhip_rules::matmul_skinny(m, n, k) && fhip_host::aligned16(a) && fhip_host::aligned16(b);
 }
 
 int matmul_skinny(void* c, const void* a, const void* b, int m, int n, int k, hipStream_t s) {

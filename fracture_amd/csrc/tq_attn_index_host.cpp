@@ -1,9 +1,9 @@
 // Host build of the MFMA decode-attention kernel's index arithmetic (tq_attn_index.h), for the
-// CPU bounds check of the kernel's global accesses, and of the launchers' rules (attn_rules.h). Each entry evaluates the same inline
+// CPU bounds check of the kernel's global accesses, and of the launchers' rules (launch_rules.h). Each entry evaluates the same inline
 // functions the kernel calls, over all 64 lanes where an index depends on the lane.
 #include <stdint.h>
 
-#include "attn_rules.h"
+#include "launch_rules.h"
 #include "tq_attn_index.h"
 
 extern "C" {
@@ -123,7 +123,7 @@ int64_t fhip_idx_partial_row(int h, int tq0, int G, int qh, int g, int nsplit, i
     return fhip_idx::partial_row(fhip_idx::partial_vector(h, tq0, G, qh, g), nsplit, blk);
 }
 
-// Route of a TurboQuant attention call (attn_rules.h): out[0..5] = kind (0 VALU, 1 decode, 2 prefill), positions per
+// Route of a TurboQuant attention call (launch_rules.h): out[0..5] = kind (0 VALU, 1 decode, 2 prefill), positions per
 // partial, waves, queries per workgroup, splits, positions per split; returns the workspace bytes of its
 // layout.
 int64_t fhip_rule_tq_route(int nq, int qh, int kvh, int hd, int kbits, int vbits, int max_tokens, int kv_len,
@@ -145,9 +145,12 @@ int64_t fhip_rule_tq_workspace(int nq, int qh, int hd, int max_tokens) {
     return (int64_t)fhip_rules::tq_workspace_bytes(nq, qh, hd, max_tokens);
 }
 
-// Waves per split of an FP16 decode launch (attn_rules.h).
+// Waves per split of an FP16 decode launch (launch_rules.h).
 int fhip_rule_paged_waves(int64_t items, int hd, int max_tokens) {
     return fhip_rules::paged_waves(items, hd, max_tokens);
 }
+
+// Whether a matmul takes the streaming kernel (launch_rules.h).
+int fhip_rule_matmul_skinny(int m, int n, int k) { return fhip_rules::matmul_skinny(m, n, k); }
 
 }  // extern "C"

@@ -1,4 +1,4 @@
-"""The launchers' rules (fracture_amd/csrc/attn_rules.h) through their host build."""
+"""The launchers' rules (fracture_amd/csrc/launch_rules.h) through their host build."""
 import ctypes as C
 from pathlib import Path
 

@@ -58,7 +58,7 @@ def test_matmul_vs_float64(dev, m, n, k):
     # few rows: rows of B past the last full 16, K of one lane's 8, short of a 32-wide step, of the
     # waves' shares and of their unrolled loads; the last m and sizes each kernel takes
     (1, 1, 8), (1, 17, 24), (2, 1000, 4088), (3, 33, 1000), (8, 1024, 4096), (16, 100, 264), (17, 100, 264),
-    (5, 64, 36), (2, 16384, 2056), (3, 16384, 2056), (1, 40, 20000)])
+    (5, 64, 36), (2, 16384, 2056), (3, 16384, 2056), (1, 40, 20000), (4, 50, 8192), (16, 50, 4096), (2, 4096, 14336)])
 def test_matmul_few_rows(dev, m, n, k):
     rng = np.random.default_rng(m * n + k)
     a = rng.standard_normal((m, k)).astype(np.float16)

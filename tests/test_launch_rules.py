@@ -1,4 +1,4 @@
-"""Which kernel and split the attention launchers choose (fracture_amd/csrc/attn_rules.h), on the CPU."""
+"""Which kernel and split the attention and matmul launchers choose (fracture_amd/csrc/launch_rules.h)."""
 import pytest
 
 import rules
@@ -54,3 +54,17 @@ def test_other_widths_and_head_dims_stay_on_the_valu_kernel(qh, kvh, hd, kbits, 
 def test_route_of_a_tq_prefill(queries, qh, kvh, kbits, vbits, kv_len, kind, part, nsplit, split_pos):
     r = rules.TqRoute(queries, qh, kvh, kbits, vbits, kv_len, causal=True)
     assert (r.kind, r.part, r.nsplit, r.split_pos) == (kind, part, nsplit, split_pos)
+
+
+@pytest.mark.parametrize("m,n,k,streamed", [
+    (1, 4096, 4096, True), (16, 1024, 4096, True), (17, 1024, 4096, False), (8, 14336, 4096, False),
+    # a workgroup's waves share K: 8192 of it with up to 4 rows, 4096 with up to 16
+    (4, 1024, 8192, True), (5, 1024, 8192, False), (16, 2048, 14336, False), (1, 16, 1 << 20, False),
+    (1, 512, 1 << 18, False),
+    # one or two rows on up to 2^27 elements of a wide B
+    (2, 14336, 4096, True), (2, 4096, 14336, True), (3, 14336, 4096, False), (2, 2048, 14336, False),
+    (1, 32000, 4096, True), (1, 128256, 4096, False),
+    # many short rows; K that is no multiple of 8
+    (1, 65536, 64, True), (16, 1 << 19, 64, False), (1, 4096, 4, False), (1, 4096, 4100, False), (0, 8, 8, False)])
+def test_route_of_a_matmul(m, n, k, streamed):
+    assert bool(rules.lib().fhip_rule_matmul_skinny(m, n, k)) == streamed
