@@ -2119,7 +2119,7 @@ struct AttnArgs {
     const float *krot, *vrot, *kcent, *vcent;
     int qh, kvh, hd, kbits, vbits;
     void* ws;
-    size_t ws_bytes = fhip_rules::kTqFineBytes;  // what `ws` holds, at least tq_layout's at kSplit positions
+    size_t ws_bytes = 0;  // what `ws` holds; 0: what the workspace size function asks for this call
 };
 
 template <int KB, int VB, class Pages>
@@ -2157,8 +2157,9 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
     if (a.nq == 0) return hipSuccess;
     const int max_tokens = a.qs.max_blocks * FHIP_PAGE_TOKENS;
     const bool causal = std::is_same_v<Pages, PtrPages> && !a.qs.seq_lens && a.qs.table_stride == 0;
+    const size_t ws_bytes = a.ws_bytes ? a.ws_bytes : fhip_rules::tq_workspace_bytes(a.nq, a.qh, a.hd, max_tokens);
     const fhip_rules::TqRoute route = fhip_rules::tq_route({a.nq, a.qh, a.kvh, a.hd, a.kbits, a.vbits, max_tokens,
-                                                            a.qs.kv_len, causal, a.ws_bytes});
+                                                            a.qs.kv_len, causal, ws_bytes});
     const fhip_rules::TqLayout layout = fhip_rules::tq_layout(a.nq, a.qh, a.hd, max_tokens, route.part);
     int nsplit = layout.nsplit, split_pos = route.part;
     if (route.kind == fhip_rules::TqRoute::kPrefill) {

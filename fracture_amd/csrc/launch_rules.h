@@ -86,11 +86,13 @@ inline TqLayout tq_layout(int nq, int qh, int hd, int max_tokens, int part) {
     return l;
 }
 // Small launches may split finer, where the layout of kTqFinePart positions stays within kTqFineBytes. The
-// size a caller is asked for covers that layout at every smaller size too (it never falls as an
-// argument grows), so a workspace warmed up at the largest call serves the smaller ones.
+// size a caller is asked for covers that layout too, of every table with as many kTqSplit-position splits,
+// and at every smaller size (it never falls as an argument grows): a workspace serves the tables that it
+// would serve if no launch split finer, and one warmed up at the largest call the smaller ones.
 inline size_t tq_workspace_bytes(int nq, int qh, int hd, int max_tokens) {
-    return std::max(tq_layout(nq, qh, hd, max_tokens, kTqSplit).bytes,
-                    std::min(tq_layout(nq, qh, hd, max_tokens, kTqFinePart).bytes, kTqFineBytes));
+    const int whole = (int)(div_up(std::max(max_tokens, 1), kTqSplit) * kTqSplit);
+    return std::max(tq_layout(nq, qh, hd, whole, kTqSplit).bytes,
+                    std::min(tq_layout(nq, qh, hd, whole, kTqFinePart).bytes, kTqFineBytes));
 }
 
 // The (K, V) code widths that the MFMA kernels are built for: the default cache, equal widths, and the

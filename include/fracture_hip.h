@@ -333,7 +333,13 @@ int fhip_launch_tq_dequant_kv_planned(const fhip_tq_plan* kplan, const fhip_tq_p
  * empty sequences only, is refused with hipErrorInvalidValue) and max_blocks * 16 at most
  * 1,048,576. Output [B, qh, hd] fp16 (zeros for an empty sequence); centroid tables hold
  * 2^bits entries.
- * The workspace holds split-K partials; size it with fhip_attention_tq_workspace_bytes. */
+ * The workspace holds split-K partials; size it with fhip_attention_tq_workspace_bytes of this
+ * call's own batch, heads, head_dim and max_blocks, or larger ones (the size never falls as one of
+ * them grows, and is the same for every max_blocks of as many 1024-position splits). The entries
+ * without a size argument take the workspace to hold that much. Small calls split the positions
+ * finer than large ones, within 24 MiB, so the size is not a multiple of one call's.
+ * How many waves and splits share a sequence's positions follows from the size of the call, so
+ * a sequence's result may differ in its last bits between batches of different sizes. */
 size_t fhip_attention_tq_workspace_bytes(int batch, int num_q_heads, int head_dim,
                                          int max_blocks);
 int fhip_launch_attention_tq_decode(void* output, const void* q, const int32_t* block_table,
@@ -366,7 +372,8 @@ int fhip_launch_attention_tq_decode_ptrs(void* output, const void* q, const int3
  * page p of K at k_pool + p * page_k_bytes holds [16, kvh, hd] fp16, likewise V; positions
  * whose page id is outside [0, num_pages) are masked out; max_blocks is at least 1, as above.
  * Output [B, qh, hd] fp16.
- * The workspace holds split partials; size it with fhip_attention_paged_workspace_bytes. */
+ * The workspace holds split partials; size it with fhip_attention_paged_workspace_bytes. As over
+ * TurboQuant pages, a sequence's last bits may depend on the size of the batch it is in. */
 size_t fhip_attention_paged_workspace_bytes(int batch, int num_q_heads, int head_dim,
                                             int max_blocks);
 int fhip_launch_attention_paged_decode(void* output, const void* q, const int32_t* block_table,

@@ -208,6 +208,44 @@ def test_code_pages_at_odd_addresses(dev, bits):
     assert_close(out.cpu().numpy()[0].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3)
 
 
+@pytest.mark.parametrize("kbits,vbits,qh,kvh", [(4, 2, 32, 8), (8, 8, 8, 2)])
+def test_workspace_of_a_shorter_table(dev, kbits, vbits, qh, kvh):
+    """A workspace sized for one block serves a table of 60, which launches in 256-position parts, in decode
+    and through the entry that is told its size; nothing is written past it."""
+    rng = np.random.default_rng(kbits)
+    n, guard = 960, 1 << 20
+    pool = build_pool(rng, [n], kvh, 128, kbits, vbits)
+    route = rules.TqRoute(1, qh, kvh, kbits, vbits, n)
+    assert (route.kind, route.part, route.nsplit) == (rules.DECODE, 256, 4)
+    size = K._L().fhip_attention_tq_workspace_bytes(1, qh, 128, 1)
+    assert size == rules.tq_workspace(1, qh, 128, n) and route.bytes <= size
+    parts = [dev_t(pool[x], dev) for x in ("KP", "KN", "VP", "VN")]
+    tabs = [dev_t(pool[x], dev) for x in ("krot", "vrot", "kc", "vc")]
+    q = rng.standard_normal((1, qh, 128)).astype(np.float16)
+    tq_, table, lens = dev_t(q, dev), dev_t(pool["table"], dev), dev_t(np.array([n], np.int32), dev)
+    ptrs = [torch.tensor([x.data_ptr() for x in t], dtype=torch.int64, device=dev) for t in parts]
+    pd = [oracle.packed_dim(128, b) for b in (kbits, vbits)]
+    s = torch.cuda.current_stream().cuda_stream
+    want = oracle.tq_attention(q[0], pool["table"][0], n, pool["KP"], pool["KN"], pool["VP"], pool["VN"],
+                               pool["krot"], pool["vrot"], pool["kc"], pool["vc"], kbits, vbits, kvh)
+    for told in (False, True):
+        ws = torch.full((size + guard,), 0x5A, dtype=torch.uint8, device=dev)
+        out = torch.empty_like(tq_)
+        if told:
+            code = K._L().fhip_launch_attention_paged_tq_ws(
+                out.data_ptr(), tq_.data_ptr(), table.data_ptr(), *(p.data_ptr() for p in ptrs),
+                *(t.data_ptr() for t in tabs), 1, qh, kvh, 128, n, n - 1, kbits, vbits, *pd, ws.data_ptr(), size, s)
+        else:
+            code = K._L().fhip_launch_attention_tq_decode(
+                out.data_ptr(), tq_.data_ptr(), table.data_ptr(), lens.data_ptr(), 1, table.shape[1],
+                parts[0].shape[0], *(p.data_ptr() for p in parts), *(p[0].nbytes for p in parts),
+                *(t.data_ptr() for t in tabs), qh, kvh, 128, kbits, vbits, ws.data_ptr(), s)
+        assert code == 0
+        torch.cuda.synchronize()
+        assert (ws[size:] == 0x5A).all()
+        assert_close(out.cpu().numpy()[0].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3, f"told {told}")
+
+
 def run_prefill(dev, pool, q, kvh, kv_len, start_pos, kbits, vbits):
     P, T, qh, hd = pool["KP"].shape[0], *q.shape
     parts = [dev_t(pool[n], dev) for n in ("KP", "KN", "VP", "VN")]

@@ -68,3 +68,26 @@ def test_route_of_a_tq_prefill(queries, qh, kvh, kbits, vbits, kv_len, kind, par
     (1, 65536, 64, True), (16, 1 << 19, 64, False), (1, 4096, 4, False), (1, 4096, 4100, False), (0, 8, 8, False)])
 def test_route_of_a_matmul(m, n, k, streamed):
     assert bool(rules.lib().fhip_rule_matmul_skinny(m, n, k)) == streamed
+
+
+@pytest.mark.parametrize("queries,qh,hd", [(1, 32, 128), (1, 8, 128), (7, 24, 128), (64, 32, 128), (300, 64, 128), (5, 8, 64)])
+def test_workspace_serves_every_table_of_its_splits(queries, qh, hd):
+    """A workspace sized for one table serves, in every layout that a launch may choose, each table of as many
+    1024-position splits, and every smaller call; the size never falls as an argument grows."""
+    G = 8 if qh % 8 == 0 else 1
+    last = 0
+    for split in (1, 2, 3, 9, 12, 13, 48, 64):
+        sizes = set()
+        for blocks in (64 * split - 63, 64 * split - 40, 64 * split - 15, 64 * split):
+            n = 16 * blocks
+            size = rules.tq_workspace(queries, qh, hd, n)
+            sizes.add(size)
+            for causal in (False, True):
+                for bits in (4, 8):
+                    smallest = rules.tq_workspace(queries, qh, hd, 16 * (64 * split - 63))
+                    r = rules.TqRoute(queries, qh, qh // G, bits, bits, n, causal, hd=hd, ws_bytes=size)
+                    assert r.bytes <= smallest, (blocks, causal, r.part)
+        assert len(sizes) == 1
+        assert last <= size and size <= rules.tq_workspace(queries + 1, qh, hd, n)
+        assert size <= rules.tq_workspace(queries, qh + G, hd, n)
+        last = size
