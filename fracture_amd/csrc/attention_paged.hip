@@ -520,8 +520,8 @@ paged_attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, PQueries qs, Page
     const int clen = qs.causal_len(q0 + nq - 1);  // the block's longest causal length
     const int clen0 = qs.causal_len(q0);          // and its shortest
     const int t_begin = split * split_pos;
-    // uniform: with several splits, a split past the block's length writes nothing
-    if (nsplit > 1 && t_begin >= clen) return;
+    // uniform: of partials, a split past the block's length writes none
+    if (!out && t_begin >= clen) return;
     const int t_end = min(clen, t_begin + split_pos);
     const int32_t* table = qs.table + (int64_t)q0 * qs.table_stride;
 
@@ -736,7 +736,7 @@ paged_attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, PQueries qs, Page
             float m, l, a[4];
             wave_attend(q + v2 * HD, table, pg, t_begin, min(t_end, qs.causal_len(q0 + cq2)), kvh, g,
                         HD, scale_log2 * 0.6931471805599453f, lane, qv, m, l, a);
-            if (lane == 0 && nsplit > 1) {  // in the units of the other splits' partials
+            if (lane == 0 && !out) {  // in the units of the other splits' partials
                 part_ml[(v2 * nsplit + split) * 2 + 0] = m;
                 part_ml[(v2 * nsplit + split) * 2 + 1] = l * kPfScale;
             }
@@ -744,10 +744,10 @@ paged_attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, PQueries qs, Page
             for (int i = 0; i < 4; ++i) {
                 const int d = lane + 64 * i;
                 if (d >= HD) continue;
-                if (nsplit > 1)
-                    part_acc[(v2 * nsplit + split) * HD + d] = a[i] * kPfScale;
-                else
+                if (out)
                     out[v2 * HD + d] = (uint16_t)f2h(l > 0.0f ? a[i] / l : 0.0f);
+                else
+                    part_acc[(v2 * nsplit + split) * HD + d] = a[i] * kPfScale;
             }
         }
         return;
@@ -755,7 +755,7 @@ paged_attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, PQueries qs, Page
 
     l_run += __shfl_xor(l_run, 32);
     if (!col_ok) return;
-    if (nsplit == 1) {
+    if (out) {
 #pragma unroll
         for (int d = 0; d < kDt; ++d)
 #pragma unroll
@@ -983,12 +983,12 @@ void launch_split_hd(const uint16_t* q, const PQueries& qs, const Pages& pg, int
 
 template <int HD, class Pages>
 void launch_prefill_t(const uint16_t* q, const PQueries& qs, const Pages& pg, int qh, int kvh,
-                      float* ml, float* acc, uint16_t* out, int nsplit, int split_pos, int nqb,
-                      int nblk, hipStream_t s) {
+                      float* ml, float* acc, uint16_t* out, const fhip_rules::PrefillSplit& ps,
+                      hipStream_t s) {
     const float scale_log2 = 1.4426950408889634f / sqrtf((float)HD);
-    hipLaunchKernelGGL((paged_attn_prefill_mfma_kernel<HD, Pages>),
-                       dim3((unsigned)((int64_t)nblk * nsplit * kvh)), dim3(64 * kPfWaves), 0, s, q,
-                       qs, pg, qh, kvh, scale_log2, ml, acc, out, nsplit, split_pos, nqb, nblk);
+    hipLaunchKernelGGL((paged_attn_prefill_mfma_kernel<HD, Pages>), dim3((unsigned)ps.workgroups),
+                       dim3(64 * kPfWaves), 0, s, q, qs, pg, qh, kvh, scale_log2, ml, acc, out, ps.nsplit,
+                       ps.split_pos, ps.nqb, ps.nblk);
 }
 
 // The merge of nsplit splits of split_pos positions per vector.
@@ -1028,31 +1028,27 @@ int launch_paged(void* out, const void* q, const PQueries& qs, int nq, const Pag
     // MFMA prefill kernel (head_dim <= 128, G <= 8), else 8 / G per wave (G < 8)
     const bool prefill = !qs.seq_lens && qs.table_stride == 0 && nq > 1;
     if (prefill && (hd == 32 || hd == 64 || hd == 128) && G <= kHeadsMax) {
-        const int nqb = kPfCols / G;
-        const int nblk = (int)ceil_div((int64_t)nq, nqb);
-        const int64_t base = (int64_t)nblk * kvh;
         // Splits only as far as the workgroups need to fill the chip (kPfGroups: 768 or 1024
         // measured 129 and 120 us where 512 took 114), at most the
-        // workspace's one per kPSplit positions: every split adds partials to write and merge.
-        const int64_t extent =
-            std::max<int64_t>(std::min<int64_t>(qs.kv_len, (int64_t)qs.max_blocks * FHIP_PAGE_TOKENS), 1);
-        const int64_t want =
-            std::min<int64_t>(std::max<int64_t>(ceil_div(kPfGroups, base), 1), nsplit);
-        const int split_pos = (int)(ceil_div(ceil_div(extent, want), kPfTile) * kPfTile);
-        const int ns = (int)ceil_div(extent, split_pos);
-        if (base * ns > 0x7fffffff || nvec > 0x7fffffff) return hipErrorInvalidValue;
+        // workspace's one per kPSplit positions: every split adds partials to write and merge. A single
+        // split writes the output itself, 8 bytes a lane, where it is aligned to them.
+        const int extent = (int)std::min<int64_t>(qs.kv_len, (int64_t)qs.max_blocks * FHIP_PAGE_TOKENS);
+        const fhip_rules::PrefillSplit ps =
+            fhip_rules::prefill_split(nq, G, kvh, kPfCols, kPfTile, kPfGroups, extent, nsplit);
+        if (ps.workgroups > 0x7fffffff || nvec > 0x7fffffff) return hipErrorInvalidValue;
+        uint16_t* direct = ps.nsplit == 1 && ((uintptr_t)out & 7) == 0 ? (uint16_t*)out : nullptr;
         switch (hd) {
             case 32:
-                launch_prefill_t<32>(qp, q2, pg, qh, kvh, ml, acc, (uint16_t*)out, ns, split_pos, nqb, nblk, s);
+                launch_prefill_t<32>(qp, q2, pg, qh, kvh, ml, acc, direct, ps, s);
                 break;
             case 64:
-                launch_prefill_t<64>(qp, q2, pg, qh, kvh, ml, acc, (uint16_t*)out, ns, split_pos, nqb, nblk, s);
+                launch_prefill_t<64>(qp, q2, pg, qh, kvh, ml, acc, direct, ps, s);
                 break;
             default:
-                launch_prefill_t<128>(qp, q2, pg, qh, kvh, ml, acc, (uint16_t*)out, ns, split_pos, nqb, nblk, s);
+                launch_prefill_t<128>(qp, q2, pg, qh, kvh, ml, acc, direct, ps, s);
                 break;
         }
-        if (ns > 1) launch_combine(q2, ml, acc, out, nvec, qh, hd, ns, split_pos, s);
+        if (!direct) launch_combine(q2, ml, acc, out, nvec, qh, hd, ps.nsplit, ps.split_pos, s);
         return hipGetLastError();
     }
     const int tok = prefill && G < kHeadsMax ? kHeadsMax / G : 1;

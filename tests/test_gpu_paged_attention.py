@@ -211,6 +211,27 @@ def test_reference_interface_prefill_causal(dev, kv_len, T, start_pos, qh, kvh, 
                      f"token {t}")
 
 
+@pytest.mark.parametrize("kv_len,T,hd", [(300, 40, 128), (70, 70, 64), (3000, 9, 128), (5000, 3, 32)])
+def test_prefill_into_an_output_of_any_alignment(dev, kv_len, T, hd):
+    """Outputs that start at an odd element: one split goes through the merge, which stores single
+    elements, instead of storing 8 bytes itself."""
+    rng = np.random.default_rng(kv_len)
+    qh, kvh = 8, 2
+    kp, vp, table = build_pool(rng, [kv_len], kvh, hd)
+    tk, tv = dev_t(kp, dev), dev_t(vp, dev)
+    ptr = [torch.tensor([x.data_ptr() for x in t], dtype=torch.int64, device=dev) for t in (tk, tv)]
+    q = dev_t((rng.standard_normal((T, qh, hd)) * 2).astype(np.float16), dev)
+    want = torch.empty_like(q)
+    K.paged_attention(want, q, dev_t(table[0], dev), *ptr, kvh, kv_len, kv_len - T)
+    held = torch.full((q.numel() + 4,), 7.0, dtype=torch.float16, device=dev)
+    K.paged_attention(held[1:-3].view(q.shape), q, dev_t(table[0], dev), *ptr, kvh, kv_len, kv_len - T)
+    torch.cuda.synchronize()
+    assert (held[[0, -3, -2, -1]] == 7.0).all()
+    # the merge divides the same sums
+    assert_close(held[1:-3].view(q.shape).cpu().numpy().astype(np.float32), want.cpu().numpy().astype(np.float32),
+                 1e-3, 1e-3)
+
+
 def test_reference_interface_rejects_unsupported_head_dim(dev):
     q = torch.zeros((1, 4, 264), dtype=torch.float16, device=dev)
     out = torch.empty_like(q)
