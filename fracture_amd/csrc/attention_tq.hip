@@ -918,15 +918,14 @@ __device__ __forceinline__ void dma_v(const PageAddrs* pages, int j0, uint32_t v
 #pragma unroll
     for (int i = 0; i < 4; ++i) dma16(addr_of_lane(v4, i), voff, vb + 1024 * i);
 }
-// 2-bit V codes (kV2): the same segments as dma_v, from rows of 32 bytes. Lane L takes 8 bytes of
+// 2-bit V codes: the same segments as dma_v, from rows of 32 bytes. Lane L takes 8 bytes of
 // position 16i + L / 4 of page j0 + i (v2_offset), and once they have arrived store_v2 widens
 // each 2-bit code to a 4-bit one and writes the 16 bytes that dma_v would have copied, so the
 // transposed reads and the pair table serve both widths (its V entries map codes 0..3).
-typedef __attribute__((address_space(1))) const u32x2 g_u32x2;
 __device__ __forceinline__ void load_v2(const PageAddrs* pages, int j0, uint32_t voff,
                                         u32x2 (&r)[4]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r[i] = *(g_u32x2*)(pages[j0 + i].v + voff);
+    for (int i = 0; i < 4; ++i) r[i] = *(g_u32x2_any*)(pages[j0 + i].v + voff);
 }
 // Bytes sel of w (two code bytes, four codes each, the first in the top bits) as four bytes
 // of 4-bit codes, the first in the high nibble: byte b -> (c0 << 4 | c1), (c2 << 4 | c3).
