@@ -29,6 +29,7 @@
 #include "launch_rules.h"
 #include "fhip_common.h"
 #include "fracture_hip.h"
+#include "tq_attn_index.h"
 
 using namespace fhip;
 
@@ -514,7 +515,7 @@ paged_attn_prefill_mfma_kernel(const uint16_t* __restrict__ q, PQueries qs, Page
     const int g = (int)(blockIdx.x % kvh);
     const int rest = (int)(blockIdx.x / kvh);
     const int split = rest % nsplit;
-    const int q0 = (nblk - 1 - rest / nsplit) * nqb;  // the block's first query
+    const int q0 = fhip_idx::prefill_block(rest / nsplit, nblk, 0) * nqb;  // the block's first query
     const int nq = min(nqb, qs.count - q0);
     const int G = qh / kvh;
     const int clen = qs.causal_len(q0 + nq - 1);  // the block's longest causal length

@@ -678,14 +678,12 @@ __global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
 // Online softmax per head (lanes n = h), lazily rescaling the accumulators.
 // ---------------------------------------------------------------------------------------
 constexpr int kChunkM = 64;     // positions per chunk
-constexpr int kSplitMfma = 512;  // positions per wave (split) at two waves per workgroup
 constexpr int kXcds = 8;         // MI355X: accelerator complex dies, each with its own L2
 constexpr int kWavesM = 2;      // waves per workgroup, large launches
 constexpr int kWavesWide = 4;   // and small ones
-static_assert(kChunkM == fhip_idx::kChunk && kSplitMfma == fhip_idx::kSplitPositions &&
-                  kWavesM == fhip_idx::kBlockWaves && kXcds == fhip_idx::kXcdCount &&
+static_assert(kChunkM == fhip_idx::kChunk && kXcds == fhip_idx::kXcdCount && kXcds == fhip_rules::kXcds &&
                   FHIP_PAGE_TOKENS == fhip_idx::kPageTokens,
-              "the kernel's shape is the one its index helpers describe");
+              "tq_attn_index.h and launch_rules.h describe this kernel");
 
 typedef int v2i_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
@@ -1750,7 +1748,7 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
     const int rest = (int)(blockIdx.x / kvh);
     const int split = rest % nsplit;
     const int bi = rest / nsplit;
-    const int q0 = (fold > 0 && bi >= fold ? bi - fold : nblk - 1 - bi) * nqb;
+    const int q0 = fhip_idx::prefill_block(bi, nblk, fold) * nqb;
     const int nq = min(nqb, qs.seq_lens_count - q0);
     const int G = qh / kvh;
     const int clen = qs.causal_len(q0 + nq - 1), clen0 = qs.causal_len(q0);
@@ -1827,9 +1825,9 @@ tq_attn_prefill_kernel(float* __restrict__ qrot, Queries qs, PtrPages pg,
     // ---- tile loads: thread -> row tid / 4, quarter tid % 4 (32 codes); threads of wave 0 the norms.
     // The row's page is looked up per thread (a wave's 16 rows are one page).
     const int row = threadIdx.x >> 2, quarter = threadIdx.x & 3;
-    const uint32_t koff = (uint32_t)((((row & 15) * kvh + g) * 16 + 4 * quarter) * KB);
-    const uint32_t voff = (uint32_t)((((row & 15) * kvh + g) * 16 + 4 * quarter) * VB);
-    const uint32_t noff = (uint32_t)(((lane & 15) * kvh + g) * 2);
+    const uint32_t koff = fhip_idx::prefill_code_offset(row, quarter, kvh, g, KB);
+    const uint32_t voff = fhip_idx::prefill_code_offset(row, quarter, kvh, g, VB);
+    const uint32_t noff = fhip_idx::norm_offset(lane, kvh, g);
     Codes32<KB> kc;
     Codes32<VB> vc;
     uint32_t kn = 0, vn = 0;
@@ -2135,10 +2133,7 @@ void launch_split(const AttnArgs& a, const Pages& pg, int nsplit, float* ml, flo
 // Launches the prefill kernel; `merged`: it leaves merged vectors in qrot.
 void launch_prefill(float* qrot, const AttnArgs& a, const PtrPages& pg, const fhip_rules::PrefillSplit& ps,
                     bool merged, float* ml, float* acc, hipStream_t s) {
-    // Blocks start from the last (the longest contexts) down. Where all fit at once, two to a CU, the
-    // second half goes up from the first instead, so that a long block shares its CU with a short one.
-    const int cus = fhip_host::cu_count();
-    const int fold = ps.nsplit == 1 && ps.workgroups > cus && ps.workgroups <= 2 * cus ? (int)(cus / a.kvh) : 0;
+    const int fold = fhip_rules::prefill_fold(ps, a.kvh, fhip_host::cu_count());
     Queries q2 = a.qs;
     q2.seq_lens_count = a.nq;
     auto kern = a.kbits == 8   ? tq_attn_prefill_kernel<8, 8>

@@ -60,6 +60,13 @@ inline PrefillSplit prefill_split(int nq, int G, int kvh, int cols, int tile, in
     return p;
 }
 
+// Blocks start from the last (the longest contexts) down. Where all of a single split's fit at once, two to a
+// CU, those of the second half go up from the first instead (their index from this one on), so that a
+// long block shares its CU with a short one.
+inline int prefill_fold(const PrefillSplit& p, int kvh, int cus) {
+    return p.nsplit == 1 && p.workgroups > cus && p.workgroups <= 2 * (int64_t)cus ? cus / kvh : 0;
+}
+
 // ---------------------------------------------------------------------------------------
 // TurboQuant attention
 // ---------------------------------------------------------------------------------------

@@ -1,8 +1,8 @@
 // Index arithmetic of the MFMA decode-attention kernel (tq_attn_mfma_kernel, head_dim 128, K and V
-// codes of 2, 3, 4 or 8 bits), shared by the kernel and by a host build of the functions
-// (tq_attn_index_host.cpp). The CPU bounds check of every global access the kernel makes
-// calls the host build, so it covers the arithmetic the kernel runs rather than a restatement
-// of it. Page layout (quantized_paged_kv_cache.rs:86-128): a page holds 16 positions; its K
+// codes of 2, 3, 4 or 8 bits) and of the tiled prefill kernels' work split and code loads, shared by the
+// kernels and by a host build of the functions (tq_attn_index_host.cpp). The CPU bounds check of the
+// decode kernel's page, table, query and partial accesses calls the host build, so it covers the
+// arithmetic the kernel runs rather than a restatement of it. Page layout (quantized_paged_kv_cache.rs:86-128): a page holds 16 positions; its K
 // codes are [16][kvh][16 bits] bytes (64 at 4 bits), its K norms [16][kvh] fp16, and the same for V.
 #pragma once
 #include <stdint.h>
@@ -18,8 +18,6 @@ namespace fhip_idx {
 constexpr int kPageTokens = 16;      // positions per page
 constexpr int kCodeRow = 64;         // bytes of one position's 4-bit codes for one kv head
 constexpr int kChunk = 64;           // positions per chunk of a wave's loop
-constexpr int kSplitPositions = 512; // positions per wave (one split)
-constexpr int kBlockWaves = 2;       // waves per workgroup: one 1024-position block
 constexpr int kXcdCount = 8;         // MI355X: workgroup b runs on XCD b % 8
 
 // Workgroup wg -> (item, kv head g). An item is a (query group, block); the 8 kv heads of one
@@ -54,10 +52,8 @@ FHIP_IDX void split_grid_item(int64_t lin, int64_t total, int nsplit, int kvh, i
     qi = (int)(eff / ((int64_t)nsplit * kvh));
 }
 
-// First position of wave `wave`'s split in block blk.
-FHIP_IDX int split_begin(int blk, int wave) { return (kBlockWaves * blk + wave) * kSplitPositions; }
-
-// The same with `waves` waves per workgroup sharing a block of `part` positions.
+// First position of wave `wave`'s split in block blk, `waves` waves per workgroup sharing a block of `part`
+// positions.
 FHIP_IDX int split_begin(int blk, int wave, int waves, int part) {
     return blk * part + wave * (part / waves);
 }
@@ -73,14 +69,9 @@ FHIP_IDX bool split_page_column(int t_begin, int t_end, int lane, int& column) {
 FHIP_IDX int chunk_first_page(int t0, int t_begin) { return (t0 - t_begin) / kPageTokens; }
 
 // K codes of a chunk: lane (n = lane & 15, rg = lane >> 4) reads split page
-// chunk_first_page + k_page(lane), 16 bytes at k_offset + pt * k_tile_stride for pt = 0..3:
-// position 4 (n & 3) + pt of the page, bytes [16 rg, 16 rg + 16) of kv head g's code row.
+// chunk_first_page + k_page(lane), 4 bits bytes (32 codes) at k_offset + pt * k_tile_stride for pt = 0..3:
+// position 4 (n & 3) + pt of the page, bytes [4 bits rg, 4 bits (rg + 1)) of kv head g's code row.
 FHIP_IDX int k_page(int lane) { return (lane & 15) >> 2; }
-FHIP_IDX uint32_t k_offset(int lane, int kvh, int g) {
-    return (uint32_t)((4 * ((lane & 15) & 3) * kvh + g) * kCodeRow + 16 * (lane >> 4));
-}
-FHIP_IDX uint32_t k_tile_stride(int kvh) { return (uint32_t)(kvh * kCodeRow); }
-// The same for rows of `bits`-bit codes: 4 bits bytes (32 codes) at 4 bits rg of the row.
 FHIP_IDX uint32_t k_offset(int lane, int kvh, int g, int bits) {
     return (uint32_t)((4 * ((lane & 15) & 3) * kvh + g) * 16 * bits + 4 * bits * (lane >> 4));
 }
@@ -136,5 +127,15 @@ FHIP_IDX int64_t partial_vector(int h, int tq0, int G, int qh, int g) {
     return (int64_t)(tq0 + ht) * qh + (int64_t)g * G + (h - ht * G);
 }
 FHIP_IDX int64_t partial_row(int64_t vec, int nsplit, int blk) { return vec * nsplit + blk; }
+
+// Tiled prefill: the query block that workgroup block `bi` of nblk takes. From the last (the longest
+// contexts) down; with fold > 0 the workgroups from `fold` on go up from the first instead.
+FHIP_IDX int prefill_block(int bi, int nblk, int fold) {
+    return fold > 0 && bi >= fold ? bi - fold : nblk - 1 - bi;
+}
+// Byte offset in its page of quarter `quarter` (32 codes, 4 bits bytes) of tile row `row`, kv head g.
+FHIP_IDX uint32_t prefill_code_offset(int row, int quarter, int kvh, int g, int bits) {
+    return (uint32_t)((((row & (kPageTokens - 1)) * kvh + g) * 16 + 4 * quarter) * bits);
+}
 
 }  // namespace fhip_idx

@@ -17,7 +17,7 @@ int fhip_idx_lane_tables(int kvh, int g, uint32_t* k_off, int32_t* k_page, uint3
         return -1;
     for (int lane = 0; lane < 64; ++lane) {
         for (int pt = 0; pt < 4; ++pt)
-            k_off[pt * 64 + lane] = fhip_idx::k_offset(lane, kvh, g) + pt * fhip_idx::k_tile_stride(kvh);
+            k_off[pt * 64 + lane] = fhip_idx::k_offset(lane, kvh, g, 4) + pt * fhip_idx::k_tile_stride(kvh, 4);
         k_page[lane] = fhip_idx::k_page(lane);
         v_off[lane] = fhip_idx::v_offset(lane, kvh, g);
         n_off[lane] = fhip_idx::norm_offset(lane, kvh, g);
@@ -87,18 +87,23 @@ int fhip_idx_split_grid_item(int64_t lin, int nsplit, int kvh, int nq, int32_t* 
     return 0;
 }
 
-// Wave `wave` of block blk: its split's first position, and per lane the block-table column
-// of split page `lane` and whether that page holds positions of [t_begin, t_end).
-int fhip_idx_split(int blk, int wave, int t_end, int32_t* t_begin, int32_t* column,
-                   uint8_t* in_split) {
-    if (blk < 0 || wave < 0 || !t_begin || !column || !in_split) return -1;
-    *t_begin = fhip_idx::split_begin(blk, wave);
+// Wave `wave` of `waves` in block blk of `part` positions: its split's first position, and per lane the
+// block-table column of split page `lane` and whether that page holds positions of [t_begin, t_end).
+int fhip_idx_wave_split(int blk, int wave, int waves, int part, int t_end, int32_t* t_begin, int32_t* column,
+                        uint8_t* in_split) {
+    if (blk < 0 || wave < 0 || waves < 1 || part < waves || !t_begin || !column || !in_split) return -1;
+    *t_begin = fhip_idx::split_begin(blk, wave, waves, part);
     for (int lane = 0; lane < 64; ++lane) {
         int c;
         in_split[lane] = fhip_idx::split_page_column(*t_begin, t_end, lane, c) ? 1 : 0;
         column[lane] = c;
     }
     return 0;
+}
+
+// The same of a 1024-position block's two waves.
+int fhip_idx_split(int blk, int wave, int t_end, int32_t* t_begin, int32_t* column, uint8_t* in_split) {
+    return fhip_idx_wave_split(blk, wave, 2, 1024, t_end, t_begin, column, in_split);
 }
 
 // The first split page of the chunk starting at t0.
@@ -152,5 +157,27 @@ int fhip_rule_paged_waves(int64_t items, int hd, int max_tokens) {
 
 // Whether a matmul takes the streaming kernel (launch_rules.h).
 int fhip_rule_matmul_skinny(int m, int n, int k) { return fhip_rules::matmul_skinny(m, n, k); }
+
+// Split of a tiled prefill (launch_rules.h): out[0..4] = queries per block, blocks, splits, positions per split,
+// workgroups.
+void fhip_rule_prefill_split(int nq, int G, int kvh, int cols, int tile, int64_t groups, int extent, int max_splits,
+                             int64_t* out) {
+    const fhip_rules::PrefillSplit p = fhip_rules::prefill_split(nq, G, kvh, cols, tile, groups, extent, max_splits);
+    out[0] = p.nqb;
+    out[1] = p.nblk;
+    out[2] = p.nsplit;
+    out[3] = p.split_pos;
+    out[4] = p.workgroups;
+}
+int fhip_rule_prefill_fold(int nsplit, int64_t workgroups, int kvh, int cus) {
+    fhip_rules::PrefillSplit p{};
+    p.nsplit = nsplit;
+    p.workgroups = workgroups;
+    return fhip_rules::prefill_fold(p, kvh, cus);
+}
+int fhip_idx_prefill_block(int bi, int nblk, int fold) { return fhip_idx::prefill_block(bi, nblk, fold); }
+uint32_t fhip_idx_prefill_code_offset(int row, int quarter, int kvh, int g, int bits) {
+    return fhip_idx::prefill_code_offset(row, quarter, kvh, g, bits);
+}
 
 }  // extern "C"

@@ -19,6 +19,10 @@ def lib():
         _LIB.fhip_rule_tq_route.restype = C.c_int64
         _LIB.fhip_rule_tq_workspace.argtypes = [C.c_int] * 4
         _LIB.fhip_rule_tq_workspace.restype = C.c_int64
+        _LIB.fhip_rule_prefill_split.argtypes = [C.c_int] * 5 + [C.c_int64, C.c_int, C.c_int, C.c_void_p]
+        _LIB.fhip_rule_prefill_split.restype = None
+        _LIB.fhip_rule_prefill_fold.argtypes = [C.c_int, C.c_int64, C.c_int, C.c_int]
+        _LIB.fhip_idx_prefill_code_offset.restype = C.c_uint32
     return _LIB
 
 
@@ -47,3 +51,10 @@ class TqRoute:
 
 def tq_workspace(queries, qh, hd, max_tokens):
     return lib().fhip_rule_tq_workspace(queries, qh, hd, max_tokens)
+
+
+def prefill_split(queries, G, kvh, extent, max_splits):
+    """Queries per block, blocks, splits, positions per split and workgroups of a tiled prefill."""
+    out = (C.c_int64 * 5)()
+    lib().fhip_rule_prefill_split(queries, G, kvh, 128, 64, 512, extent, max_splits, out)
+    return tuple(out)

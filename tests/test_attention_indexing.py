@@ -4,9 +4,9 @@ against the buffers the launcher hands them.
 
 The MFMA kernel's addresses come from its own index functions (fracture_amd/csrc/
 tq_attn_index.h), called through their host build (libfracture_hip_index.so), for every
-workgroup of the launch grid, every wave (one 512-position split of the workgroup's
-1024-position block) and every 64-position chunk, with numpy over the 64 lanes. What they
-compute:
+workgroup of the launch grid, every wave (an equal split of the workgroup's block: two or four
+waves of a 1024-position block, four of a 256-position one) and every 64-position chunk, with
+numpy over the 64 lanes, at every pair of code widths. What they compute (K and V at 4 bits):
 
   split pages        entry j = table[t_begin / 16 + j] for pages holding positions of the split,
                      in the pool; every other entry is the split's first valid page (no valid
@@ -33,11 +33,10 @@ import pytest
 PAGE = 16
 CHUNK = 64
 SPLIT = 1024       # positions per partial (the MFMA kernel's workgroup block, the VALU kernel's split)
-WAVE_SPLIT = 512   # positions per MFMA wave
 
 
-def ws_layout(nq, qh, hd, max_tokens):
-    ns = (max_tokens + SPLIT - 1) // SPLIT if max_tokens > 0 else 1
+def ws_layout(nq, qh, hd, max_tokens, part=SPLIT):
+    ns = (max_tokens + part - 1) // part if max_tokens > 0 else 1
     al = lambda x: (x + 255) & ~255
     qrot = nq * qh * hd * 4
     ml = nq * qh * ns * 2 * 4
@@ -86,7 +85,8 @@ class IndexLib:
         L.fhip_idx_partial_row.argtypes = [C.c_int] * 7
         L.fhip_idx_partial_row.restype = C.c_int64
         L.fhip_idx_lane_tables.argtypes = [C.c_int, C.c_int] + [C.c_void_p] * 6
-        L.fhip_idx_v2_offsets.argtypes = [C.c_int, C.c_int, C.c_void_p]
+        L.fhip_idx_wave_split.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int32), C.c_void_p, C.c_void_p]
+        L.fhip_idx_code_tables.argtypes = [C.c_int] * 4 + [C.c_void_p] * 3 + [C.POINTER(C.c_int32)] * 2
         L.fhip_idx_split_grid_item.argtypes = [C.c_int64, C.c_int, C.c_int, C.c_int] + [C.POINTER(C.c_int32)] * 3
         self._tables = {}
 
@@ -105,10 +105,14 @@ class IndexLib:
                                  n_off.astype(np.int64), n_page, q_off)
         return self._tables[key]
 
-    def v2_offsets(self, kvh, g):
-        out = np.zeros(64, np.uint32)
-        assert self.lib.fhip_idx_v2_offsets(kvh, g, out.ctypes.data) == 0
-        return out.astype(np.int64)
+    def code_tables(self, kvh, g, kbits, vbits):
+        """K load offsets [4][64], V load offsets [4 or 8][64] and their pages, bytes of a K and a V load."""
+        k_off, v_off = np.zeros((4, 64), np.uint32), np.zeros((8, 64), np.uint32)
+        v_page, kw, vw = np.zeros(8, np.int32), self.C.c_int32(), self.C.c_int32()
+        assert self.lib.fhip_idx_code_tables(kvh, g, kbits, vbits, k_off.ctypes.data, v_off.ctypes.data,
+                                             v_page.ctypes.data, self.C.byref(kw), self.C.byref(vw)) == 0
+        n = 8 if vbits == 8 else 4
+        return k_off.astype(np.int64), v_off[:n].astype(np.int64), v_page[:n], kw.value, vw.value
 
     def split_grid_item(self, lin, nsplit, kvh, nq):
         s, h, q = self.C.c_int32(), self.C.c_int32(), self.C.c_int32()
@@ -121,12 +125,12 @@ class IndexLib:
         assert self.lib.fhip_idx_wg_item(wg, kvh, self.C.byref(item), self.C.byref(g)) == 0
         return item.value, g.value
 
-    def split(self, blk, wave, t_end):
+    def split(self, blk, wave, t_end, waves=2, part=SPLIT):
         t_begin = self.C.c_int32()
         col = np.zeros(64, np.int32)
         ins = np.zeros(64, np.uint8)
-        assert self.lib.fhip_idx_split(blk, wave, t_end, self.C.byref(t_begin), col.ctypes.data,
-                                       ins.ctypes.data) == 0
+        assert self.lib.fhip_idx_wave_split(blk, wave, waves, part, t_end, self.C.byref(t_begin), col.ctypes.data,
+                                            ins.ctypes.data) == 0
         return t_begin.value, col, ins.astype(bool)
 
     def q_vectors(self, tq0, tok, G, nq, qh, g):
@@ -147,18 +151,20 @@ def index_lib():
     return _IDX
 
 
-def model_mfma_kernel(lens, table, num_pages, qh, kvh, page_bytes, pool_bytes, tok=1, vbits=4):
-    """Every access of tq_attn_mfma_kernel<PoolPages> for one launch (hd 128, K4 and V4 or V2),
-    from the kernel's own index functions. With tok > 1, `table` has one row that every query
-    reads (causal prefill). Walks every workgroup of the launcher's grid."""
+def model_mfma_kernel(lens, table, num_pages, qh, kvh, page_bytes, pool_bytes, tok=1, kbits=4, vbits=4,
+                      waves=2, part=SPLIT):
+    """Every access of tq_attn_mfma_kernel<PoolPages> for one launch (hd 128, K and V of kbits and
+    vbits, `waves` waves per block of `part` positions), from the kernel's own index functions. With
+    tok > 1, `table` has one row that every query reads (causal prefill). Walks every workgroup of
+    the launcher's grid."""
     ix = index_lib()
-    hd, pd = 128, 64
+    hd = 128
     B = len(lens)
     rows, max_blocks = table.shape
     stride = 0 if tok > 1 else max_blocks
     assert tok == 1 or rows == 1
     G = qh // kvh
-    nsplit, _, ml_bytes, acc_bytes = ws_layout(B, qh, hd, max_blocks * PAGE)
+    nsplit, _, ml_bytes, acc_bytes = ws_layout(B, qh, hd, max_blocks * PAGE, part)
     bnd = Bounds({"table": table.size * 4, "kp": pool_bytes["kp"], "kn": pool_bytes["kn"],
                   "vp": pool_bytes["vp"], "vn": pool_bytes["vn"], "qrot": B * qh * hd * 4,
                   "part_ml": ml_bytes, "part_acc": acc_bytes})
@@ -174,23 +180,20 @@ def model_mfma_kernel(lens, table, num_pages, qh, kvh, page_bytes, pool_bytes, t
             continue  # padding workgroup: leaves at once
         tq_last = min(tq0 + tok, B) - 1
         clen = causal_len(lens[tq_last], max_blocks)
-        if blk * SPLIT >= clen:
+        if blk * part >= clen:
             continue  # the workgroup leaves before building its tables
-        k_off, k_page, v_off, n_off, n_page, q_off = ix.lane_tables(kvh, g)
-        for k in range(4):
-            assert (k_off[k] + 16 <= PAGE * kvh * pd).all() and (k_off[k] + 16 <= page_bytes["kp"]).all()
-        vpd, vw = (pd, 16) if vbits == 4 else (pd // 2, 8)  # V row bytes, bytes per V load
-        if vbits == 2:
-            v_off = ix.v2_offsets(kvh, g)
-        assert (v_off + vw <= min(PAGE * kvh * vpd, page_bytes["vp"])).all()
+        _, k_page, _, n_off, n_page, q_off = ix.lane_tables(kvh, g)
+        k_off, v_off, v_page, kw, vw = ix.code_tables(kvh, g, kbits, vbits)
+        assert (k_off + kw <= min(PAGE * kvh * 16 * kbits, page_bytes["kp"])).all()
+        assert (v_off + vw <= min(PAGE * kvh * 16 * vbits, page_bytes["vp"])).all()
         for nm in ("kn", "vn"):
             assert (n_off + 2 <= min(PAGE * kvh * 2, page_bytes[nm])).all()
-        for w in range(SPLIT // WAVE_SPLIT):
-            t_begin, col, has = ix.split(blk, w, SPLIT * nsplit)
+        for w in range(waves):
+            t_begin, col, has = ix.split(blk, w, part * nsplit, waves, part)
             if t_begin >= clen:
                 continue  # empty state, nothing read
-            t_end = min(clen, t_begin + WAVE_SPLIT)
-            _, col, has = ix.split(blk, w, t_end)
+            t_end = min(clen, t_begin + part // waves)
+            _, col, has = ix.split(blk, w, t_end, waves, part)
             tidx = col[has]
             assert tidx.max() < max_blocks
             bnd.check("table", (tq0 * stride + tidx) * 4, 4)
@@ -199,15 +202,15 @@ def model_mfma_kernel(lens, table, num_pages, qh, kvh, page_bytes, pool_bytes, t
             ok = has & (ids >= 0) & (ids < num_pages)
             if not ok.any():
                 continue
-            entry = np.where(ok, ids, ids[np.flatnonzero(ok)[0]])[:WAVE_SPLIT // PAGE]
+            entry = np.where(ok, ids, ids[np.flatnonzero(ok)[0]])[:part // waves // PAGE]
             assert ((entry >= 0) & (entry < num_pages)).all()
             for t0 in range(t_begin, t_end, CHUNK):
                 j0 = ix.lib.fhip_idx_chunk_first_page(t0, t_begin)
                 assert j0 + 3 < len(entry), "page entry index past the wave's table"
                 for pt in range(4):  # K codes
-                    bnd.check("kp", entry[j0 + k_page] * page_bytes["kp"] + k_off[pt], 16)
-                for i in range(4):  # V copies: copy i reads entry j0 + i
-                    bnd.check("vp", entry[j0 + i] * page_bytes["vp"] + v_off, vw)
+                    bnd.check("kp", entry[j0 + k_page] * page_bytes["kp"] + k_off[pt], kw)
+                for i, j in enumerate(v_page):  # V loads: load i reads entry j0 + v_page[i]
+                    bnd.check("vp", entry[j0 + j] * page_bytes["vp"] + v_off[i], vw)
                 for nm in ("kn", "vn"):  # norms
                     bnd.check(nm, entry[j0 + n_page] * page_bytes[nm] + n_off, 2)
             vec, live = ix.q_vectors(tq0, tok, G, B, qh, g)
@@ -225,7 +228,7 @@ def model_mfma_kernel(lens, table, num_pages, qh, kvh, page_bytes, pool_bytes, t
     return bnd, nsplit
 
 
-def model_combine(lens, max_blocks, qh, hd, nsplit, ml_bytes, acc_bytes):
+def model_combine(lens, max_blocks, qh, hd, nsplit, ml_bytes, acc_bytes, part=SPLIT):
     """tq_attn_combine_kernel: partial reads (clamped split index), rotation reads, output."""
     B = len(lens)
     nvec = B * qh
@@ -235,7 +238,7 @@ def model_combine(lens, max_blocks, qh, hd, nsplit, ml_bytes, acc_bytes):
     c0 = np.arange(256)[:, None] + 256 * np.arange(16)[None, :]
     bnd.check("vrot", 4 * np.minimum(c0, n16 - 1) * 4, 16)
     heads = np.arange(nvec)
-    ns = np.array([(causal_len(lens[h // qh], max_blocks) + SPLIT - 1) // SPLIT for h in heads])
+    ns = np.array([(causal_len(lens[h // qh], max_blocks) + part - 1) // part for h in heads])
     assert ns.max() <= nsplit
     for hh, k in zip(heads, ns):
         sp = np.arange(k)
@@ -303,6 +306,29 @@ def test_mfma_decode_accesses_in_bounds(which, vbits):
     assert bnd.count["kp"] > 0 and bnd.count["vp"] > 0
     _, _, ml, acc = ws_layout(len(lens), qh, 128, table.shape[1] * PAGE)
     model_combine(lens, table.shape[1], qh, 128, nsplit, ml, acc)
+
+
+@pytest.mark.parametrize("waves,part", [(2, SPLIT), (4, SPLIT), (4, 256)])
+@pytest.mark.parametrize("kbits,vbits", [(4, 4), (4, 2), (3, 3), (2, 2), (8, 8)])
+def test_mfma_variants_in_bounds(waves, part, kbits, vbits):
+    """Every variant that the route may take, at every pair of widths: lengths on the edges of chunks,
+    pages, waves and blocks, an empty sequence, a length past its table, pages outside the pool."""
+    lens = np.array([1, 17, 64, 65, 255, 256, 257, 511, 513, 1024, 1025, 0, 3000], np.int32)
+    max_blocks, qh, kvh = 160, 16, 8
+    rng = np.random.default_rng(waves + part)
+    P = 700
+    table = np.full((len(lens), max_blocks), -7, np.int32)
+    for b, n in enumerate(lens):
+        nb = min((int(n) + 15) // 16, max_blocks)
+        table[b, :nb] = rng.integers(0, P, nb)
+    table[9, 3], table[10, 64] = P, -1
+    page = {"kp": PAGE * kvh * 16 * kbits, "kn": PAGE * kvh * 2, "vp": PAGE * kvh * 16 * vbits, "vn": PAGE * kvh * 2}
+    pool = {k: v * P for k, v in page.items()}
+    bnd, nsplit = model_mfma_kernel(lens, table, P, qh, kvh, page, pool, kbits=kbits, vbits=vbits, waves=waves,
+                                    part=part)
+    assert bnd.count["kp"] > 0 and bnd.count["vp"] > 0 and nsplit == -(-max_blocks * PAGE // part)
+    _, _, ml, acc = ws_layout(len(lens), qh, 128, max_blocks * PAGE, part)
+    model_combine(lens, max_blocks, qh, 128, nsplit, ml, acc, part)
 
 
 @pytest.mark.parametrize("qh,kvh,T,kv_len", [(32, 8, 37, 3000), (16, 8, 9, 1100), (8, 8, 20, 2100),

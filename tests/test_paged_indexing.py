@@ -1,23 +1,24 @@
-"""CPU model of the work split of the FP16 paged-attention kernels (paged_attn_split_kernel
-and paged_attn_prefill_mfma_kernel in fracture_amd/csrc/attention_paged.hip): which query rows
-each wave reads and which split partials it writes, checked against the combine kernel's reads.
+"""CPU models of the work split of the FP16 paged-attention kernels: which query rows each wave of
+paged_attn_split_kernel reads and which split partials it writes, checked against the combine kernel's
+reads, and the tiled prefill kernels' blocks and splits (FP16 and TurboQuant), through the functions
+that the launchers and kernels call.
 
-A wave item is (query group, kv head g, head block hb, split). In causal prefill over one
-shared block table, a group is tok consecutive queries: 16 / G of them on the MFMA prefill
-kernel (head_dim <= 128, G = qh / kvh <= 8), else 8 / G (G < 8); MFMA column c is head
-g G + c % G of query tq0 + c / G. Otherwise tok = 1 and column c is head g G + 8 hb + c. Each
-column scores positions below min(split end, its own causal length). The combine reads partial
-(vector, split) for every split below the vector's causal length; the model asserts that each
-of those is written by exactly one wave, with the causal length of that vector, and that
-nothing else is read. No GPU is used.
+A workgroup item of the split kernel is (query group, kv head g, head block hb, split). In causal
+prefill over one shared block table at head_dim 256, a group is tok = 8 / G consecutive queries
+(G = qh / kvh < 8); MFMA column c is head g G + c % G of query tq0 + c / G. Otherwise tok = 1 and
+column c is head g G + 8 hb + c. Each column scores positions below min(split end, its own causal
+length). The combine reads partial (vector, split) for every split below the vector's causal length;
+the model asserts that each of those is written by exactly one item, with the causal length of
+that vector, and that nothing else is read. No GPU is used.
 """
 import numpy as np
 import pytest
 
+import rules
+
 PAGE = 16
 SPLIT = 1024
 HEADS_MAX = 8
-PF_WAVES = 4  # query groups per workgroup of the MFMA prefill kernel
 
 
 def causal_len(qi, kv_len, start_pos, max_blocks, seq_lens=None):
@@ -26,54 +27,33 @@ def causal_len(qi, kv_len, start_pos, max_blocks, seq_lens=None):
 
 
 def model_split_kernel(nq, qh, kvh, kv_len, start_pos, shared_table=True, seq_lens=None,
-                       wrap=None, hd=128):
+                       wrap=None):
     G = qh // kvh
     wrap = G if wrap is None else wrap  # head count at which the acc loop's counter wraps
     nhb = (G + HEADS_MAX - 1) // HEADS_MAX
     max_blocks = (max(kv_len, int(max(seq_lens)) if seq_lens is not None else 0) + 15) // 16
     nsplit = max(1, (max_blocks * PAGE + SPLIT - 1) // SPLIT)
     prefill = seq_lens is None and shared_table and nq > 1
-    mfma = prefill and hd <= 128 and G <= HEADS_MAX
-    tok = (2 * HEADS_MAX // G if mfma else
-           HEADS_MAX // G if prefill and G < HEADS_MAX else 1)
-    NH = 16 if mfma else 4 if G * tok <= 4 else 8
+    tok = HEADS_MAX // G if prefill and G < HEADS_MAX else 1
+    NH = 4 if G * tok <= 4 else 8
     per_q = kvh * nhb * nsplit
-    waves = []  # (tp0, tq0, ntok, g, hb, split, t_begin, t_end) of each wave that runs the loop
-    if mfma:
-        # workgroup (PF_WAVES groups, kv head, split); wave w takes the set's group w, and
-        # all run the chunks of the set's longest causal length (uniform exits only)
-        for wg in range(-(-(-(-nq // tok)) // PF_WAVES) * kvh * nsplit):
-            tp0 = (wg // per_q) * PF_WAVES * tok
-            if tp0 >= nq:
-                continue
-            g, split = wg % kvh, (wg // kvh) % nsplit
-            clen = causal_len(min(tp0 + PF_WAVES * tok, nq) - 1, kv_len, start_pos, max_blocks,
-                              seq_lens)
-            t_begin = split * SPLIT
-            if t_begin >= clen:
-                continue
-            for w in range(PF_WAVES):
-                tq0 = tp0 + w * tok
-                waves.append((tp0, tq0, max(0, min(tok, nq - tq0)), g, 0, split, t_begin,
-                              min(clen, t_begin + SPLIT)))
-    else:
-        for item in range(-(-nq // tok) * per_q):
-            tq0 = (item // per_q) * tok
-            if tq0 >= nq:
-                continue
-            ntok = min(tok, nq - tq0)
-            g = item % kvh
-            hb = (item // kvh) % nhb
-            split = (item // (kvh * nhb)) % nsplit
-            clen = causal_len(tq0 + ntok - 1, kv_len, start_pos, max_blocks, seq_lens)
-            t_begin = split * SPLIT
-            if t_begin >= clen:
-                continue
-            waves.append((tq0, tq0, ntok, g, hb, split, t_begin, min(clen, t_begin + SPLIT)))
+    items = []  # (tq0, ntok, g, hb, split, t_begin, t_end) of each item that runs the loop
+    for item in range(-(-nq // tok) * per_q):
+        tq0 = (item // per_q) * tok
+        if tq0 >= nq:
+            continue
+        ntok = min(tok, nq - tq0)
+        g = item % kvh
+        hb = (item // kvh) % nhb
+        split = (item // (kvh * nhb)) % nsplit
+        clen = causal_len(tq0 + ntok - 1, kv_len, start_pos, max_blocks, seq_lens)
+        t_begin = split * SPLIT
+        if t_begin >= clen:
+            continue
+        items.append((tq0, ntok, g, hb, split, t_begin, min(clen, t_begin + SPLIT)))
     written = {}
     q_rows = set()
-    for tp0, tq0, ntok, g, hb, split, t_begin, t_end in waves:
-        clen = t_end  # only its bound on the column lengths matters below
+    for tq0, ntok, g, hb, split, t_begin, t_end in items:
         h0 = g * G + hb * HEADS_MAX
         ncols = ntok * G if tok > 1 else min(HEADS_MAX, G - hb * HEADS_MAX)
         assert ncols <= NH
@@ -82,8 +62,8 @@ def model_split_kernel(nq, qh, kvh, kv_len, start_pos, shared_table=True, seq_le
             col_ok = n < ncols
             ct = n // G if col_ok else 0
             hn = n - ct * G if col_ok else 0
-            # a column past the queries reads the workgroup's first query row (unused)
-            row = ((tq0 + ct) if col_ok else tp0) * qh + h0 + hn
+            # a column past the queries reads the group's first query row (unused)
+            row = (tq0 + ct) * qh + h0 + hn
             assert 0 <= row < nq * qh
             if not col_ok:
                 continue
@@ -92,20 +72,14 @@ def model_split_kernel(nq, qh, kvh, kv_len, start_pos, shared_table=True, seq_le
                 if tok > 1 else t_end
             lim = min(t_end, col_len)
             q_rows.add(row)
-            if mfma:
-                # the MFMA kernel's partial write of product h, row 4 kg + e: column 8h + 4kg + e
-                for col in range(ncols):
-                    if col == n:
-                        assert (tq0 + col // G) * qh + h0 + col % G == row
-            else:
-                # the partial write of lane n (== column n) and of the acc loop's column n
-                hc, hh = 0, 0
-                for h in range(NH):
-                    if h == n:
-                        assert (tq0 + hc) * qh + h0 + hh == row
-                    hh += 1
-                    if hh == wrap:
-                        hh, hc = 0, hc + 1
+            # the partial write of lane n (== column n) and of the acc loop's column n
+            hc, hh = 0, 0
+            for h in range(NH):
+                if h == n:
+                    assert (tq0 + hc) * qh + h0 + hh == row
+                hh += 1
+                if hh == wrap:
+                    hh, hc = 0, hc + 1
             key = (row, split)
             assert key not in written, f"partial {key} written twice"
             written[key] = (lim, t_begin)
@@ -126,13 +100,12 @@ def model_split_kernel(nq, qh, kvh, kv_len, start_pos, shared_table=True, seq_le
     return tok
 
 
-@pytest.mark.parametrize("nq,qh,kvh,kv_len,start_pos,hd,tok", [
-    (19, 4, 4, 1050, 1020, 128, 16), (13, 8, 4, 300, 0, 32, 8), (11, 6, 2, 1100, 1019, 256, 2),
-    (11, 6, 2, 1100, 1019, 64, 5), (70, 8, 2, 70, 0, 128, 4), (9, 16, 16, 2100, 2040, 64, 16),
-    (7, 16, 2, 50, 43, 64, 2), (37, 32, 8, 3000, 2963, 128, 4), (5, 24, 2, 1030, 1025, 128, 1),
-    (1, 8, 8, 40, 39, 128, 1), (33, 32, 4, 2100, 2067, 128, 2), (21, 8, 8, 600, 579, 256, 8)])
-def test_prefill_groups_cover_every_partial(nq, qh, kvh, kv_len, start_pos, hd, tok):
-    assert model_split_kernel(nq, qh, kvh, kv_len, start_pos, hd=hd) == tok
+@pytest.mark.parametrize("nq,qh,kvh,kv_len,start_pos,tok", [
+    (19, 4, 4, 1050, 1020, 8), (13, 8, 4, 300, 0, 4), (11, 6, 2, 1100, 1019, 2), (70, 8, 2, 70, 0, 2),
+    (9, 16, 16, 2100, 2040, 8), (7, 16, 2, 50, 43, 1), (37, 32, 8, 3000, 2963, 2), (5, 24, 2, 1030, 1025, 1),
+    (1, 8, 8, 40, 39, 1), (33, 32, 4, 2100, 2067, 1), (21, 8, 8, 600, 579, 8)])
+def test_prefill_groups_cover_every_partial(nq, qh, kvh, kv_len, start_pos, tok):
+    assert model_split_kernel(nq, qh, kvh, kv_len, start_pos) == tok
 
 
 def test_decode_rows_keep_one_query_per_wave():
@@ -143,34 +116,28 @@ def test_decode_rows_keep_one_query_per_wave():
 def test_column_mapping_error_is_caught():
     """The model fails when the acc loop's column counter wraps at the wrong head count."""
     with pytest.raises(AssertionError):
-        model_split_kernel(13, 8, 4, 300, 0, wrap=3, hd=256)
-
-
-def prefill_split(nq, qh, kvh, extent, nsplit_ws, cols=128, tile=64, groups=512):
-    """The launchers' choice for the tiled prefill kernels: queries per block, blocks, splits."""
-    nqb = cols // (qh // kvh)
-    nblk = -(-nq // nqb)
-    base = nblk * kvh
-    want = min(max(-(-groups // base), 1), nsplit_ws)
-    pos = -(-(-(-extent // want)) // tile) * tile
-    return nqb, nblk, -(-extent // pos), pos
+        model_split_kernel(13, 8, 4, 300, 0, wrap=3)
 
 
 @pytest.mark.parametrize("nq,qh,kvh,kv_len,start_pos", [
     (2, 8, 8, 40, 38), (130, 32, 8, 1130, 1000), (129, 128, 128, 2100, 1971), (37, 24, 3, 1200, 1163),
     (1000, 32, 8, 4001, 3001), (70, 7, 1, 70, 0), (65, 16, 2, 5000, 4000)])
-@pytest.mark.parametrize("fold", [False, True])
-def test_tiled_prefill_covers_every_partial(nq, qh, kvh, kv_len, start_pos, fold):
-    """Workgroups of the tiled prefill kernels (128 columns of one kv head, one split): each
-    (vector, split) below the vector's causal length is written once, no split count exceeds the
-    workspace's, tiles start inside a 64-page window with their four pages, and the order of blocks
-    (from the last down, or folded) is a permutation."""
+@pytest.mark.parametrize("part", [SPLIT, 256])
+@pytest.mark.parametrize("cus", [0, 8, 64, 256])
+def test_tiled_prefill_covers_every_partial(nq, qh, kvh, kv_len, start_pos, part, cus):
+    """Workgroups of the tiled prefill kernels (128 columns of one kv head, one split), as the launchers'
+    functions split them over a workspace of `part`-position partials: each (vector, split) below the
+    vector's causal length is written once, no split count exceeds the workspace's, tiles start inside a
+    64-page window with their four pages, and the order of blocks (from the last down, folded where
+    they fit `cus` CUs twice) is a permutation."""
     G = qh // kvh
-    ws = max(1, -(-(-(-kv_len // PAGE) * PAGE) // SPLIT))
-    nqb, nblk, nsplit, pos = prefill_split(nq, qh, kvh, kv_len, ws)
-    assert nsplit <= ws and pos % 64 == 0
-    half = max(1, nblk // 2) if fold else 0
-    order = [bi - half if fold and bi >= half else nblk - 1 - bi for bi in range(nblk)]
+    ws = max(1, -(-(-(-kv_len // PAGE) * PAGE) // part))
+    nqb, nblk, nsplit, pos, wgs = rules.prefill_split(nq, G, kvh, kv_len, ws)
+    assert nsplit <= ws and pos % 64 == 0 and wgs == nblk * kvh * nsplit
+    assert nqb * G <= 128 and (nblk - 1) * nqb < nq <= nblk * nqb and (nsplit - 1) * pos < kv_len <= nsplit * pos
+    fold = rules.lib().fhip_rule_prefill_fold(nsplit, wgs, kvh, cus)
+    assert 0 <= fold < max(nblk, 1)
+    order = [rules.lib().fhip_idx_prefill_block(bi, nblk, fold) for bi in range(nblk)]
     assert sorted(order) == list(range(nblk))
     written = {}
     for blk in order:
@@ -196,3 +163,27 @@ def test_tiled_prefill_covers_every_partial(nq, qh, kvh, kv_len, start_pos, fold
         for s in range(-(-c // pos)):
             for h in range(qh):
                 assert written[(qi * qh + h, s)] >= min(c, (s + 1) * pos)
+
+
+def test_prefill_folds_a_single_split():
+    """2048 queries of 32 / 8 heads: 512 workgroups on 256 CUs, the second half from the first block up."""
+    nqb, nblk, nsplit, pos, wgs = rules.prefill_split(2048, 4, 8, 2048, 8)
+    assert (nqb, nblk, nsplit, wgs) == (32, 64, 1, 512)
+    fold = rules.lib().fhip_rule_prefill_fold(nsplit, wgs, 8, 256)
+    assert fold == 32
+    order = [rules.lib().fhip_idx_prefill_block(bi, nblk, fold) for bi in range(nblk)]
+    assert order == list(range(63, 31, -1)) + list(range(32))
+
+
+@pytest.mark.parametrize("bits", [2, 3, 4, 8])
+@pytest.mark.parametrize("kvh", [1, 3, 8])
+def test_prefill_code_loads_cover_each_row_once(bits, kvh):
+    """A tile's 64 rows of four quarters: each byte of kv head g's codes on the tile's four pages once."""
+    for g in range(kvh):
+        seen = np.zeros((4, PAGE * kvh * 16 * bits), np.int32)
+        for row in range(64):
+            for quarter in range(4):
+                off = rules.lib().fhip_idx_prefill_code_offset(row, quarter, kvh, g, bits)
+                seen[row // PAGE, off:off + 4 * bits] += 1
+        rows = seen.reshape(4, PAGE, kvh, 16 * bits)
+        assert (rows[:, :, g] == 1).all() and rows.sum() == 64 * 16 * bits
