@@ -9,10 +9,11 @@
 // online softmax each, merged by a second kernel: up to 1,048,576 positions per sequence.
 //
 // Work split: one workgroup per (query, kv head, block of up to 8 of its q heads, split). Each K
-// row crosses HBM once per (query, kv head) for up to 8 q heads. In causal prefill with fewer
-// than 8 q heads per kv head, it takes 8 / G consecutive queries instead, its columns
+// row crosses HBM once per (query, kv head) for up to 8 q heads. In causal prefill at head_dim 256 with
+// fewer than 8 q heads per kv head, it takes 8 / G consecutive queries instead, its columns
 // being (query, head) pairs each masked to its own causal length, so that a K or V row is
-// read once for all of them. Per 32-position chunk (16 when head_dim is 256):
+// read once for all of them (head_dim 32, 64 and 128 have a prefill kernel of their own, below). Per
+// 32-position chunk (16 when head_dim is 256):
 //   QK on v_mfma_f32_16x16x32_f16: A = K rows (row = position, 8 consecutive dims per lane,
 //      exactly their memory layout), B = Q^T (column = q head): fp16 x fp16 products are
 //      exact in fp32, the sums are fp32;
@@ -26,9 +27,9 @@
 
 #include <algorithm>
 
-#include "launch_rules.h"
 #include "fhip_common.h"
 #include "fracture_hip.h"
+#include "launch_rules.h"
 #include "tq_attn_index.h"
 
 using namespace fhip;
@@ -480,17 +481,6 @@ constexpr float kPfScale = 4096.0f;        // 2^kPfBias
 constexpr float kPfSlack = 3.75f;          // log2 that p may exceed it by (2^15.75 < fp16's largest)
 constexpr int64_t kPfGroups = 512;         // workgroups wanted: the two per CU that fit at once
 typedef float f16x_t __attribute__((ext_vector_type(16)));
-
-// (a, b) as fp16 pairs hi + lo, hi rounded to nearest, lo the fp16 of what it leaves.
-typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
-typedef float f2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
-    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t{a, b}), h2_t));
-    float la, lb;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(la) : "v"(hi), "v"(a));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(lb) : "v"(hi), "v"(b));
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2_t{la, lb}), h2_t));
-}
 
 template <int HD, class Pages>
 __global__ __launch_bounds__(64 * kPfWaves) __attribute__((amdgpu_waves_per_eu(2))) void

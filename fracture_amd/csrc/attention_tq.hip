@@ -578,8 +578,8 @@ __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
 // (vector, d) up to 16 splits' (m, l) and accumulator d, folded as an online softmax over chunks of
 // 16 splits. The merged vectors cross LDS once, then each lane sums its 32 products for the 4
 // vectors and the quarters meet in LDS. The general kernel above stages Pi_v in LDS, then waits for
-// (m, l), for the accumulators and for 128 LDS reads in turn: 8.3 us for 32 vectors of 4 splits
-// against 5.3 here (2048 vectors of up to 32 splits are bound by their 34 MB either way: 20 us).
+// (m, l), for the accumulators and for 128 LDS reads in turn: 8.3 us for 32 vectors of 4 splits and
+// 19.9 for 2048 of up to 32 against 4.6 (of 16 parts) and 13.7 here (kernel trace, as above).
 constexpr int kComb128Vecs = 4;
 __global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
     Queries qs, const float* __restrict__ part_ml, const float* __restrict__ part_acc,
@@ -1197,7 +1197,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
 #pragma unroll
     for (int c = 0; c < 8; ++c) acc[c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // The split's pages , read once: the chunk loop then issues no memory
+    // The split's pages, read once: the chunk loop then issues no memory
     // instruction besides its loads and copies. A wave with no position to read (its split
     // starts past the end, or no page is in the pool) keeps the empty state.
     PageAddrs* pages = pagebuf[wave];
@@ -1234,7 +1234,6 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     float colscale;
     uint32_t bq[8][4];
     {
-        // heads past G read head 0 and are zeroed by the multiplier
         // columns past the group's heads read the group's first vector and are zeroed
         const float* qsrc = qrot + qvec * hd;
         f32x4_t qv[8];
@@ -1310,7 +1309,7 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
         const uint32_t pmask_n = tn < t_end ? (uint32_t)(vmask >> jn) & 0xfu : 0u;
         const bool full = pmask == 0xfu && tn <= t_end && tn <= min_len;
 
-        // ---- QK: 4 tiles x 8 steps, K codes from this wave's DMA buffer
+        // ---- QK: 4 tiles x 8 steps
         float sc[4][4];  // !kG4 [pt][e]: position 16rg + 4e + pt, head n & 7
         float scc[4];    // kG4 [e]: position 16rg + 4e + ptc, head n & 3
         // all loads of this chunk are in (the V copies included)
@@ -1670,17 +1669,6 @@ constexpr float kPqBias = 13.0f;        // log2 of the scale that p carries
 // its power of two), which fp16 holds
 constexpr float kPqSlack = 3.0f;
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef _Float16 f16x2c_t __attribute__((ext_vector_type(2)));
-typedef float f32x2c_t __attribute__((ext_vector_type(2)));
-
-// x = hi + lo as fp16 pairs, hi rounded to nearest, lo the fp16 of what it leaves.
-__device__ __forceinline__ void split_pair(float a, float b, uint32_t& hi, uint32_t& lo) {
-    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2c_t{a, b}), f16x2c_t));
-    float la, lb;
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(la) : "v"(hi), "v"(a));
-    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(lb) : "v"(hi), "v"(b));
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2c_t{la, lb}), f16x2c_t));
-}
 // Codes of one thread's quarter row (32 codes) of a tile: 4 B bytes.
 template <int B>
 struct Codes32 {

@@ -214,7 +214,6 @@ __device__ __forceinline__ float partner_f(float x) {
 
 // Sum of squares of 8 fp16 values with fp32 accumulation (products of fp16 are exact).
 __device__ __forceinline__ float sumsq8(const f16x8& b, float acc) {
-    typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const f16x2 p = {b[2 * e], b[2 * e + 1]};
