@@ -1174,8 +1174,14 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
     }
     __syncthreads();
 
-    const int t_begin = fhip_idx::split_begin(blk, wave, W, kPart);
-    const int t_end = min(clen, t_begin + kPart / W);
+    // (a constant where it can only be one chunk: the loop below is then straight code. Two waves of 8-bit
+    // codes keep halves of the block: with two waves per SIMD a large launch is bound by the waves' fixed
+    // part, 128 sequences of 400, 8 / 8 heads 40.4 us and 43.2 in halves of their positions)
+    const int span = kPart / W == kChunkM || (KB == 8 && W == 2)
+                         ? kPart / W
+                         : fhip_idx::wave_span(min(kPart, clen - blk * kPart), W);
+    const int t_begin = fhip_idx::split_begin(blk, wave, kPart, span);
+    const int t_end = min(clen, t_begin + span);
     const int G = qh / kvh;
     const int32_t* table = qs.table + (int64_t)tq0 * qs.table_stride;
     uint8_t* vb = vbuf[wave][0];

@@ -138,10 +138,14 @@ constexpr int kMergeSplits = 8;     // ... and the splits that the merge before 
 //   The decode kernel in 256-position parts, four waves of one chunk each, where that makes at most three
 //   workgroups per CU and 48 parts: four times the workgroups of 1024-position parts (one sequence of
 //   1000, 32 / 8 heads: 16.5 us; 23.3 in 1024-position blocks of four waves, 31.2 of two). More
-//   workgroups run in turns (512 queries' worth, 64 sequences of 1000: 39.9 and 35.5), and more parts
-//   make the merge the larger half (one sequence of 20000, 79 parts: 28.3 and 25.6; 32000: 37.3 and 26.8).
-//   Else 1024-position parts: four waves up to 512 workgroups (64 sequences of 1000: 35.5 us, with two
-//   42.8, with eight 39.6; of 16: 21.3, 21.5, 24.1), two beyond (64 of 3000, 1536 workgroups: 62.6 us,
+//   parts make the merge the larger half (one sequence of 20000, 79 parts: 28.3 and 25.6; 32000: 37.3 and
+//   26.8). More workgroups run in turns; up to 1536 of them are still the shorter way where the
+//   1024-position parts are more than one per CU, whose second turn is nearly empty or short: with up to 384 of
+//   those, or 512 where some hold only a sequence's rest (K4/V4, 32 / 8 heads: 20 sequences of 1200 23.9 and
+//   29.7, 40 of 1000 32.3 and 34.8, 32 of 1400 32.0 and 32.0, of 175 .. 1400 25.1 and 30.3; but 64 of 378
+//   28.4 and 26.8, 28 of 1000 25.2 and 25.2).
+//   Else 1024-position parts: four waves up to 512 workgroups (64 sequences of 1000: 35.4 us, with two
+//   42.4, with eight 38.7; 32 of 2000 32.5, 39.7, 35.7), two beyond (64 of 3000, 1536 workgroups: 62.6 us,
 //   with four 64.8).
 //   Causal calls of more workgroups than that (than 256 where the codes' expansion is dearer, at 3 and 8
 //   bits) go to the prefill kernel where it is the shorter one: a tile takes a workgroup 4.3 us, with up to
@@ -164,7 +168,10 @@ inline TqRoute tq_route(const TqCall& c) {
     const bool fits = fine.bytes <= std::min(c.ws_bytes, kTqFineBytes);
     const int nsplit = tq_layout(c.nq, c.qh, c.hd, c.max_tokens, kTqSplit).nsplit;
     const int64_t wgs = tq_decode_workgroups(c.nq, r.tok, c.kvh, nsplit);
-    if (fits && fine.nsplit <= 48 && tq_decode_workgroups(c.nq, r.tok, c.kvh, fine.nsplit) <= 768) {
+    // decode in a second turn of 1024-position parts
+    const bool second = wgs > 256 && wgs <= (nsplit > 1 ? 512 : 384) && !(c.causal && c.nq > 1);
+    if (fits && fine.nsplit <= 48 &&
+        tq_decode_workgroups(c.nq, r.tok, c.kvh, fine.nsplit) <= (second ? 1536 : 768)) {
         r.part = kTqFinePart;
         r.waves = 4;
         return r;

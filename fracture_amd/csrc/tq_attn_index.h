@@ -52,11 +52,15 @@ FHIP_IDX void split_grid_item(int64_t lin, int64_t total, int nsplit, int kvh, i
     qi = (int)(eff / ((int64_t)nsplit * kvh));
 }
 
-// First position of wave `wave`'s split in block blk, `waves` waves per workgroup sharing a block of `part`
-// positions.
-FHIP_IDX int split_begin(int blk, int wave, int waves, int part) {
-    return blk * part + wave * (part / waves);
+// Positions of each wave's split of a block of which `len` positions are live: `waves` equal shares in whole
+// chunks, so that a short context or a ragged last block has no wave with all of it (55 sequences of 378,
+// 8 / 8 heads, K4/V2, four waves: 24.2 us in fixed quarters of 1024, 20.9 so).
+FHIP_IDX int wave_span(int len, int waves) {
+    return (len + kChunk * waves - 1) / (kChunk * waves) * kChunk;
 }
+
+// First position of wave `wave`'s split in block blk of `part` positions.
+FHIP_IDX int split_begin(int blk, int wave, int part, int span) { return blk * part + wave * span; }
 
 // Lane j of a wave reads the block-table column of its split's page j, if that page holds
 // positions of the split [t_begin, t_end).

@@ -3,6 +3,8 @@
 // functions the kernel calls, over all 64 lanes where an index depends on the lane.
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "launch_rules.h"
 #include "tq_attn_index.h"
 
@@ -59,9 +61,9 @@ int fhip_idx_code_tables(int kvh, int g, int kbits, int vbits, uint32_t* k_off, 
     return 0;
 }
 
-// First position of wave `wave` of `waves` in block blk of `part` positions.
+// First position of wave `wave` of `waves` in block blk of `part` positions, all of them live.
 int32_t fhip_idx_split_begin(int blk, int wave, int waves, int part) {
-    return fhip_idx::split_begin(blk, wave, waves, part);
+    return fhip_idx::split_begin(blk, wave, part, fhip_idx::wave_span(part, waves));
 }
 
 // Workgroup wg of a launch with kvh kv heads -> its item and kv head.
@@ -87,23 +89,35 @@ int fhip_idx_split_grid_item(int64_t lin, int nsplit, int kvh, int nq, int32_t* 
     return 0;
 }
 
-// Wave `wave` of `waves` in block blk of `part` positions: its split's first position, and per lane the
-// block-table column of split page `lane` and whether that page holds positions of [t_begin, t_end).
-int fhip_idx_wave_split(int blk, int wave, int waves, int part, int t_end, int32_t* t_begin, int32_t* column,
-                        uint8_t* in_split) {
-    if (blk < 0 || wave < 0 || waves < 1 || part < waves || !t_begin || !column || !in_split) return -1;
-    *t_begin = fhip_idx::split_begin(blk, wave, waves, part);
+// Wave `wave` of `waves` in block blk of `part` positions, `clen` the longest causal length that it sees: its
+// split [t_begin, t_end), and per lane the block-table column of split page `lane` and whether that page holds
+// positions of the split.
+int fhip_idx_wave_split(int blk, int wave, int waves, int part, int clen, int32_t* t_begin, int32_t* t_end,
+                        int32_t* column, uint8_t* in_split) {
+    if (blk < 0 || wave < 0 || waves < 1 || part < waves || clen <= blk * part || !t_begin || !t_end || !column ||
+        !in_split)
+        return -1;
+    const int span = fhip_idx::wave_span(std::min(part, clen - blk * part), waves);
+    *t_begin = fhip_idx::split_begin(blk, wave, part, span);
+    *t_end = std::min(clen, *t_begin + span);
+    for (int lane = 0; lane < 64; ++lane) {
+        int c;
+        in_split[lane] = fhip_idx::split_page_column(*t_begin, *t_end, lane, c) ? 1 : 0;
+        column[lane] = c;
+    }
+    return 0;
+}
+
+// A whole 1024-position block's two waves, the split ending at t_end.
+int fhip_idx_split(int blk, int wave, int t_end, int32_t* t_begin, int32_t* column, uint8_t* in_split) {
+    if (blk < 0 || wave < 0 || !t_begin || !column || !in_split) return -1;
+    *t_begin = fhip_idx_split_begin(blk, wave, 2, 1024);
     for (int lane = 0; lane < 64; ++lane) {
         int c;
         in_split[lane] = fhip_idx::split_page_column(*t_begin, t_end, lane, c) ? 1 : 0;
         column[lane] = c;
     }
     return 0;
-}
-
-// The same of a 1024-position block's two waves.
-int fhip_idx_split(int blk, int wave, int t_end, int32_t* t_begin, int32_t* column, uint8_t* in_split) {
-    return fhip_idx_wave_split(blk, wave, 2, 1024, t_end, t_begin, column, in_split);
 }
 
 // The first split page of the chunk starting at t0.

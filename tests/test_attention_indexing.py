@@ -85,7 +85,7 @@ class IndexLib:
         L.fhip_idx_partial_row.argtypes = [C.c_int] * 7
         L.fhip_idx_partial_row.restype = C.c_int64
         L.fhip_idx_lane_tables.argtypes = [C.c_int, C.c_int] + [C.c_void_p] * 6
-        L.fhip_idx_wave_split.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int32), C.c_void_p, C.c_void_p]
+        L.fhip_idx_wave_split.argtypes = [C.c_int] * 5 + [C.POINTER(C.c_int32)] * 2 + [C.c_void_p] * 2
         L.fhip_idx_code_tables.argtypes = [C.c_int] * 4 + [C.c_void_p] * 3 + [C.POINTER(C.c_int32)] * 2
         L.fhip_idx_split_grid_item.argtypes = [C.c_int64, C.c_int, C.c_int, C.c_int] + [C.POINTER(C.c_int32)] * 3
         self._tables = {}
@@ -125,13 +125,13 @@ class IndexLib:
         assert self.lib.fhip_idx_wg_item(wg, kvh, self.C.byref(item), self.C.byref(g)) == 0
         return item.value, g.value
 
-    def split(self, blk, wave, t_end, waves=2, part=SPLIT):
-        t_begin = self.C.c_int32()
+    def split(self, blk, wave, clen, waves=2, part=SPLIT):
+        t_begin, t_end = self.C.c_int32(), self.C.c_int32()
         col = np.zeros(64, np.int32)
         ins = np.zeros(64, np.uint8)
-        assert self.lib.fhip_idx_wave_split(blk, wave, waves, part, t_end, self.C.byref(t_begin), col.ctypes.data,
-                                            ins.ctypes.data) == 0
-        return t_begin.value, col, ins.astype(bool)
+        assert self.lib.fhip_idx_wave_split(blk, wave, waves, part, clen, self.C.byref(t_begin),
+                                            self.C.byref(t_end), col.ctypes.data, ins.ctypes.data) == 0
+        return t_begin.value, t_end.value, col, ins.astype(bool)
 
     def q_vectors(self, tq0, tok, G, nq, qh, g):
         vec = np.zeros(64, np.int64)
@@ -189,11 +189,9 @@ def model_mfma_kernel(lens, table, num_pages, qh, kvh, page_bytes, pool_bytes, t
         for nm in ("kn", "vn"):
             assert (n_off + 2 <= min(PAGE * kvh * 2, page_bytes[nm])).all()
         for w in range(waves):
-            t_begin, col, has = ix.split(blk, w, part * nsplit, waves, part)
+            t_begin, t_end, col, has = ix.split(blk, w, clen, waves, part)
             if t_begin >= clen:
                 continue  # empty state, nothing read
-            t_end = min(clen, t_begin + part // waves)
-            _, col, has = ix.split(blk, w, t_end, waves, part)
             tidx = col[has]
             assert tidx.max() < max_blocks
             bnd.check("table", (tq0 * stride + tidx) * 4, 4)
@@ -481,10 +479,21 @@ def test_transposed_reads_of_8_bit_codes():
                         assert got == pos * 128 + 16 * c + n
 
 
-@pytest.mark.parametrize("waves,part", [(2, SPLIT), (8, SPLIT), (4, 256)])
+@pytest.mark.parametrize("waves,part", [(2, SPLIT), (4, SPLIT), (8, SPLIT), (4, 256)])
 def test_split_begin_tiles_the_block(waves, part):
     L = index_lib().lib
     begins = [L.fhip_idx_split_begin(3, w, waves, part) for w in range(waves)]
     assert begins == [3 * part + w * (part // waves) for w in range(waves)]
-    if (waves, part) == (2, SPLIT):  # the split that the model above walks
-        assert begins[1] == index_lib().split(3, 1, 1 << 20)[0]
+    # the splits that the model above walks: together the block's live positions, in whole chunks of
+    # which no wave has more than its share
+    for live in (1, 15, 63, 64, 65, 128, 129, 200, part // 2, part // 2 + 1, part - 1, part, part + 1):
+        end, clen = 3 * part, 3 * part + live
+        for w in range(waves):
+            t_begin, t_end, _, _ = index_lib().split(3, w, clen, waves, part)
+            if t_begin >= clen:
+                assert end == clen
+                continue
+            assert t_begin == end < t_end and (t_begin - 3 * part) % CHUNK == 0
+            assert t_end - t_begin <= -(-min(live, part) // (CHUNK * waves)) * CHUNK <= part // waves
+            end = t_end
+        assert end == min(clen, 4 * part)

@@ -148,7 +148,8 @@ def test_decode_widths_and_waves(dev, kbits, vbits, qh, kvh, reps, part, waves):
     waves' splits and of pages, a masked page, an empty sequence."""
     rng = np.random.default_rng(kbits * 10 + vbits + qh)
     hd = 128
-    lens = ([1, 65, 128, 0, 300] if waves == 2 else [1, 63, 64, 65, 127, 129, 255, 257, 511, 513, 0, 1023, 1025])
+    lens = ([1, 65, 128, 0, 300] if waves == 2 else
+            [1, 63, 64, 65, 127, 129, 255, 257, 511, 513, 0, 1023, 1025 if part == 256 else 1800])
     route = rules.TqRoute(len(lens) * reps, qh, kvh, kbits, vbits, max(lens))
     assert (route.kind, route.part, route.waves) == (rules.DECODE, part, waves)
     pool = build_pool(rng, lens, kvh, hd, kbits, vbits)

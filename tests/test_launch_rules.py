@@ -22,7 +22,10 @@ def test_waves_of_a_paged_decode(queries, qh, kvh, hd, tokens, waves):
     # 256-position parts: at most 768 of their workgroups and 48 parts
     (1, 32, 8, 4, 2, 4001, 256, 4), (32, 32, 8, 4, 2, 700, 256, 4), (64, 32, 8, 4, 4, 16, 256, 4),
     (1, 32, 8, 4, 2, 12288, 256, 4), (1, 32, 8, 4, 2, 12289, 1024, 4), (1, 32, 8, 8, 8, 32000, 1024, 4),
-    (40, 32, 8, 4, 2, 700, 1024, 4), (64, 32, 8, 3, 3, 1000, 1024, 4), (8, 32, 8, 8, 8, 8000, 1024, 4),
+    (64, 32, 8, 3, 3, 1000, 1024, 4), (8, 32, 8, 8, 8, 8000, 1024, 4), (32, 32, 8, 4, 2, 1000, 1024, 4),
+    # up to 1536 where 1024-position parts would be a second turn: 257 .. 384 workgroups, 512 of several parts
+    (40, 32, 8, 4, 2, 700, 256, 4), (48, 32, 8, 4, 2, 1024, 256, 4), (49, 32, 8, 4, 2, 700, 1024, 4),
+    (24, 32, 8, 8, 8, 1400, 256, 4), (32, 32, 8, 4, 4, 1400, 256, 4), (32, 32, 8, 4, 4, 1600, 1024, 4),
     # above 512 workgroups two waves
     (65, 32, 8, 4, 2, 1024, 1024, 2), (64, 32, 8, 4, 2, 32768, 1024, 2), (256, 32, 8, 2, 2, 16, 1024, 2)])
 def test_route_of_a_tq_decode(queries, qh, kvh, kbits, vbits, kv_len, part, waves):
