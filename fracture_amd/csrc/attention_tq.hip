@@ -575,17 +575,17 @@ __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
 
 // Merge and unrotation at head_dim 128: 4 vectors per workgroup of 512 lanes. Everything that does not
 // depend on the rest is loaded at once: lane (i, quarter jq) its 32 entries of Pi_v's column i, lane
-// (vector, d) up to 16 splits' (m, l) and accumulator d, folded as an online softmax over chunks of
-// 16 splits. The merged vectors cross LDS once, then each lane sums its 32 products for the 4
+// (vector, d) up to kChunk splits' (m, l) and accumulator d, folded as an online softmax over chunks of
+// kChunk splits, 16 or, where there are no more, 4 (32 vectors of one split: 5.4 us and 3.9; 2048: 6.9 and 4.6). The merged vectors cross LDS once, then each lane sums its 32 products for the 4
 // vectors and the quarters meet in LDS. The general kernel above stages Pi_v in LDS, then waits for
 // (m, l), for the accumulators and for 128 LDS reads in turn: 8.3 us for 32 vectors of 4 splits and
 // 19.9 for 2048 of up to 32 against 4.6 (of 16 parts) and 13.7 here (kernel trace, as above).
 constexpr int kComb128Vecs = 4;
+template <int kChunk>
 __global__ __launch_bounds__(512) void tq_attn_combine128_kernel(
     Queries qs, const float* __restrict__ part_ml, const float* __restrict__ part_acc,
     const float* __restrict__ vrot, uint16_t* __restrict__ out, int qh, int nsplit, int64_t nvec,
     int split_pos) {
-    constexpr int kChunk = 16;
     __shared__ __attribute__((aligned(16))) float o[kComb128Vecs][128];
     __shared__ float red[4][kComb128Vecs][128];
     const int tid = threadIdx.x, i = tid & 127;
@@ -2205,7 +2205,8 @@ int launch_attention(const AttnArgs& a, const Pages& pg, hipStream_t s) {
         return fhip_internal::tq_rotate_back_rows(qrot, a.vrot, a.out, nvec, s);
     }
     if (a.hd == 128) {
-        hipLaunchKernelGGL(tq_attn_combine128_kernel, dim3((unsigned)ceil_div(nvec, kComb128Vecs)),
+        auto merge = nsplit <= 4 ? tq_attn_combine128_kernel<4> : tq_attn_combine128_kernel<16>;
+        hipLaunchKernelGGL(merge, dim3((unsigned)ceil_div(nvec, kComb128Vecs)),
                            dim3(512), 0, s, a.qs, ml, acc, a.vrot, (uint16_t*)a.out, a.qh, nsplit,
                            (int64_t)nvec, split_pos);
         return hipGetLastError();

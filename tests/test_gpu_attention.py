@@ -209,6 +209,28 @@ def test_code_pages_at_odd_addresses(dev, bits):
     assert_close(out.cpu().numpy()[0].astype(np.float32), want.astype(np.float32), 1e-3, 1e-3)
 
 
+@pytest.mark.parametrize("splits", [1, 3, 4, 5, 16, 17, 33])
+def test_merge_of_splits(dev, splits):
+    """The head_dim 128 merge at the edges of its chunks of 4 and of 16 splits, beside sequences that end in
+    an earlier split and an empty one."""
+    rng = np.random.default_rng(splits)
+    qh, kvh = 8, 2
+    lens = [256 * splits, 256 * splits - 255, 1, 0, max(1, 256 * (splits - 2)), 256 * splits - 16]
+    route = rules.TqRoute(len(lens), qh, kvh, 4, 4, lens[0])
+    assert (route.kind, route.part, route.nsplit) == (rules.DECODE, 256, splits)
+    pool = build_pool(rng, lens, kvh, 128, 4, 4)
+    q = rng.standard_normal((len(lens), qh, 128)).astype(np.float16)
+    out = torch.empty(q.shape, dtype=torch.float16, device=dev)
+    K.attention_tq_decode(out, dev_t(q, dev), dev_t(pool["table"], dev), dev_t(np.array(lens, np.int32), dev),
+                          *(dev_t(pool[n], dev) for n in ("KP", "KN", "VP", "VN", "krot", "vrot", "kc", "vc")),
+                          4, 4, kvh)
+    got = out.cpu().numpy().astype(np.float32)
+    for b, n in enumerate(lens):
+        want = oracle.tq_attention(q[b], pool["table"][b], n, pool["KP"], pool["KN"], pool["VP"], pool["VN"],
+                                   pool["krot"], pool["vrot"], pool["kc"], pool["vc"], 4, 4, kvh)
+        assert_close(got[b], want.astype(np.float32), 1e-3, 1e-3, f"sequence {b}")
+
+
 @pytest.mark.parametrize("kbits,vbits,qh,kvh", [(4, 2, 32, 8), (8, 8, 8, 2)])
 def test_workspace_of_a_shorter_table(dev, kbits, vbits, qh, kvh):
     """A workspace sized for one block serves a table of 60, which launches in 256-position parts, in decode
