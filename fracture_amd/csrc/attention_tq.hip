@@ -576,7 +576,8 @@ __global__ __launch_bounds__(256) void tq_attn_combine_kernel(
 // Merge and unrotation at head_dim 128: 4 vectors per workgroup of 512 lanes. Everything that does not
 // depend on the rest is loaded at once: lane (i, quarter jq) its 32 entries of Pi_v's column i, lane
 // (vector, d) up to kChunk splits' (m, l) and accumulator d, folded as an online softmax over chunks of
-// kChunk splits, 16 or, where there are no more, 4 (32 vectors of one split: 5.4 us and 3.9; 2048: 6.9 and 4.6). The merged vectors cross LDS once, then each lane sums its 32 products for the 4
+// kChunk splits, 16 or, where there are no more, 4 (32 vectors of one split: 5.4 us and 3.9; 2048: 6.9
+// and 4.6). The merged vectors cross LDS once, then each lane sums its 32 products for the 4
 // vectors and the quarters meet in LDS. The general kernel above stages Pi_v in LDS, then waits for
 // (m, l), for the accumulators and for 128 LDS reads in turn: 8.3 us for 32 vectors of 4 splits and
 // 19.9 for 2048 of up to 32 against 4.6 (of 16 parts) and 13.7 here (kernel trace, as above).

@@ -134,6 +134,26 @@ constexpr int64_t kPqGroups = 512;  // workgroups wanted: the two per CU that fi
 constexpr int kRotBatch = 4096;     // vectors from which both rotations are batched MFMA products ...
 constexpr int kMergeSplits = 8;     // ... and the splits that the merge before the second takes in one wave
 
+// The prefill kernel's splits, at most `most`: the shortest of those that fill kPqGroups, those that stay
+// within it and those of the wave merge. A tile takes a workgroup 4.3 us alone on its CU and 6.3 beside another;
+// more than kMergeSplits splits of a batch are merged in LDS, 25 us slower. 32 / 8 heads unless said otherwise:
+// 64 queries at 3000 of 64 / 8 heads 8 splits (96 us in 12), at 30000 16 (223 us, 269 in 8), 130 at 30000 12
+// (264; 288 in 13, 299 in 8), 200 at 30000 8 or 9 (359; 475 in 10).
+inline PrefillSplit tq_prefill_split(int nq, int G, int kvh, int extent, int most, bool batch) {
+    const int64_t base = div_up(nq, kPqCols / G) * kvh;
+    PrefillSplit best = {};
+    int64_t least = 0;
+    for (const int64_t limit : {(int64_t)most, kPqGroups / base, batch ? (int64_t)kMergeSplits : (int64_t)most}) {
+        const PrefillSplit p = prefill_split(nq, G, kvh, kPqCols, kPqTile, kPqGroups, extent,
+                                             (int)std::max<int64_t>(std::min<int64_t>(limit, most), 1));
+        const int64_t rest = p.workgroups % kPqGroups;
+        const int64_t ns = p.split_pos / kPqTile * (p.workgroups / kPqGroups * 6300 + (rest > 256 ? 6300 : rest ? 4300 : 0)) +
+                           (batch && p.nsplit > kMergeSplits ? 25000 : 0);
+        if (!least || ns < least) best = p, least = ns;
+    }
+    return best;
+}
+
 // The route of a call. Times in us at K4/V2 unless said otherwise.
 //   The decode kernel in 256-position parts, four waves of one chunk each, where that makes at most three
 //   workgroups per CU and 48 parts: four times the workgroups of 1024-position parts (one sequence of
@@ -150,9 +170,10 @@ constexpr int kMergeSplits = 8;     // ... and the splits that the merge before 
 //   Causal calls of more workgroups than that (than 256 where the codes' expansion is dearer, at 3 and 8
 //   bits) go to the prefill kernel where it is the shorter one: a tile takes a workgroup 4.3 us, with up to
 //   one workgroup per CU, and a decode workgroup of 1024 positions 0.042 us of the whole chip, twice that at
-//   3 and 8 bits. It also has to have 96 workgroups, 128 where its partials are merged by a kernel of their
-//   own. 32 / 8 heads, decoded and tiled: 8 queries at 8000 26.6 and 31.9, 32 at 3000 33.2 and 32.9, 32 at
-//   8000 52 and 40, 8 at 30000 51 and 59, 200 at 1000 of 64 / 8 heads (104 workgroups of 16 tiles) 90 and 92.
+//   3 and 8 bits. It also has to have 96 workgroups, 128 at 4 and 2 bits where its partials are merged by a
+//   kernel of their own (130 queries at 3000, 120 workgroups: 88 us decoded and 95, at 8 bits 122 and 101).
+//   32 / 8 heads, decoded and tiled: 8 queries at 8000 26.6 and 31.9, 32 at 3000 33.2 and 32.9, 32 at 8000 52
+//   and 40, 8 at 30000 51 and 59, 200 at 1000 of 64 / 8 heads (104 workgroups of 16 tiles) 90 and 92.
 inline TqRoute tq_route(const TqCall& c) {
     TqRoute r;
     const int G = c.qh / c.kvh;
@@ -180,13 +201,11 @@ inline TqRoute tq_route(const TqCall& c) {
     const bool dear = c.kbits == 3 || c.kbits == 8;
     if (c.causal && c.nq > 1 && wgs > (dear ? 256 : 512)) {
         const bool batch = (int64_t)c.nq * c.qh >= kRotBatch;
-        // splits beyond what the wave merge takes would go to the merge in LDS, 25 us slower (64 queries at
-        // 3000, 64 / 8 heads: 96 us in 12 splits)
-        const int most = std::min(fits ? fine.nsplit : nsplit, batch ? kMergeSplits : 1 << 30);
-        r.prefill = prefill_split(c.nq, G, c.kvh, kPqCols, kPqTile, kPqGroups,
-                                  std::min(c.kv_len, c.max_tokens), most);
+        r.prefill = tq_prefill_split(c.nq, G, c.kvh, std::min(c.kv_len, c.max_tokens),
+                                     fits ? fine.nsplit : nsplit, batch);
         const int64_t tiles = r.prefill.split_pos / kPqTile * div_up(r.prefill.workgroups, 256);
-        if (r.prefill.workgroups >= (batch && r.prefill.nsplit > 1 ? 128 : 96) && tiles * (dear ? 50 : 105) < wgs) {
+        if (r.prefill.workgroups >= (batch && !dear && r.prefill.nsplit > 1 ? 128 : 96) &&
+            tiles * (dear ? 50 : 105) < wgs) {
             r.kind = TqRoute::kPrefill;
             r.part = fits ? kTqFinePart : kTqSplit;
         }

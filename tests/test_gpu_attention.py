@@ -294,7 +294,9 @@ def run_prefill(dev, pool, q, kvh, kv_len, start_pos, kbits, vbits):
     # one split and a batch of vectors that skips the merge, blocks going up after those going down
     (4, 2, 32, 8, 2048, 2048, True),
     # a batch of vectors whose splits the wave merge takes
-    (4, 2, 32, 8, 130, 2560, True)])
+    (4, 2, 32, 8, 130, 2560, True),
+    # a batch in fewer and longer splits, and in 16 that the merge in LDS takes
+    (3, 3, 32, 8, 130, 3000, True), (4, 4, 16, 2, 256, 20000, True)])
 def test_prefill_tiles(dev, kbits, vbits, qh, kvh, T, kv_len, tiled):
     """The causal prefill kernel against the oracle, with a masked page and with a value norm of
     infinity and a key norm of NaN at late positions, which no earlier query may see; the value norms

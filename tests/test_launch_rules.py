@@ -50,8 +50,12 @@ def test_other_widths_and_head_dims_stay_on_the_valu_kernel(qh, kvh, hd, kbits, 
     (2048, 32, 8, 4, 2, 2048, rules.PREFILL, 1024, 1, 2048), (130, 32, 8, 4, 4, 1000, rules.PREFILL, 256, 4, 256),
     # the codes' expansion is dearer at 8 and 3 bits
     (32, 32, 8, 8, 8, 3000, rules.PREFILL, 256, 12, 256), (32, 32, 8, 3, 3, 3000, rules.PREFILL, 256, 12, 256),
-    # from 4096 vectors on at most the 8 splits that a wave merges, and 128 workgroups
+    # from 4096 vectors on 128 workgroups at 4 and 2 bits, and the 8 splits that a wave merges or, of long
+    # contexts, as many as fit at once
     (130, 32, 8, 4, 2, 2560, rules.PREFILL, 256, 8, 320), (600, 8, 8, 4, 4, 600, rules.DECODE, 1024, 1, 1024),
+    (64, 64, 8, 4, 4, 30000, rules.PREFILL, 1024, 16, 1920), (130, 32, 8, 4, 4, 30000, rules.PREFILL, 1024, 12, 2560),
+    (200, 32, 8, 4, 4, 30000, rules.PREFILL, 1024, 9, 3392), (130, 64, 8, 4, 4, 30000, rules.PREFILL, 1024, 7, 4288),
+    (130, 32, 8, 4, 4, 3000, rules.DECODE, 1024, 3, 1024), (600, 8, 8, 8, 8, 3000, rules.PREFILL, 1024, 3, 1024),
     # long tiles on a part of the chip lose to the decode kernel
     (200, 64, 8, 4, 2, 1000, rules.DECODE, 1024, 1, 1024), (8, 32, 8, 4, 2, 30000, rules.DECODE, 1024, 30, 1024)])
 def test_route_of_a_tq_prefill(queries, qh, kvh, kbits, vbits, kv_len, kind, part, nsplit, split_pos):
