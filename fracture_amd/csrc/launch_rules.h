@@ -16,24 +16,31 @@ inline int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 // 128 unless said otherwise; one wave is what there was before waves shared a split.
 //   Up to 256 items eight waves hide one another's memory latency (one sequence of 1000: 67 / 31 / 23 /
 //     19), up to 512 four (64 of 1000: 109 / 51 / 45 / 48), up to 1024 two (64 of 2000: 145 / 99 / 109 /
-//     106; of 250 .. 2000: 130 / 66 / 83 / 76). Beyond, one wave per split fills the chip, and more only
+//     106; of 250 .. 2000: 130 / 66 / 83 / 76). Far beyond, one wave per split fills the chip, and more only
 //     add merges and idle waves (64 of 4000: 185 / 214 / 199 / 202; 256 of 200: 40 / 48 / 58 / 83).
+//   Between, to 1536 items, one wave is a second turn that is half empty, or emptier where the batch is ragged.
+//     Four waves: 48 of 3000 160 / 124 / 121, of 375 .. 3000 134 / 72 / 79; 64 / 8 heads, 64 of 3000 154 / 175
+//     / 162, of 375 .. 3000 137 / 112 / 110. At head_dim 64 two: 96 of 2000, 16 / 8 heads, 96 / 86 / 95, of
+//     250 .. 2000 74 / 54 / 58. Not on tables below half a split (192 of 300, 64 / 8 heads).
+//   Head_dim 256 takes two waves to 1024 items (64 of 4000, 16 / 4 heads: 194 / 195 / 218, of 500 .. 4000 176 /
+//     133 / 170), head_dim 32 to 768 (8 / 8 heads, 32 of 3000: 41 / 36 / 40, of 375 .. 3000 40 / 27 / 28; 64
+//     of 2000, 1024 items: 41 / 48 / 50).
 //   A wave takes 1024 / W positions of the split, so waves past the end of a short table are idle. At
 //     head_dim 128 they cost less than two splits sharing a workgroup, as one wave per split has them
 //     (64 of 100: 16.9 with one, 14.1 with two or four): halved while one wave would hold the table, not
 //     below two. Elsewhere they lose from about two thirds of the table on (64 of 16, 16 / 8 heads of 64: 7.5
 //     / 8.3 / 8.6 / 11.0; of 300, 8 / 8 heads of 32: 15.2 / 18.5 / 17.3 / 15.1; of 400: 18.2 / 21.7 /
-//     17.9 / 16.4).
-//   Head_dim 32 and 256 take one wave from 513 items: uniform batches lose (64 of 2000, 8 / 8 heads of
-//     32: 41 / 47; of 4000, 16 / 4 heads of 256: 186 / 196).
+//     17.9 / 16.4), but for two waves of head_dim 64 and 256 (128 of 300, 16 / 8 heads of 64: 26.6 / 26.5;
+//     of 700 49 / 41).
 inline int paged_waves(int64_t items, int hd, int max_tokens) {
-    if (items > 1024) return 1;
-    int w = items <= 256 ? 8 : items <= 512 ? 4 : hd == 64 || hd == 128 ? 2 : 1;
     const int span = std::min(max_tokens, 1024);
+    if (items > 1024) return items <= 1536 && span > 512 ? (hd == 128 ? 4 : hd == 64 ? 2 : 1) : 1;
+    int w = items <= 256 ? 8 : items <= 512 ? 4 : 2;
     if (hd == 128) {
         while (w > 2 && span * w <= 1024) w /= 2;
         return w;
     }
+    if (w == 2) return hd == 32 ? (items <= 768 && span >= 768 ? 2 : 1) : span > 128 ? 2 : 1;
     return span * w >= 1536 ? w : 1;
 }
 

@@ -69,7 +69,8 @@ def test_decode_small_contexts(dev, hd, qh, kvh):
 
 @pytest.mark.parametrize("nseq,qh,kvh,hd,waves", [
     (32, 8, 8, 64, 8), (33, 8, 8, 64, 4), (33, 32, 8, 128, 4), (64, 16, 8, 32, 4), (65, 16, 8, 128, 2),
-    (65, 16, 8, 64, 2), (65, 16, 8, 256, 1), (65, 64, 64, 32, 1)])
+    (65, 16, 8, 64, 2), (65, 16, 8, 256, 2), (65, 8, 8, 32, 2), (65, 16, 16, 128, 4), (65, 16, 16, 64, 2),
+    (65, 64, 64, 32, 1)])
 def test_decode_waves_per_split(dev, nseq, qh, kvh, hd, waves):
     """8, 4, 2 and 1 waves per split: lengths that leave waves empty, end inside each wave's piece and on
     its edges, and a masked page that is a wave's whole piece of one chunk."""
@@ -95,8 +96,8 @@ def test_decode_waves_per_split(dev, nseq, qh, kvh, hd, waves):
 
 
 @pytest.mark.parametrize("nseq,qh,kvh,hd,widest", [
-    (343, 4, 1, 128, 2100),   # 1029 splits: the last workgroup's second wave has none
-    (343, 8, 1, 128, 2100), (172, 16, 2, 128, 2100), (172, 8, 2, 64, 3000), (515, 4, 2, 256, 20),
+    (513, 4, 1, 128, 2100),   # 1539 splits: the last workgroup's second wave has none
+    (513, 8, 1, 128, 2100), (257, 16, 2, 128, 2100), (257, 8, 2, 64, 3000), (515, 4, 2, 256, 20),
     (257, 8, 2, 256, 1100), (1025, 1, 1, 32, 100)])
 def test_decode_one_wave_per_split(dev, nseq, qh, kvh, hd, widest):
     """Two splits of neighbouring kv heads to a workgroup, each a wave's own: odd counts of splits, pairs

@@ -7,9 +7,13 @@ import rules
 @pytest.mark.parametrize("queries,qh,kvh,hd,tokens,waves", [
     # up to 256, 512, 1024 splits and more, tables of whole splits
     (1, 32, 8, 128, 4000, 8), (32, 32, 8, 128, 1024, 8), (33, 32, 8, 128, 1024, 4), (64, 32, 8, 128, 1000, 4),
-    (65, 32, 8, 128, 1024, 2), (128, 32, 8, 128, 1024, 2), (129, 32, 8, 128, 1024, 1),
+    (65, 32, 8, 128, 1024, 2), (128, 32, 8, 128, 1024, 2), (193, 32, 8, 128, 1024, 1),
     (64, 32, 8, 128, 4000, 1), (256, 32, 8, 128, 1100, 1), (64, 32, 32, 128, 1000, 1),
-    (16, 64, 8, 64, 8000, 2), (16, 8, 8, 32, 8000, 1), (256, 16, 4, 256, 1000, 1), (128, 16, 4, 256, 1000, 4),
+    (16, 64, 8, 64, 8000, 2), (16, 8, 8, 32, 8000, 1), (257, 16, 4, 256, 1000, 1), (128, 16, 4, 256, 1000, 4),
+    # between 512 and 1536 splits, by head_dim
+    (129, 32, 8, 128, 1024, 4), (192, 32, 8, 128, 1024, 4), (129, 32, 8, 128, 528, 4), (129, 32, 8, 128, 512, 1),
+    (96, 16, 8, 64, 2000, 2), (97, 16, 8, 64, 2000, 1), (192, 32, 8, 64, 512, 1), (128, 16, 8, 64, 300, 2),
+    (128, 16, 8, 64, 128, 1), (256, 16, 4, 256, 1000, 2), (32, 8, 8, 32, 3000, 2), (33, 8, 8, 32, 3000, 1),
     # short tables: no waves past their end, at head_dim 128 not below two
     (1, 32, 8, 128, 128, 2), (1, 32, 8, 128, 144, 8), (64, 32, 8, 128, 256, 2), (64, 32, 8, 128, 272, 4),
     (128, 32, 8, 128, 100, 2), (256, 32, 8, 128, 16, 1), (8, 16, 8, 64, 64, 1), (8, 16, 8, 64, 208, 8),
