@@ -17,8 +17,8 @@
 #include <algorithm>
 #include <type_traits>
 
-#include "launch_rules.h"
 #include "fhip_internal.h"
+#include "launch_rules.h"
 #include "tq_attn_index.h"
 #include "tq_quant.h"
 
@@ -1156,7 +1156,8 @@ tq_attn_mfma_kernel(const float* __restrict__ qrot, Queries qs, Pages pg,
             if (bits == 8) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    if (k % W == wave) ((uint32_t*)tab)[64 * k + lane] = hi_lo_pair(ldexpf(c.v[k % (sizeof(c.v) / 4)], c.e), hf);
+                    if (k % W == wave)
+                        ((uint32_t*)tab)[64 * k + lane] = hi_lo_pair(ldexpf(c.v[k % (sizeof(c.v) / 4)], c.e), hf);
             } else {
                 const int word = (int)hi_lo_pair(ldexpf(c.v[0], c.e), hf);  // lane: its code's
                 const int low = __shfl(word, lane & 15);
